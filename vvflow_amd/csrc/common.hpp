@@ -212,6 +212,26 @@ struct PList {
     }
 };
 
+// State of the merge rounds (epsilon.hip), grown to the list they run on.
+struct MergeBufs {
+    DBuf<int2> info;                              // per element: partner, death
+    DBuf<double4> rec, cand, cbox;                // records, next records, boxes of the changes
+    DBuf<double> fd2;                             // second-neighbour distance before a merge
+    DBuf<int32_t> stamp, list, chg, chg_p, ever;
+    DBuf<uint64_t> maxd2;                         // per leaf: bound of the second-neighbour distance
+    DBuf<int32_t> hn1, hn2, hlist;                // heat list: search results
+    DBuf<double> hd1, hd2;
+    DBuf<uint8_t> hflag;
+    void release() {
+        info.release();
+        for (auto* b : {&rec, &cand, &cbox}) b->release();
+        for (auto* b : {&fd2, &hd1, &hd2}) b->release();
+        for (auto* b : {&stamp, &list, &chg, &chg_p, &ever, &hn1, &hn2, &hlist}) b->release();
+        maxd2.release();
+        hflag.release();
+    }
+};
+
 struct Ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -263,9 +283,6 @@ struct Ctx {
     DBuf<int32_t> heat_cond;
     DBuf<float> heat_const;                  // per segment
     DBuf<int64_t> heat_layer;                // per segment
-    DBuf<double> hres;                       // per heat particle: epsh result
-    DBuf<uint8_t> hflag;
-    DBuf<uint8_t> hdirty;                    // per leaf: a heat merge touched it
 
     // segments and bodies (host copy is authoritative between calls)
     std::vector<vvhd_seg> segs_h;
@@ -297,12 +314,8 @@ struct Ctx {
     DBuf<double> leaf_crit, leaf_restr;
     DBuf<uint8_t> eflag;                     // per target: bit0 processed, bit1 merge flag
     DBuf<int32_t> flag_list;                 // targets flagged by the parallel pass
-    DBuf<int32_t> ecount;                    // [0]=flags, [1]=merged, ...
-    DBuf<int64_t> rnear_off;                 // transposed near lists (repair)
-    DBuf<int32_t> rnear_list, rnear_cnt, leaf_stamp;
-    DBuf<uint64_t> leaf_maxd2;                       // per-leaf bound of the second-neighbour distance
-    DBuf<uint8_t> leaf_mark;                         // leaves whose reverse near lists are built
-    DBuf<int64_t> rep_state;                         // per simulation: resume target, commit count
+    DBuf<int32_t> ecount;                    // [0]=flags, [1..4]=the merge rounds' counters, [5]=merges
+    MergeBufs mg;
 
     // learned far-field correction
     DBuf<double> fm;                         // per-node moments after epsilon: kMomArrays x node capacity

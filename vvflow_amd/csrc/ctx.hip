@@ -205,20 +205,16 @@ void vvhd_destroy(vvhd_ctx* ctx) {
     for (auto* b : {&c.x, &c.y, &c.g, &c.vx, &c.vy, &c.ie, &c.x2, &c.y2, &c.g2, &c.vx2, &c.vy2, &c.ie2, &c.snap,
                     &c.d1, &c.d2, &c.leaf_crit, &c.leaf_restr, &c.fric})
         b->release();
-    for (auto* b : {&c.id, &c.id2, &c.iscratch0, &c.iscratch1, &c.iscratch2, &c.iscratch3, &c.nn1, &c.nn2, &c.ecount,
-                    &c.rnear_list})
+    for (auto* b : {&c.id, &c.id2, &c.iscratch0, &c.iscratch1, &c.iscratch2, &c.iscratch3, &c.nn1, &c.nn2, &c.ecount})
         b->release();
-    for (auto* b : {&c.flag_list, &c.rnear_cnt, &c.leaf_stamp, &c.seg_root, &c.sim_body}) b->release();
+    for (auto* b : {&c.flag_list, &c.seg_root, &c.sim_body}) b->release();
     c.sim_off.release();
     c.sim_re.release();
-    c.leaf_maxd2.release();
-    c.leaf_mark.release();
-    c.rep_state.release();
+    c.mg.release();
     c.near_v.release();
     c.taylor.release();
     c.src_ge.release();
     c.lscratch0.release();
-    c.rnear_off.release();
     c.tmp.release();
     c.eflag.release();
     c.segs.release();
@@ -261,9 +257,6 @@ void vvhd_destroy(vvhd_ctx* ctx) {
     c.heat_cond.release();
     c.heat_const.release();
     c.heat_layer.release();
-    c.hres.release();
-    c.hflag.release();
-    c.hdirty.release();
     for (auto* b : {&t.h0, &t.h1, &t.s0, &t.s1, &t.seg_keys, &t.seg_ids}) b->release();
     for (auto* b : {&c.fld_a, &c.fld_b, &c.fld_gtmp}) b->release();
     c.fld_map.release();
@@ -523,7 +516,7 @@ int vvhd_epsilon(vvhd_ctx* ctx, int merge, int32_t* nn1, int32_t* nn2, int32_t* 
     epsilon(c, merge, nn1, nn2, merged);
     VVHD_HIP(hipEventRecord(c.ev[3], c.stream));
     c.phase_recorded[1] = true;
-    if (nn1 || nn2 || merged) sync(c);
+    if (nn1 || nn2) sync(c);   // the merge count is known on the host already
     API_END(ctx)
 }
 

@@ -12,11 +12,13 @@
 // A merge (:111-126) mutates the target and zeroes its partner; every later
 // target sees the mutated state.  Pass 1 computes every target on the
 // unmodified state and flags the targets that would merge.  When flags exist,
-// a single-workgroup pass commits merges in target order: after each commit
-// it updates the targets that come later and have the merged leaves in their
-// near lists -- in O(1) when the moved vortex only enters their top-2, by a
-// full rescan when one of their two neighbours changed -- and re-evaluates
-// their merge flags, exactly reproducing the sequential outcome.
+// the sequential outcome is found as a fixed point, in parallel (merge_rounds
+// below): the visit of target i depends only on the merges of targets before
+// it, so each round evaluates every target whose surroundings the last round
+// changed against the merges assumed so far, seen as of i, until no merge
+// changes.  After k rounds every target whose chain of dependencies is
+// shorter than k holds its sequential result, and a state that a round leaves
+// unchanged is the sequential one.
 //
 // Pass 1 prunes near leaves by box distance: leaves touching the target leaf
 // are scanned first, then only leaves whose box distance does not exceed the
@@ -25,11 +27,9 @@
 
 #include "common.hpp"
 
-#include <cstring>
-#include <rocprim/device/device_scan.hpp>
-
 #include <algorithm>
 #include <cmath>
+#include <vector>
 
 #pragma clang fp contract(off)
 
@@ -301,458 +301,382 @@ __device__ inline double point_box_dist2(const TreeDev& T, int M, double px, dou
     return dx * dx + dy * dy;
 }
 
-// Sources of the near leaves of leaf l selected by sel(M) for one target i,
-// lanes over each selected leaf's vortices.
-// Chunks of kWave entries starting at chunk `first`, every `stride`-th.
-template <typename Sel>
-__device__ inline void scan_one(const TreeDev& T, int l, const double* x, const double* y, const double* g, int i,
-                                double tx, double ty, Top2& st, Sel sel, int first = 0, int stride = 1) {
-    const int64_t e0 = T.near_off[l], e1 = T.near_off[l + 1];
-    for (int64_t eb = e0 + (int64_t)first * kWave; eb < e1; eb += (int64_t)stride * kWave) {
-        const int64_t e = eb + lane_id();
-        int M = -1;
-        bool q = false;
-        if (e < e1) {
-            M = T.near_list[e];
-            q = sel(M);
-        }
-        uint64_t mask = __ballot(q);
-        while (mask) {
-            const int b = (int)__builtin_ctzll(mask);
-            mask &= mask - 1;
-            const int Mb = __shfl(M, b, kWave);
-            const int s0 = T.v0[Mb], s1 = T.v1[Mb];
-            for (int j = s0 + lane_id(); j < s1; j += kWave) {
-                const double gj = g[j];
-                if (gj != 0 && j != i) top2_insert(st, dist2(tx, ty, x[j], y[j]), j);
-            }
-        }
-    }
-}
-
 __device__ inline Top2 wave_top2(Top2 st) {
     for (int o = kWave / 2; o > 0; o >>= 1) top2_merge(st, top2_shfl_xor(st, o));
     return st;
 }
 
-// Full top-2 searches of the targets tg[0..nt) over their near leaves by
-// the NW waves of a workgroup: leaves touching the target's leaf first, then
-// those whose box lies within the second-neighbour distance found.  Groups
-// of G waves (G the largest
-// power of two with G * nt <= NW, at least 1) take one target each; within
-// a group, wave k scans every G-th chunk of the near list, and the partial
-// top-2s combine through LDS (the top-2 under (d, index) does not depend on
-// the order of the candidates).  out(i, st) runs on one lane per target.
-// Every thread of the workgroup must call it; it starts and ends with a
-// barrier.
-template <int NW, typename Out>
-__device__ void group_rescans(const TreeDev& T, const double* x, const double* y, const double* g, const int* tg,
-                              int nt, Top2* s_part, Out out) {
-    int G = 1;
-    while (2 * G * nt <= NW && 2 * G <= NW) G *= 2;
-    const int ngroups = NW / G;
-    const int wave = threadIdx.x / kWave, grp = wave / G, k = wave % G;
-    for (int r0 = 0; r0 < nt; r0 += ngroups) {
-        const int h = r0 + grp;
-        const int i = h < nt ? tg[h] : -1;
-        int l = 0, L = 0;
-        double tx = 0, ty = 0;
-        if (i >= 0) {
-            l = T.vleaf[i];
-            L = T.leaf_node[l];
-            tx = x[i];
-            ty = y[i];
-        }
-        Top2 st = top2_empty();
-        if (i >= 0) scan_one(T, l, x, y, g, i, tx, ty, st, [&](int M) { return box_dist2(T, L, M) <= 0.0; }, k, G);
-        st = wave_top2(st);
-        __syncthreads();
-        if (lane_id() == 0) s_part[wave] = st;
-        __syncthreads();
-        Top2 c = top2_empty();
-        for (int w = grp * G; w < grp * G + G; w++) top2_merge(c, s_part[w]);
-        const double bound = c.i2 >= 0 ? c.d2 : INFINITY;
-        st = top2_empty();
-        if (i >= 0)
-            scan_one(T, l, x, y, g, i, tx, ty, st,
-                     [&](int M) { return box_dist2(T, L, M) > 0.0 && point_box_dist2(T, M, tx, ty) <= bound; }, k, G);
-        st = wave_top2(st);
-        __syncthreads();
-        if (lane_id() == 0) s_part[wave] = st;
-        __syncthreads();
-        if (i >= 0 && k == 0 && lane_id() == 0) {
-            for (int w = grp * G; w < grp * G + G; w++) top2_merge(c, s_part[w]);
-            out(i, c);
-        }
-    }
-    __syncthreads();
-}
-
-__device__ inline bool merge_flag(const double* g, int i, const Top2& st, double crit) {
-    if (st.i1 < 0 || st.i2 < 0 || isnan(crit)) return false;
-    const double s1 = sgn(g[st.i1]), s2 = sgn(g[st.i2]), si = sgn(g[i]);
-    return (st.d1 < crit) || ((s1 == s2) && (s1 != si));
-}
-
-// Transposed near lists: for every leaf M the leaves L with M in near(L).
-// With mark set, only the lists of marked leaves are built (the others stay
-// empty).
-__global__ void k_rnear_count(TreeDev T, int32_t* cnt, const uint8_t* mark) {
-    const int l = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
-    if (l >= T.nleaf) return;
-    for (int64_t e = T.near_off[l] + lane_id(); e < T.near_off[l + 1]; e += kWave) {
-        const int m = T.leaf_rank[T.near_list[e]];
-        if (!mark || mark[m]) atomicAdd(&cnt[m], 1);
-    }
-}
-
-// The same lists for a few marked leaves, flat over all near-list entries
-// (one thread per entry, coalesced; the owner leaf of a kept entry is found
-// by binary search over the list offsets).
-__global__ void k_rnear_count_flat(TreeDev T, int64_t nnear, int32_t* cnt, const uint8_t* mark) {
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < nnear; e += (int64_t)gridDim.x * blockDim.x) {
-        const int m = T.leaf_rank[T.near_list[e]];
-        if (mark[m]) atomicAdd(&cnt[m], 1);
-    }
-}
-__global__ void k_rnear_fill_flat(TreeDev T, int64_t nnear, const int64_t* roff, int32_t* fillc, int32_t* rlist,
-                                  const uint8_t* mark) {
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < nnear; e += (int64_t)gridDim.x * blockDim.x) {
-        const int m = T.leaf_rank[T.near_list[e]];
-        if (!mark[m]) continue;
-        int lo = 0, hi = T.nleaf;   // the leaf l with near_off[l] <= e < near_off[l + 1]
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (T.near_off[mid] <= e)
-                lo = mid;
-            else
-                hi = mid;
-        }
-        rlist[roff[m] + atomicAdd(&fillc[m], 1)] = lo;
-    }
-}
-
-// Leaves of the flagged targets and of their first neighbours: the commits
-// of pass 1's flags need their reverse lists.
-__global__ void k_mark_flag_leaves(TreeDev T, const int32_t* flag_list, const int32_t* ecount, const int32_t* nn1,
-                                   uint8_t* mark) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= ecount[0]) return;
-    const int q = flag_list[k];
-    mark[T.vleaf[q]] = 1;
-    mark[T.vleaf[nn1[q]]] = 1;
-}
-
-__global__ void k_rnear_fill(TreeDev T, const int64_t* roff, int32_t* fillc, int32_t* rlist, const uint8_t* mark) {
-    const int l = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
-    if (l >= T.nleaf) return;
-    for (int64_t e = T.near_off[l] + lane_id(); e < T.near_off[l + 1]; e += kWave) {
-        const int m = T.leaf_rank[T.near_list[e]];
-        if (!mark || mark[m]) rlist[roff[m] + atomicAdd(&fillc[m], 1)] = l;
-    }
-}
-
-constexpr int kRepairThreads = 1024;
-constexpr int kMaxHard = 2048;
-constexpr int kMaxPend = 8192;
-constexpr int kMaxLive = 2048;
-constexpr int kMarkedFlags = 256;   // up to this many flags, reverse lists of their leaves only
-
-struct RepairArgs {
-    TreeDev T;
-    double *x, *y, *g;
-    const double* leaf_crit;
-    const int64_t* roff;
-    const int32_t* rlist;
-    int32_t* stamp;
-    int32_t *nn1, *nn2;
-    double *d1a, *d2a;
-    uint8_t* eflag;
-    int32_t* ecount;
-    uint64_t *box_lo_x, *box_lo_y, *box_hi_x, *box_hi_y;
-    uint64_t* maxd2;   // per leaf: upper bound of d2 over its searched targets (ordered image)
-};
-
-struct CommitShared {
-    int nhard;
-    int overflow;
-    int nlive;
-    int hard[kMaxHard];
-    int live[kMaxLive];
-    double qx0, qy0, px0, py0;
-    Top2 part[kRepairThreads / kWave];
-};
-
-// Upper bound of the second-neighbour distance over the searched targets of
-// every leaf, as an ordered integer (-1 for a leaf without one; NaN counts
-// as DBL_MAX).  Commits prune leaves whose box is farther from the merged
-// vortices than this bound: none of their targets can change.
+// Second-neighbour distance as an ordered integer (NaN counts as DBL_MAX).
 __device__ inline uint64_t d2_key(double d2) { return ord_from_double(isnan(d2) ? DBL_MAX : d2); }
 
-__global__ void k_leaf_maxd2(TreeDev T, const double* d2a, const uint8_t* eflag, uint64_t* maxd2) {
+// Upper bound of the second-neighbour distance over the searched targets of
+// every leaf (-1 for a leaf without one): a merge farther from the leaf's box
+// than this changes none of its targets.
+__global__ void k_leaf_maxd2(TreeDev T, const int32_t* r0, const int32_t* r1, int base, const double* d2a,
+                             const uint8_t* eflag, uint64_t* maxd2) {
     const int l = blockIdx.x * blockDim.x + threadIdx.x;
     if (l >= T.nleaf) return;
     const int L = T.leaf_node[l];
     uint64_t m = ord_from_double(-1.0);
-    for (int i = T.v0[L]; i < T.v1[L]; i++)
-        if (eflag[i] & 1) m = max(m, d2_key(d2a[i]));
+    if (d2a)
+        for (int i = r0[L] - base; i < r1[L] - base; i++)
+            if (eflag[i] & 1) m = max(m, d2_key(d2a[i]));
     maxd2[l] = m;
 }
 
-// One merge, MergeVortexes(q, nn1[q]) (MEpsilonFast.cpp:111-126), by a
-// workgroup of NT threads, and its consequences for the targets that come
-// later: q itself is searched again without merging; every later target
-// whose near list holds leaf(q) takes q into its top-2 in O(1), and those
-// that had q or its partner p among their two neighbours (or see only
-// leaf(p)) are searched again.  Of the leaves whose near lists hold leaf(q)
-// or leaf(p), only those whose box lies within their targets' largest
-// second-neighbour distance of the old or new position of q or of p are
-// visited: no target elsewhere can take q or have had q or p as neighbour.
-// Targets whose merge flag becomes set are passed to on_flag(i).  `mark`
-// tags the leaves of leaf(q)'s reverse near list in stamp[] for this
-// commit.  Starts and ends with a barrier.
-template <int NT, typename OnFlag>
-__device__ void commit_one(const RepairArgs& A, int q, int mark, CommitShared& sh, OnFlag on_flag) {
-    const TreeDev& T = A.T;
-    const int tid = threadIdx.x;
-    constexpr int kWaves = NT / kWave;
-    double* x = A.x;
-    double* y = A.y;
-    double* g = A.g;
-    const int p = A.nn1[q];
-    __syncthreads();
-    if (tid == 0) {
-        sh.qx0 = x[q];
-        sh.qy0 = y[q];
-        sh.px0 = x[p];
-        sh.py0 = y[p];
-        const double gq = g[q], gp = g[p];
-        if (sgn(gq) == sgn(gp)) {
-            const double inv = 1. / (gq + gp);
-            const double nx = (x[q] * gq + x[p] * gp) * inv;
-            const double ny = (y[q] * gq + y[p] * gp) * inv;
-            x[q] = nx;
-            y[q] = ny;
-        } else if (fabs(gq) < fabs(gp)) {
-            x[q] = x[p];
-            y[q] = y[p];
-        }
-        g[q] = gq + gp;
-        g[p] = 0;
-        atomicAdd(&A.ecount[1], 1);
-        // the merged vortex may leave its leaf's box: grow the box so box
-        // distances stay lower bounds (pruned rescans, diffusive cutoff)
-        const int Lq = T.leaf_node[T.vleaf[q]];
-        if (!isnan(x[q])) {
-            atomicMin((unsigned long long*)&A.box_lo_x[Lq], (unsigned long long)ord_from_double(x[q]));
-            atomicMax((unsigned long long*)&A.box_hi_x[Lq], (unsigned long long)ord_from_double(x[q]));
-        }
-        if (!isnan(y[q])) {
-            atomicMin((unsigned long long*)&A.box_lo_y[Lq], (unsigned long long)ord_from_double(y[q]));
-            atomicMax((unsigned long long*)&A.box_hi_y[Lq], (unsigned long long)ord_from_double(y[q]));
-        }
-        if (p > q) {   // skipped later by the reference (g == 0)
-            A.eflag[p] = 0;
-            A.nn1[p] = -1;
-            A.nn2[p] = -1;
-        }
-        sh.nhard = 0;
+// The list being merged (the vortices, or the heat particles) and the state
+// of the rounds.  Elements are numbered within the list; r0/r1 minus base are
+// a node's range, vleaf[base + i] the leaf of element i.
+//   info[i]  {partner, death}: the element that i merges with at its visit
+//            (-1: none; -2: none now, but once), and the smallest target that
+//            absorbs i (INT_MAX: none).  Target t sees i when death >= t.
+//   rec[i]   position and circulation of i after its merge: what targets
+//            after i see while info[i].x >= 0
+//   fd2[i]   second-neighbour distance of i before its merge
+//   cand     a changed element's next record {x, y, g, partner}
+struct MergeArgs {
+    TreeDev T;
+    const double *x, *y, *g;
+    const int32_t *r0, *r1;
+    int base, n;
+    int heat;              // epsh: the distance criterion only
+    const double* crit;    // per leaf
+    int32_t *nn1, *nn2;
+    double *d1, *d2;
+    uint8_t* eflag;
+    uint64_t* maxd2;
+    int2* info;
+    double4 *rec, *cand;
+    double* fd2;
+    int32_t *stamp, *list0, *list1, *chg, *chg_p, *ever;
+    double4* cbox;         // per changed element: box of every position its change involves
+    int32_t* ctr;          // [0..1] targets to evaluate, [2..3] changed elements, [4] elements with a record
+    uint64_t *blx, *bly, *trx, *try_;
+    const int32_t *leaf_sim, *root_first;
+};
+
+constexpr int kMergeTab = 512;   // candidates staged per wave
+
+// What target i sees of element j (j != i).
+struct Seen {
+    double x, y, g;
+};
+__device__ inline Seen seen_of(const MergeArgs& A, int j, int i, int2 f) {
+    if (j < i && f.x >= 0) {
+        const double4 r = A.rec[j];
+        return Seen{r.x, r.y, r.z};
     }
-    __threadfence_block();
-    __syncthreads();
-    // the target itself: search again without merging
-    group_rescans<kWaves>(T, x, y, g, &q, 1, sh.part, [&](int i, const Top2& st) {
-        A.nn1[i] = st.i1;
-        A.nn2[i] = st.i2;
-        A.d1a[i] = st.d1;
-        A.d2a[i] = st.d2;
-        A.eflag[i] = 1;
-        atomicMax((unsigned long long*)&A.maxd2[T.vleaf[i]], (unsigned long long)d2_key(st.d2));
-    });
-    // mark the leaves whose near list contains leaf(q)
-    const int lq = T.vleaf[q], lp = T.vleaf[p];
-    for (int64_t e = A.roff[lq] + tid; e < A.roff[lq + 1]; e += NT) A.stamp[A.rlist[e]] = mark;
-    __threadfence_block();
-    __syncthreads();
-    const double qx = x[q], qy = y[q];
-    const double qx0 = sh.qx0, qy0 = sh.qy0, px0 = sh.px0, py0 = sh.py0;
-    // later targets that see leaf(q) (then those that see only leaf(p))
-    for (int pass = 0; pass < 2; pass++) {
-        const int lm = pass == 0 ? lq : lp;
-        if (pass == 1 && lp == lq) break;
-        const int64_t r0 = A.roff[lm], r1 = A.roff[lm + 1];
-        // leaves that can hold a changed target, one thread per leaf
-        if (tid == 0) sh.nlive = 0;
-        __syncthreads();
-        for (int64_t e = r0 + tid; e < r1; e += NT) {
-            const int L = A.rlist[e];
-            if (pass == 1 && A.stamp[L] == mark) continue;
-            const int Ln = T.leaf_node[L];
-            const double m = double_from_ord(A.maxd2[L]);
-            bool need = !(point_box_dist2(T, Ln, qx0, qy0) > m) || !(point_box_dist2(T, Ln, px0, py0) > m);
-            if (pass == 0) need = need || !(point_box_dist2(T, Ln, qx, qy) > m);
-            if (need) {
-                const int k = atomicAdd(&sh.nlive, 1);
-                if (k < kMaxLive) sh.live[k] = L;
-            }
-        }
-        __syncthreads();
-        const int nlive = sh.nlive;
-        const bool all = nlive > kMaxLive;   // list overflow: visit every leaf
-        const int64_t nvis = all ? r1 - r0 : nlive;
-        // NT / 16 leaves at a time, 16 threads per leaf
-        for (int64_t e0 = 0; e0 < nvis; e0 += NT / 16) {
-            const int64_t e = e0 + tid / 16;
-            if (e >= nvis) continue;
-            const int L = all ? A.rlist[r0 + e] : sh.live[e];
-            if (all && pass == 1 && A.stamp[L] == mark) continue;
-            const int Ln = T.leaf_node[L];
-            const int a0 = T.v0[Ln], a1 = T.v1[Ln];
-            for (int i = a0 + (tid & 15); i < a1; i += 16) {
-                if (i <= q || !(A.eflag[i] & 1)) continue;
-                const bool hard = A.nn1[i] == q || A.nn1[i] == p || A.nn2[i] == q || A.nn2[i] == p;
-                if (hard) {
-                    const int h = atomicAdd(&sh.nhard, 1);
-                    if (h < kMaxHard)
-                        sh.hard[h] = i;
-                    else
-                        sh.overflow = 1;
-                    continue;
-                }
-                if (pass == 1) continue;   // q is not in the near set of i
-                Top2 st{A.d1a[i], A.d2a[i], A.nn1[i], A.nn2[i]};
-                top2_insert(st, dist2(x[i], y[i], qx, qy), q);
-                A.nn1[i] = st.i1;
-                A.nn2[i] = st.i2;
-                A.d1a[i] = st.d1;
-                A.d2a[i] = st.d2;   // only decreases: the leaf bound holds
-                const bool f = merge_flag(g, i, st, A.leaf_crit[L]);
-                A.eflag[i] = 1 | (f ? 2 : 0);
-                if (f) on_flag(i);
-            }
-        }
-        __syncthreads();
-    }
-    __threadfence_block();
-    __syncthreads();
-    const int nh = min(sh.nhard, kMaxHard);
-    group_rescans<kWaves>(T, x, y, g, sh.hard, nh, sh.part, [&](int i, const Top2& st) {
-        A.nn1[i] = st.i1;
-        A.nn2[i] = st.i2;
-        A.d1a[i] = st.d1;
-        A.d2a[i] = st.d2;
-        const bool f = merge_flag(g, i, st, A.leaf_crit[T.vleaf[i]]);
-        A.eflag[i] = 1 | (f ? 2 : 0);
-        atomicMax((unsigned long long*)&A.maxd2[T.vleaf[i]], (unsigned long long)d2_key(st.d2));
-        if (f) on_flag(i);
-    });
-    __threadfence_block();
-    __syncthreads();
+    return Seen{A.x[j], A.y[j], A.g[j]};
 }
 
-// Pass 2: commits merges in target order, one workgroup per simulation
-// (targets [sim_off[s], sim_off[s+1]); simulations share no leaf).
-// Candidates are kept in an LDS list (the flags of pass 1 plus targets
-// flagged by later updates); the next commit is the smallest listed index at
-// or after the cursor whose flag is still set.  If the list overflows, the
-// remaining commits find their target by scanning the flags.
-// With mark set, only the reverse near lists of marked leaves exist: a commit
-// that needs another one stops the simulation's pass (state[2s] = its
-// target, state[2s+1] = the commit count, ecount[3] set); a second launch
-// with resume set continues from there once all lists are built, taking its
-// candidates from the flags at or after the cursor.  state[2s] = -1 marks a
-// finished simulation.
-__global__ __launch_bounds__(kRepairThreads) void k_eps_repair(RepairArgs A, const int64_t* sim_off,
-                                                               const int32_t* flag_list, const uint8_t* mark,
-                                                               int64_t* state, int resume) {
-    __shared__ int s_q;
-    __shared__ int s_np;
-    __shared__ int s_pend[kMaxPend];
-    __shared__ CommitShared sh;
-    int32_t* ecount = A.ecount;
-    const int tid = threadIdx.x;
-    const int64_t lo = sim_off[blockIdx.x], n = sim_off[blockIdx.x + 1];
-    int64_t cursor = lo;
-    int commit = 0;
-    if (resume) {
-        cursor = state[2 * blockIdx.x];
-        commit = (int)state[2 * blockIdx.x + 1];
-        if (cursor < 0) return;   // finished in the first launch
+// The two nearest of target i among what it sees in its near leaves, at
+// (px, py), without itself and excl: the leaves touching its own first, then
+// those whose box lies within the second-neighbour distance found.  One wave;
+// all lanes get the result.  Latency-bound: the entries of 256 list places,
+// their boxes and ranges load together, and the candidates of all of them
+// are listed in LDS, so that a search is about four dependent loads.
+__device__ Top2 seen_top2(const MergeArgs& A, int l, int L, int i, int excl, double px, double py, int* tab) {
+    const TreeDev& T = A.T;
+    const int lane = lane_id();
+    const int64_t e0 = T.near_off[l], e1 = T.near_off[l + 1];
+    constexpr int kPer = 4;
+    auto wave_sync = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    auto scan = [&](bool touching, double bound) {
+        Top2 st = top2_empty();
+        for (int64_t eb = e0; eb < e1; eb += kPer * kWave) {
+            int M[kPer], j0[kPer], cnt[kPer], mine = 0;
+#pragma unroll
+            for (int k = 0; k < kPer; k++) {
+                const int64_t e = eb + k * kWave + lane;
+                M[k] = e < e1 ? T.near_list[e] : -1;
+            }
+#pragma unroll
+            for (int k = 0; k < kPer; k++) {
+                const int m = M[k] >= 0 ? M[k] : L;
+                const double bd = box_dist2(T, L, m);
+                const bool take = M[k] >= 0 && (touching ? bd <= 0.0 : bd > 0.0 && point_box_dist2(T, m, px, py) <= bound);
+                j0[k] = A.r0[m] - A.base;
+                cnt[k] = take ? A.r1[m] - A.base - j0[k] : 0;
+                mine += cnt[k];
+            }
+            const int incl = wave_incl_scan(mine);
+            const int total = __shfl(incl, kWave - 1, kWave);
+            for (int done = 0; done < total; done += kMergeTab) {
+                int o = incl - mine - done;
+#pragma unroll
+                for (int k = 0; k < kPer; k++) {
+                    for (int t = max(0, -o); t < cnt[k] && o + t < kMergeTab; t++) tab[o + t] = j0[k] + t;
+                    o += cnt[k];
+                }
+                wave_sync();
+                const int m = min(kMergeTab, total - done);
+                for (int q = lane; q < m; q += kWave) {
+                    const int j = tab[q];
+                    if (j == i || j == excl) continue;
+                    const int2 f = A.info[j];
+                    if (f.y < i) continue;
+                    const Seen v = seen_of(A, j, i, f);
+                    if (v.g != 0) top2_insert(st, dist2(px, py, v.x, v.y), j);
+                }
+                wave_sync();
+            }
+        }
+        return wave_top2(st);
+    };
+    Top2 c = scan(true, 0.0);
+    top2_merge(c, scan(false, c.i2 >= 0 ? c.d2 : INFINITY));
+    return c;
+}
+
+// Elements start without a merge.
+__global__ void k_merge_init(MergeArgs A) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= A.n) return;
+    A.info[i] = make_int2(-1, INT32_MAX);
+    A.stamp[i] = 0;
+    if (A.heat) {   // no parallel pass before the rounds: every particle is a target of the first
+        A.list0[i] = i;
+        A.d2[i] = -1.;
+    }
+}
+
+// One round, first part: every listed target is visited as the reference does
+// when the merges of the targets before it are those of the last round; one
+// wave per target.  Its search results are written in place (only the marking
+// pass reads them), its merge goes to cand and the list of changes.
+__global__ __launch_bounds__(kBlock) void k_merge_eval(MergeArgs A, int parity) {
+    __shared__ int s_tab[kWavesPerBlock][kMergeTab];
+    const TreeDev& T = A.T;
+    const int w = threadIdx.x / kWave, lane = lane_id();
+    const int nd = A.ctr[parity];
+    const int32_t* list = parity ? A.list1 : A.list0;
+    for (int k = blockIdx.x * kWavesPerBlock + w; k < nd; k += gridDim.x * kWavesPerBlock) {
+        const int i = list[k];
+        const double gi = A.g[i];
+        const int2 own = A.info[i];
+        const int l = T.vleaf[A.base + i], L = T.leaf_node[l];
+        Top2 st = top2_empty();
+        int partner = -1;
+        double4 rec = make_double4(0, 0, 0, 0);
+        const bool alive = gi != 0 && own.y >= i;
+        double first_d2 = -1.;
+        if (alive) {
+            double px = A.x[i], py = A.y[i];
+            st = seen_top2(A, l, L, i, -1, px, py, s_tab[w]);
+            first_d2 = st.d2;
+            const double crit = A.crit[l];
+            if (st.i1 >= 0 && st.i2 >= 0 && !isnan(crit)) {
+                const Seen a = seen_of(A, st.i1, i, A.info[st.i1]), b = seen_of(A, st.i2, i, A.info[st.i2]);
+                const double s1 = sgn(a.g), s2 = sgn(b.g), si = sgn(gi);
+                if ((st.d1 < crit) || (!A.heat && (s1 == s2) && (s1 != si))) {
+                    // MergeVortexes (:111-126), then the search without merging
+                    partner = st.i1;
+                    if (si == s1) {
+                        const double inv = 1. / (gi + a.g);
+                        const double nx = (px * gi + a.x * a.g) * inv;
+                        const double ny = (py * gi + a.y * a.g) * inv;
+                        px = nx;
+                        py = ny;
+                    } else if (fabs(gi) < fabs(a.g)) {
+                        px = a.x;
+                        py = a.y;
+                    }
+                    rec = make_double4(px, py, gi + a.g, 0);
+                    st = seen_top2(A, l, L, i, partner, px, py, s_tab[w]);
+                }
+            }
+        }
+        if (lane != 0) continue;
+        A.nn1[i] = st.i1;
+        A.nn2[i] = st.i2;
+        A.d1[i] = st.d1;
+        A.d2[i] = alive ? st.d2 : -1.;
+        A.fd2[i] = first_d2;
+        A.eflag[i] = alive ? 1 : 0;
+        if (alive) {
+            const uint64_t key = max(d2_key(st.d2), d2_key(first_d2));
+            atomicMax((unsigned long long*)&A.maxd2[l], (unsigned long long)key);
+        }
+        bool changed = partner != max(own.x, -1);
+        if (!changed && partner >= 0) {
+            const double4 o = A.rec[i];
+            changed = __double_as_longlong(o.x) != __double_as_longlong(rec.x) ||
+                      __double_as_longlong(o.y) != __double_as_longlong(rec.y) ||
+                      __double_as_longlong(o.z) != __double_as_longlong(rec.z);
+        }
+        if (changed) {
+            rec.w = (double)partner;
+            A.cand[i] = rec;
+            A.chg[atomicAdd(&A.ctr[2 + parity], 1)] = i;
+        }
+    }
+}
+
+// Second part, one workgroup: the changed records take effect, the deaths
+// follow from all records, and every change gets the box of the positions it
+// involves (the element's own before and after, and its old and new
+// partner's).  Node boxes grow by the new positions, so that box distances
+// stay lower bounds.
+constexpr int kMergeThreads = 1024;
+__global__ __launch_bounds__(kMergeThreads) void k_merge_apply(MergeArgs A, int parity) {
+    const int nc = A.ctr[2 + parity], tid = threadIdx.x;
+    auto grow = [](double4& b, double px, double py) {
+        b.x = fmin(b.x, px);
+        b.y = fmin(b.y, py);
+        b.z = fmax(b.z, px);
+        b.w = fmax(b.w, py);
+    };
+    for (int e = tid; e < nc; e += kMergeThreads) {
+        const int q = A.chg[e], p = A.info[q].x;
+        double4 b = make_double4(A.x[q], A.y[q], A.x[q], A.y[q]);
+        A.chg_p[e] = p;
+        if (p >= 0) {
+            const double4 r = A.rec[q];
+            grow(b, r.x, r.y);
+            grow(b, A.x[p], A.y[p]);
+            A.info[p].y = INT32_MAX;
+        }
+        A.cbox[e] = b;
+    }
+    __threadfence();
+    __syncthreads();
+    for (int e = tid; e < nc; e += kMergeThreads) {
+        const int q = A.chg[e];
+        const double4 r = A.cand[q];
+        const int p = (int)r.w;
+        if (A.info[q].x == -1) A.ever[atomicAdd(&A.ctr[4], 1)] = q;
+        A.info[q].x = p >= 0 ? p : -2;
+        A.rec[q] = r;
+        if (p >= 0) {
+            double4 b = A.cbox[e];
+            grow(b, r.x, r.y);
+            grow(b, A.x[p], A.y[p]);
+            A.cbox[e] = b;
+            const int Lq = A.T.leaf_node[A.T.vleaf[A.base + q]];
+            if (!isnan(r.x)) {
+                atomicMin((unsigned long long*)&A.blx[Lq], (unsigned long long)ord_from_double(r.x));
+                atomicMax((unsigned long long*)&A.trx[Lq], (unsigned long long)ord_from_double(r.x));
+            }
+            if (!isnan(r.y)) {
+                atomicMin((unsigned long long*)&A.bly[Lq], (unsigned long long)ord_from_double(r.y));
+                atomicMax((unsigned long long*)&A.try_[Lq], (unsigned long long)ord_from_double(r.y));
+            }
+        }
+    }
+    __threadfence();
+    __syncthreads();
+    const int ne = A.ctr[4];
+    for (int k = tid; k < ne; k += kMergeThreads) {
+        const int q = A.ever[k], p = A.info[q].x;
+        if (p >= 0) atomicMin(&A.info[p].y, q);
+    }
+    // a partner that has merged itself is seen at its merged position too
+    for (int e = tid; e < nc; e += kMergeThreads) {
+        const int q = A.chg[e];
+        double4 b = A.cbox[e];
+        for (int which = 0; which < 2; which++) {
+            const int p = which ? A.chg_p[e] : A.info[q].x;
+            if (p < 0 || A.info[p].x < 0) continue;
+            const double4 r = A.rec[p];
+            grow(b, r.x, r.y);
+        }
+        A.cbox[e] = b;
     }
     if (tid == 0) {
-        sh.overflow = 0;
-        s_np = 0;
+        A.ctr[parity] = 0;
+        A.ctr[2 + (parity ^ 1)] = 0;
     }
+}
+
+// Third part: the targets after a changed element whose second-neighbour
+// distance reaches its box are visited again in the next round (those it
+// does not reach cannot take or lose a neighbour by it), and so are its old
+// and new partner, which it kills or revives.  Work items are (change, 256
+// leaves): leaves before the element's hold no later target.
+__global__ __launch_bounds__(kBlock) void k_merge_mark(MergeArgs A, int parity, int chunks, int tag) {
+    const TreeDev& T = A.T;
+    const int nc = A.ctr[2 + parity];
+    int32_t* list = parity ? A.list0 : A.list1;
+    auto push = [&](int i) {
+        if (atomicExch(&A.stamp[i], tag) != tag) list[atomicAdd(&A.ctr[parity ^ 1], 1)] = i;
+    };
+    for (int64_t it = blockIdx.x; it < (int64_t)nc * chunks; it += gridDim.x) {
+        const int e = (int)(it / chunks), ch = (int)(it % chunks);
+        const int q = A.chg[e];
+        const int lq = T.vleaf[A.base + q];
+        const int lend = A.root_first[A.leaf_sim[lq] + 1];
+        if (ch == 0 && threadIdx.x == 0) {
+            const int p0 = A.chg_p[e], p1 = A.info[q].x;
+            if (p0 > q) push(p0);
+            if (p1 > q) push(p1);
+        }
+        const int l = lq + ch * kBlock + threadIdx.x;
+        if (l >= lend) continue;
+        const double4 b = A.cbox[e];
+        const int L = T.leaf_node[l];
+        const double m = double_from_ord(A.maxd2[l]);
+        {
+            const double dx = fmax(0.0, fmax(b.x - double_from_ord(T.trx[L]), double_from_ord(T.blx[L]) - b.z));
+            const double dy = fmax(0.0, fmax(b.y - double_from_ord(T.try_[L]), double_from_ord(T.bly[L]) - b.w));
+            if (dx * dx + dy * dy > m) continue;
+        }
+        auto reach = [&](double px, double py, double d2) {
+            const double dx = fmax(0.0, fmax(b.x - px, px - b.z)), dy = fmax(0.0, fmax(b.y - py, py - b.w));
+            return !(dx * dx + dy * dy > d2);
+        };
+        for (int i = A.r0[L] - A.base; i < A.r1[L] - A.base; i++) {
+            if (i <= q || !(A.eflag[i] & 1)) continue;
+            bool hit;
+            if (A.info[i].x >= 0) {
+                const double4 r = A.rec[i];
+                hit = reach(A.x[i], A.y[i], A.fd2[i]) || reach(r.x, r.y, A.d2[i]);
+            } else {
+                hit = reach(A.x[i], A.y[i], A.d2[i]);
+            }
+            if (hit) push(i);
+        }
+    }
+}
+
+// The converged merges written to the list, one workgroup: every merging
+// element takes its record, then every partner loses its circulation.
+__global__ __launch_bounds__(kMergeThreads) void k_merge_finish(MergeArgs A, double* x, double* y, double* g,
+                                                                int32_t* merged) {
+    __shared__ int s_n;
+    const int ne = A.ctr[4], tid = threadIdx.x;
+    if (tid == 0) s_n = 0;
     __syncthreads();
-    if (!resume) {
-        for (int k = tid; k < ecount[0]; k += kRepairThreads) {
-            const int i = flag_list[k];
-            if (i >= lo && i < n) {
-                const int idx = atomicAdd(&s_np, 1);
-                if (idx < kMaxPend) s_pend[idx] = i;
-            }
-        }
-    } else {
-        for (int64_t i = cursor + tid; i < n; i += kRepairThreads)
-            if (A.eflag[i] & 2) {
-                const int idx = atomicAdd(&s_np, 1);
-                if (idx < kMaxPend) s_pend[idx] = (int)i;
-            }
+    int cnt = 0;
+    for (int k = tid; k < ne; k += kMergeThreads) {
+        const int q = A.ever[k];
+        if (A.info[q].x < 0) continue;
+        const double4 r = A.rec[q];
+        x[q] = r.x;
+        y[q] = r.y;
+        g[q] = r.z;
+        cnt++;
     }
+    atomicAdd(&s_n, cnt);
+    __threadfence();
     __syncthreads();
-    const bool scan_mode0 = s_np > kMaxPend;
-    while (true) {
-        if (tid == 0) s_q = INT32_MAX;
-        __syncthreads();
-        const bool scan_mode = scan_mode0 || s_np > kMaxPend;
-        if (!scan_mode) {
-            for (int k = tid; k < s_np; k += kRepairThreads) {
-                const int i = s_pend[k];
-                if (i >= cursor && (A.eflag[i] & 2)) atomicMin(&s_q, i);
-            }
-            __syncthreads();
-        } else {
-            for (int64_t b = cursor; b < n; b += kRepairThreads) {
-                const int64_t i = b + tid;
-                if (i < n && (A.eflag[i] & 2)) atomicMin(&s_q, (int)i);
-                __syncthreads();
-                if (s_q != INT32_MAX) break;
-                __syncthreads();
-            }
-            __syncthreads();
-        }
-        const int q = s_q;
-        if (q == INT32_MAX) break;
-        if (mark && !(mark[A.T.vleaf[q]] && mark[A.T.vleaf[A.nn1[q]]])) {
-            if (tid == 0) {
-                state[2 * blockIdx.x] = q;
-                state[2 * blockIdx.x + 1] = commit;
-                atomicExch(&ecount[3], 1);
-            }
-            return;   // uniform: q comes from LDS
-        }
-        commit++;
-        commit_one<kRepairThreads>(A, q, commit, sh, [&](int i) {
-            const int k = atomicAdd(&s_np, 1);
-            if (k < kMaxPend) s_pend[k] = i;
-        });
-        cursor = q + 1;
+    for (int k = tid; k < ne; k += kMergeThreads) {
+        const int p = A.info[A.ever[k]].x;
+        if (p >= 0) g[p] = 0;
     }
-    if (tid == 0) {
-        state[2 * blockIdx.x] = -1;
-        if (sh.overflow) ecount[2] = 1;
-    }
+    if (tid == 0) *merged = s_n;
 }
 
 // Applies _1_eps = 1/max(eps, floor) to every processed target (:49-54) and
-// packs the FP32 {g, eps^2} copy the pair kernels read.  Does nothing while
-// the merge pass still has to resume (ecount[3]): it must see the final
-// state only once.
+// packs the FP32 {g, eps^2} copy the pair kernels read.
 __global__ void k_eps_apply(const TreeDev T, const double* g, double* ie, int64_t n, const int32_t* nn1,
                             const int32_t* nn2, const double* d1a, const double* d2a, const uint8_t* eflag,
-                            const double* leaf_restr, float2* src_ge, const int32_t* ecount) {
+                            const double* leaf_restr, float2* src_ge) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n || ecount[3]) return;
+    if (i >= n) return;
     double iv = ie[i];
     if (eflag[i] & 1) {
         double eps;
@@ -794,6 +718,65 @@ void pack_sources(Ctx& c) {
         hipLaunchKernelGGL(k_pack, dim3(nblocks(c.n)), dim3(kBlock), 0, c.stream, c.g.p, c.ie.p, c.n, c.src_ge.p);
 }
 
+namespace {
+
+// Finds the sequential merges of the list in A (see MergeArgs) and writes
+// them to x, y, g; the number goes to *merged on the device.  The first
+// round's targets are in list0, their count in ctr[0].  Rounds are queued a
+// few at a time and end when one leaves nothing to visit: at most one per
+// element, in practice the longest chain of merges that wait for each other
+// (three to about ten).  One workgroup committing merge after merge took
+// about 45 us each (5.8 ms a step for a cylinder wake of 3k vortices); a
+// round of all of them takes about 25 us.
+void merge_rounds(Ctx& c, MergeArgs A, double* x, double* y, double* g, int32_t* merged) {
+    hipStream_t s = c.stream;
+    int most = 1;   // most leaves of one simulation
+    if (c.nsim == 1) {
+        most = A.T.nleaf;
+    } else {
+        std::vector<int32_t> rf(c.nsim + 1);
+        VVHD_HIP(hipMemcpyAsync(rf.data(), c.t.root_first.p, rf.size() * 4, hipMemcpyDeviceToHost, s));
+        VVHD_HIP(hipStreamSynchronize(s));
+        for (int q = 0; q < c.nsim; q++) most = std::max(most, rf[q + 1] - rf[q]);
+    }
+    const int chunks = (most + kBlock - 1) / kBlock;
+    int32_t left = 1;
+    for (int64_t round = 0; left > 0; ) {
+        VVHD_CHECK(round <= (int64_t)A.n + 8, VVHD_EHIP, "epsilon: the merges do not settle");
+        for (int k = 0; k < 4; k++, round++) {
+            const int par = (int)(round & 1);
+            hipLaunchKernelGGL(k_merge_eval, dim3(1024), dim3(kBlock), 0, s, A, par);
+            hipLaunchKernelGGL(k_merge_apply, dim3(1), dim3(kMergeThreads), 0, s, A, par);
+            hipLaunchKernelGGL(k_merge_mark, dim3(1024), dim3(kBlock), 0, s, A, par, chunks, (int)round + 1);
+        }
+        VVHD_HIP(hipMemcpyAsync(&left, A.ctr + (round & 1), 4, hipMemcpyDeviceToHost, s));
+        VVHD_HIP(hipStreamSynchronize(s));
+    }
+    hipLaunchKernelGGL(k_merge_finish, dim3(1), dim3(kMergeThreads), 0, s, A, x, y, g, merged);
+}
+
+// Buffers of the rounds for a list of n elements.
+MergeArgs merge_args(Ctx& c, const double* x, const double* y, const double* g, const int32_t* r0, const int32_t* r1,
+                     int base, int64_t n, int heat, int32_t* nn1, int32_t* nn2, double* d1, double* d2,
+                     uint8_t* eflag, int32_t* list0) {
+    MergeBufs& b = c.mg;
+    b.info.grow(n);
+    b.rec.grow(n);
+    b.cand.grow(n);
+    b.cbox.grow(n);
+    b.fd2.grow(n);
+    for (auto* p : {&b.stamp, &b.list, &b.chg, &b.chg_p, &b.ever}) p->grow(n);
+    b.maxd2.grow(c.t.nleaves_h + 1);
+    TreeArrays& t = c.t;
+    return MergeArgs{tree_dev(t), x, y, g, r0, r1, base, (int)n, heat, c.leaf_crit.p, nn1, nn2, d1, d2, eflag,
+                     b.maxd2.p, b.info.p, b.rec.p, b.cand.p, b.fd2.p, b.stamp.p, list0, b.list.p, b.chg.p, b.chg_p.p,
+                     b.ever.p, b.cbox.p, c.ecount.p, t.blx.p, t.bly.p, t.trx.p, t.try_.p, t.leaf_sim.p,
+                     t.root_first.p};
+}
+
+}  // namespace
+
+// ecount: [0..4] the rounds' counters ([0] pass 1's flags), [5] merges.
 void epsilon(Ctx& c, int merge, int32_t* nn1_out, int32_t* nn2_out, int32_t* merged_out) {
     const int64_t n = c.n;
     const TreeDev T = tree_dev(c.t);
@@ -816,87 +799,71 @@ void epsilon(Ctx& c, int merge, int32_t* nn1_out, int32_t* nn2_out, int32_t* mer
         hipLaunchKernelGGL(k_eps_top2, dim3((nl + kWavesPerBlock - 1) / kWavesPerBlock), dim3(kBlock), 0, s, T, c.x.p,
                            c.y.p, c.g.p, merge, c.leaf_crit.p, c.nn1.p, c.nn2.p, c.d1.p, c.d2.p, c.eflag.p,
                            c.ecount.p, c.flag_list.p);
-    int32_t hc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    VVHD_HIP(hipMemcpyAsync(hc, c.ecount.p, 16, hipMemcpyDeviceToHost, s));
+    int32_t flags = 0, merged = 0;
+    VVHD_HIP(hipMemcpyAsync(&flags, c.ecount.p, 4, hipMemcpyDeviceToHost, s));
     VVHD_HIP(hipStreamSynchronize(s));
-    // reverse near lists: all of them, or with few flags only those of the
-    // flagged targets' leaves (a commit that needs another one resumes after
-    // the full build)
-    auto build_rnear = [&](const uint8_t* mark) {
-        VVHD_HIP(hipMemsetAsync(c.rnear_cnt.p, 0, (size_t)(nl + 1) * 4, s));
-        const int flat_grid = (int)std::min<int64_t>(8192, std::max<int64_t>(1, (c.t.nnear + kBlock - 1) / kBlock));
-        if (mark)
-            hipLaunchKernelGGL(k_rnear_count_flat, dim3(flat_grid), dim3(kBlock), 0, s, T, (int64_t)c.t.nnear,
-                               c.rnear_cnt.p, mark);
-        else
-            hipLaunchKernelGGL(k_rnear_count, dim3(nblocks(nl, kWavesPerBlock)), dim3(kBlock), 0, s, T,
-                               c.rnear_cnt.p, mark);
-        size_t bytes = 0;
-        VVHD_HIP(rocprim::exclusive_scan(nullptr, bytes, c.rnear_cnt.p, c.rnear_off.p, (int64_t)0, (size_t)nl + 1,
-                                         rocprim::plus<int64_t>(), s));
-        c.tmp.grow(bytes + 16);
-        VVHD_HIP(rocprim::exclusive_scan(c.tmp.p, bytes, c.rnear_cnt.p, c.rnear_off.p, (int64_t)0, (size_t)nl + 1,
-                                         rocprim::plus<int64_t>(), s));
-        VVHD_HIP(hipMemsetAsync(c.rnear_cnt.p, 0, (size_t)(nl + 1) * 4, s));
-        if (mark)
-            hipLaunchKernelGGL(k_rnear_fill_flat, dim3(flat_grid), dim3(kBlock), 0, s, T, (int64_t)c.t.nnear,
-                               c.rnear_off.p, c.rnear_cnt.p, c.rnear_list.p, mark);
-        else
-            hipLaunchKernelGGL(k_rnear_fill, dim3(nblocks(nl, kWavesPerBlock)), dim3(kBlock), 0, s, T,
-                               c.rnear_off.p, c.rnear_cnt.p, c.rnear_list.p, mark);
-    };
-    // (buffers grown first: the arguments hold their pointers)
-    auto repair_args = [&] {
-        return RepairArgs{T,         c.x.p,         c.y.p,       c.g.p,     c.leaf_crit.p, c.rnear_off.p,
-                          c.rnear_list.p, c.leaf_stamp.p, c.nn1.p, c.nn2.p, c.d1.p,        c.d2.p,
-                          c.eflag.p, c.ecount.p,    c.t.blx.p,   c.t.bly.p, c.t.trx.p,     c.t.try_.p,
-                          c.leaf_maxd2.p};
-    };
-    const bool marked = hc[0] > 0 && hc[0] <= kMarkedFlags;
-    if (hc[0] > 0) {
-        c.rnear_off.grow(nl + 1);
-        c.rnear_cnt.grow(nl + 1);
-        c.leaf_stamp.grow(nl + 1);
-        c.rnear_list.grow(c.t.nnear + 1);
-        c.rep_state.grow(2 * (size_t)c.nsim);
-        c.leaf_mark.grow(nl + 1);
-        c.leaf_maxd2.grow(nl + 1);
-        VVHD_HIP(hipMemsetAsync(c.leaf_stamp.p, 0, (size_t)(nl + 1) * 4, s));
-        if (marked) {
-            VVHD_HIP(hipMemsetAsync(c.leaf_mark.p, 0, (size_t)(nl + 1), s));
-            hipLaunchKernelGGL(k_mark_flag_leaves, dim3(nblocks(hc[0])), dim3(kBlock), 0, s, T,
-                               (const int32_t*)c.flag_list.p, (const int32_t*)c.ecount.p, (const int32_t*)c.nn1.p,
-                               c.leaf_mark.p);
-        }
-        build_rnear(marked ? c.leaf_mark.p : nullptr);
-        hipLaunchKernelGGL(k_leaf_maxd2, dim3(nblocks(nl)), dim3(kBlock), 0, s, T, c.d2.p, c.eflag.p, c.leaf_maxd2.p);
-        hipLaunchKernelGGL(k_eps_repair, dim3(c.nsim), dim3(kRepairThreads), 0, s, repair_args(),
-                           (const int64_t*)c.sim_off.p,
-                           c.flag_list.p, marked ? (const uint8_t*)c.leaf_mark.p : (const uint8_t*)nullptr,
-                           c.rep_state.p, 0);
+    if (flags > 0) {
+        const MergeArgs A = merge_args(c, c.x.p, c.y.p, c.g.p, T.v0, T.v1, 0, n, 0, c.nn1.p, c.nn2.p, c.d1.p, c.d2.p,
+                                       c.eflag.p, c.flag_list.p);
+        hipLaunchKernelGGL(k_merge_init, dim3(nblocks(n)), dim3(kBlock), 0, s, A);
+        hipLaunchKernelGGL(k_leaf_maxd2, dim3(nblocks(nl)), dim3(kBlock), 0, s, T, A.r0, A.r1, 0,
+                           (const double*)c.d2.p, (const uint8_t*)c.eflag.p, A.maxd2);
+        merge_rounds(c, A, c.x.p, c.y.p, c.g.p, c.ecount.p + 5);
     }
-    auto finish = [&] {
-        hipLaunchKernelGGL(k_eps_apply, dim3(nblocks(n)), dim3(kBlock), 0, s, T, c.g.p, c.ie.p, n, c.nn1.p, c.nn2.p,
-                           c.d1.p, c.d2.p, c.eflag.p, c.leaf_restr.p, c.src_ge.p, (const int32_t*)c.ecount.p);
-        VVHD_HIP(hipMemcpyAsync(hc, c.ecount.p, 32, hipMemcpyDeviceToHost, s));
+    hipLaunchKernelGGL(k_eps_apply, dim3(nblocks(n)), dim3(kBlock), 0, s, T, c.g.p, c.ie.p, n, c.nn1.p, c.nn2.p,
+                       c.d1.p, c.d2.p, c.eflag.p, c.leaf_restr.p, c.src_ge.p);
+    if (flags > 0) {
+        VVHD_HIP(hipMemcpyAsync(&merged, c.ecount.p + 5, 4, hipMemcpyDeviceToHost, s));
         VVHD_HIP(hipStreamSynchronize(s));
-    };
-    finish();
-    if (marked && hc[3]) {   // a merge reached a leaf without its reverse list
-        VVHD_HIP(hipMemsetAsync(c.ecount.p + 3, 0, 4, s));
-        build_rnear(nullptr);
-        hipLaunchKernelGGL(k_eps_repair, dim3(c.nsim), dim3(kRepairThreads), 0, s, repair_args(),
-                           (const int64_t*)c.sim_off.p,
-                           c.flag_list.p, (const uint8_t*)nullptr, c.rep_state.p, 1);
-        finish();
     }
     if (nn1_out && n) VVHD_HIP(hipMemcpyAsync(nn1_out, c.nn1.p, (size_t)n * 4, hipMemcpyDeviceToHost, s));
     if (nn2_out && n) VVHD_HIP(hipMemcpyAsync(nn2_out, c.nn2.p, (size_t)n * 4, hipMemcpyDeviceToHost, s));
-    VVHD_HIP(hipStreamSynchronize(s));
-    VVHD_CHECK(hc[2] == 0, VVHD_EUNSUPPORTED, "epsilon: too many targets to rescan after one merge");
-    if (hc[1] > 0) pack_boxes(c);   // merges grew leaf boxes
+    if (flags > 0) pack_boxes(c);   // merges grew leaf boxes
     const int heat_merged = heat_epsilon(c, merge);   // epsh on the heat list (MEpsilonFast.cpp:53-60)
-    if (merged_out) *merged_out = hc[1] + heat_merged;
+    if (merged_out) *merged_out = merged + heat_merged;
+}
+
+// _1_eps = 1 / max(eps, floor) of the heat particles (MEpsilonFast.cpp:55-60).
+__global__ void k_heat_eps_apply(const int32_t* vleaf, const int32_t* nn1, const int32_t* nn2, const double* d1,
+                                 const double* d2, const uint8_t* eflag, const double* restr, double* hie, int64_t nh) {
+    const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (j >= nh || !(eflag[j] & 1)) return;
+    const double e = nn1[j] < 0 ? DBL_MIN : (nn2[j] < 0 ? sqrt(d1[j]) : sqrt(d2[j]));
+    const double r = restr[vleaf[j]];
+    hie[j] = 1.0 / ((e < r) ? r : e);   // std::max(e, r)
+}
+
+// epsh (MEpsilonFast.cpp:175-212) on the heat list: the same rounds, every
+// particle a target of the first (without merging the criterion is NaN and
+// the first round is all there is).
+int heat_epsilon(Ctx& c, int merge) {
+    const int64_t nh = c.heat.n;
+    if (nh == 0) return 0;
+    const TreeDev T = tree_dev(c.t);
+    hipStream_t s = c.stream;
+    MergeBufs& b = c.mg;
+    for (auto* p : {&b.hn1, &b.hn2, &b.hlist}) p->grow(nh);
+    for (auto* p : {&b.hd1, &b.hd2}) p->grow(nh);
+    b.hflag.grow(nh);
+    const MergeArgs A = merge_args(c, c.heat.x.p, c.heat.y.p, c.heat.g.p, T.h0, T.h1, T.hbase, nh, 1, b.hn1.p,
+                                   b.hn2.p, b.hd1.p, b.hd2.p, b.hflag.p, b.hlist.p);
+    const int32_t start[8] = {(int32_t)nh, 0, 0, 0, 0, 0, 0, 0};
+    VVHD_HIP(hipMemcpyAsync(c.ecount.p, start, sizeof(start), hipMemcpyHostToDevice, s));
+    hipLaunchKernelGGL(k_merge_init, dim3(nblocks(nh)), dim3(kBlock), 0, s, A);
+    hipLaunchKernelGGL(k_leaf_maxd2, dim3(nblocks(T.nleaf)), dim3(kBlock), 0, s, T, A.r0, A.r1, A.base,
+                       (const double*)nullptr, (const uint8_t*)nullptr, A.maxd2);
+    merge_rounds(c, A, c.heat.x.p, c.heat.y.p, c.heat.g.p, c.ecount.p + 5);
+    hipLaunchKernelGGL(k_heat_eps_apply, dim3(nblocks(nh)), dim3(kBlock), 0, s, T.vleaf + T.hbase,
+                       (const int32_t*)b.hn1.p, (const int32_t*)b.hn2.p, (const double*)b.hd1.p,
+                       (const double*)b.hd2.p, (const uint8_t*)b.hflag.p, (const double*)c.leaf_restr.p, c.heat.ie.p,
+                       nh);
+    int32_t merged = 0;
+    if (merge) {
+        VVHD_HIP(hipMemcpyAsync(&merged, c.ecount.p + 5, 4, hipMemcpyDeviceToHost, s));
+        VVHD_HIP(hipStreamSynchronize(s));
+    }
+    VVHD_HIP(hipGetLastError());
+    return merged;
 }
 
 }  // namespace vvhd

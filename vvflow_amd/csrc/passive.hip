@@ -3,14 +3,7 @@
 //
 // The tree build partitions both lists with the vortices (one range per list
 // and node, tree.hip).  On the built tree:
-//  * epsh (MEpsilonFast.cpp:175-212): the two nearest heat particles of every
-//    heat particle among the heat particles of its leaf's near leaves, with
-//    the reference's sequential merges.  A parallel pass evaluates every
-//    target on the unmodified list and flags the targets that would merge;
-//    when flags exist, one wave walks the leaves in DFS order and re-evaluates,
-//    target by target, exactly the leaves that hold a flagged target or have
-//    a near leaf touched by an earlier merge; every other leaf's targets
-//    keep their parallel result, which the merges before them did not change.
+//  * epsh (MEpsilonFast.cpp:175-212) runs with the vortices' (epsilon.hip).
 //  * process_all_lists on the hRange and sRange targets (MConvectiveFast.cpp:
 //    87-110): FP64 near sum over the near leaves' vortices plus the leaf's
 //    Taylor far terms, one wave per target.
@@ -48,149 +41,6 @@ constexpr double kRemoveEps = 1e-10;   // MFlowmove.hpp:8
 inline int nblocks(int64_t n, int b = kBlock) { return (int)std::max<int64_t>(1, (n + b - 1) / b); }
 
 __device__ inline double sgn(double x) { return (x > 0) ? 1 : ((x < 0) ? -1 : 0); }
-
-// ------------------------------------------------------------------ epsh --
-
-// Two nearest under the order (d^2, index): the reference keeps the first
-// found on ties, and the near leaves' heat ranges come in increasing index
-// order.
-struct Near2 {
-    double d1, d2;
-    int i1, i2;
-};
-
-__device__ inline bool before(double d, int j, double dc, int ic) { return d < dc || (d == dc && ic >= 0 && j < ic); }
-
-__device__ inline void near2_add(Near2& t, double d, int j) {
-    if (before(d, j, t.d1, t.i1)) {
-        t.d2 = t.d1;
-        t.i2 = t.i1;
-        t.d1 = d;
-        t.i1 = j;
-    } else if (before(d, j, t.d2, t.i2)) {
-        t.d2 = d;
-        t.i2 = j;
-    }
-}
-
-// The wave's two nearest heat particles (g != 0, not j itself) to (px, py)
-// among the heat ranges of leaf l's near leaves; every lane gets the result.
-__device__ Near2 wave_near2(const TreeDev& T, const double* hx, const double* hy, const double* hg, int l, int j,
-                            double px, double py) {
-    Near2 t{DBL_MAX, DBL_MAX, -1, -1};
-    for (int64_t e = T.near_off[l]; e < T.near_off[l + 1]; e++) {
-        const int M = T.near_list[e];
-        const int k1 = T.h1[M] - T.hbase;
-        for (int k = T.h0[M] - T.hbase + lane_id(); k < k1; k += kWave) {
-            if (k == j || hg[k] == 0) continue;
-            const double dx = px - hx[k], dy = py - hy[k];
-            near2_add(t, dx * dx + dy * dy, k);
-        }
-    }
-    for (int o = kWave / 2; o > 0; o >>= 1) {
-        Near2 u;
-        u.d1 = __shfl_xor(t.d1, o, kWave);
-        u.d2 = __shfl_xor(t.d2, o, kWave);
-        u.i1 = __shfl_xor(t.i1, o, kWave);
-        u.i2 = __shfl_xor(t.i2, o, kWave);
-        if (u.i1 >= 0) near2_add(t, u.d1, u.i1);
-        if (u.i2 >= 0) near2_add(t, u.d2, u.i2);
-    }
-    return t;
-}
-
-// epsh's value for a target whose search found t and that does not merge:
-// DBL_MIN without candidates, sqrt(d1) with one, sqrt(d2) otherwise.
-__device__ inline double epsh_value(const Near2& t) {
-    if (t.i1 < 0) return DBL_MIN;
-    if (t.i2 < 0) return sqrt(t.d1);
-    return sqrt(t.d2);
-}
-
-// Parallel pass, one wave per heat particle.  res = NaN marks "keep _1_eps"
-// (g = 0) or "to be decided by the sequential pass" (flagged).
-__global__ void k_heat_eps(TreeDev T, const double* hx, const double* hy, const double* hg, int64_t nh,
-                           const double* crit, double* res, uint8_t* flag, int32_t* counters) {
-    const int64_t j = (int64_t)blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
-    if (j >= nh) return;
-    if (hg[j] == 0) {
-        if (lane_id() == 0) {
-            res[j] = __builtin_nan("");
-            flag[j] = 0;
-        }
-        return;
-    }
-    const int l = T.vleaf[T.hbase + j];
-    const Near2 t = wave_near2(T, hx, hy, hg, l, (int)j, hx[j], hy[j]);
-    if (lane_id() != 0) return;
-    const bool merge = t.i1 >= 0 && t.i2 >= 0 && t.d1 < crit[l];
-    flag[j] = merge ? 1 : 0;
-    res[j] = merge ? __builtin_nan("") : epsh_value(t);
-    if (merge) atomicAdd(&counters[0], 1);
-}
-
-// Sequential pass (one wave): the reference's order, leaf by leaf (DFS),
-// target by target, for the leaves that can differ from the parallel pass.
-__global__ __launch_bounds__(kWave) void k_heat_eps_seq(TreeDev T, double* hx, double* hy, double* hg,
-                                                        const double* crit, double* res, const uint8_t* flag,
-                                                        uint8_t* dirty, int32_t* counters) {
-    const int lane = lane_id();
-    int merged = 0;
-    for (int l = 0; l < T.nleaf; l++) {
-        const int L = T.leaf_node[l];
-        const int jb = T.h0[L] - T.hbase, je = T.h1[L] - T.hbase;
-        if (jb == je) continue;
-        bool need = false;
-        for (int j = jb + lane; j < je; j += kWave) need = need || flag[j];
-        for (int64_t e = T.near_off[l] + lane; e < T.near_off[l + 1]; e += kWave)
-            need = need || dirty[T.leaf_rank[T.near_list[e]]];
-        if (!__ballot(need)) continue;
-        for (int j = jb; j < je; j++) {
-            if (hg[j] == 0) {
-                if (lane == 0) res[j] = __builtin_nan("");
-                continue;
-            }
-            Near2 t = wave_near2(T, hx, hy, hg, l, j, hx[j], hy[j]);
-            if (t.i1 >= 0 && t.i2 >= 0 && t.d1 < crit[l]) {
-                // MergeVortexes (MEpsilonFast.cpp:111-126), then epsh without merging
-                if (lane == 0) {
-                    const int k = t.i1;
-                    const double ga = hg[j], gb = hg[k];
-                    if (sgn(ga) == sgn(gb)) {
-                        const double inv = 1. / (ga + gb);
-                        const double nx = (hx[j] * ga + hx[k] * gb) * inv;
-                        const double ny = (hy[j] * ga + hy[k] * gb) * inv;
-                        hx[j] = nx;
-                        hy[j] = ny;
-                    } else if (fabs(ga) < fabs(gb)) {
-                        hx[j] = hx[k];
-                        hy[j] = hy[k];
-                    }
-                    hg[j] = ga + gb;
-                    hg[k] = 0;
-                    dirty[l] = 1;
-                    dirty[T.vleaf[T.hbase + k]] = 1;
-                }
-                merged++;
-                __threadfence();   // lane 0's stores, seen by every lane's loads
-                __builtin_amdgcn_wave_barrier();
-                t = wave_near2(T, hx, hy, hg, l, j, hx[j], hy[j]);
-            }
-            if (lane == 0) res[j] = epsh_value(t);
-        }
-    }
-    if (lane == 0) counters[1] = merged;
-}
-
-// _1_eps = 1 / max(eps, floor) (MEpsilonFast.cpp:55-60); NaN keeps _1_eps.
-__global__ void k_heat_eps_apply(TreeDev T, const double* res, const double* restr, double* hie, int64_t nh) {
-    const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= nh) return;
-    const double e = res[j];
-    if (isnan(e)) return;
-    const double r = restr[T.vleaf[T.hbase + j]];
-    hie[j] = 1.0 / ((e < r) ? r : e);   // std::max(e, r)
-}
 
 // ------------------------------------------------------------ convective --
 
@@ -567,35 +417,6 @@ __global__ void k_leaf_lists(TreeDev T, int32_t* out) {
     out[4 * l + 1] = T.h1[L] - T.hbase;
     out[4 * l + 2] = T.s0[L] - T.sbase;
     out[4 * l + 3] = T.s1[L] - T.sbase;
-}
-
-int heat_epsilon(Ctx& c, int merge) {
-    const int64_t nh = c.heat.n;
-    if (nh == 0) return 0;
-    const TreeDev T = tree_dev(c.t);
-    hipStream_t s = c.stream;
-    c.hres.grow(nh + 1);
-    c.hflag.grow(nh + 1);
-    c.iscratch4.grow(4);
-    int32_t* counters = c.iscratch4.p;
-    hipLaunchKernelGGL(k_fill_i32v, dim3(1), dim3(64), 0, s, counters, (int64_t)4, 0);
-    hipLaunchKernelGGL(k_heat_eps, dim3(nblocks(nh, kWavesPerBlock)), dim3(kBlock), 0, s, T, c.heat.x.p, c.heat.y.p,
-                       c.heat.g.p, nh, (const double*)c.leaf_crit.p, c.hres.p, c.hflag.p, counters);
-    int32_t hc[2] = {0, 0};
-    VVHD_HIP(hipMemcpyAsync(hc, counters, 8, hipMemcpyDeviceToHost, s));
-    VVHD_HIP(hipStreamSynchronize(s));
-    if (hc[0] > 0 && merge) {
-        c.hdirty.grow(T.nleaf + 1);
-        VVHD_HIP(hipMemsetAsync(c.hdirty.p, 0, (size_t)T.nleaf + 1, s));
-        hipLaunchKernelGGL(k_heat_eps_seq, dim3(1), dim3(kWave), 0, s, T, c.heat.x.p, c.heat.y.p, c.heat.g.p,
-                           (const double*)c.leaf_crit.p, c.hres.p, (const uint8_t*)c.hflag.p, c.hdirty.p, counters);
-        VVHD_HIP(hipMemcpyAsync(hc, counters, 8, hipMemcpyDeviceToHost, s));
-    }
-    hipLaunchKernelGGL(k_heat_eps_apply, dim3(nblocks(nh)), dim3(kBlock), 0, s, T, (const double*)c.hres.p,
-                       (const double*)c.leaf_restr.p, c.heat.ie.p, nh);
-    VVHD_HIP(hipStreamSynchronize(s));
-    VVHD_HIP(hipGetLastError());
-    return hc[0] > 0 && merge ? hc[1] : 0;
 }
 
 void passive_convective(Ctx& c, const double4* taylor, double inf_x, double inf_y) {
