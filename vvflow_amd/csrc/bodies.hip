@@ -2,12 +2,13 @@
 // and the FP64 boundary-condition system, on the device.
 //
 //  * TBody::doUpdateSegments / doFillProperties (TBody.cpp:200-215, 283-343)
-//    and TBody::move (:179-198): one thread per body, sequential in segment
-//    order, so every FP64 quantity rounds as in the reference.
+//    and TBody::move (:179-198): one block per body, sums in segment order,
+//    so every FP64 quantity rounds as in the reference.
 //  * MFlowmove::move_and_clean (MFlowmove.cpp:11-215) for rigid bodies
-//    without collisions: two passes (k_fm_count, k_fm_scatter) advect, flag
-//    |g| < 1e-10 and in-body vortices (TBody::isPointInvalid, TBody.cpp:
-//    217-281) and compact the survivors stably; then the bodies' dead force,
+//    without collisions: the vortices that end in a body (TBody::
+//    isPointInvalid, TBody.cpp:217-281) are found first, then two passes
+//    (k_fm_count, k_fm_scatter) advect, flag |g| < 1e-10 and those, and
+//    compact the survivors stably; then the bodies' dead force,
 //    moment and circulation accumulated in vortex order and the zero/slip
 //    segment loop.
 //  * MFlowmove::vortex_shed (MFlowmove.cpp:217-235): appended behind the
@@ -49,11 +50,45 @@ __device__ inline double dot2(double ax, double ay, double bx, double by) { retu
 
 // ------------------------------------------------------------ body geometry
 
+// The kernels over a body's segments run one block per body: the terms of a
+// chunk of segments are computed by all threads and staged in LDS, then one
+// lane per sum adds them in segment order, so every FP64 quantity rounds as
+// in the reference.  One thread per body waited for each segment's loads in
+// turn (290-410 us for 350-500 segments; 5-12 us so).
+constexpr int kBodyBlock = 256;
+constexpr int kBodyChunk = 512;
+
+// Q running sums over segments 0..n-1 of terms term(q, k), added in order by
+// lane q of the block; acc holds them in shared memory, set by the caller
+// (barrier before and after).  sh: Q x kBodyChunk.
+template <int Q, typename Term>
+__device__ inline void ordered_sums(int n, double (*sh)[kBodyChunk], double* acc, Term term) {
+    const int t = threadIdx.x;
+    for (int k0 = 0; k0 < n; k0 += kBodyChunk) {
+        const int m = min(kBodyChunk, n - k0);
+        for (int k = t; k < m; k += kBodyBlock) {
+            double v[Q];
+            term(k0 + k, v);
+            for (int q = 0; q < Q; q++) sh[q][k] = v[q];
+        }
+        __syncthreads();
+        if (t < Q) {
+            double a = acc[t];
+            const double* v = sh[t];
+#pragma unroll 8
+            for (int k = 0; k < m; k++) a += v[k];
+            acc[t] = a;
+        }
+        __syncthreads();
+    }
+}
+
 // doUpdateSegments + doFillProperties of one body; geo receives the
 // bounding disc radius squared and the bounding box used by isPointInvalid.
-__device__ void body_properties(vvhd_body& B, vvhd_seg* segs, double* geo) {
-    const int f = B.first_seg, n = B.nseg;
-    for (int k = 0; k < n; k++) {
+// Subtracted terms are added with their sign turned, which rounds the same.
+__device__ void body_properties(vvhd_body& B, vvhd_seg* segs, double* geo, double (*sh)[kBodyChunk], double* acc) {
+    const int f = B.first_seg, n = B.nseg, t = threadIdx.x;
+    for (int k = t; k < n; k += kBodyBlock) {
         vvhd_seg& s = segs[f + k];
         const vvhd_seg& nx = segs[f + (k + 1) % n];
         s.dlx = nx.cx - s.cx;
@@ -62,79 +97,91 @@ __device__ void body_properties(vvhd_body& B, vvhd_seg* segs, double* geo) {
         s.x = (nx.cx + s.cx) * 0.5;
         s.y = (nx.cy + s.cy) * 0.5;
     }
-    double slen = 0, area = 0;
-    for (int k = 0; k < n; k++) {
+    if (t < 5) acc[t] = 0;
+    __threadfence_block();
+    __syncthreads();
+    ordered_sums<2>(n, sh, acc, [&](int k, double* v) {
         const vvhd_seg& s = segs[f + k];
-        slen += sqrt(s.dlx * s.dlx + s.dly * s.dly);
-        area += s.y * s.dlx;
-    }
+        v[0] = sqrt(s.dlx * s.dlx + s.dly * s.dly);
+        v[1] = s.y * s.dlx;
+    });
+    const double slen = acc[0], area = acc[1];
+    __syncthreads();
+    if (t < 5) acc[t] = 0;
+    __syncthreads();
     double cx, cy, moi;
     if (area == 0) {
-        double Lx = 0., Ly = 0.;
-        for (int k = 0; k < n; k++) {
+        ordered_sums<2>(n, sh, acc, [&](int k, double* v) {
             const vvhd_seg& s = segs[f + k];
             const double a = sqrt(s.dlx * s.dlx + s.dly * s.dly);
-            Lx += s.x * a;
-            Ly += s.y * a;
-        }
+            v[0] = s.x * a;
+            v[1] = s.y * a;
+        });
         const double inv = 1. / slen;
-        cx = Lx * inv;
-        cy = Ly * inv;
+        cx = acc[0] * inv;
+        cy = acc[1] * inv;
         moi = 0.;
     } else {
-        double Sx = 0., Sy = 0., m12 = 0.;
-        for (int k = 0; k < n; k++) {
+        ordered_sums<3>(n, sh, acc, [&](int k, double* v) {
             const vvhd_seg& s = segs[f + k];
             const vvhd_seg& nx = segs[f + (k + 1) % n];
             const double cr = dot2(-s.cy, s.cx, nx.cx, nx.cy);
-            Sx -= s.x * cr;
-            Sy -= s.y * cr;
-            m12 -= (dot2(s.cx, s.cy, s.cx, s.cy) + dot2(s.cx, s.cy, nx.cx, nx.cy) + dot2(nx.cx, nx.cy, nx.cx, nx.cy)) *
-                   cr;
-        }
+            v[0] = -(s.x * cr);
+            v[1] = -(s.y * cr);
+            v[2] = -((dot2(s.cx, s.cy, s.cx, s.cy) + dot2(s.cx, s.cy, nx.cx, nx.cy) + dot2(nx.cx, nx.cy, nx.cx, nx.cy)) *
+                     cr);
+        });
         const double inv = 1. / (3 * area);
-        cx = Sx * inv;
-        cy = Sy * inv;
-        moi = m12 / 12. - area * (cx * cx + cy * cy);
+        cx = acc[0] * inv;
+        cy = acc[1] * inv;
+        moi = acc[2] / 12. - area * (cx * cx + cy * cy);
     }
-    B.slen = slen;
-    B.area = area;
-    B.cofm[0] = cx;
-    B.cofm[1] = cy;
-    B.moi_cofm = moi;
-    double r2max = 0, blx = INFINITY, bly = INFINITY, trx = -INFINITY, try_ = -INFINITY;
-    for (int k = 0; k < n; k++) {
+    __syncthreads();
+    double v[5] = {0, INFINITY, INFINITY, -INFINITY, -INFINITY};   // r2max, box
+    for (int k = t; k < n; k += kBodyBlock) {
         const vvhd_seg& s = segs[f + k];
         const double r2 = (s.cx - cx) * (s.cx - cx) + (s.cy - cy) * (s.cy - cy);
-        if (r2 > r2max) r2max = r2;
-        if (s.cx > trx) trx = s.cx;
-        if (s.cy > try_) try_ = s.cy;
-        if (s.cx < blx) blx = s.cx;
-        if (s.cy < bly) bly = s.cy;
+        if (r2 > v[0]) v[0] = r2;
+        if (s.cx < v[1]) v[1] = s.cx;
+        if (s.cy < v[2]) v[2] = s.cy;
+        if (s.cx > v[3]) v[3] = s.cx;
+        if (s.cy > v[4]) v[4] = s.cy;
     }
-    geo[0] = r2max;
-    geo[1] = blx;
-    geo[2] = bly;
-    geo[3] = trx;
-    geo[4] = try_;
+    for (int q = 0; q < 5; q++) sh[q][t] = v[q];
+    __syncthreads();
+    if (t < 5) {
+        double r = sh[t][0];
+        for (int k = 1; k < kBodyBlock; k++) {
+            const double u = sh[t][k];
+            if (t == 1 || t == 2 ? u < r : u > r) r = u;
+        }
+        geo[t] = r;
+    }
+    if (t == 0) {
+        B.slen = slen;
+        B.area = area;
+        B.cofm[0] = cx;
+        B.cofm[1] = cy;
+        B.moi_cofm = moi;
+    }
 }
 
-__global__ void k_body_properties(vvhd_body* bodies, int nbody, vvhd_seg* segs, double* geo) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b < nbody) body_properties(bodies[b], segs, geo + 5 * b);
+__global__ __launch_bounds__(kBodyBlock) void k_body_properties(vvhd_body* bodies, vvhd_seg* segs, double* geo) {
+    __shared__ double sh[5][kBodyChunk], acc[5];
+    body_properties(bodies[blockIdx.x], segs, geo + 5 * blockIdx.x, sh, acc);
 }
 
 // TBody::move for a body with no prescribed motion, moved by the speed of
 // the last solution (TBody.cpp:179-198, MFlowmove.cpp:200-246).
-__global__ void k_body_move(vvhd_body* bodies, int nbody, vvhd_seg* segs, double* geo, double dt) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nbody) return;
+__global__ __launch_bounds__(kBodyBlock) void k_body_move(vvhd_body* bodies, vvhd_seg* segs, double* geo, double dt) {
+    __shared__ double sh[5][kBodyChunk], acc[5];
+    const int b = blockIdx.x;
     vvhd_body& B = bodies[b];
     const double dH[3] = {0. * dt, 0. * dt, 0. * dt};
     const double dB[3] = {B.speed_slae[0] * dt, B.speed_slae[1] * dt, B.speed_slae[2] * dt};
     const double ax = B.holder[0] + B.dpos[0], ay = B.holder[1] + B.dpos[1];
     const double cs = cos(dB[2]), sn = sin(dB[2]);
-    for (int k = 0; k < B.nseg; k++) {
+    for (int k = threadIdx.x; k < B.nseg; k += kBodyBlock) {
         vvhd_seg& s = segs[B.first_seg + k];
         const double drx = s.cx - ax, dry = s.cy - ay;
         const double nx = ax + dB[0] + drx * cs + (-dry) * sn;
@@ -142,12 +189,15 @@ __global__ void k_body_move(vvhd_body* bodies, int nbody, vvhd_seg* segs, double
         s.cx = nx;
         s.cy = ny;
     }
-    for (int i = 0; i < 3; i++) {
-        B.holder[i] += dH[i];
-        B.dpos[i] += dB[i] - dH[i];
-        B.speed_slae_prev[i] = B.speed_slae[i];
-    }
-    body_properties(B, segs, geo + 5 * b);
+    __threadfence_block();
+    __syncthreads();
+    if (threadIdx.x == 0)
+        for (int i = 0; i < 3; i++) {
+            B.holder[i] += dH[i];
+            B.dpos[i] += dB[i] - dH[i];
+            B.speed_slae_prev[i] = B.speed_slae[i];
+        }
+    body_properties(B, segs, geo + 5 * b, sh, acc);
 }
 
 __device__ inline int body_of_seg(const vvhd_body* bodies, int nbody, int s) {
@@ -175,7 +225,7 @@ struct FmArgs {
     const double *x, *y, *vx, *vy, *g, *ie;
     int64_t n;
     double dt;
-    int remove;
+    const int32_t* seg;   // per vortex: the segment it is removed at, or -1 (null: none is)
     const vvhd_body* bodies;
     int nbody;
     const vvhd_seg* segs;
@@ -200,6 +250,55 @@ __device__ inline int sim_of(const int64_t* sim_off, int nsim, int64_t i) {
     return lo;
 }
 
+// Which vortices end inside a body (only with bodies and removal): seg[i] the
+// nearest segment, or -1.  k_fm_inside tests every moved vortex against the
+// bodies' boxes and discs and lists the ones that need the contour test;
+// k_fm_contour gives each of those a wave, whose lanes share the segments.
+// One thread per vortex and contour (in the counting pass and again in the
+// scattering pass) took 2 x 310 us for 3k vortices and 350 segments.
+__global__ void k_fm_inside(FmArgs A, int32_t* seg, int32_t* cand, int32_t* ncand) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    bool test = false;
+    if (i < A.n) {
+        seg[i] = -1;
+        if (!(fabs(A.g[i]) < kRemoveEps)) {
+            const double px = A.x[i] + A.vx[i] * A.dt, py = A.y[i] + A.vy[i] * A.dt;
+            int b0 = 0, b1 = A.nbody;
+            if (A.nsim > 1) {
+                const int sm = sim_of(A.sim_off, A.nsim, i);
+                b0 = A.sim_body[sm];
+                b1 = A.sim_body[sm + 1];
+            }
+            for (int b = b0; b < b1 && !test; b++) test = may_be_invalid(A.bodies[b], A.geo + 5 * b, px, py);
+        }
+    }
+    const uint64_t m = __ballot(test);
+    if (!m) return;
+    int at = 0;
+    if (lane_id() == 0) at = atomicAdd(ncand, __popcll(m));
+    at = __shfl(at, 0, kWave);
+    if (test) cand[at + __popcll(m & ((1ull << lane_id()) - 1))] = (int32_t)i;
+}
+
+__global__ __launch_bounds__(kFmBlock) void k_fm_contour(FmArgs A, int32_t* seg, const int32_t* cand,
+                                                         const int32_t* ncand) {
+    const int nc = *ncand;
+    for (int c = blockIdx.x * kFmWaves + threadIdx.x / kWave; c < nc; c += gridDim.x * kFmWaves) {
+        const int64_t i = cand[c];
+        const double px = A.x[i] + A.vx[i] * A.dt, py = A.y[i] + A.vy[i] * A.dt;
+        int b0 = 0, b1 = A.nbody;
+        if (A.nsim > 1) {
+            const int sm = sim_of(A.sim_off, A.nsim, i);
+            b0 = A.sim_body[sm];
+            b1 = A.sim_body[sm + 1];
+        }
+        int at = -1;
+        for (int b = b0; b < b1 && at < 0; b++)
+            at = wave_point_invalid(A.bodies[b], A.segs, A.geo + 5 * b, px, py);
+        if (at >= 0 && lane_id() == 0) seg[i] = at;
+    }
+}
+
 // Moved position and removal class of vortex i: 1 kept, 2 removed in a body
 // (segment in *bs), 0 removed for |g| < remove_eps or past the list.
 __device__ inline int fm_classify(const FmArgs& A, int64_t i, double& px, double& py, int& bs) {
@@ -208,21 +307,8 @@ __device__ inline int fm_classify(const FmArgs& A, int64_t i, double& px, double
     px = A.x[i] + A.vx[i] * A.dt;
     py = A.y[i] + A.vy[i] * A.dt;
     if (fabs(A.g[i]) < kRemoveEps) return 0;
-    int b0 = 0, b1 = A.nbody;
-    if (A.nsim > 1) {
-        const int sm = sim_of(A.sim_off, A.nsim, i);
-        b0 = A.sim_body[sm];
-        b1 = A.sim_body[sm + 1];
-    }
-    if (A.remove)
-        for (int b = b0; b < b1; b++) {
-            const int sgi = point_invalid(A.bodies[b], A.segs, A.geo + 5 * b, px, py);
-            if (sgi >= 0) {
-                bs = sgi;
-                return 2;
-            }
-        }
-    return 1;
+    if (A.seg) bs = A.seg[i];
+    return bs >= 0 ? 2 : 1;
 }
 
 __global__ __launch_bounds__(kFmBlock) void k_fm_count(FmArgs A, int32_t* tile_cnt) {
@@ -349,15 +435,18 @@ __global__ void k_fill_u64(uint64_t* p, int64_t n) {
 
 // Dead force, moment and circulation of the removed vortices in vortex order
 // (MFlowmove.cpp:124-144), then the zero/slip segment loop (:205-214).
-// One thread per body: the dead records of its simulation's vortices (a
+// One block per body: the dead records of its simulation's vortices (a
 // contiguous run of the records, in vortex order) whose segment is its own,
 // then its zero and slip segments.  With one simulation the run is every
 // record.  dead_off: per simulation, the records before its first vortex
-// (nullptr: one simulation).
-__global__ void k_dead(vvhd_body* bodies, int nbody, vvhd_seg* segs, const double4* dead, const int32_t* counts,
-                       const int32_t* body_sim, const int32_t* dead_off) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nbody) return;
+// (nullptr: one simulation).  A record or segment that is not the body's, or
+// adds nothing, contributes no addition (not +0: a sum may be -0).
+__global__ __launch_bounds__(kBodyBlock) void k_dead(vvhd_body* bodies, vvhd_seg* segs, const double4* dead,
+                                                     const int32_t* counts, const int32_t* body_sim,
+                                                     const int32_t* dead_off) {
+    __shared__ double sh[4][kBodyChunk];
+    __shared__ int s_seg[kBodyChunk];
+    const int b = blockIdx.x, t = threadIdx.x;
     vvhd_body& B = bodies[b];
     const int f0 = B.first_seg, f1 = B.first_seg + B.nseg;
     int q0 = 0, q1 = counts[1];
@@ -365,29 +454,57 @@ __global__ void k_dead(vvhd_body* bodies, int nbody, vvhd_seg* segs, const doubl
         q0 = dead_off[body_sim[b]];
         q1 = dead_off[body_sim[b] + 1];
     }
-    for (int q = q0; q < q1; q++) {
-        const double4 r = dead[q];
-        const int s = (int)r.w;
-        if (s < f0 || s >= f1) continue;
-        const double gi = r.z, xi = r.x, yi = r.y;
-        B.fdt_dead[0] += (-yi) * gi;
-        B.fdt_dead[1] += xi * gi;
-        const double ax = B.holder[0] + B.dpos[0], ay = B.holder[1] + B.dpos[1];
-        B.fdt_dead[2] += ((xi - ax) * (xi - ax) + (yi - ay) * (yi - ay)) * gi;
-        segs[s].gsum -= gi;
-        B.g_dead += gi;
-    }
     const double ax = B.holder[0] + B.dpos[0], ay = B.holder[1] + B.dpos[1];
-    for (int k = 0; k < B.nseg; k++) {
-        vvhd_seg& s = segs[B.first_seg + k];
-        if (fabs(s.g) < kRemoveEps || s.slip) {
-            B.fdt_dead[0] += (-s.cy) * s.g;
-            B.fdt_dead[1] += s.cx * s.g;
-            B.fdt_dead[2] += ((s.cx - ax) * (s.cx - ax) + (s.cy - ay) * (s.cy - ay)) * s.g;
-            s.gsum -= s.g;
-            B.g_dead += s.g;
+    double acc = t < 3 ? B.fdt_dead[t] : (t == 3 ? B.g_dead : 0);   // lane t < 4 keeps one sum
+    auto add = [&](int m) {
+        __syncthreads();
+        if (t < 4)
+            for (int k = 0; k < m; k++)
+                if (s_seg[k] >= 0) acc += sh[t][k];
+    };
+    for (int r0 = q0; r0 < q1; r0 += kBodyChunk) {
+        const int m = min(kBodyChunk, q1 - r0);
+        for (int k = t; k < m; k += kBodyBlock) {
+            const double4 r = dead[r0 + k];
+            const int s = (int)r.w;
+            const double gi = r.z, xi = r.x, yi = r.y;
+            sh[0][k] = (-yi) * gi;
+            sh[1][k] = xi * gi;
+            sh[2][k] = ((xi - ax) * (xi - ax) + (yi - ay) * (yi - ay)) * gi;
+            sh[3][k] = gi;
+            s_seg[k] = s >= f0 && s < f1 ? s : -1;
         }
+        add(m);
+        for (int s = f0 + t; s < f1; s += kBodyBlock) {   // gsum of every segment, its records in order
+            double gs = segs[s].gsum;
+            bool any = false;
+            for (int k = 0; k < m; k++)
+                if (s_seg[k] == s) {
+                    gs -= sh[3][k];
+                    any = true;
+                }
+            if (any) segs[s].gsum = gs;
+        }
+        __syncthreads();
     }
+    for (int k0 = 0; k0 < B.nseg; k0 += kBodyChunk) {
+        const int m = min(kBodyChunk, B.nseg - k0);
+        for (int k = t; k < m; k += kBodyBlock) {
+            vvhd_seg& s = segs[f0 + k0 + k];
+            const bool on = fabs(s.g) < kRemoveEps || s.slip;
+            s_seg[k] = on ? 0 : -1;
+            if (!on) continue;
+            sh[0][k] = (-s.cy) * s.g;
+            sh[1][k] = s.cx * s.g;
+            sh[2][k] = ((s.cx - ax) * (s.cx - ax) + (s.cy - ay) * (s.cy - ay)) * s.g;
+            sh[3][k] = s.g;
+            s.gsum -= s.g;
+        }
+        add(m);
+        __syncthreads();
+    }
+    if (t < 3) B.fdt_dead[t] = acc;
+    if (t == 3) B.g_dead = acc;
 }
 
 // Per simulation s: the dead records before its first vortex, from the
@@ -463,44 +580,60 @@ __global__ void k_shed_write(const vvhd_seg* segs, int nseg, const int32_t* flag
     ie[w] = 0;
 }
 
-// Space::calc_forces (TSpace.cpp:94-120); fric holds the diffusive friction.
-__global__ void k_calc_forces(vvhd_body* bodies, int nbody, vvhd_seg* segs, const double* fric, double re_one,
-                              double dt, double pr, const double* sim_re, const int32_t* body_sim) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nbody) return;
+// Space::calc_forces (TSpace.cpp:94-120), one block per body; fric holds the
+// diffusive friction.
+__global__ __launch_bounds__(kBodyBlock) void k_calc_forces(vvhd_body* bodies, vvhd_seg* segs, const double* fric,
+                                                            double re_one, double dt, double pr, const double* sim_re,
+                                                            const int32_t* body_sim) {
+    __shared__ double sh[5][kBodyChunk];
+    const int b = blockIdx.x, t = threadIdx.x;
     const double re = sim_re ? sim_re[body_sim[b]] : re_one;   // the body's simulation's Reynolds number
     const double C_NyuDt_Pi = dt / (M_PI * re);
     const double C_Nyu_Pi = 1. / (M_PI * re);
     vvhd_body& B = bodies[b];
-    double tmp = 0;
-    B.friction[0] = B.friction[1] = B.friction[2] = 0;
-    for (int k = 0; k < B.nseg; k++) {
-        vvhd_seg& s = segs[B.first_seg + k];
-        s.fric = fric[B.first_seg + k];
-        const double a = sqrt(s.dlx * s.dlx + s.dly * s.dly);
-        tmp += s.gsum;
-        s.Cp += tmp;
-        s.Fr += s.fric * C_NyuDt_Pi;
-        s.Nu += s.hsum * (re * pr / a);
-        const double c = s.fric * C_Nyu_Pi / a;
-        B.friction[0] -= s.dlx * c;
-        B.friction[1] -= s.dly * c;
-        B.friction[2] -= dot2(-s.y, s.x, s.dlx, s.dly) * c;
-        B.nusselt += s.hsum * (re * pr);
+    double acc = t == 4 ? B.nusselt : 0;   // lane t < 5: running gsum, friction x, y, moment, Nusselt
+    for (int k0 = 0; k0 < B.nseg; k0 += kBodyChunk) {
+        const int m = min(kBodyChunk, B.nseg - k0);
+        for (int k = t; k < m; k += kBodyBlock) {
+            vvhd_seg& s = segs[B.first_seg + k0 + k];
+            const double fr = fric[B.first_seg + k0 + k];
+            s.fric = fr;
+            const double a = sqrt(s.dlx * s.dlx + s.dly * s.dly);
+            s.Fr += fr * C_NyuDt_Pi;
+            s.Nu += s.hsum * (re * pr / a);
+            const double c = fr * C_Nyu_Pi / a;
+            sh[0][k] = s.gsum;
+            sh[1][k] = -(s.dlx * c);
+            sh[2][k] = -(s.dly * c);
+            sh[3][k] = -(dot2(-s.y, s.x, s.dlx, s.dly) * c);
+            sh[4][k] = s.hsum * (re * pr);
+        }
+        __syncthreads();
+        if (t < 5) {
+            double* v = sh[t];
+#pragma unroll 8
+            for (int k = 0; k < m; k++) {
+                acc += v[k];
+                v[k] = acc;
+            }
+        }
+        __syncthreads();
+        for (int k = t; k < m; k += kBodyBlock) segs[B.first_seg + k0 + k].Cp += sh[0][k];
+        __syncthreads();
     }
-    B.nusselt /= dt;
+    if (t >= 1 && t < 4) B.friction[t - 1] = acc;
+    if (t == 4) B.nusselt = acc / dt;
 }
 
 // Space::zero_forces (TSpace.cpp:122-143).
-__global__ void k_zero_forces(vvhd_body* bodies, int nbody, vvhd_seg* segs, double* fric) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nbody) return;
-    vvhd_body& B = bodies[b];
-    for (int k = 0; k < B.nseg; k++) {
+__global__ __launch_bounds__(kBodyBlock) void k_zero_forces(vvhd_body* bodies, vvhd_seg* segs, double* fric) {
+    vvhd_body& B = bodies[blockIdx.x];
+    for (int k = threadIdx.x; k < B.nseg; k += kBodyBlock) {
         vvhd_seg& s = segs[B.first_seg + k];
         s.gsum = s.fric = s.hsum = 0;
         fric[B.first_seg + k] = 0;
     }
+    if (threadIdx.x != 0) return;
     for (int i = 0; i < 3; i++) {
         B.force_hydro[i] = 0;
         B.force_holder[i] = 0;
@@ -689,18 +822,32 @@ __global__ __launch_bounds__(64) void k_slip_rhs(SlaeMap M, TreeDev T, const vvh
 }
 
 // Special-segment rows and the nine body rows (:484-862, :896-975), one
-// thread per system: the steady-circulation rows depend on a counter over
-// the system's bodies.  gsum_all holds each system's vortex circulation.
-__global__ void k_body_rows(SlaeMap M, const vvhd_seg* segs, const double* gsum_all, double inf_g, double dt,
-                            double* A, double* rhs) {
-    const int sys = blockIdx.x * blockDim.x + threadIdx.x;
-    if (sys >= M.nsys) return;
+// block per system whose threads share the segments' cells: the
+// steady-circulation rows depend on a counter over the system's bodies.  gsum_all holds each system's vortex circulation.
+__global__ __launch_bounds__(kBodyBlock) void k_body_rows(SlaeMap M, const vvhd_seg* segs, const double* gsum_all,
+                                                          double inf_g, double dt, double* A, double* rhs_) {
+    const int sys = blockIdx.x, t = threadIdx.x;
     const int n = M.n;
     A += (size_t)sys * n * n;
-    rhs += (size_t)sys * n;
+    rhs_ += (size_t)sys * n;
     gsum_all += sys;
     const int b0 = M.sys_body[sys], b1 = M.sys_body[sys + 1];
-    auto cell = [&](int row, int col) -> double& { return A[(size_t)col * n + row]; };
+    // single cells and right-hand sides are written by thread 0, the cells of
+    // the segments by all threads
+    struct One {
+        double* p;
+        bool on;
+        __device__ void operator=(double v) const {
+            if (on) *p = v;
+        }
+    };
+    auto cell = [&](int row, int col) { return One{A + (size_t)col * n + row, t == 0}; };
+    auto seg_cell = [&](int row, int col) -> double& { return A[(size_t)col * n + row]; };
+    struct Rhs {
+        double* p;
+        bool on;
+        __device__ One operator[](int row) const { return One{p + row, on}; }
+    } const rhs{rhs_, t == 0};
     int once = 0;
     for (int b = b0; b < b1; b++) {
         const vvhd_body& B = M.bodies[b];
@@ -714,12 +861,12 @@ __global__ void k_body_rows(SlaeMap M, const vvhd_seg* segs, const double* gsum_
             } else if (!once++) {   // fillInfSteadyEquationForSegment (:508-522)
                 rhs[row] = -(*gsum_all) - inf_g;
                 for (int jb = b0; jb < b1; jb++) {
-                    for (int m = 0; m < M.bodies[jb].nseg; m++) cell(row, M.base[jb] + m) = 1;
+                    for (int m = t; m < M.bodies[jb].nseg; m += kBodyBlock) seg_cell(row, M.base[jb] + m) = 1;
                     cell(row, M.base[jb] + M.bodies[jb].nseg + 2) = 2 * M.bodies[jb].area;
                 }
             } else {   // fillSteadyEquationForSegment (:494-506)
                 rhs[row] = B.g_dead + 2 * B.area * B.speed_slae_prev[2];
-                for (int m = 0; m < ns; m++) cell(row, base + m) = 1;
+                for (int m = t; m < ns; m += kBodyBlock) seg_cell(row, base + m) = 1;
                 cell(row, cs + 2) = 2 * B.area;
             }
         }
@@ -738,7 +885,7 @@ __global__ void k_body_rows(SlaeMap M, const vvhd_seg* segs, const double* gsum_
         // fillHydroXEquation (:533-562)
         rhs[eq] = +area * _1_dt * sp[0] + area * _1_dt * (-(2 * B.cofm[1] + ry)) * sp[2] + (sp[2] * sp[2]) * area * rx -
                   B.friction_prev[0] + B.fdt_dead[0] * _1_dt;
-        for (int m = 0; m < ns; m++) cell(eq, base + m) = _1_dt * (-segs[B.first_seg + m].cy);
+        for (int m = t; m < ns; m += kBodyBlock) seg_cell(eq, base + m) = _1_dt * (-segs[B.first_seg + m].cy);
         cell(eq, cs + 0) = area * _1_dt;
         cell(eq, cs + 1) = 0;
         cell(eq, cs + 2) = area * _1_dt * (-2 * B.cofm[1] - ry);
@@ -747,7 +894,7 @@ __global__ void k_body_rows(SlaeMap M, const vvhd_seg* segs, const double* gsum_
         // fillHydroYEquation (:564-593)
         rhs[eq] = +area * _1_dt * sp[1] + area * _1_dt * (2 * B.cofm[0] + rx) * sp[2] + (sp[2] * sp[2]) * area * ry -
                   B.friction_prev[1] + B.fdt_dead[1] * _1_dt;
-        for (int m = 0; m < ns; m++) cell(eq, base + m) = _1_dt * (segs[B.first_seg + m].cx);
+        for (int m = t; m < ns; m += kBodyBlock) seg_cell(eq, base + m) = _1_dt * (segs[B.first_seg + m].cx);
         cell(eq, cs + 0) = 0;
         cell(eq, cs + 1) = area * _1_dt;
         cell(eq, cs + 2) = area * _1_dt * (2 * B.cofm[0] + rx);
@@ -759,9 +906,9 @@ __global__ void k_body_rows(SlaeMap M, const vvhd_seg* segs, const double* gsum_
             rhs[eq] = +((-ry) * c * sp[0] + rx * c * sp[1]) + 2 * moi_axis * _1_dt * sp[2] - B.friction_prev[2] +
                       B.fdt_dead[2] * _1_2dt;
         }
-        for (int m = 0; m < ns; m++) {
+        for (int m = t; m < ns; m += kBodyBlock) {
             const vvhd_seg& sm = segs[B.first_seg + m];
-            cell(eq, base + m) = _1_2dt * ((sm.cx - axx) * (sm.cx - axx) + (sm.cy - axy) * (sm.cy - axy));
+            seg_cell(eq, base + m) = _1_2dt * ((sm.cx - axx) * (sm.cx - axx) + (sm.cy - axy) * (sm.cy - axy));
         }
         cell(eq, cs + 0) = area * _1_dt * (-ry);
         cell(eq, cs + 1) = area * _1_dt * (rx);
@@ -837,15 +984,15 @@ __global__ void k_differ(const double* a, const double* b, size_t n, int32_t* di
     if (i < n && __double_as_longlong(a[i]) != __double_as_longlong(b[i])) atomicOr(differ, 1);
 }
 
-__global__ void k_writeback(SlaeMap M, vvhd_body* bodies, vvhd_seg* segs, const double* xsol,
-                            const int32_t* body_sys) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= M.nbody) return;
+__global__ __launch_bounds__(kBodyBlock) void k_writeback(SlaeMap M, vvhd_body* bodies, vvhd_seg* segs,
+                                                          const double* xsol, const int32_t* body_sys) {
+    const int b = blockIdx.x;
     vvhd_body& B = bodies[b];
     const int base = M.base[b];
     xsol += (size_t)body_sys[b] * M.n;
-    for (int k = 0; k < B.nseg; k++) segs[B.first_seg + k].g = xsol[base + k];
-    for (int i = 0; i < 3; i++) {
+    for (int k = threadIdx.x; k < B.nseg; k += kBodyBlock) segs[B.first_seg + k].g = xsol[base + k];
+    if (threadIdx.x < 3) {
+        const int i = threadIdx.x;
         B.speed_slae[i] = xsol[base + B.nseg + i];
         B.force_hydro[i] = xsol[base + B.nseg + 3 + i];
         B.force_holder[i] = xsol[base + B.nseg + 6 + i];
@@ -881,7 +1028,7 @@ void bodies_prepare(Ctx& c) {
     if (!nb) return;
     VVHD_HIP(hipMemcpyAsync(c.bodies_d.p, c.bodies_h.data(), (size_t)nb * sizeof(vvhd_body), hipMemcpyHostToDevice,
                             c.stream));
-    hipLaunchKernelGGL(k_body_properties, dim3(nblocks(nb, 64)), dim3(64), 0, c.stream, c.bodies_d.p, nb, c.segs.p,
+    hipLaunchKernelGGL(k_body_properties, dim3(nb), dim3(kBodyBlock), 0, c.stream, c.bodies_d.p, c.segs.p,
                        c.body_geo.p);
     sync_bodies_to_host(c);
 }
@@ -890,7 +1037,7 @@ void bodies_release(Ctx& c) {
     c.bodies_d.release();
     c.body_geo.release();
     for (auto* b : {&c.slae_A, &c.slae_Acached, &c.slae_LU, &c.slae_b, &c.slae_x}) b->release();
-    for (auto* b : {&c.slae_base, &c.slae_ipiv, &c.slae_info, &c.iscratch4}) b->release();
+    for (auto* b : {&c.slae_base, &c.slae_ipiv, &c.slae_info, &c.iscratch4, &c.fm_seg}) b->release();
     if (c.rocblas) (void)rocblas_destroy_handle((rocblas_handle)c.rocblas);
     c.rocblas = nullptr;
     c.slae_n = -1;
@@ -901,8 +1048,8 @@ void move_and_clean(Ctx& c, int remove, int64_t* cleaned) {
     hipStream_t s = c.stream;
     if (c.nsim > 1) sim_sync(c);   // the device copy of the simulations' ranges
     if (nb)
-        hipLaunchKernelGGL(k_body_move, dim3(nblocks(nb, 64)), dim3(64), 0, s, c.bodies_d.p, nb, c.segs.p,
-                           c.body_geo.p, c.dt);
+        hipLaunchKernelGGL(k_body_move, dim3(nb), dim3(kBodyBlock), 0, s, c.bodies_d.p, c.segs.p, c.body_geo.p,
+                           c.dt);
     const int64_t n = c.n;
     VVHD_CHECK(n < (int64_t(1) << 31), VVHD_EUNSUPPORTED, "move_and_clean: more than 2^31 - 1 vortices");
     const int ntiles = (int)std::max<int64_t>(1, (n + kFmTile - 1) / kFmTile);
@@ -920,8 +1067,18 @@ void move_and_clean(Ctx& c, int remove, int64_t* cleaned) {
             c.iscratch2.grow((size_t)ntiles * kFmTile + 1);
             c.iscratch3.grow((size_t)ntiles * kFmTile + 1);
         }
-        const FmArgs A{c.x.p, c.y.p, c.vx.p, c.vy.p, c.g.p, c.ie.p, n, c.dt, remove, c.bodies_d.p, nb, c.segs.p,
+        const bool inside = remove && nb;
+        if (inside) c.fm_seg.grow(2 * (size_t)n + 1);   // segments, candidates, their number
+        const FmArgs A{c.x.p, c.y.p, c.vx.p, c.vy.p, c.g.p, c.ie.p, n, c.dt,
+                       inside ? c.fm_seg.p : (const int32_t*)nullptr, c.bodies_d.p, nb, c.segs.p,
                        c.body_geo.p, (const int64_t*)c.sim_off.p, (const int32_t*)c.sim_body.p, c.nsim};
+        if (inside) {
+            int32_t* ncand = c.fm_seg.p + 2 * n;
+            VVHD_HIP(hipMemsetAsync(ncand, 0, 4, s));
+            hipLaunchKernelGGL(k_fm_inside, dim3(nblocks(n)), dim3(kBlock), 0, s, A, c.fm_seg.p, c.fm_seg.p + n, ncand);
+            hipLaunchKernelGGL(k_fm_contour, dim3(1024), dim3(kFmBlock), 0, s, A, c.fm_seg.p,
+                               (const int32_t*)(c.fm_seg.p + n), (const int32_t*)ncand);
+        }
         hipLaunchKernelGGL(k_fm_count, dim3(ntiles), dim3(kFmBlock), 0, s, A, tile_cnt);
         hipLaunchKernelGGL(k_fm_scatter, dim3(ntiles), dim3(kFmBlock), 0, s, A, (const int32_t*)tile_cnt, ntiles,
                            c.x2.p, c.y2.p, c.g2.p, c.vx2.p, c.vy2.p, c.ie2.p, dead, counts,
@@ -941,8 +1098,8 @@ void move_and_clean(Ctx& c, int remove, int64_t* cleaned) {
             hipLaunchKernelGGL(k_dead_off, dim3(nblocks(c.nsim + 1)), dim3(kBlock), 0, s, (const int64_t*)c.sim_off.p,
                                c.nsim, (const int32_t*)c.iscratch3.p, (const int32_t*)counts, n, dead_off);
         }
-        hipLaunchKernelGGL(k_dead, dim3(nblocks(nb, 64)), dim3(64), 0, s, c.bodies_d.p, nb, c.segs.p, dead, counts,
-                           body_sim, (const int32_t*)dead_off);
+        hipLaunchKernelGGL(k_dead, dim3(nb), dim3(kBodyBlock), 0, s, c.bodies_d.p, c.segs.p, dead, counts, body_sim,
+                           (const int32_t*)dead_off);
     }
     VVHD_HIP(hipGetLastError());
     VVHD_HIP(hipEventRecord(c.ev[9], s));   // end of the device work of the phase
@@ -1038,8 +1195,8 @@ void calc_forces(Ctx& c) {
         body_sim = c.iscratch3.p;
         VVHD_HIP(hipMemcpyAsync(body_sim, bs.data(), (size_t)nb * 4, hipMemcpyHostToDevice, c.stream));
     }
-    hipLaunchKernelGGL(k_calc_forces, dim3(nblocks(nb, 64)), dim3(64), 0, c.stream, c.bodies_d.p, nb, c.segs.p,
-                       c.fric.p, c.re, c.dt, c.pr, batch ? (const double*)c.sim_re.p : (const double*)nullptr,
+    hipLaunchKernelGGL(k_calc_forces, dim3(nb), dim3(kBodyBlock), 0, c.stream, c.bodies_d.p, c.segs.p, c.fric.p,
+                       c.re, c.dt, c.pr, batch ? (const double*)c.sim_re.p : (const double*)nullptr,
                        (const int32_t*)body_sim);
     sync_bodies_to_host(c);
 }
@@ -1047,8 +1204,7 @@ void calc_forces(Ctx& c) {
 void zero_forces(Ctx& c) {
     const int nb = (int)c.bodies_h.size();
     if (!nb) return;
-    hipLaunchKernelGGL(k_zero_forces, dim3(nblocks(nb, 64)), dim3(64), 0, c.stream, c.bodies_d.p, nb, c.segs.p,
-                       c.fric.p);
+    hipLaunchKernelGGL(k_zero_forces, dim3(nb), dim3(kBodyBlock), 0, c.stream, c.bodies_d.p, c.segs.p, c.fric.p);
     heat_layer_reset(c);
     sync_bodies_to_host(c);
 }
@@ -1098,7 +1254,7 @@ void calc_circulation(Ctx& c, double infx, double infy) {
     hipLaunchKernelGGL(k_slip_rhs, dim3(nseg), dim3(kWave), 0, s, M, tree_dev(c.t), c.segs.p, nseg, c.x.p, c.y.p,
                        c.g.p, c.ie.p, infx, infy, c.slae_A.p, c.slae_b.p);
     hipLaunchKernelGGL(k_gsum, dim3(nsys), dim3(1024), 0, s, c.g.p, (const int64_t*)c.sim_off.p, gsum);
-    hipLaunchKernelGGL(k_body_rows, dim3(nblocks(nsys, 64)), dim3(64), 0, s, M, c.segs.p, (const double*)gsum,
+    hipLaunchKernelGGL(k_body_rows, dim3(nsys), dim3(kBodyBlock), 0, s, M, c.segs.p, (const double*)gsum,
                        c.inf_g, c.dt, c.slae_A.p, c.slae_b.p);
     c.slae_filled = n;
     c.slae_nsys = nsys;
@@ -1145,7 +1301,7 @@ void calc_circulation(Ctx& c, double infx, double infy) {
                                                 c.slae_ipiv.p, (rocblas_stride)n, c.slae_x.p, n, (rocblas_stride)n,
                                                 nsys) == rocblas_status_success,
                VVHD_EHIP, "rocsolver_dgetrs_strided_batched failed");
-    hipLaunchKernelGGL(k_writeback, dim3(nblocks(nb, 64)), dim3(64), 0, s, M, c.bodies_d.p, c.segs.p, c.slae_x.p,
+    hipLaunchKernelGGL(k_writeback, dim3(nb), dim3(kBodyBlock), 0, s, M, c.bodies_d.p, c.segs.p, c.slae_x.p,
                        (const int32_t*)d_body_sys);
     sync_bodies_to_host(c);
 }

@@ -291,6 +291,7 @@ struct Ctx {
     DBuf<double> fric;                       // per segment friction accumulator
     DBuf<int32_t> body_range;                // per body: first segment, count
     DBuf<vvhd_body> bodies_d;                // device copy of the body records
+    DBuf<int32_t> fm_seg;                    // flow-move: in-body segment per vortex, contour-test candidates
     DBuf<double> body_geo;                   // per body: r2max, bbox (blx, bly, trx, try)
 
     // boundary-condition system (column-major, LAPACK convention)

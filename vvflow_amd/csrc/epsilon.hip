@@ -88,48 +88,78 @@ __device__ inline double dist2(double tx, double ty, double sx, double sy) {
 }
 
 // nearestBodySegment (MEpsilonFast.cpp:214-253) for every leaf centre, then
-// the merge criterion and the epsilon floor (:29-47).  The bodies searched
-// are those of the leaf's simulation, [sim_body[s], sim_body[s+1]).
-__global__ void k_leaf_criteria(TreeDev T, const vvhd_seg* segs, const int32_t* body_range, const int32_t* sim_body,
-                                const int32_t* leaf_sim, int merge, double* crit_out, double* restr_out) {
-    const int l = blockIdx.x * blockDim.x + threadIdx.x;
+// the merge criterion and the epsilon floor (:29-47), one wave per leaf.  The
+// bodies searched are those of the leaf's simulation, [sim_body[s],
+// sim_body[s+1]).  Among the segments of the near leaves the reference keeps
+// the first nearest in list order: the lanes take the near entries in turn
+// and the first of equal distances wins.  Without one it walks the bodies'
+// segments, skipping nine after each that is no nearer: the lanes compute 64
+// distances at a time and the walk reads them from the lanes.  (One thread
+// per leaf, every load waiting for the one before: 210-640 us a call.)
+__global__ __launch_bounds__(kBlock) void k_leaf_criteria(TreeDev T, const vvhd_seg* segs, const int32_t* body_range,
+                                                          const int32_t* sim_body, const int32_t* leaf_sim, int merge,
+                                                          double* crit_out, double* restr_out) {
+    const int l = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
     if (l >= T.nleaf) return;
+    const int lane = lane_id();
     const int sim = leaf_sim[l];
     const int b0 = sim_body[sim], b1 = sim_body[sim + 1];
     if (b0 == b1) {   // no segment in the simulation: criterion 0 (or NaN), floor 0
-        crit_out[l] = merge ? 0.0 : __builtin_nan("");
-        restr_out[l] = 0;
+        if (lane == 0) {
+            crit_out[l] = merge ? 0.0 : __builtin_nan("");
+            restr_out[l] = 0;
+        }
         return;
     }
     const int L = T.leaf_node[l];
     const double px = T.nx[L], py = T.ny[L];
     int att = -1;
     double res = DBL_MAX;
-    for (int64_t e = T.near_off[l]; e < T.near_off[l + 1]; e++) {
+    int64_t where = INT64_MAX;   // near entry of the candidate
+    for (int64_t e = T.near_off[l] + lane; e < T.near_off[l + 1]; e += kWave) {
         const int m = T.leaf_rank[T.near_list[e]];
-        for (int64_t q = T.seg_off[m]; q < T.seg_off[m + 1]; q++) {
+        const int64_t q1 = T.seg_off[m + 1];
+        for (int64_t q = T.seg_off[m]; q < q1; q++) {
             const int s = T.seg_list[q];
             const double d2 = dist2(px, py, segs[s].x, segs[s].y);
             if (d2 < res) {
                 res = d2;
                 att = s;
+                where = e;
             }
         }
     }
+    for (int o = kWave / 2; o > 0; o >>= 1) {
+        const double d = __shfl_xor(res, o, kWave);
+        const int a = __shfl_xor(att, o, kWave);
+        const int64_t w = __shfl_xor(where, o, kWave);
+        if (a >= 0 && (d < res || (d == res && w < where))) {
+            res = d;
+            att = a;
+            where = w;
+        }
+    }
     if (att < 0) {
+        res = DBL_MAX;
         for (int b = b0; b < b1; b++) {
             const int f = body_range[2 * b], cnt = body_range[2 * b + 1];
-            for (int k = 0; k < cnt; k++) {
-                const double d2 = dist2(px, py, segs[f + k].x, segs[f + k].y);
-                if (d2 < res) {
-                    res = d2;
-                    att = f + k;
-                } else {
-                    k += 9;   // the reference's "speed up" skip
+            for (int k = 0; k < cnt;) {
+                const int k0 = k, s = f + min(k0 + lane, cnt - 1);
+                const double mine = dist2(px, py, segs[s].x, segs[s].y);
+                while (k < min(k0 + kWave, cnt)) {
+                    const double d2 = __shfl(mine, k - k0, kWave);
+                    if (d2 < res) {
+                        res = d2;
+                        att = f + k;
+                        k++;
+                    } else {
+                        k += 10;   // the reference's "speed up" skip
+                    }
                 }
             }
         }
     }
+    if (lane != 0) return;
     double crit;
     if (merge) {
         if (att >= 0) {
@@ -792,7 +822,7 @@ void epsilon(Ctx& c, int merge, int32_t* nn1_out, int32_t* nn2_out, int32_t* mer
     c.leaf_crit.grow(nl + 1);
     c.leaf_restr.grow(nl + 1);
     VVHD_HIP(hipMemsetAsync(c.ecount.p, 0, 8 * 4, s));
-    hipLaunchKernelGGL(k_leaf_criteria, dim3(nblocks(nl)), dim3(kBlock), 0, s, T, c.segs.p, c.body_range.p,
+    hipLaunchKernelGGL(k_leaf_criteria, dim3(nblocks(nl, kWavesPerBlock)), dim3(kBlock), 0, s, T, c.segs.p, c.body_range.p,
                        (const int32_t*)c.sim_body.p, (const int32_t*)c.t.leaf_sim.p,
                        merge, c.leaf_crit.p, c.leaf_restr.p);
     if (nl > 0)

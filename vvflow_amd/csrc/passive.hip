@@ -156,34 +156,12 @@ __global__ void k_heat_diffusive(TreeDev T, const double* hx, const double* hy, 
 // TBody::isPointInHeatLayer (TBody.cpp:222-233): isPointInContour over the
 // points r + rotl(dl) of the segments, with the body's own box and disc as
 // the pre-test; the nearest segment, or -1.
-__device__ inline int point_in_heat_layer(const vvhd_body& B, const vvhd_seg* segs, const double* geo, double px,
-                                          double py) {
-    bool in = B.area <= 0;
-    if (!in && (px < geo[1] || py < geo[2] || px > geo[3] || py > geo[4] ||
-                (px - B.cofm[0]) * (px - B.cofm[0]) + (py - B.cofm[1]) * (py - B.cofm[1]) > geo[0]))
-        return -1;
-    const int f = B.first_seg, n = B.nseg;
-    for (int i = 0, j = n - 1; i < n; j = i++) {
-        const vvhd_seg& a = segs[f + i];
-        const vvhd_seg& b = segs[f + j];
-        const double vix = a.x + (-a.dly), viy = a.y + a.dlx;
-        const double vjx = b.x + (-b.dly), vjy = b.y + b.dlx;
-        if (((viy < vjy) && (viy < py) && (py <= vjy) && ((vjy - viy) * (px - vix) > (vjx - vix) * (py - viy))) ||
-            ((viy > vjy) && (viy > py) && (py >= vjy) && ((vjy - viy) * (px - vix) < (vjx - vix) * (py - viy))))
-            in = !in;
-    }
-    if (!in) return -1;
-    int best = -1;
-    double bd = DBL_MAX;
-    for (int k = 0; k < n; k++) {
-        const double dx = segs[f + k].x - px, dy = segs[f + k].y - py;
-        const double d2 = dx * dx + dy * dy;
-        if (d2 < bd) {
-            best = f + k;
-            bd = d2;
-        }
-    }
-    return best;
+__device__ inline int wave_in_heat_layer(const vvhd_body& B, const vvhd_seg* segs, const double* geo, double px,
+                                         double py) {
+    return wave_in_contour(B, segs, geo, px, py, [](const vvhd_seg& s, double& x, double& y) {
+        x = s.x + (-s.dly);
+        y = s.y + s.dlx;
+    });
 }
 
 struct PMove {
@@ -201,17 +179,17 @@ struct PMove {
 // (|g| < remove_eps), 1 in a body (seg: nearest segment), 2 in the heat layer
 // of a const_t body (seg: nearest segment), 3 kept.  Positions move in place.
 // Streak particles (heat = false): 1 in a body, 3 kept.
-__global__ void k_passive_classify(PMove A, bool heat, int32_t* cls, int32_t* seg, int32_t* first_in_layer) {
-    const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// One wave per particle: lanes share the contours' segments.
+__global__ __launch_bounds__(kBlock) void k_passive_classify(PMove A, bool heat, int32_t* cls, int32_t* seg,
+                                                             int32_t* first_in_layer) {
+    const int64_t j = (int64_t)blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
     if (j >= A.n) return;
     const double px = A.x[j] + A.vx[j] * A.dt, py = A.y[j] + A.vy[j] * A.dt;
-    A.x[j] = px;
-    A.y[j] = py;
     int c = 3, s = -1;
     if (heat && fabs(A.g[j]) < kRemoveEps) c = 0;
     if (c == 3)
         for (int b = 0; b < A.nbody; b++) {
-            s = point_invalid(A.bodies[b], A.segs, A.geo + 5 * b, px, py);
+            s = wave_point_invalid(A.bodies[b], A.segs, A.geo + 5 * b, px, py);
             if (s >= 0) {
                 c = 1;
                 break;
@@ -219,17 +197,20 @@ __global__ void k_passive_classify(PMove A, bool heat, int32_t* cls, int32_t* se
         }
     if (heat && c == 3) {
         for (int b = 0; b < A.nbody; b++) {
-            const int q = point_in_heat_layer(A.bodies[b], A.segs, A.geo + 5 * b, px, py);
+            const int q = wave_in_heat_layer(A.bodies[b], A.segs, A.geo + 5 * b, px, py);
             if (q >= 0) {
                 if (A.cond[b] == 2) {
                     c = 2;
                     s = q;
-                    atomicMin(&first_in_layer[q], (int32_t)j);
+                    if (lane_id() == 0) atomicMin(&first_in_layer[q], (int32_t)j);
                 }
                 break;
             }
         }
     }
+    if (lane_id() != 0) return;
+    A.x[j] = px;
+    A.y[j] = py;
     cls[j] = c;
     seg[j] = s;
 }
@@ -461,7 +442,7 @@ void passive_move_and_clean(Ctx& c) {
                                      (int64_t)nseg, INT32_MAX);
         const PMove A{L.x.p, L.y.p, L.g.p, L.vx.p, L.vy.p, n, c.dt, c.bodies_d.p, nb, c.segs.p, c.body_geo.p,
                       c.heat_cond.p};
-        hipLaunchKernelGGL(k_passive_classify, dim3(nblocks(n)), dim3(kBlock), 0, s, A, q == 0, c.iscratch0.p,
+        hipLaunchKernelGGL(k_passive_classify, dim3(nblocks(n, kWavesPerBlock)), dim3(kBlock), 0, s, A, q == 0, c.iscratch0.p,
                            c.iscratch1.p, c.iscratch4.p);
         hipLaunchKernelGGL(k_passive_keep, dim3(nblocks(n + 1)), dim3(kBlock), 0, s, n, (const int32_t*)c.iscratch0.p,
                            (const int32_t*)c.iscratch1.p, (const int32_t*)c.iscratch4.p,
