@@ -17,10 +17,12 @@
 //  * MConvectiveFast::calc_circulation (MConvectiveFast.cpp:235-273, fill
 //    :459-1017): FP64 fill of the column-major matrix and right-hand side
 //    (influence cells one thread each; the vortex influence on a slip row one
-//    wave per segment, summed in the reference's order; body rows one
-//    thread), LU factorisation and solve with rocSOLVER.  The factors are
-//    reused while the matrix is bit-identical to the factorised one, the
-//    condition under which the reference reuses its inverse
+//    wave per segment, summed in the reference's order; body rows one block
+//    per system).  The solve uses that the system of rigid bodies is block
+//    triangular: the speeds are given, the segments' circulations follow from
+//    the segment rows alone (the core), the forces from the circulations.  The
+//    core's inverse is kept while the core is bit-identical to the inverted
+//    one, the condition under which the reference reuses its inverse
 //    (TMatrix.cpp:225-259).
 
 #include "api.hpp"
@@ -946,18 +948,18 @@ __global__ __launch_bounds__(kBodyBlock) void k_body_rows(SlaeMap M, const vvhd_
 
 // Total vortex circulation (Space::gsum, TSpace.hpp:93-99) of every
 // simulation, one block each over its range [sim_off[s], sim_off[s + 1]):
-// per-thread Neumaier sums over contiguous chunks combined in a fixed tree,
-// so the result is deterministic and at least as accurate as the serial sum.
+// per-thread Neumaier sums over every 1024th vortex (coalesced loads)
+// combined in a fixed tree, so the result is deterministic and at least as
+// accurate as the serial sum.
 __global__ __launch_bounds__(1024) void k_gsum(const double* g, const int64_t* sim_off, double* out) {
     __shared__ double ss[1024], sc[1024];
     const int t = threadIdx.x;
     g += sim_off[blockIdx.x];
     const int64_t n = sim_off[blockIdx.x + 1] - sim_off[blockIdx.x];
     out += blockIdx.x;
-    const int64_t chunk = (n + 1023) / 1024;
-    const int64_t a = min(n, (int64_t)t * chunk), b = min(n, a + chunk);
     double s = 0, c = 0;
-    for (int64_t i = a; i < b; i++) {
+#pragma unroll 8
+    for (int64_t i = t; i < n; i += 1024) {
         const double v = g[i];
         const double u = s + v;
         c += (fabs(s) >= fabs(v)) ? ((s - u) + v) : ((v - u) + s);
@@ -979,24 +981,137 @@ __global__ __launch_bounds__(1024) void k_gsum(const double* g, const int64_t* s
     if (t == 0) *out = ss[0] + sc[0];
 }
 
-__global__ void k_differ(const double* a, const double* b, size_t n, int32_t* differ) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n && __double_as_longlong(a[i]) != __double_as_longlong(b[i])) atomicOr(differ, 1);
+// The core of every system: the rows and columns of its segments (core index
+// = the segment's number within the system), row-major, order nc (the most
+// segments of a system: a system of the same order with more bodies has fewer,
+// its core continues as the unit matrix), with what the solve reads of it.
+struct CoreMap {
+    SlaeMap M;
+    int nc;
+    double *A, *inv;        // nsys x nc x nc
+    double *b, *x, *r;      // nsys x nc
+};
+
+// Segments of a system.
+__device__ inline int core_size(const SlaeMap& M, int sys) {
+    const vvhd_body &a = M.bodies[M.sys_body[sys]], &z = M.bodies[M.sys_body[sys + 1] - 1];
+    return z.first_seg + z.nseg - a.first_seg;
 }
 
-__global__ __launch_bounds__(kBodyBlock) void k_writeback(SlaeMap M, vvhd_body* bodies, vvhd_seg* segs,
-                                                          const double* xsol, const int32_t* body_sys) {
-    const int b = blockIdx.x;
-    vvhd_body& B = bodies[b];
-    const int base = M.base[b];
-    xsol += (size_t)body_sys[b] * M.n;
-    for (int k = threadIdx.x; k < B.nseg; k += kBodyBlock) segs[B.first_seg + k].g = xsol[base + k];
-    if (threadIdx.x < 3) {
-        const int i = threadIdx.x;
-        B.speed_slae[i] = xsol[base + B.nseg + i];
-        B.force_hydro[i] = xsol[base + B.nseg + 3 + i];
-        B.force_holder[i] = xsol[base + B.nseg + 6 + i];
+// Equation of core index i < core_size.
+__device__ inline int core_eq(const SlaeMap& M, int sys, int i) {
+    const int b0 = M.sys_body[sys], b1 = M.sys_body[sys + 1];
+    const int s = M.bodies[b0].first_seg + i;
+    const int b = body_of_seg_in(M.bodies, b0, b1, s);
+    return M.base[b] + (s - M.bodies[b].first_seg);
+}
+
+// Core from the filled systems (column-major) by 32 x 32 tiles through LDS;
+// *differ is set when a cell is not bit-identical to the one it replaces.
+__global__ __launch_bounds__(kBlock) void k_core_gather(CoreMap C, const double* A, int32_t* differ) {
+    __shared__ double tile[32][33];
+    __shared__ int eqr[32], eqc[32];
+    const int sys = blockIdx.z, n = C.M.n, nc = C.nc;
+    const int r0 = blockIdx.y * 32, c0 = blockIdx.x * 32, tx = threadIdx.x % 32, ty = threadIdx.x / 32;
+    const int ns = core_size(C.M, sys);
+    if (threadIdx.x < 64) {
+        const int q = threadIdx.x % 32, i = (threadIdx.x < 32 ? r0 : c0) + q;
+        (threadIdx.x < 32 ? eqr : eqc)[q] = i < ns ? core_eq(C.M, sys, i) : 0;
     }
+    __syncthreads();
+    A += (size_t)sys * n * n;
+    for (int j = ty; j < 32; j += kBlock / 32)
+        tile[tx][j] = r0 + tx < ns && c0 + j < ns ? A[(size_t)eqc[j] * n + eqr[tx]] : (r0 + tx == c0 + j ? 1. : 0.);
+    __syncthreads();
+    double* out = C.A + (size_t)sys * nc * nc;
+    bool diff = false;
+    for (int j = ty; j < 32; j += kBlock / 32)
+        if (r0 + j < nc && c0 + tx < nc) {
+            double* o = out + (size_t)(r0 + j) * nc + c0 + tx;
+            const double v = tile[j][tx];
+            diff |= __double_as_longlong(*o) != __double_as_longlong(v);
+            *o = v;
+        }
+    if (__ballot(diff) && lane_id() == 0) atomicOr(differ, 1);
+}
+
+// Right-hand side of the core: the given speeds (each speed row holds one 1)
+// taken over.
+__global__ void k_core_rhs(CoreMap C, const double* A, const double* rhs) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, sys = blockIdx.y, n = C.M.n;
+    if (i >= C.nc) return;
+    if (i >= core_size(C.M, sys)) {
+        C.b[(size_t)sys * C.nc + i] = 0;
+        return;
+    }
+    A += (size_t)sys * n * n;
+    rhs += (size_t)sys * n;
+    const int row = core_eq(C.M, sys, i);
+    double v = rhs[row];
+    for (int b = C.M.sys_body[sys]; b < C.M.sys_body[sys + 1]; b++) {
+        const int sc = C.M.base[b] + C.M.bodies[b].nseg;
+        for (int q = 0; q < 3; q++) v -= A[(size_t)(sc + q) * n + row] * rhs[sc + q];
+    }
+    C.b[(size_t)sys * C.nc + i] = v;
+}
+
+// One product with the core or its inverse, a wave per row (the rows stream
+// once: 2 MB at 500 segments, 3 us): x = inv b; r = b - A x; x += inv r.  The
+// residual step makes the solution as accurate as one from the factors.
+// (rocSOLVER's dgetrs: about 35 launches of 8-20 us in a row, 0.4 ms.)
+enum { kMvFirst, kMvResidual, kMvCorrect };
+template <int kMode>
+__global__ __launch_bounds__(kBlock) void k_core_mv(CoreMap C) {
+    const int i = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave, sys = blockIdx.y, nc = C.nc;
+    if (i >= nc) return;
+    const double* m = (kMode == kMvResidual ? C.A : C.inv) + ((size_t)sys * nc + i) * nc;
+    const size_t o = (size_t)sys * nc;
+    const double* v = (kMode == kMvFirst ? C.b : kMode == kMvResidual ? C.x : C.r) + o;
+    double a = 0;
+    for (int j = lane_id(); j < nc; j += kWave) a = __builtin_fma(m[j], v[j], a);
+    a = wave_sum(a);
+    if (lane_id() != 0) return;
+    if (kMode == kMvFirst) C.x[o + i] = a;
+    if (kMode == kMvResidual) C.r[o + i] = C.b[o + i] - a;
+    if (kMode == kMvCorrect) C.x[o + i] += a;
+}
+
+// Circulations from the core, speeds as given, forces from their rows
+// (hydro: cells . (circulations, speeds) - force = rhs; Newton: cells .
+// speeds + hydro force - holder force = rhs), one block per body.
+__global__ __launch_bounds__(kBodyBlock) void k_writeback(CoreMap C, vvhd_body* bodies, vvhd_seg* segs,
+                                                          const double* A, const double* rhs,
+                                                          const int32_t* body_sys) {
+    __shared__ double part[3][kBodyBlock / kWave];
+    const int b = blockIdx.x, t = threadIdx.x, n = C.M.n;
+    vvhd_body& B = bodies[b];
+    const int sys = body_sys[b], base = C.M.base[b], ns = B.nseg;
+    A += (size_t)sys * n * n;
+    rhs += (size_t)sys * n;
+    const double* x = C.x + (size_t)sys * C.nc + (B.first_seg - bodies[C.M.sys_body[sys]].first_seg);
+    const int cs = base + ns, ch = cs + 3, ck = cs + 6;
+    double f[3] = {0, 0, 0};
+    for (int k = t; k < ns; k += kBodyBlock) {
+        const double g = x[k];
+        segs[B.first_seg + k].g = g;
+        for (int q = 0; q < 3; q++) f[q] += A[(size_t)(base + k) * n + ch + q] * g;
+    }
+    for (int q = 0; q < 3; q++) {
+        f[q] = wave_sum(f[q]);
+        if (lane_id() == 0) part[q][t / kWave] = f[q];
+    }
+    __syncthreads();
+    if (t >= 3) return;
+    double h = 0, k = 0;
+    for (int w = 0; w < kBodyBlock / kWave; w++) h += part[t][w];
+    for (int q = 0; q < 3; q++) {
+        h += A[(size_t)(cs + q) * n + ch + t] * rhs[cs + q];
+        k += A[(size_t)(cs + q) * n + ck + t] * rhs[cs + q];
+    }
+    h -= rhs[ch + t];
+    B.speed_slae[t] = rhs[cs + t];
+    B.force_hydro[t] = h;
+    B.force_holder[t] = k + h - rhs[ck + t];
 }
 
 }  // namespace
@@ -1036,7 +1151,7 @@ void bodies_prepare(Ctx& c) {
 void bodies_release(Ctx& c) {
     c.bodies_d.release();
     c.body_geo.release();
-    for (auto* b : {&c.slae_A, &c.slae_Acached, &c.slae_LU, &c.slae_b, &c.slae_x}) b->release();
+    for (auto* b : {&c.slae_A, &c.slae_core, &c.slae_inv, &c.slae_v, &c.slae_b, &c.slae_x}) b->release();
     for (auto* b : {&c.slae_base, &c.slae_ipiv, &c.slae_info, &c.iscratch4, &c.fm_seg}) b->release();
     if (c.rocblas) (void)rocblas_destroy_handle((rocblas_handle)c.rocblas);
     c.rocblas = nullptr;
@@ -1244,11 +1359,11 @@ void calc_circulation(Ctx& c, double infx, double infy) {
     const size_t nn = (size_t)n * n, nall = nn * nsys;
     c.slae_A.grow(nall);
     c.slae_b.grow((size_t)n * nsys + 1);
-    c.slae_x.grow((size_t)n * nsys + nsys + 1);
+    c.slae_x.grow((size_t)nsys + 1);
     VVHD_HIP(hipMemsetAsync(c.slae_A.p, 0, nall * 8, s));
     VVHD_HIP(hipMemsetAsync(c.slae_b.p, 0, ((size_t)n * nsys + 1) * 8, s));
     SlaeMap M{c.bodies_d.p, d_base, nb, n, d_sys_body, c.seg_root.p, nsys, max_segs};
-    double* gsum = c.slae_x.p + (size_t)n * nsys;   // per system, after the solutions
+    double* gsum = c.slae_x.p;   // per system
     hipLaunchKernelGGL(k_slip_cells, dim3(nblocks((int64_t)nseg * max_segs)), dim3(kBlock), 0, s, M, c.segs.p, nseg,
                        c.slae_A.p);
     hipLaunchKernelGGL(k_slip_rhs, dim3(nseg), dim3(kWave), 0, s, M, tree_dev(c.t), c.segs.p, nseg, c.x.p, c.y.p,
@@ -1258,33 +1373,41 @@ void calc_circulation(Ctx& c, double infx, double infy) {
                        c.inf_g, c.dt, c.slae_A.p, c.slae_b.p);
     c.slae_filled = n;
     c.slae_nsys = nsys;
-    bool refactor = !(c.time > 0) || c.slae_n != n || c.slae_nsys_factored != nsys;
+    // the core of each system, and whether its inverse is kept
+    const int nc = max_segs;
+    const size_t cc = (size_t)nc * nc, call = cc * nsys;
+    c.slae_core.grow(call);
+    c.slae_inv.grow(call);
+    c.slae_v.grow(3 * (size_t)nc * nsys);
     c.slae_info.grow((size_t)nsys + 2);
+    const CoreMap C{M, nc, c.slae_core.p, c.slae_inv.p, c.slae_v.p, c.slae_v.p + (size_t)nc * nsys,
+                    c.slae_v.p + 2 * (size_t)nc * nsys};
+    int32_t* d_differ = c.slae_info.p + nsys;
+    VVHD_HIP(hipMemsetAsync(d_differ, 0, 4, s));
+    const int tiles = (nc + 31) / 32;
+    hipLaunchKernelGGL(k_core_gather, dim3(tiles, tiles, nsys), dim3(kBlock), 0, s, C, (const double*)c.slae_A.p,
+                       d_differ);
+    bool refactor = !(c.time > 0) || c.slae_n != nc || c.slae_nsys_factored != nsys;
     if (!refactor) {
-        VVHD_HIP(hipMemsetAsync(c.slae_info.p + nsys, 0, 4, s));
-        hipLaunchKernelGGL(k_differ, dim3(nblocks((int64_t)nall)), dim3(kBlock), 0, s, c.slae_A.p, c.slae_Acached.p,
-                           nall, c.slae_info.p + nsys);
         int32_t differ = 0;
-        VVHD_HIP(hipMemcpyAsync(&differ, c.slae_info.p + nsys, 4, hipMemcpyDeviceToHost, s));
+        VVHD_HIP(hipMemcpyAsync(&differ, d_differ, 4, hipMemcpyDeviceToHost, s));
         VVHD_HIP(hipStreamSynchronize(s));
         refactor = differ != 0;
     }
-    if (!c.rocblas) {
-        rocblas_handle h = nullptr;
-        VVHD_CHECK(rocblas_create_handle(&h) == rocblas_status_success, VVHD_EHIP, "rocblas_create_handle failed");
-        c.rocblas = h;
-    }
-    rocblas_handle h = (rocblas_handle)c.rocblas;
-    VVHD_CHECK(rocblas_set_stream(h, s) == rocblas_status_success, VVHD_EHIP, "rocblas_set_stream failed");
     if (refactor) {
+        if (!c.rocblas) {
+            rocblas_handle h = nullptr;
+            VVHD_CHECK(rocblas_create_handle(&h) == rocblas_status_success, VVHD_EHIP, "rocblas_create_handle failed");
+            c.rocblas = h;
+        }
+        rocblas_handle h = (rocblas_handle)c.rocblas;
+        VVHD_CHECK(rocblas_set_stream(h, s) == rocblas_status_success, VVHD_EHIP, "rocblas_set_stream failed");
         c.slae_n = -1;
-        c.slae_Acached.grow(nall);
-        c.slae_LU.grow(nall);
-        c.slae_ipiv.grow((size_t)n * nsys + 1);
-        VVHD_HIP(hipMemcpyAsync(c.slae_Acached.p, c.slae_A.p, nall * 8, hipMemcpyDeviceToDevice, s));
-        VVHD_HIP(hipMemcpyAsync(c.slae_LU.p, c.slae_A.p, nall * 8, hipMemcpyDeviceToDevice, s));
-        VVHD_CHECK(rocsolver_dgetrf_strided_batched(h, n, n, c.slae_LU.p, n, (rocblas_stride)nn, c.slae_ipiv.p,
-                                                    (rocblas_stride)n, c.slae_info.p, nsys) == rocblas_status_success,
+        c.slae_ipiv.grow((size_t)nc * nsys + 1);
+        VVHD_HIP(hipMemcpyAsync(c.slae_inv.p, c.slae_core.p, call * 8, hipMemcpyDeviceToDevice, s));
+        // a row-major core is the transpose to the library, whose inverse is the row-major inverse
+        VVHD_CHECK(rocsolver_dgetrf_strided_batched(h, nc, nc, c.slae_inv.p, nc, (rocblas_stride)cc, c.slae_ipiv.p,
+                                                    (rocblas_stride)nc, c.slae_info.p, nsys) == rocblas_status_success,
                    VVHD_EHIP, "rocsolver_dgetrf_strided_batched failed");
         std::vector<int32_t> info(nsys);
         VVHD_HIP(hipMemcpyAsync(info.data(), c.slae_info.p, (size_t)nsys * 4, hipMemcpyDeviceToHost, s));
@@ -1293,16 +1416,20 @@ void calc_circulation(Ctx& c, double infx, double infy) {
             if (info[q] != 0)
                 throw Error(VVHD_ESINGULAR, "calc_circulation: singular matrix of simulation " + std::to_string(q) +
                                                 ", column " + std::to_string(info[q]));
-        c.slae_n = n;
+        VVHD_CHECK(rocsolver_dgetri_strided_batched(h, nc, c.slae_inv.p, nc, (rocblas_stride)cc, c.slae_ipiv.p,
+                                                    (rocblas_stride)nc, c.slae_info.p, nsys) == rocblas_status_success,
+                   VVHD_EHIP, "rocsolver_dgetri_strided_batched failed");
+        c.slae_n = nc;
         c.slae_nsys_factored = nsys;
     }
-    VVHD_HIP(hipMemcpyAsync(c.slae_x.p, c.slae_b.p, (size_t)n * nsys * 8, hipMemcpyDeviceToDevice, s));
-    VVHD_CHECK(rocsolver_dgetrs_strided_batched(h, rocblas_operation_none, n, 1, c.slae_LU.p, n, (rocblas_stride)nn,
-                                                c.slae_ipiv.p, (rocblas_stride)n, c.slae_x.p, n, (rocblas_stride)n,
-                                                nsys) == rocblas_status_success,
-               VVHD_EHIP, "rocsolver_dgetrs_strided_batched failed");
-    hipLaunchKernelGGL(k_writeback, dim3(nb), dim3(kBodyBlock), 0, s, M, c.bodies_d.p, c.segs.p, c.slae_x.p,
-                       (const int32_t*)d_body_sys);
+    hipLaunchKernelGGL(k_core_rhs, dim3(nblocks(nc), nsys), dim3(kBlock), 0, s, C, (const double*)c.slae_A.p,
+                       (const double*)c.slae_b.p);
+    const dim3 rows((nc + kBlock / kWave - 1) / (kBlock / kWave), nsys);
+    hipLaunchKernelGGL(k_core_mv<kMvFirst>, rows, dim3(kBlock), 0, s, C);
+    hipLaunchKernelGGL(k_core_mv<kMvResidual>, rows, dim3(kBlock), 0, s, C);
+    hipLaunchKernelGGL(k_core_mv<kMvCorrect>, rows, dim3(kBlock), 0, s, C);
+    hipLaunchKernelGGL(k_writeback, dim3(nb), dim3(kBodyBlock), 0, s, C, c.bodies_d.p, c.segs.p,
+                       (const double*)c.slae_A.p, (const double*)c.slae_b.p, (const int32_t*)d_body_sys);
     sync_bodies_to_host(c);
 }
 
