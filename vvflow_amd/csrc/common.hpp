@@ -8,6 +8,7 @@
 #include <cfloat>
 #include <cstdint>
 #include <cstdio>
+#include <functional>
 #include <stdexcept>
 #include <map>
 #include <string>
@@ -123,6 +124,8 @@ __device__ inline int xcd_block(int b, int nblocks) {
 
 // ------------------------------------------------------------------ context --
 
+constexpr int kSubLevels = 128;   // levels of a subtree in TreeArrays::sub_lev
+
 struct TreeArrays {
     // node table (capacity ncap)
     DBuf<double> x, y, h, w;              // Stretch() geometry
@@ -150,7 +153,7 @@ struct TreeArrays {
     DBuf<int32_t> seg_leaf;               // per segment: leaf (DFS)
     DBuf<int32_t> seg_keys, seg_ids;      // sort scratch of the per-leaf segment lists
     DBuf<int32_t> vleaf;                  // per element (vortex, heat, streak): leaf (DFS)
-    DBuf<int32_t> node_L, node_m, leaf_tmp, seg_node;   // build scratch
+    DBuf<int32_t> node_L, node_m, seg_node;             // build scratch
     DBuf<int32_t> cnt_near, cnt_far, err;               // list scratch
     DBuf<int64_t> slot_near, slot_far;                  // per (leaf, top entry) list offsets
     DBuf<uint8_t> entries;                              // top-of-tree entry tables of the list builder (per root)
@@ -163,7 +166,12 @@ struct TreeArrays {
     int32_t nnodes = 0, nleaves_h = 0;
     int64_t nnear = 0, nfar = 0;
     int max_depth = 0;
-    std::vector<std::pair<int, int>> levels;   // node id range per depth
+    // node ids: the levels over the whole list (host, and {begin, end} on the
+    // device), and per subtree its levels {begin, count} below its root
+    std::vector<std::pair<int, int>> levels;
+    DBuf<int2> lev_d, sub_lev;
+    DBuf<int32_t> sub_nlev;
+    int nsub = 0;
     bool built = false;
     int far_criteria = 8;
     double min_node = 0, max_node = DBL_MAX;
@@ -355,10 +363,7 @@ struct Ctx {
 
     // timing
     hipEvent_t ev[16] = {};
-    // tree build: per-level counters copied asynchronously (pinned, two slots)
-    static constexpr int kLevSlots = 2;   // tree levels in flight (pinned counter slots and events)
-    hipEvent_t lev_ev[kLevSlots] = {};
-    int32_t* lev_counters = nullptr;      // kLevSlots x 8 pinned counters
+    int32_t* lev_counters = nullptr;      // pinned: the tree build's counters
     int32_t* fm_counts = nullptr;         // pinned: flow-move survivors, removals in bodies, scan error
     bool phase_recorded[8] = {false, false, false, false, false, false, false, false};
 
@@ -425,6 +430,9 @@ void sync(Ctx& c);
 // phase entry points (one translation unit each)
 void tree_build(Ctx& c, int far_criteria, double min_node, double max_node, int32_t* perm_out);
 void tree_lists(Ctx& c);
+// Calls run(first level, end level, blocks) for the levels over the whole list,
+// deepest first when up: consecutive small levels together for one block.
+void for_level_runs(const TreeArrays& t, bool up, const std::function<void(int, int, int)>& run);
 void epsilon(Ctx& c, int merge, int32_t* nn1, int32_t* nn2, int32_t* merged);
 void convective(Ctx& c, double inf_x, double inf_y, int kahan);
 // beside: the near field runs beside the far-field kernels (tuned among the

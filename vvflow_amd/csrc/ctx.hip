@@ -157,11 +157,6 @@ int vvhd_create(int device, vvhd_ctx** out) {
             delete ctx;
             return VVHD_EHIP;
         }
-    for (auto& e : ctx->c.lev_ev)
-        if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
-            delete ctx;
-            return VVHD_EHIP;
-        }
     for (auto& e : ctx->c.tune_ev)
         if (hipEventCreate(&e) != hipSuccess) {
             delete ctx;
@@ -179,7 +174,7 @@ int vvhd_create(int device, vvhd_ctx** out) {
         delete ctx;
         return VVHD_EHIP;
     }
-    if (hipHostMalloc((void**)&ctx->c.lev_counters, Ctx::kLevSlots * 8 * sizeof(int32_t), hipHostMallocDefault) !=
+    if (hipHostMalloc((void**)&ctx->c.lev_counters, 16 * sizeof(int32_t), hipHostMallocDefault) !=
             hipSuccess ||
         hipHostMalloc((void**)&ctx->c.fm_counts, 4 * sizeof(int32_t), hipHostMallocDefault) != hipSuccess) {
         delete ctx;
@@ -226,11 +221,13 @@ void vvhd_destroy(vvhd_ctx* ctx) {
     for (auto* b : {&t.blx, &t.bly, &t.trx, &t.try_, &t.path}) b->release();
     for (auto* b : {&t.v0, &t.v1, &t.ch1, &t.parent, &t.depth, &t.nseg, &t.split, &t.nleaves, &t.arrive, &t.leaf_rank,
                     &t.counters, &t.leaf_node, &t.near_list, &t.far_list, &t.seg_list, &t.seg_leaf, &t.vleaf,
-                    &t.node_L, &t.node_m, &t.leaf_tmp, &t.seg_node, &t.cnt_near, &t.cnt_far, &t.err})
+                    &t.node_L, &t.node_m, &t.sub_nlev, &t.seg_node, &t.cnt_near, &t.cnt_far, &t.err})
         b->release();
     for (auto* b : {&t.near_off, &t.far_off, &t.seg_off, &t.slot_near, &t.slot_far}) b->release();
     for (auto* b : {&t.groups, &t.leaf_sim, &t.root_first, &t.pre}) b->release();
     t.entries.release();
+    t.lev_d.release();
+    t.sub_lev.release();
     t.trav.release();
     t.pbox.release();
     t.cmp_ie.release();
@@ -260,8 +257,6 @@ void vvhd_destroy(vvhd_ctx* ctx) {
     for (auto* b : {&t.h0, &t.h1, &t.s0, &t.s1, &t.seg_keys, &t.seg_ids}) b->release();
     for (auto* b : {&c.fld_a, &c.fld_b, &c.fld_gtmp}) b->release();
     c.fld_map.release();
-    for (auto& e : c.lev_ev)
-        if (e) (void)hipEventDestroy(e);
     if (c.lev_counters) (void)hipHostFree(c.lev_counters);
     if (c.fm_counts) (void)hipHostFree(c.fm_counts);
     (void)hipStreamDestroy(c.stream);

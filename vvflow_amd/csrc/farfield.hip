@@ -229,13 +229,10 @@ __global__ void k_moments_leaves(const int32_t* leaf_node, int nleaf, const int3
     leaf_moments(leaf_node[l], v0, v1, nx, ny, x, y, g, ie, M);
 }
 
-// The internal nodes of one tree level from their two children (parallel-axis
-// combination of the second moments); leaves are done beforehand.
-__global__ void k_moments_level(const int32_t* ch1, const int32_t* split, const double* nx, const double* ny,
-                                MomView M, int lb, int le) {
+// An internal node from its two children (parallel-axis combination of the
+// second moments); leaves are done beforehand.
+__device__ inline void node_moments(const int32_t* ch1, const double* nx, const double* ny, MomView M, int id) {
 #pragma clang fp contract(off)
-    const int id = lb + blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= le || split[id] != 2) return;
     for (int s = 0; s < 2; s++) {
         double G, zx, zy, qr = 0, qi = 0, E;
         const int a = ch1[id], b = a + 1;
@@ -259,6 +256,33 @@ __global__ void k_moments_level(const int32_t* ch1, const int32_t* split, const 
         M(6 + 2 * s, id) = qr;
         M(7 + 2 * s, id) = qi;
         M(10 + s, id) = E;
+    }
+}
+
+// Bottom-up over the levels [l0, l1) of the whole list (one block for several,
+// or one level spread over the grid), and over each subtree's levels (one
+// block per subtree).
+constexpr int kMomThreads = 1024;
+__global__ __launch_bounds__(kMomThreads) void k_moments_levels(const int32_t* ch1, const int32_t* split,
+                                                                const double* nx, const double* ny, MomView M,
+                                                                const int2* lev, int l0, int l1) {
+    for (int d = l1 - 1; d >= l0; d--) {
+        for (int id = lev[d].x + blockIdx.x * kMomThreads + threadIdx.x; id < lev[d].y; id += gridDim.x * kMomThreads)
+            if (split[id] == 2) node_moments(ch1, nx, ny, M, id);
+        __threadfence_block();
+        __syncthreads();
+    }
+}
+
+__global__ __launch_bounds__(kBlock) void k_moments_subs(const int32_t* ch1, const int32_t* split, const double* nx,
+                                                         const double* ny, MomView M, const int2* sub_lev,
+                                                         const int32_t* sub_nlev) {
+    const int2* lev = sub_lev + (size_t)blockIdx.x * kSubLevels;
+    for (int d = sub_nlev[blockIdx.x] - 2; d >= 0; d--) {   // the last level holds leaves only
+        for (int i = threadIdx.x; i < lev[d].y; i += kBlock)
+            if (split[lev[d].x + i] == 2) node_moments(ch1, nx, ny, M, lev[d].x + i);
+        __threadfence_block();
+        __syncthreads();
     }
 }
 
@@ -1226,13 +1250,14 @@ MomView moments(Ctx& c) {
     if (t.nleaves_h > 0)
         hipLaunchKernelGGL(k_moments_leaves, dim3(nblocks(t.nleaves_h)), dim3(kBlock), 0, c.stream, t.leaf_node.p,
                            t.nleaves_h, t.v0.p, t.v1.p, t.x.p, t.y.p, c.x.p, c.y.p, c.g.p, c.ie.p, M);
-    // internal nodes level by level from the deepest one that has any (the
-    // last level holds leaves only)
-    for (int d = (int)t.levels.size() - 2; d >= 0; d--) {
-        const int lb = t.levels[d].first, le = t.levels[d].second;
-        hipLaunchKernelGGL(k_moments_level, dim3(nblocks(le - lb)), dim3(kBlock), 0, c.stream, t.ch1.p, t.split.p,
-                           t.x.p, t.y.p, M, lb, le);
-    }
+    // internal nodes: the subtrees, then the levels above them
+    if (t.nsub)
+        hipLaunchKernelGGL(k_moments_subs, dim3(t.nsub), dim3(kBlock), 0, c.stream, t.ch1.p, t.split.p, t.x.p, t.y.p, M,
+                           (const int2*)t.sub_lev.p, (const int32_t*)t.sub_nlev.p);
+    for_level_runs(t, true, [&](int l0, int l1, int grid) {
+        hipLaunchKernelGGL(k_moments_levels, dim3(grid), dim3(kMomThreads), 0, c.stream, t.ch1.p, t.split.p, t.x.p,
+                           t.y.p, M, (const int2*)t.lev_d.p, l0, l1);
+    });
     return M;
 }
 

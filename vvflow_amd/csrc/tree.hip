@@ -18,12 +18,16 @@
 // the build are the vortices, then the heat particles, then the streak
 // particles, and every node holds one range per list.
 //
-// Node ids are allocated level by level, so every level is a contiguous id
-// range.  After the levels: subtree leaf counts (bottom-up) and leaf DFS
-// ranks (top-down) give the bottomNodes order; per-sign monopoles
-// (CalculateCMass, :150-197) are combined bottom-up level by level; and the
-// near/far lists of every leaf (FindNearNodes, :199-217) come from one
-// traversal per wave of 64 DFS-consecutive leaves with a shared stack.
+// The levels run over the whole list only while nodes are large: a node with
+// at most kSubElems elements and kSubSegs segments is taken by one workgroup,
+// which builds its whole subtree in LDS (k_subtree).  Node ids of the levels
+// over the whole list are contiguous per level (TreeArrays::levels), those of
+// a subtree contiguous per level of the subtree (sub_lev).  After the build,
+// subtree leaf counts and monopoles (CalculateCMass, :150-197) go bottom-up
+// and leaf DFS ranks (the bottomNodes order) top-down, one workgroup per
+// subtree and one for the levels above; and the near/far lists of every leaf
+// (FindNearNodes, :199-217) come from walks of waves of 64 DFS-consecutive
+// leaves.
 
 #include "common.hpp"
 
@@ -32,7 +36,9 @@
 #include <rocprim/device/device_scan.hpp>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
+#include <functional>
 
 #pragma clang fp contract(off)
 
@@ -107,7 +113,7 @@ __device__ inline void init_node(NodeView nv, int id, int parent, int depth, uin
 // One root per simulation: root s holds the vortices [sim_off[s], sim_off[s+1]).
 // The heat elements [hbase, sbase) and streak elements [sbase, nelem) belong
 // to root 0 (one simulation only).
-__global__ void k_init_roots(NodeView nv, int nroots, const int64_t* sim_off, int32_t* counters, int hbase,
+__global__ void k_init_roots(NodeView nv, int nroots, const int64_t* sim_off, int32_t* counters, int2* lev, int hbase,
                              int sbase, int nelem) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s < nroots) {
@@ -121,8 +127,13 @@ __global__ void k_init_roots(NodeView nv, int nroots, const int64_t* sim_off, in
         counters[1] = 0;        // leaves
         counters[2] = 0;        // level begin
         counters[3] = nroots;   // level end
-        counters[4] = 0;        // overflow flag
+        counters[4] = 0;        // 1: node capacity exceeded, 2: tree too deep
         counters[5] = 0;        // max depth
+        counters[6] = 0;        // nodes of the level that k_subtree left
+        counters[7] = 0;        // subtrees
+        counters[8] = 0;        // nodes of the level handed to k_subtree
+        counters[9] = nroots;   // first id of the next level
+        lev[0] = make_int2(0, nroots);
     }
 }
 
@@ -372,8 +383,7 @@ __global__ void k_leaf_sim(const int32_t* root_first, int nroots, int nleaf, int
 
 // snode::Stretch tail + DivideNode decision (TSortedTree.cpp:36-56, 122-125)
 // for the nodes of the current level; split nodes get a pair of children.
-__global__ void k_decide(NodeView nv, int32_t* counters, int32_t* leaf_tmp, int cap, double min_node,
-                         double max_node) {
+__global__ void k_decide(NodeView nv, int32_t* counters, int cap, double min_node, double max_node) {
     const int lb = counters[2], le = counters[3];
     const int lane = lane_id();
     const uint64_t below = (1ull << lane) - 1;
@@ -382,7 +392,7 @@ __global__ void k_decide(NodeView nv, int32_t* counters, int32_t* leaf_tmp, int 
     const int stride = gridDim.x * blockDim.x;
     for (int b0 = lb + blockIdx.x * blockDim.x + threadIdx.x - lane; b0 < le; b0 += stride) {
         const int id = b0 + lane;
-        const bool valid = id < le;
+        const bool valid = id < le && nv.split[id] == 0;   // not taken as a subtree
         bool leaf = false;
         int depth = 0;
         if (valid) {
@@ -404,21 +414,19 @@ __global__ void k_decide(NodeView nv, int32_t* counters, int32_t* leaf_tmp, int 
             depth = nv.depth[id] + 1;
         }
         const uint64_t lm = __ballot(valid && leaf), sm = __ballot(valid && !leaf);
-        int lbase = 0, sbase = 0, dmax = depth;
+        int sbase = 0, dmax = depth;
         for (int o = kWave / 2; o > 0; o >>= 1) dmax = max(dmax, __shfl_xor(dmax, o, kWave));
         if (lane == 0) {
-            if (lm) lbase = atomicAdd(&counters[1], __popcll(lm));
+            if (lm) atomicAdd(&counters[1], __popcll(lm));
             if (sm) {
                 sbase = atomicAdd(&counters[0], 2 * __popcll(sm));
                 atomicMax(&counters[5], dmax);
             }
         }
-        lbase = __shfl(lbase, 0, kWave);
         sbase = __shfl(sbase, 0, kWave);
         if (!valid) continue;
         if (leaf) {
             nv.split[id] = 1;
-            leaf_tmp[lbase + __popcll(lm & below)] = id;
             continue;
         }
         const int c = sbase + 2 * __popcll(sm & below);
@@ -460,17 +468,21 @@ struct GoesLeftFlag {
 // of a split node's range also records that list's split position and number
 // of misplaced pairs (node_L / node_m at list * cap + node) and sets the
 // children's ranges.  Thread 0 advances the level range (the nodes of the
-// next level were allocated by k_decide).
+// next level were allocated by k_decide) and records it in lev[depth].
 // The flags come from k_flag_count, before any swap of this level: k_swap
 // reads them too and must not derive them from coordinates that the swaps
 // may be rewriting.
 __global__ void k_ranks(NodeView nv, const int32_t* enode, const int32_t* P, int n, int hbase, int sbase, int cap,
                         int32_t* node_L, int32_t* node_m, int32_t* left_pos, int32_t* right_pos, int32_t* counters,
-                        const int32_t* flag) {
+                        const int32_t* flag, int2* lev, int depth) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k == 0) {
-        counters[2] = counters[3];
+        counters[2] = counters[9];
         counters[3] = counters[0];
+        counters[9] = counters[0];
+        counters[6] = 0;
+        counters[8] = 0;
+        lev[depth] = make_int2(counters[2], counters[3]);
     }
     if (k >= n) return;
     const int node = enode[k];
@@ -564,6 +576,381 @@ __global__ void k_seg_step(NodeView nv, const vvhd_seg* segs, int nseg, int32_t*
 }
 
 
+// The ids that k_subtree took lie before the children of the level's other
+// nodes.
+__global__ void k_level_begin(int32_t* counters) {
+    if (threadIdx.x == 0) counters[9] = counters[0];
+}
+
+// Subtrees in LDS.  A block takes one undecided node of the level after
+// another (queue counters[8]); a node that fits is split down to its leaves
+// by one workgroup, level by level, with the same steps as the kernels above:
+// boxes, decisions, goes-left flags and their prefix, ranks, Hoare swaps.  The
+// others are counted in counters[6] and stay for the level kernels.  What
+// bounds a level over the whole list is its five to seven launches and passes
+// over all elements (45-55 us, 22 levels at 1M and in a cylinder wake of 3k);
+// in LDS a level is eight barriers, which wait for LDS operations only (the
+// node records go out to memory meanwhile), and all subtrees run at once.
+// The sizes keep two blocks on a compute unit (160 KiB of LDS).  A node of a
+// subtree holds an element or segment of its own, and unless the box is still
+// above max_node only nodes of kLeafMaxList or more split, which bounds the
+// nodes of a level (fits_subtree); 64 spare ones are for empty children of
+// boxes too small to halve.
+constexpr int kSubElems = 1536, kSubSegs = 256, kSubNodes = 512;
+constexpr int kSubThreads = 512, kSubWaves = kSubThreads / kWave;
+constexpr int kSubPer = kSubElems / kSubThreads;   // elements per thread
+constexpr uint16_t kDone = 0xFFFF;
+static_assert(kSubNodes <= kSubThreads && kSubElems % kSubThreads == 0, "one node per thread");
+
+__device__ inline bool fits_subtree(int ne, int ns, double mx, double max_node) {
+    if (ne > kSubElems || ns > kSubSegs) return false;
+    const int all = ne + ns;
+    return (mx < max_node ? 2 * (all / kLeafMaxList) : all) + 64 <= kSubNodes;
+}
+
+struct SubShared {
+    double x[kSubElems], y[kSubElems];
+    unsigned long long lx[kSubNodes], ly[kSubNodes], hx[kSubNodes], hy[kSubNodes], path[kSubNodes];
+    double sx[kSubSegs], sy[kSubSegs];
+    int gid[kSubNodes], nsg[kSubNodes], sid[kSubSegs];
+    uint16_t r0[3][kSubNodes], r1[3][kSubNodes];   // per list: a node's range (local elements)
+    uint16_t kid[kSubNodes];                       // first child in the next level, or kDone
+    uint16_t perm[kSubElems], node[kSubElems], P[kSubElems + 1], pos[kSubElems], snode[kSubSegs];
+    int cnt[kSubWaves], cnt2[kSubPer * kSubWaves];
+    int cur, slot, base, fail, nseg;
+};
+
+// Barrier of the block that waits for LDS operations only.
+__device__ inline void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+__global__ __launch_bounds__(kSubThreads, 4) void k_subtree(NodeView nv, int32_t* counters, int cap, double min_node,
+                                                            double max_node, int32_t* enode, double* gx, double* gy,
+                                                            int32_t* id, const vvhd_seg* segs, int nseg,
+                                                            int32_t* seg_node, int2* sub_lev, int32_t* sub_nlev,
+                                                            int sub_cap) {
+    __shared__ SubShared S;
+    const int t = threadIdx.x, w = t / kWave, lane = lane_id();
+    const uint64_t below = (1ull << lane) - 1;
+    const unsigned long long lo0 = ord_from_double(DBL_MAX), hi0 = ord_from_double(-DBL_MAX);
+    const int first = counters[2], last = counters[3];
+    int next = 0;   // thread 0: the node after this one
+    if (t == 0) next = first + atomicAdd(&counters[8], 1);
+    for (;;) {
+        __syncthreads();   // (also the id loads and stores of the node before)
+        if (t == 0) {
+            S.cur = next;
+            S.fail = 0;
+            S.nseg = 0;
+            S.slot = sub_cap;
+        }
+        lds_barrier();
+        const int r = S.cur;
+        if (r >= last) return;   // every block gets here: the queue only grows
+        const int gv0 = nv.v0[r], gh0 = nv.h0[r], gs0 = nv.s0[r];
+        const int nvt = nv.v1[r] - gv0, nh = nv.h1[r] - gh0, nst = nv.s1[r] - gs0;
+        const int ne = nvt + nh + nst, ns = nv.nseg[r], depth0 = nv.depth[r];
+        const unsigned long long rlx = nv.blx[r], rly = nv.bly[r], rhx = nv.trx[r], rhy = nv.try_[r];
+        if (t == 0) {
+            next = first + atomicAdd(&counters[8], 1);
+            const double h = double_from_ord(rhy) - double_from_ord(rly), wd = double_from_ord(rhx) - double_from_ord(rlx);
+            if (fits_subtree(ne, ns, (h < wd) ? wd : h, max_node)) S.slot = atomicAdd(&counters[7], 1);
+            if (S.slot >= sub_cap) atomicAdd(&counters[6], 1);
+        }
+        lds_barrier();
+        const int slot = S.slot;
+        if (slot >= sub_cap) continue;
+        auto global_of = [&](int k) { return k < nvt ? gv0 + k : (k < nvt + nh ? gh0 + (k - nvt) : gs0 + (k - nvt - nh)); };
+        for (int k = t; k < ne; k += kSubThreads) {
+            const int gk = global_of(k);
+            S.x[k] = gx[gk];
+            S.y[k] = gy[gk];
+            S.perm[k] = (uint16_t)k;
+            S.node[k] = 0;
+        }
+        if (ns) {
+            for (int q = t; q < nseg; q += kSubThreads)
+                if (seg_node[q] == r) {
+                    const int p = atomicAdd(&S.nseg, 1);
+                    S.sid[p] = q;
+                    S.sx[p] = segs[q].x;
+                    S.sy[p] = segs[q].y;
+                    S.snode[p] = 0;
+                }
+        }
+        if (t == 0) {
+            S.gid[0] = r;
+            S.nsg[0] = 0;
+            S.path[0] = nv.path[r];
+            S.lx[0] = rlx;
+            S.ly[0] = rly;
+            S.hx[0] = rhx;
+            S.hy[0] = rhy;
+            S.r0[0][0] = 0;
+            S.r1[0][0] = S.r0[1][0] = (uint16_t)nvt;
+            S.r1[1][0] = S.r0[2][0] = (uint16_t)(nvt + nh);
+            S.r1[2][0] = (uint16_t)ne;
+        }
+        lds_barrier();
+        // does a point of node i go to its first child (goes_left)
+        auto left_of = [&](int i, double px, double py) {
+            const double blx = double_from_ord(S.lx[i]), bly = double_from_ord(S.ly[i]);
+            const double trx = double_from_ord(S.hx[i]), try_ = double_from_ord(S.hy[i]);
+            return (try_ - bly < trx - blx) ? px < (blx + trx) * 0.5 : py < (bly + try_) * 0.5;
+        };
+        auto add_box = [&](int i, double px, double py) {
+            if (!isnan(px)) {
+                const unsigned long long o = ord_from_double(px);
+                atomicMin(&S.lx[i], o);
+                atomicMax(&S.hx[i], o);
+            }
+            if (!isnan(py)) {
+                const unsigned long long o = ord_from_double(py);
+                atomicMin(&S.ly[i], o);
+                atomicMax(&S.hy[i], o);
+            }
+        };
+        int m = 1, lev = 0;
+        for (;; lev++) {
+            // boxes of this level's nodes (the root's is known) and their segments:
+            // L lanes per node over its ranges, about three elements per lane
+            // (one LDS atomic per element and side queues 64 deep on a node's
+            // slots: 5 us a level).  Below eight nodes several waves share one.
+            if (lev > 0) {
+                int L = kWave;
+                while (L > 1 && L * m > kSubThreads) L >>= 1;
+                const int parts = max(1, kSubThreads / (L * m));   // groups per node
+                const int grp = t / L, i = grp / parts, sub = (grp % parts) * L + (t & (L - 1)), step = parts * L;
+                double bx0 = DBL_MAX, by0 = DBL_MAX, bx1 = -DBL_MAX, by1 = -DBL_MAX;
+                if (i < m)
+                    for (int c = 0; c < 3; c++) {
+                        const int b = S.r1[c][i];
+                        for (int k = S.r0[c][i] + sub; k < b; k += step) {
+                            const double px = S.x[k], py = S.y[k];   // fmin and fmax pass over NaN
+                            bx0 = fmin(bx0, px);
+                            by0 = fmin(by0, py);
+                            bx1 = fmax(bx1, px);
+                            by1 = fmax(by1, py);
+                        }
+                    }
+                for (int o = L / 2; o > 0; o >>= 1) {
+                    bx0 = fmin(bx0, __shfl_xor(bx0, o, kWave));
+                    by0 = fmin(by0, __shfl_xor(by0, o, kWave));
+                    bx1 = fmax(bx1, __shfl_xor(bx1, o, kWave));
+                    by1 = fmax(by1, __shfl_xor(by1, o, kWave));
+                }
+                if (i < m && (t & (L - 1)) == 0) {
+                    if (bx0 != DBL_MAX) atomicMin(&S.lx[i], (unsigned long long)ord_from_double(bx0));
+                    if (by0 != DBL_MAX) atomicMin(&S.ly[i], (unsigned long long)ord_from_double(by0));
+                    if (bx1 != -DBL_MAX) atomicMax(&S.hx[i], (unsigned long long)ord_from_double(bx1));
+                    if (by1 != -DBL_MAX) atomicMax(&S.hy[i], (unsigned long long)ord_from_double(by1));
+                }
+            }
+            if (t < ns && S.snode[t] != kDone) {
+                const int i = S.snode[t];
+                atomicAdd(&S.nsg[i], 1);
+                if (lev > 0) add_box(i, S.sx[t], S.sy[t]);
+            }
+            lds_barrier();
+            // decisions (k_decide), one node per thread
+            bool split = false;
+            if (t < m) {
+                const int gi = S.gid[t];
+                const double blx = double_from_ord(S.lx[t]), bly = double_from_ord(S.ly[t]);
+                const double trx = double_from_ord(S.hx[t]), try_ = double_from_ord(S.hy[t]);
+                const double h = try_ - bly, wd = trx - blx;
+                const double mx = (h < wd) ? wd : h;   // std::max(h, w)
+                const double mn = (wd < h) ? wd : h;   // std::min(h, w)
+                int nlist = S.nsg[t];
+                for (int c = 0; c < 3; c++) nlist = max(nlist, (int)S.r1[c][t] - (int)S.r0[c][t]);
+                split = !((mx < max_node && mn <= min_node) || (mx < max_node && nlist < kLeafMaxList));
+                nv.x[gi] = (blx + trx) * 0.5;
+                nv.y[gi] = (bly + try_) * 0.5;
+                nv.h[gi] = h;
+                nv.w[gi] = wd;
+                nv.split[gi] = split ? 2 : 1;
+                if (lev > 0) {
+                    nv.blx[gi] = S.lx[t];
+                    nv.bly[gi] = S.ly[t];
+                    nv.trx[gi] = S.hx[t];
+                    nv.try_[gi] = S.hy[t];
+                    nv.nseg[gi] = S.nsg[t];
+                }
+            }
+            const uint64_t sm = __ballot(split);
+            if (lane == 0) S.cnt[w] = __popcll(sm);
+            lds_barrier();
+            int nsplit = 0, rank = 0;
+            for (int q = 0; q < kSubWaves; q++) {
+                if (q == w) rank = nsplit;
+                nsplit += S.cnt[q];
+            }
+            rank += __popcll(sm & below);
+            if (t < m) S.kid[t] = split ? (uint16_t)(2 * rank) : kDone;
+            // ids of the children: the counter's answer is needed only when
+            // they are written
+            int claim = 0;
+            if (t == 0) {
+                atomicAdd(&counters[1], m - nsplit);
+                if (nsplit) {
+                    atomicMax(&counters[5], depth0 + lev + 1);
+                    claim = atomicAdd(&counters[0], 2 * nsplit);
+                }
+            }
+            lds_barrier();
+            // goes-left flags and their counts; the elements of leaves are done
+            uint64_t fmask[kSubPer];
+            for (int j = 0; j < kSubPer; j++) {
+                const int k = j * kSubThreads + t;
+                bool f = false;
+                if (k < ne && S.node[k] != kDone) {
+                    const int i = S.node[k];
+                    if (S.kid[i] == kDone) {
+                        enode[global_of(k)] = S.gid[i];
+                        S.node[k] = kDone;
+                    } else {
+                        f = left_of(i, S.x[k], S.y[k]);
+                    }
+                }
+                fmask[j] = __ballot(f);
+                if (lane == 0) S.cnt2[j * kSubWaves + w] = __popcll(fmask[j]);
+            }
+            if (t < ns && S.snode[t] != kDone) {
+                const int i = S.snode[t];
+                if (S.kid[i] == kDone) {
+                    seg_node[S.sid[t]] = S.gid[i];
+                    S.snode[t] = kDone;
+                } else {
+                    S.snode[t] = (uint16_t)(S.kid[i] + (left_of(i, S.sx[t], S.sy[t]) ? 0 : 1));
+                }
+            }
+            if (nsplit == 0) break;
+            lds_barrier();
+            {
+                int run = 0;
+                for (int q = 0; q < kSubPer * kSubWaves; q++) {
+                    if (q % kSubWaves == w) {
+                        const int j = q / kSubWaves, k = j * kSubThreads + t;
+                        if (k < ne) S.P[k] = (uint16_t)(run + __popcll(fmask[j] & below));
+                    }
+                    run += S.cnt2[q];
+                }
+                if (t == 0) S.P[ne] = (uint16_t)run;
+            }
+            lds_barrier();
+            // ranks of misplaced elements: a node's left ones from the front of
+            // its range of pos, the right ones from the back
+            for (int j = 0; j < kSubPer; j++) {
+                const int k = j * kSubThreads + t;
+                if (k >= ne || S.node[k] == kDone) continue;
+                const int i = S.node[k], c = k < nvt ? 0 : (k < nvt + nh ? 1 : 2);
+                const int a = S.r0[c][i], b = S.r1[c][i];
+                const int Pa = S.P[a], Labs = a + S.P[b] - Pa;
+                const bool f = (fmask[j] >> lane) & 1;
+                if (k < Labs && !f)
+                    S.pos[k - (S.P[k] - Pa)] = (uint16_t)k;
+                else if (k >= Labs && f)
+                    S.pos[b - 1 - (S.P[k] - S.P[Labs])] = (uint16_t)k;
+            }
+            lds_barrier();
+            for (int j = 0; j < kSubPer; j++) {
+                const int k = j * kSubThreads + t;
+                if (k >= ne || S.node[k] == kDone) continue;
+                const int i = S.node[k], c = k < nvt ? 0 : (k < nvt + nh ? 1 : 2);
+                const int a = S.r0[c][i], b = S.r1[c][i];
+                const int Pa = S.P[a], Lc = S.P[b] - Pa, Labs = a + Lc;
+                const bool f = (fmask[j] >> lane) & 1;
+                if (k < Labs && !f) {   // the left thread of a pair swaps
+                    const int pairs = Lc - (S.P[Labs] - Pa);
+                    const int q = S.pos[b - pairs + (k - a) - (S.P[k] - Pa)];
+                    const double px = S.x[k], py = S.y[k];
+                    const uint16_t pk = S.perm[k];
+                    S.x[k] = S.x[q];
+                    S.y[k] = S.y[q];
+                    S.perm[k] = S.perm[q];
+                    S.x[q] = px;
+                    S.y[q] = py;
+                    S.perm[q] = pk;
+                }
+                S.node[k] = (uint16_t)(S.kid[i] + (k < Labs ? 0 : 1));
+            }
+            // children: the parents' records are read before any is replaced
+            const int pk = t < m ? S.kid[t] : kDone;
+            int pg = 0, pr[3][3];
+            unsigned long long ppath = 0;
+            if (pk != kDone) {
+                pg = S.gid[t];
+                ppath = S.path[t] << 1;
+                for (int c = 0; c < 3; c++) {
+                    const int a = S.r0[c][t], b = S.r1[c][t];
+                    pr[c][0] = a;
+                    pr[c][1] = a + S.P[b] - S.P[a];
+                    pr[c][2] = b;
+                }
+            }
+            if (t == 0) {
+                S.base = claim;
+                if (claim + 2 * nsplit > cap || 2 * nsplit > kSubNodes) S.fail = 1;
+                if (depth0 + lev + 2 >= kMaxLevels) S.fail = 2;
+                if (S.fail)
+                    counters[4] = S.fail;
+                else
+                    sub_lev[(size_t)slot * kSubLevels + lev] = make_int2(claim, 2 * nsplit);
+            }
+            lds_barrier();
+            if (S.fail) return;   // uniform; the host reports counters[4]
+            const int base = S.base;
+            if (pk != kDone) {
+                nv.ch1[pg] = base + pk;
+                for (int q = 0; q < 2; q++) {
+                    const int i = pk + q, gi = base + i;
+                    S.gid[i] = gi;
+                    S.nsg[i] = 0;
+                    S.path[i] = ppath | (unsigned long long)q;
+                    S.lx[i] = S.ly[i] = lo0;
+                    S.hx[i] = S.hy[i] = hi0;
+                    for (int c = 0; c < 3; c++) {
+                        S.r0[c][i] = (uint16_t)pr[c][q];
+                        S.r1[c][i] = (uint16_t)pr[c][q + 1];
+                    }
+                    nv.parent[gi] = pg;
+                    nv.depth[gi] = depth0 + lev + 1;
+                    nv.path[gi] = ppath | (unsigned long long)q;
+                    nv.ch1[gi] = -1;
+                    nv.v0[gi] = gv0 + pr[0][q];
+                    nv.v1[gi] = gv0 + pr[0][q + 1];
+                    nv.h0[gi] = gh0 + pr[1][q] - nvt;
+                    nv.h1[gi] = gh0 + pr[1][q + 1] - nvt;
+                    nv.s0[gi] = gs0 + pr[2][q] - nvt - nh;
+                    nv.s1[gi] = gs0 + pr[2][q + 1] - nvt - nh;
+                }
+            }
+            lds_barrier();
+            m = 2 * nsplit;
+        }
+        if (t == 0) sub_nlev[slot] = lev;
+        // positions and ids back; the old ids are read before any is replaced
+        int32_t ids[kSubPer];
+        for (int j = 0; j < kSubPer; j++) {
+            const int k = j * kSubThreads + t;
+            if (k < ne) {
+                const int gk = global_of(k);
+                ids[j] = id[global_of(S.perm[k])];
+                gx[gk] = S.x[k];
+                gy[gk] = S.y[k];
+            }
+        }
+        __syncthreads();
+        for (int j = 0; j < kSubPer; j++) {
+            const int k = j * kSubThreads + t;
+            if (k < ne) id[global_of(k)] = ids[j];
+        }
+    }
+}
+
 // A heat or streak list in tree order: positions from the element arrays,
 // the other fields gathered from the list's own arrays (id holds element
 // numbers, base is the list's first element).
@@ -598,107 +985,286 @@ struct CMView {
     float *pie, *mie;
 };
 
-// Bottom-up over one level: subtree leaf counts, and monopoles --
-// CalculateCMassFromScratch (TSortedTree.cpp:176-197) for leaves (array
-// order) and CalculateCMass (:150-174) from the children otherwise.
-__global__ void k_up_level(NodeView nv, CMView cm, int lb, int le, const double* x, const double* y, const double* g,
-                           int32_t* nleaves) {
-    const int id = lb + blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= le) return;
+// Per-sign monopoles of a node (CMp, CMm); ie is _1_eps, infinite or 0.
+struct Monopoles {
+    double px, py, pg, mx, my, mg;
+    float pie, mie;
+};
+
+__device__ inline Monopoles get_monopoles(const CMView& cm, int id) {
+    return Monopoles{cm.px[id], cm.py[id], cm.pg[id], cm.mx[id], cm.my[id], cm.mg[id], cm.pie[id], cm.mie[id]};
+}
+
+__device__ inline void put_monopoles(const CMView& cm, int id, const Monopoles& q) {
+    cm.px[id] = q.px;
+    cm.py[id] = q.py;
+    cm.pg[id] = q.pg;
+    cm.mx[id] = q.mx;
+    cm.my[id] = q.my;
+    cm.mg[id] = q.mg;
+    cm.pie[id] = q.pie;
+    cm.mie[id] = q.mie;
+}
+
+// CalculateCMassFromScratch (TSortedTree.cpp:176-197), in array order.
+__device__ inline Monopoles leaf_monopoles(const NodeView& nv, int id, const double* x, const double* y,
+                                           const double* g) {
+    Monopoles q{0, 0, 0, 0, 0, 0, INFINITY, INFINITY};
+    for (int k = nv.v0[id]; k < nv.v1[id]; k++) {
+        const double gk = g[k];
+        if (gk > 0) {
+            q.px += x[k] * gk;
+            q.py += y[k] * gk;
+            q.pg += gk;
+        } else {
+            q.mx += x[k] * gk;
+            q.my += y[k] * gk;
+            q.mg += gk;
+        }
+    }
+    if (q.pg) {
+        q.px *= (1. / q.pg);
+        q.py *= (1. / q.pg);
+    } else {
+        q.px = nv.x[id];
+        q.py = nv.y[id];
+    }
+    if (q.mg) {
+        q.mx *= (1. / q.mg);
+        q.my *= (1. / q.mg);
+    } else {
+        q.mx = nv.x[id];
+        q.my = nv.y[id];
+    }
+    return q;
+}
+
+// CalculateCMass (:150-174) from the children; without circulation
+// TObj(x, y, 0): _1_eps = 0.
+__device__ inline Monopoles node_monopoles(const NodeView& nv, int id, const Monopoles& a, const Monopoles& b) {
+    Monopoles q;
+    auto combine = [&](double ax, double ay, double ag, double bx, double by, double bg, double& x, double& y,
+                       double& g, float& ie) {
+        const double s = ag + bg;
+        if (s) {
+            const double inv = 1. / s;
+            x = (ax * ag + bx * bg) * inv;
+            y = (ay * ag + by * bg) * inv;
+            g = s;
+            ie = INFINITY;
+        } else {
+            x = nv.x[id];
+            y = nv.y[id];
+            g = 0;
+            ie = 0;
+        }
+    };
+    combine(a.px, a.py, a.pg, b.px, b.py, b.pg, q.px, q.py, q.pg, q.pie);
+    combine(a.mx, a.my, a.mg, b.mx, b.my, b.mg, q.mx, q.my, q.mg, q.mie);
+    return q;
+}
+
+// Leaf count and monopoles of a node.
+__device__ inline void up_node(const NodeView& nv, const CMView& cm, int id, const double* x, const double* y,
+                               const double* g, int32_t* nleaves) {
     if (nv.split[id] != 2) {
         nleaves[id] = 1;
-        double px = 0, py = 0, pg = 0, mx = 0, my = 0, mg = 0;
-        for (int k = nv.v0[id]; k < nv.v1[id]; k++) {
-            const double gk = g[k];
-            if (gk > 0) {
-                px += x[k] * gk;
-                py += y[k] * gk;
-                pg += gk;
-            } else {
-                mx += x[k] * gk;
-                my += y[k] * gk;
-                mg += gk;
-            }
-        }
-        if (pg) {
-            px *= (1. / pg);
-            py *= (1. / pg);
-        } else {
-            px = nv.x[id];
-            py = nv.y[id];
-        }
-        if (mg) {
-            mx *= (1. / mg);
-            my *= (1. / mg);
-        } else {
-            mx = nv.x[id];
-            my = nv.y[id];
-        }
-        cm.px[id] = px;
-        cm.py[id] = py;
-        cm.pg[id] = pg;
-        cm.mx[id] = mx;
-        cm.my[id] = my;
-        cm.mg[id] = mg;
-        cm.pie[id] = INFINITY;
-        cm.mie[id] = INFINITY;
+        put_monopoles(cm, id, leaf_monopoles(nv, id, x, y, g));
         return;
     }
-    const int a = nv.ch1[id], b = a + 1;
-    nleaves[id] = nleaves[a] + nleaves[b];
-    {
-        const double ag = cm.pg[a], bg = cm.pg[b];
-        const double s = ag + bg;
-        if (s) {
-            const double inv = 1. / s;
-            cm.px[id] = (cm.px[a] * ag + cm.px[b] * bg) * inv;
-            cm.py[id] = (cm.py[a] * ag + cm.py[b] * bg) * inv;
-            cm.pg[id] = s;
-            cm.pie[id] = INFINITY;
-        } else {   // TObj(x, y, 0): _1_eps = 0
-            cm.px[id] = nv.x[id];
-            cm.py[id] = nv.y[id];
-            cm.pg[id] = 0;
-            cm.pie[id] = 0;
-        }
+    const int a = nv.ch1[id];
+    nleaves[id] = nleaves[a] + nleaves[a + 1];
+    put_monopoles(cm, id, node_monopoles(nv, id, get_monopoles(cm, a), get_monopoles(cm, a + 1)));
+}
+
+// Leaf f (DFS rank) is node id.
+__device__ inline void down_leaf(const NodeView& nv, int id, int f, int32_t* leaf_rank, int32_t* leaf_node,
+                                 int32_t* vleaf) {
+    leaf_rank[id] = f;
+    leaf_node[f] = id;
+    for (int k = nv.v0[id]; k < nv.v1[id]; k++) vleaf[k] = f;
+    for (int k = nv.h0[id]; k < nv.h1[id]; k++) vleaf[k] = f;
+    for (int k = nv.s0[id]; k < nv.s1[id]; k++) vleaf[k] = f;
+}
+
+// First leaf rank of a node's children (DFS order), or the leaf itself.
+__device__ inline void down_node(const NodeView& nv, int id, const int32_t* nleaves, int32_t* first,
+                                 int32_t* leaf_rank, int32_t* leaf_node, int32_t* vleaf, int32_t* pre) {
+    const int f = first[id];
+    if (nv.split[id] != 2) {
+        down_leaf(nv, id, f, leaf_rank, leaf_node, vleaf);
+        return;
     }
-    {
-        const double ag = cm.mg[a], bg = cm.mg[b];
-        const double s = ag + bg;
-        if (s) {
-            const double inv = 1. / s;
-            cm.mx[id] = (cm.mx[a] * ag + cm.mx[b] * bg) * inv;
-            cm.my[id] = (cm.my[a] * ag + cm.my[b] * bg) * inv;
-            cm.mg[id] = s;
-            cm.mie[id] = INFINITY;
-        } else {
-            cm.mx[id] = nv.x[id];
-            cm.my[id] = nv.y[id];
-            cm.mg[id] = 0;
-            cm.mie[id] = 0;
-        }
+    const int a = nv.ch1[id];
+    first[a] = f;
+    first[a + 1] = f + nleaves[a];
+    const int p = pre[id];   // the first child's subtree (2 nleaves - 1 nodes) follows the node
+    pre[a] = p + 1;
+    pre[a + 1] = p + 2 * nleaves[a];
+}
+
+// The passes over the finished nodes.  In the levels over the whole list one
+// launch takes several consecutive levels, a block for all of them (levels
+// [l0, l1) of lev, at most kPassNodes nodes each: a level of a launch of its
+// own waits 4-7 us); larger levels are launched by themselves (one = true:
+// level l0 spread over the grid).  In the subtrees one block takes one
+// subtree.  Bottom-up, leaves go first, all at once.
+constexpr int kPassNodes = 8192, kPassThreads = 1024;
+
+__global__ __launch_bounds__(kPassThreads) void k_up_levels(NodeView nv, CMView cm, const int2* lev, int l0, int l1,
+                                                            const double* x, const double* y, const double* g,
+                                                            int32_t* nleaves) {
+    const int t = blockIdx.x * kPassThreads + threadIdx.x, step = gridDim.x * kPassThreads;
+    if (l1 - l0 > 1) {
+        for (int d = l0; d < l1; d++)
+            for (int id = lev[d].x + t; id < lev[d].y; id += step)
+                if (nv.split[id] != 2) up_node(nv, cm, id, x, y, g, nleaves);
+        __threadfence_block();
+        __syncthreads();
+    }
+    for (int d = l1 - 1; d >= l0; d--) {
+        for (int id = lev[d].x + t; id < lev[d].y; id += step)
+            if (l1 - l0 == 1 || nv.split[id] == 2) up_node(nv, cm, id, x, y, g, nleaves);
+        __threadfence_block();
+        __syncthreads();
     }
 }
 
-// Top-down over one level: first leaf rank of every subtree (DFS order).
-__global__ void k_down_level(NodeView nv, int lb, int le, const int32_t* nleaves, int32_t* first, int32_t* leaf_rank,
-                             int32_t* leaf_node, int32_t* vleaf, int32_t* pre) {
-    const int id = lb + blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= le) return;
-    const int f = first[id];
-    if (nv.split[id] == 2) {
-        const int a = nv.ch1[id];
-        first[a] = f;
-        first[a + 1] = f + nleaves[a];
-        const int p = pre[id];   // the first child's subtree (2 nleaves - 1 nodes) follows the node
-        pre[a] = p + 1;
-        pre[a + 1] = p + 2 * nleaves[a];
-    } else {
-        leaf_rank[id] = f;
-        leaf_node[f] = id;
-        for (int k = nv.v0[id]; k < nv.v1[id]; k++) vleaf[k] = f;
-        for (int k = nv.h0[id]; k < nv.h1[id]; k++) vleaf[k] = f;
-        for (int k = nv.s0[id]; k < nv.s1[id]; k++) vleaf[k] = f;
+__global__ __launch_bounds__(kPassThreads) void k_down_levels(NodeView nv, const int2* lev, int l0, int l1,
+                                                              const int32_t* nleaves, int32_t* first,
+                                                              int32_t* leaf_rank, int32_t* leaf_node, int32_t* vleaf,
+                                                              int32_t* pre) {
+    const int t = blockIdx.x * kPassThreads + threadIdx.x, step = gridDim.x * kPassThreads;
+    for (int d = l0; d < l1; d++) {
+        for (int id = lev[d].x + t; id < lev[d].y; id += step)
+            down_node(nv, id, nleaves, first, leaf_rank, leaf_node, vleaf, pre);
+        __threadfence_block();
+        __syncthreads();
+    }
+}
+
+// A subtree's nodes in LDS for the passes: numbered level after level, children
+// and leaf counts (and monopoles) of the first kPassLds; nodes beyond them are
+// read back from memory.  With every level's children behind two or three
+// dependent loads from memory a pass took 15-23 us for nine levels.
+constexpr int kPassLds = 1024;
+struct SubNodes {
+    int2 lev[kSubLevels];
+    int off[kSubLevels + 1];   // first node of a level in the numbering
+    int kid[kPassLds];         // first child (numbering), or -1
+    int nl[kPassLds];          // leaves under the node
+    int nlev, count;
+};
+
+__device__ inline void load_sub(SubNodes& N, const NodeView& nv, const int2* sub_lev, const int32_t* sub_nlev) {
+    const int t = threadIdx.x, nl = sub_nlev[blockIdx.x];
+    for (int d = t; d < nl; d += kBlock) N.lev[d] = sub_lev[(size_t)blockIdx.x * kSubLevels + d];
+    __syncthreads();
+    if (t == 0) {
+        int o = 0;
+        for (int d = 0; d < nl; d++) {
+            N.off[d] = o;
+            o += N.lev[d].y;
+        }
+        N.off[nl] = o;
+        N.nlev = nl;
+        N.count = o;
+    }
+    __syncthreads();
+    for (int n = t, d = 0; n < min(N.count, kPassLds); n += kBlock) {
+        while (N.off[d + 1] <= n) d++;
+        const int id = N.lev[d].x + (n - N.off[d]), sp = nv.split[id], ch = nv.ch1[id];
+        N.kid[n] = sp == 2 ? N.off[d + 1] + (ch - N.lev[d + 1].x) : -1;
+    }
+}
+
+__global__ __launch_bounds__(kBlock) void k_up_subs(NodeView nv, CMView cm, const int2* sub_lev,
+                                                    const int32_t* sub_nlev, const double* x, const double* y,
+                                                    const double* g, int32_t* nleaves) {
+    __shared__ SubNodes N;
+    __shared__ Monopoles M[kPassLds];
+    load_sub(N, nv, sub_lev, sub_nlev);
+    __syncthreads();
+    const int t = threadIdx.x;
+    auto is_leaf = [&](int n, int id) { return n < kPassLds ? N.kid[n] < 0 : nv.split[id] != 2; };
+    for (int n = t, d = 0; n < N.count; n += kBlock) {
+        while (N.off[d + 1] <= n) d++;
+        const int id = N.lev[d].x + (n - N.off[d]);
+        if (!is_leaf(n, id)) continue;
+        const Monopoles q = leaf_monopoles(nv, id, x, y, g);
+        put_monopoles(cm, id, q);
+        nleaves[id] = 1;
+        if (n < kPassLds) {
+            M[n] = q;
+            N.nl[n] = 1;
+        }
+    }
+    __threadfence_block();
+    __syncthreads();
+    for (int d = N.nlev - 2; d >= 0; d--) {   // the last level holds leaves only
+        for (int i = t; i < N.lev[d].y; i += kBlock) {
+            const int id = N.lev[d].x + i, n = N.off[d] + i;
+            if (is_leaf(n, id)) continue;
+            const int a = nv.ch1[id], ka = N.off[d + 1] + (a - N.lev[d + 1].x);
+            const bool in = ka + 1 < kPassLds;
+            const Monopoles q = in ? node_monopoles(nv, id, M[ka], M[ka + 1])
+                                   : node_monopoles(nv, id, get_monopoles(cm, a), get_monopoles(cm, a + 1));
+            const int cnt = in ? N.nl[ka] + N.nl[ka + 1] : nleaves[a] + nleaves[a + 1];
+            put_monopoles(cm, id, q);
+            nleaves[id] = cnt;
+            if (n < kPassLds) {
+                M[n] = q;
+                N.nl[n] = cnt;
+            }
+        }
+        __threadfence_block();
+        __syncthreads();
+    }
+}
+
+__global__ __launch_bounds__(kBlock) void k_down_subs(NodeView nv, const int2* sub_lev, const int32_t* sub_nlev,
+                                                      const int32_t* nleaves, int32_t* first, int32_t* leaf_rank,
+                                                      int32_t* leaf_node, int32_t* vleaf, int32_t* pre) {
+    __shared__ SubNodes N;
+    __shared__ int s_first[kPassLds], s_pre[kPassLds];
+    load_sub(N, nv, sub_lev, sub_nlev);
+    const int t = threadIdx.x;
+    for (int n = t, d = 0; n < min(N.count, kPassLds); n += kBlock) {
+        while (N.off[d + 1] <= n) d++;
+        N.nl[n] = nleaves[N.lev[d].x + (n - N.off[d])];
+    }
+    if (t < 2 && N.nlev > 0) {   // the root's children: k_down_levels set them
+        s_first[t] = first[N.lev[0].x + t];
+        s_pre[t] = pre[N.lev[0].x + t];
+    }
+    __syncthreads();
+    for (int d = 0; d < N.nlev; d++) {
+        for (int i = t; i < N.lev[d].y; i += kBlock) {
+            const int id = N.lev[d].x + i, n = N.off[d] + i;
+            if (n >= kPassLds) {
+                down_node(nv, id, nleaves, first, leaf_rank, leaf_node, vleaf, pre);
+                continue;
+            }
+            const int ka = N.kid[n];
+            if (ka < 0) {
+                down_leaf(nv, id, s_first[n], leaf_rank, leaf_node, vleaf);
+                continue;
+            }
+            const int a = N.lev[d + 1].x + (ka - N.off[d + 1]);
+            const int na = ka < kPassLds ? N.nl[ka] : nleaves[a];
+            const int f[2] = {s_first[n], s_first[n] + na}, q[2] = {s_pre[n] + 1, s_pre[n] + 2 * na};
+            for (int k = 0; k < 2; k++) {
+                pre[a + k] = q[k];
+                if (ka + k < kPassLds) {
+                    s_first[ka + k] = f[k];
+                    s_pre[ka + k] = q[k];
+                } else {
+                    first[a + k] = f[k];
+                }
+            }
+        }
+        __threadfence_block();
+        __syncthreads();
     }
 }
 
@@ -1031,6 +1597,21 @@ void scan_flags(Ctx& c, const GoesLeftFlag& f, int32_t* flag, int32_t* P, int32_
 
 }  // namespace
 
+void for_level_runs(const TreeArrays& t, bool up, const std::function<void(int, int, int)>& run) {
+    const int n = (int)t.levels.size();
+    auto size = [&](int d) { return t.levels[d].second - t.levels[d].first; };
+    std::vector<std::array<int, 3>> runs;
+    for (int d = 0; d < n;) {
+        int e = d + 1;
+        if (size(d) <= kPassNodes)
+            while (e < n && size(e) <= kPassNodes) e++;
+        runs.push_back({d, e, size(d) <= kPassNodes ? 1 : nblocks(size(d), kPassThreads)});
+        d = e;
+    }
+    if (up) std::reverse(runs.begin(), runs.end());
+    for (const auto& r : runs) run(r[0], r[1], r[2]);
+}
+
 void tree_build(Ctx& c, int far_criteria, double min_node, double max_node, int32_t* perm_out) {
     TreeArrays& t = c.t;
     const int nvort = (int)c.n;
@@ -1086,17 +1667,21 @@ void tree_build(Ctx& c, int far_criteria, double min_node, double max_node, int3
     int32_t* right_pos = c.iscratch3.p + n + 1;
     DBuf<int32_t>& node_L = t.node_L;
     DBuf<int32_t>& node_m = t.node_m;
-    DBuf<int32_t>& leaf_tmp = t.leaf_tmp;
     DBuf<int32_t>& seg_node = t.seg_node;
     node_L.grow(3 * (size_t)cap);
     node_m.grow(3 * (size_t)cap);
-    leaf_tmp.grow(cap);
+    // subtrees: about n / kSubElems of them are expected; nodes beyond the
+    // table stay with the level kernels
+    const int sub_cap = 4 * (n / kSubElems + nroots) + 4096;
+    t.sub_lev.grow((size_t)sub_cap * kSubLevels);
+    t.sub_nlev.grow(sub_cap);
+    t.lev_d.grow(kMaxLevels + 2);
     seg_node.grow(nseg + 1);
     NodeView nv = view(t);
     hipStream_t s = c.stream;
 
     hipLaunchKernelGGL(k_init_roots, dim3(nblocks(nroots)), dim3(kBlock), 0, s, nv, nroots, (const int64_t*)c.sim_off.p,
-                       t.counters.p, t.hbase, t.sbase, n);
+                       t.counters.p, t.lev_d.p, t.hbase, t.sbase, n);
     hipLaunchKernelGGL(k_iota, dim3(nblocks(n)), dim3(kBlock), 0, s, c.id.p, n);
     hipLaunchKernelGGL(k_fill_roots, dim3(nblocks(n)), dim3(kBlock), 0, s, enode.p, n, (const int64_t*)c.sim_off.p,
                        nroots);
@@ -1113,22 +1698,17 @@ void tree_build(Ctx& c, int far_criteria, double min_node, double max_node, int3
         hipLaunchKernelGGL(k_root_segs, dim3(nblocks(nseg)), dim3(kBlock), 0, s, nv, c.segs.p,
                            (const int32_t*)c.seg_root.p, nseg);
 
-    std::vector<std::pair<int, int>>& levels = t.levels;   // node id range of every level
-    levels.clear();
-    levels.push_back({0, nroots});
-    // One level per iteration.  The kernels take their node range from the
-    // device counters; the host reads a level's counters (copied to a pinned
-    // slot) only to record the range and to stop, and it keeps kLevSlots - 1
-    // further levels enqueued meanwhile, so the device does not wait for the
-    // host between levels.  Levels after the last one find an empty range and
-    // do nothing.
+    // One level per iteration over the whole list, its kernels taking their node
+    // range from the device counters.  No node can fit a workgroup before the
+    // largest root has been halved down to kSubElems elements, so the levels up
+    // to there are queued without asking; from there on k_subtree takes what
+    // fits, and the host reads after it whether anything is left.
     auto launch_level = [&](int d) {
         const int node_blocks = 1024;
-        hipLaunchKernelGGL(k_decide, dim3(node_blocks), dim3(kBlock), 0, s, nv, t.counters.p, leaf_tmp.p, cap,
-                           min_node, max_node);
+        hipLaunchKernelGGL(k_decide, dim3(node_blocks), dim3(kBlock), 0, s, nv, t.counters.p, cap, min_node, max_node);
         scan_flags(c, GoesLeftFlag{nv, enode.p, c.x.p, c.y.p, n}, flag, P, reinterpret_cast<int32_t*>(c.tmp.p), n + 1);
         hipLaunchKernelGGL(k_ranks, dim3(nblocks(n + 1)), dim3(kBlock), 0, s, nv, enode.p, P, n, t.hbase, t.sbase, cap,
-                           node_L.p, node_m.p, left_pos, right_pos, t.counters.p, (const int32_t*)flag);
+                           node_L.p, node_m.p, left_pos, right_pos, t.counters.p, (const int32_t*)flag, t.lev_d.p, d + 1);
         // the children of level d number at most nroots 2^(d+1)
         const bool top = ((int64_t)nroots << std::min<int>(d + 1, 30)) <= kTopNodes;
         hipLaunchKernelGGL(k_swap, dim3(nblocks(n)), dim3(kBlock), 0, s, nv, enode.p, flag, P, n, t.hbase, t.sbase,
@@ -1151,25 +1731,40 @@ void tree_build(Ctx& c, int far_criteria, double min_node, double max_node, int3
         }
         if (nseg)
             hipLaunchKernelGGL(k_seg_step, dim3(nblocks(nseg)), dim3(kBlock), 0, s, nv, c.segs.p, nseg, seg_node.p);
-        int32_t* slot = c.lev_counters + 8 * (d % Ctx::kLevSlots);
-        VVHD_HIP(hipMemcpyAsync(slot, t.counters.p, 8 * sizeof(int32_t), hipMemcpyDeviceToHost, s));
-        VVHD_HIP(hipEventRecord(c.lev_ev[d % Ctx::kLevSlots], s));
     };
-    int32_t hc[8];
-    constexpr int ahead = Ctx::kLevSlots - 1;
-    for (int d = 0; d < ahead; d++) launch_level(d);
-    for (int d = 0;; d++) {
-        launch_level(d + ahead);
-        VVHD_HIP(hipEventSynchronize(c.lev_ev[d % Ctx::kLevSlots]));
-        std::memcpy(hc, c.lev_counters + 8 * (d % Ctx::kLevSlots), sizeof(hc));
-        VVHD_CHECK(hc[4] == 0, VVHD_ENOMEM, "tree_build: node capacity exceeded");
-        if (hc[3] == hc[2]) break;   // level d made no new nodes; the levels after it did nothing
-        levels.push_back({hc[2], hc[3]});
-        VVHD_CHECK((int)levels.size() < kMaxLevels, VVHD_EUNSUPPORTED, "tree_build: tree deeper than supported");
+    int64_t largest = n;   // elements of the largest root
+    if (nroots > 1) {
+        largest = 0;
+        for (int q = 0; q < nroots; q++) largest = std::max(largest, c.sim_off_h[q + 1] - c.sim_off_h[q]);
+    }
+    int depth = 0;
+    for (; (largest >> depth) > kSubElems; depth++) launch_level(depth);
+    int32_t* hc = c.lev_counters;   // pinned
+    for (;; depth++) {
+        const int grid = (int)std::min<int64_t>(2 * c.n_cu, (int64_t)nroots << std::min(depth, 20));
+        hipLaunchKernelGGL(k_subtree, dim3(grid), dim3(kSubThreads), 0, s, nv, t.counters.p, cap, min_node, max_node,
+                           enode.p, c.x.p, c.y.p, c.id.p, (const vvhd_seg*)c.segs.p, nseg, seg_node.p, t.sub_lev.p,
+                           t.sub_nlev.p, sub_cap);
+        VVHD_HIP(hipMemcpyAsync(hc, t.counters.p, 10 * sizeof(int32_t), hipMemcpyDeviceToHost, s));
+        VVHD_HIP(hipStreamSynchronize(s));
+        VVHD_CHECK(hc[4] != 1, VVHD_ENOMEM, "tree_build: node capacity exceeded");
+        VVHD_CHECK(hc[4] == 0 && depth < kMaxLevels - 1, VVHD_EUNSUPPORTED, "tree_build: tree deeper than supported");
+        if (hc[6] == 0) break;   // the level's nodes are all decided
+        hipLaunchKernelGGL(k_level_begin, dim3(1), dim3(64), 0, s, t.counters.p);
+        launch_level(depth);
     }
     t.nnodes = hc[0];
     t.nleaves_h = hc[1];
     t.max_depth = hc[5];
+    t.nsub = std::min(hc[7], sub_cap);
+    // node ranges of the levels over the whole list
+    const int nlev = depth + 1;
+    std::vector<int2> lv(nlev);
+    VVHD_HIP(hipMemcpyAsync(lv.data(), t.lev_d.p, nlev * sizeof(int2), hipMemcpyDeviceToHost, s));
+    VVHD_HIP(hipStreamSynchronize(s));
+    std::vector<std::pair<int, int>>& levels = t.levels;
+    levels.clear();
+    for (const int2& q : lv) levels.push_back({q.x, q.y});
     const int nl = t.nleaves_h;
 
     // tree order of the remaining fields
@@ -1193,19 +1788,24 @@ void tree_build(Ctx& c, int far_criteria, double min_node, double max_node, int3
 
     // leaf counts and monopoles bottom-up, DFS ranks top-down
     CMView cm{t.cmp_x.p, t.cmp_y.p, t.cmp_g.p, t.cmm_x.p, t.cmm_y.p, t.cmm_g.p, t.cmp_ie.p, t.cmm_ie.p};
-    for (int d = (int)levels.size() - 1; d >= 0; d--) {
-        const int lb = levels[d].first, le = levels[d].second;
-        hipLaunchKernelGGL(k_up_level, dim3(nblocks(le - lb)), dim3(kBlock), 0, s, nv, cm, lb, le, c.x.p, c.y.p,
-                           c.g.p, t.nleaves.p);
-    }
+    if (t.nsub)
+        hipLaunchKernelGGL(k_up_subs, dim3(t.nsub), dim3(kBlock), 0, s, nv, cm, (const int2*)t.sub_lev.p,
+                           (const int32_t*)t.sub_nlev.p, c.x.p, c.y.p, c.g.p, t.nleaves.p);
+    for_level_runs(t, true, [&](int l0, int l1, int grid) {
+        hipLaunchKernelGGL(k_up_levels, dim3(grid), dim3(kPassThreads), 0, s, nv, cm, (const int2*)t.lev_d.p, l0, l1,
+                           c.x.p, c.y.p, c.g.p, t.nleaves.p);
+    });
     int32_t* first = t.arrive.p;
     t.root_first.grow(nroots + 1);
     hipLaunchKernelGGL(k_root_first, dim3(1), dim3(1), 0, s, t.nleaves.p, nroots, first, t.root_first.p, t.pre.p);
-    for (int d = 0; d < (int)levels.size(); d++) {
-        const int lb = levels[d].first, le = levels[d].second;
-        hipLaunchKernelGGL(k_down_level, dim3(nblocks(le - lb)), dim3(kBlock), 0, s, nv, lb, le, t.nleaves.p, first,
-                           t.leaf_rank.p, t.leaf_node.p, t.vleaf.p, t.pre.p);
-    }
+    for_level_runs(t, false, [&](int l0, int l1, int grid) {
+        hipLaunchKernelGGL(k_down_levels, dim3(grid), dim3(kPassThreads), 0, s, nv, (const int2*)t.lev_d.p, l0, l1,
+                           t.nleaves.p, first, t.leaf_rank.p, t.leaf_node.p, t.vleaf.p, t.pre.p);
+    });
+    if (t.nsub)
+        hipLaunchKernelGGL(k_down_subs, dim3(t.nsub), dim3(kBlock), 0, s, nv, (const int2*)t.sub_lev.p,
+                           (const int32_t*)t.sub_nlev.p, t.nleaves.p, first, t.leaf_rank.p, t.leaf_node.p, t.vleaf.p,
+                           t.pre.p);
     // leaf -> simulation and the list builder's leaf groups (64 leaves of one root)
     t.leaf_sim.grow(nl + 1);
     std::vector<int32_t> grp;
