@@ -401,11 +401,14 @@ __device__ inline Seen seen_of(const MergeArgs& A, int j, int i, int2 f) {
 
 // The two nearest of target i among what it sees in its near leaves, at
 // (px, py), without itself and excl: the leaves touching its own first, then
-// those whose box lies within the second-neighbour distance found.  One wave;
-// all lanes get the result.  Latency-bound: the entries of 256 list places,
-// their boxes and ranges load together, and the candidates of all of them
-// are listed in LDS, so that a search is about four dependent loads.
-__device__ Top2 seen_top2(const MergeArgs& A, int l, int L, int i, int excl, double px, double py, int* tab) {
+// those whose box lies within the second-neighbour distance found.  G waves
+// (1, or all of the block) share the list; all lanes get the result.
+// Latency-bound: the entries of 256 list places, their boxes and ranges load
+// together, and the candidates of all of them are listed in LDS, so that a
+// search is about four dependent loads.
+template <int G>
+__device__ Top2 seen_top2(const MergeArgs& A, int l, int L, int i, int excl, double px, double py, int* tab,
+                          Top2* parts) {
     const TreeDev& T = A.T;
     const int lane = lane_id();
     const int64_t e0 = T.near_off[l], e1 = T.near_off[l + 1];
@@ -417,7 +420,8 @@ __device__ Top2 seen_top2(const MergeArgs& A, int l, int L, int i, int excl, dou
     };
     auto scan = [&](bool touching, double bound) {
         Top2 st = top2_empty();
-        for (int64_t eb = e0; eb < e1; eb += kPer * kWave) {
+        const int w = G == 1 ? 0 : threadIdx.x / kWave;
+        for (int64_t eb = e0 + (int64_t)w * kPer * kWave; eb < e1; eb += (int64_t)G * kPer * kWave) {
             int M[kPer], j0[kPer], cnt[kPer], mine = 0;
 #pragma unroll
             for (int k = 0; k < kPer; k++) {
@@ -455,7 +459,15 @@ __device__ Top2 seen_top2(const MergeArgs& A, int l, int L, int i, int excl, dou
                 wave_sync();
             }
         }
-        return wave_top2(st);
+        st = wave_top2(st);
+        if (G > 1) {
+            __syncthreads();   // parts of the search before are read
+            if (lane == 0) parts[w] = st;
+            __syncthreads();
+            st = parts[0];
+            for (int q = 1; q < G; q++) top2_merge(st, parts[q]);
+        }
+        return st;
     };
     Top2 c = scan(true, 0.0);
     top2_merge(c, scan(false, c.i2 >= 0 ? c.d2 : INFINITY));
@@ -475,16 +487,19 @@ __global__ void k_merge_init(MergeArgs A) {
 }
 
 // One round, first part: every listed target is visited as the reference does
-// when the merges of the targets before it are those of the last round; one
-// wave per target.  Its search results are written in place (only the marking
-// pass reads them), its merge goes to cand and the list of changes.
-__global__ __launch_bounds__(kBlock) void k_merge_eval(MergeArgs A, int parity) {
-    __shared__ int s_tab[kWavesPerBlock][kMergeTab];
+// when the merges of the targets before it are those of the last round.  Its
+// search results are written in place (only the marking pass reads them), its
+// merge goes to cand and the list of changes.  A wave takes a target, or while
+// there are no more targets than blocks a whole block: the near list of a wide
+// leaf at a cluster's rim runs to thousands of leaves, 300 us for one wave.
+constexpr int kEvalThreads = 512, kEvalWaves = kEvalThreads / kWave, kEvalBlocks = 512;
+template <int G>
+__device__ void merge_eval(const MergeArgs& A, int parity, int nd, int (*s_tab)[kMergeTab], Top2* parts) {
     const TreeDev& T = A.T;
     const int w = threadIdx.x / kWave, lane = lane_id();
-    const int nd = A.ctr[parity];
     const int32_t* list = parity ? A.list1 : A.list0;
-    for (int k = blockIdx.x * kWavesPerBlock + w; k < nd; k += gridDim.x * kWavesPerBlock) {
+    const int k0 = G == 1 ? blockIdx.x * kEvalWaves + w : blockIdx.x;
+    for (int k = k0; k < nd; k += G == 1 ? gridDim.x * kEvalWaves : gridDim.x) {
         const int i = list[k];
         const double gi = A.g[i];
         const int2 own = A.info[i];
@@ -496,7 +511,7 @@ __global__ __launch_bounds__(kBlock) void k_merge_eval(MergeArgs A, int parity) 
         double first_d2 = -1.;
         if (alive) {
             double px = A.x[i], py = A.y[i];
-            st = seen_top2(A, l, L, i, -1, px, py, s_tab[w]);
+            st = seen_top2<G>(A, l, L, i, -1, px, py, s_tab[w], parts);
             first_d2 = st.d2;
             const double crit = A.crit[l];
             if (st.i1 >= 0 && st.i2 >= 0 && !isnan(crit)) {
@@ -516,11 +531,11 @@ __global__ __launch_bounds__(kBlock) void k_merge_eval(MergeArgs A, int parity) 
                         py = a.y;
                     }
                     rec = make_double4(px, py, gi + a.g, 0);
-                    st = seen_top2(A, l, L, i, partner, px, py, s_tab[w]);
+                    st = seen_top2<G>(A, l, L, i, partner, px, py, s_tab[w], parts);
                 }
             }
         }
-        if (lane != 0) continue;
+        if (lane != 0 || (G > 1 && w != 0)) continue;
         A.nn1[i] = st.i1;
         A.nn2[i] = st.i2;
         A.d1[i] = st.d1;
@@ -544,6 +559,16 @@ __global__ __launch_bounds__(kBlock) void k_merge_eval(MergeArgs A, int parity) 
             A.chg[atomicAdd(&A.ctr[2 + parity], 1)] = i;
         }
     }
+}
+
+__global__ __launch_bounds__(kEvalThreads) void k_merge_eval(MergeArgs A, int parity) {
+    __shared__ int s_tab[kEvalWaves][kMergeTab];
+    __shared__ Top2 s_parts[kEvalWaves];
+    const int nd = A.ctr[parity];
+    if (nd <= (int)gridDim.x)
+        merge_eval<kEvalWaves>(A, parity, nd, s_tab, s_parts);
+    else
+        merge_eval<1>(A, parity, nd, s_tab, s_parts);
 }
 
 // Second part, one workgroup: the changed records take effect, the deaths
@@ -775,7 +800,7 @@ void merge_rounds(Ctx& c, MergeArgs A, double* x, double* y, double* g, int32_t*
         VVHD_CHECK(round <= (int64_t)A.n + 8, VVHD_EHIP, "epsilon: the merges do not settle");
         for (int k = 0; k < 4; k++, round++) {
             const int par = (int)(round & 1);
-            hipLaunchKernelGGL(k_merge_eval, dim3(1024), dim3(kBlock), 0, s, A, par);
+            hipLaunchKernelGGL(k_merge_eval, dim3(kEvalBlocks), dim3(kEvalThreads), 0, s, A, par);
             hipLaunchKernelGGL(k_merge_apply, dim3(1), dim3(kMergeThreads), 0, s, A, par);
             hipLaunchKernelGGL(k_merge_mark, dim3(1024), dim3(kBlock), 0, s, A, par, chunks, (int)round + 1);
         }
