@@ -124,6 +124,35 @@ __device__ inline int xcd_block(int b, int nblocks) {
 
 // ------------------------------------------------------------------ context --
 
+// Log of the list builder (tree.hip: ListLog): R records and S items a group.
+struct ListLogBufs {
+    int R = 512, S = 64;
+    DBuf<int32_t> tid, gnodes, item_n, rid, most;
+    DBuf<uint64_t> tfar, tnear, item_mask, rfar, rnear;
+    DBuf<int64_t> gbase, totals;
+    DBuf<int2> head, item, lanes, after;
+    void grow(int64_t groups, int64_t records) {
+        for (auto* b : {&tfar, &tnear}) b->grow(groups * R + 1);
+        tid.grow(groups * R + 1);
+        gnodes.grow(groups + 1);
+        gbase.grow(groups + 1);
+        head.grow(groups + 1);
+        item.grow(groups * S + 1);
+        item_mask.grow(groups * S + 1);
+        item_n.grow(groups * S + 1);
+        for (auto* b : {&lanes, &after}) b->grow((groups * S + 1) * 64);
+        rid.grow(records + 1);
+        for (auto* b : {&rfar, &rnear}) b->grow(rid.cap);
+    }
+    void release() {
+        for (auto* b : {&tid, &gnodes, &item_n, &rid, &most}) b->release();
+        for (auto* b : {&tfar, &tnear, &item_mask, &rfar, &rnear}) b->release();
+        gbase.release();
+        totals.release();
+        for (auto* b : {&head, &item, &lanes, &after}) b->release();
+    }
+};
+
 constexpr int kSubLevels = 128;   // levels of a subtree in TreeArrays::sub_lev
 
 struct TreeArrays {
@@ -154,9 +183,8 @@ struct TreeArrays {
     DBuf<int32_t> seg_keys, seg_ids;      // sort scratch of the per-leaf segment lists
     DBuf<int32_t> vleaf;                  // per element (vortex, heat, streak): leaf (DFS)
     DBuf<int32_t> node_L, node_m, seg_node;             // build scratch
-    DBuf<int32_t> cnt_near, cnt_far, err;               // list scratch
-    DBuf<int64_t> slot_near, slot_far;                  // per (leaf, top entry) list offsets
-    DBuf<uint8_t> entries;                              // top-of-tree entry tables of the list builder (per root)
+    DBuf<int32_t> cnt_near, cnt_far;                    // list entries per leaf
+    ListLogBufs log;                                    // records of the list builder's walks
     DBuf<uint8_t> trav;                                 // packed node records of the list builder
     DBuf<double4> pbox;                                 // packed node boxes (pack_boxes)
     DBuf<int32_t> groups;                               // list builder leaf groups: {first leaf, count, root}

@@ -221,11 +221,11 @@ void vvhd_destroy(vvhd_ctx* ctx) {
     for (auto* b : {&t.blx, &t.bly, &t.trx, &t.try_, &t.path}) b->release();
     for (auto* b : {&t.v0, &t.v1, &t.ch1, &t.parent, &t.depth, &t.nseg, &t.split, &t.nleaves, &t.arrive, &t.leaf_rank,
                     &t.counters, &t.leaf_node, &t.near_list, &t.far_list, &t.seg_list, &t.seg_leaf, &t.vleaf,
-                    &t.node_L, &t.node_m, &t.sub_nlev, &t.seg_node, &t.cnt_near, &t.cnt_far, &t.err})
+                    &t.node_L, &t.node_m, &t.sub_nlev, &t.seg_node, &t.cnt_near, &t.cnt_far})
         b->release();
-    for (auto* b : {&t.near_off, &t.far_off, &t.seg_off, &t.slot_near, &t.slot_far}) b->release();
+    for (auto* b : {&t.near_off, &t.far_off, &t.seg_off}) b->release();
     for (auto* b : {&t.groups, &t.leaf_sim, &t.root_first, &t.pre}) b->release();
-    t.entries.release();
+    t.log.release();
     t.lev_d.release();
     t.sub_lev.release();
     t.trav.release();

@@ -1268,86 +1268,6 @@ __global__ __launch_bounds__(kBlock) void k_down_subs(NodeView nv, const int2* s
     }
 }
 
-// FindNearNodes (TSortedTree.cpp:199-217) split over the top of the tree:
-// the "entries" are the nodes at depth kSplitDepth plus the shallower
-// leaves, in DFS order (at most 2^kSplitDepth).  One wave handles one entry
-// for 64 DFS-consecutive leaves: each lane first tests the entry's
-// ancestors for its leaf, then the wave walks the entry's subtree once (a
-// node is expanded while any lane still needs it; a lane that classifies a
-// node as far ignores the rest of that subtree).  The split gives
-// 2^kSplitDepth times more independent waves than leaf groups, which hides
-// the latency of the dependent node loads.  Emissions follow the
-// reference's preorder: a far ancestor is emitted by the first entry beneath
-// it only, and the per-(leaf, entry) segments are concatenated in entry
-// order.
-#ifndef VVHD_LIST_SPLIT_DEPTH
-#define VVHD_LIST_SPLIT_DEPTH 6
-#endif
-constexpr int kSplitDepth = VVHD_LIST_SPLIT_DEPTH;
-constexpr int kMaxEntries = 1 << kSplitDepth;
-
-struct ListEntries {
-    int n;                                 // number of entries
-    int node[kMaxEntries];                 // entry node (preorder position)
-    int depth[kMaxEntries];                // its depth (<= kSplitDepth)
-    int anc[kMaxEntries][kSplitDepth];     // ancestors, root first (preorder positions)
-    int lead[kMaxEntries];                 // bit d: first entry beneath anc[d]
-};
-
-// Entry table of every root, one wave per root: the frontier starts at the
-// root and is expanded kSplitDepth times (an internal node above the split
-// depth is replaced by its two children in place), which keeps it in DFS
-// order; at most 2^kSplitDepth = 64 entries, one per lane.
-__global__ void k_list_entries(NodeView nv, const int32_t* pre, int nroots, ListEntries* Etab) {
-    __shared__ int fr[2][kMaxEntries];
-    const int r = blockIdx.x;
-    const int lane = threadIdx.x;
-    ListEntries* E = Etab + r;
-    if (lane == 0) fr[0][0] = r;
-    int n = 1, cur = 0;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    for (int step = 0; step < kSplitDepth; step++) {
-        const int T = lane < n ? fr[cur][lane] : -1;
-        int c = -1;
-        if (T >= 0 && nv.depth[T] < kSplitDepth) c = nv.ch1[T];
-        const int out = T < 0 ? 0 : (c >= 0 ? 2 : 1);
-        const int incl = wave_incl_scan(out);
-        const int pos = incl - out;
-        if (c >= 0) {
-            fr[cur ^ 1][pos] = c;
-            fr[cur ^ 1][pos + 1] = c + 1;
-        } else if (T >= 0) {
-            fr[cur ^ 1][pos] = T;
-        }
-        n = __shfl(incl, kWave - 1, kWave);
-        cur ^= 1;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-    if (lane < n) {
-        const int T = fr[cur][lane];
-        const int d = nv.depth[T];
-        E->node[lane] = pre[T];
-        E->depth[lane] = d;
-        // ancestors, root first; T is the first entry beneath an ancestor when
-        // every step from it down is to a first child
-        int c = T, lead = 0;
-        bool first = true;
-        for (int k = d - 1; k >= 0; k--) {
-            const int p = nv.parent[c];
-            E->anc[lane][k] = pre[p];
-            first = first && (nv.ch1[p] == c);
-            if (first) lead |= 1 << k;
-            c = p;
-        }
-        E->lead[lane] = lead;
-    }
-    if (lane == 0) E->n = n;
-}
-
 __global__ void k_pack_boxes(NodeView nv, int nnodes, double4* out) {
     const int id = blockIdx.x * blockDim.x + threadIdx.x;
     if (id >= nnodes) return;
@@ -1366,8 +1286,10 @@ struct TravNode {
 };
 static_assert(sizeof(TravNode) == 32, "TravNode layout");
 
-__global__ void k_trav_nodes(NodeView nv, int nnodes, const int32_t* pre, const int32_t* nleaves, TravNode* out) {
+__global__ void k_trav_nodes(NodeView nv, int nnodes, const int32_t* pre, const int32_t* nleaves, TravNode* out,
+                             int32_t* most) {
     const int id = blockIdx.x * blockDim.x + threadIdx.x;
+    if (id < 2) most[id] = 0;
     if (id >= nnodes) return;
     TravNode r;
     r.x = nv.x[id];
@@ -1379,38 +1301,80 @@ __global__ void k_trav_nodes(NodeView nv, int nnodes, const int32_t* pre, const 
     out[p] = r;
 }
 
-// Near and far lists of every leaf, two passes (counts, then entries at the
-// scanned offsets).  A wave takes one entry of one root for a group of up to
-// 64 DFS-consecutive leaves (one leaf per lane) and writes slot (leaf,
-// entry).  The wave walks the entry's subtree in preorder without a stack:
-// from a node it moves to the next position (the first child) when some lane
-// still needs the node's subtree, otherwise past the subtree.  A lane that
-// classifies a node as far (or reaches a near leaf) waits until the walk
-// leaves that subtree.
-__global__ __launch_bounds__(kBlock) void k_lists(NodeView nv, const TravNode* __restrict__ tn,
-                                                  const ListEntries* __restrict__ Etab,
-                                                  const int32_t* __restrict__ groups, int ngroups,
-                                                  const int32_t* leaf_node, double fc, int nnodes,
-                                                  const int64_t* near_off, const int64_t* far_off,
-                                                  int32_t* near_list, int32_t* far_list, int32_t* near_cnt,
-                                                  int32_t* far_cnt) {
-    const int w = threadIdx.x / kWave;
-    const int wave = blockIdx.x * (kBlock / kWave) + w;
-    const int q = wave % kMaxEntries;
-    const int grp = wave / kMaxEntries;
-    if (grp >= ngroups) return;
-    const int lane = lane_id();
-    // a group: up to 64 DFS-consecutive leaves of one root
-    const int l = groups[3 * grp] + lane;
-    const ListEntries* E = Etab + groups[3 * grp + 2];
-    if (q >= E->n) return;   // uniform over the wave
-    const bool valid = lane < groups[3 * grp + 1];
-    if (__ballot(valid) == 0) return;
-    const int L = valid ? leaf_node[l] : 0;
-    const double lx = nv.x[L], ly = nv.y[L], lh = nv.h[L], lw = nv.w[L];   // (h_T + w_T) + lh + lw below
-    const size_t slot = (size_t)l * kMaxEntries + q;
-    int64_t pn = (valid && near_off) ? near_off[slot] : 0, pf = (valid && far_off) ? far_off[slot] : 0;
-    int cn = 0, cf = 0;
+// FindNearNodes (TSortedTree.cpp:199-217) of every leaf: one walk that logs
+// its steps, then a replay of the log at the scanned offsets.
+// A wave walks for a group of up to 64 DFS-consecutive leaves of one root, a
+// leaf per lane, in preorder without a stack: from a node it moves to the next
+// position (the first child) while some lane still needs the node's subtree,
+// otherwise past the subtree.  A lane that classifies a node as far (or
+// reaches a near leaf) waits until the walk leaves that subtree.  Every step
+// at which some lane lists the node is a record {node, far lanes, near lanes}.
+// k_list_top walks a group's nodes with more than item_nodes nodes below
+// them; a smaller subtree that is still needed becomes an item, noted in the
+// group's log and walked by a wave of its own (k_list_items).  k_list_sums
+// adds up, in the order of the group's log, what each lane has listed before
+// every item and in all; k_list_replay writes the records at these offsets,
+// so that the lists hold the reference's preorder.
+// Bound by the instructions and load latency of the steps (3.9 M for 57.7 M
+// entries at 1M) and by how evenly they spread: cut at depth 6, the longest of
+// 98k walks had 3101 steps and 1200 walks held nearly all of them, and the
+// steps were walked twice, to count and to write.  No counter is shared
+// between waves (50k claims of one address cost 0.7 ms).
+struct ListLog {
+    int R, S;                    // records and items a group has room for
+    int64_t cap;                 // records of all items
+    int32_t* tid;                // groups x R: node, or -(item of the group + 1)
+    uint64_t *tfar, *tnear;
+    int2* head;                  // per group: records, items
+    int32_t* gnodes;             // per group: nodes of its items (their records at most)
+    const int64_t* gbase;        // their exclusive sums
+    int2* item;                  // groups x S: position, first record within the group's
+    uint64_t* item_mask;         // lanes that need it
+    int32_t* item_n;             // its records
+    int2 *lanes, *after;         // groups x S x 64: near and far nodes a lane lists in the item, then before it; and after it
+    int32_t* rid;
+    uint64_t *rfar, *rnear;
+    int32_t* most;               // [0] records, [1] items of a group beyond its room
+};
+
+// The records of one walk at [o, o + limit): record k of every 64 is collected
+// in lane k, 64 go out in one coalesced store.  Records past the limit are
+// counted only.
+struct LogWriter {
+    int32_t* id;
+    uint64_t *far, *near;
+    int64_t limit;
+    const int lane;
+    int32_t rid = 0;
+    uint64_t rf = 0, rn = 0;
+    int cnt = 0;
+    int64_t done = 0;
+    __device__ inline void push(int32_t i, uint64_t F, uint64_t N) {
+        if (lane == cnt) {
+            rid = i;
+            rf = F;
+            rn = N;
+        }
+        if (++cnt == kWave) flush();
+    }
+    __device__ inline void flush() {
+        if (lane < cnt && done + lane < limit) {
+            id[done + lane] = rid;
+            far[done + lane] = rf;
+            near[done + lane] = rn;
+        }
+        done += cnt;
+        cnt = 0;
+    }
+};
+
+// Walks positions [P, end) for the lanes' leaves (a lane takes part at
+// positions >= resume); subtrees of at most item_nodes nodes go to item(P,
+// nodes, lanes) and are passed over.  cn, cf: the lane's listed nodes.
+template <typename Item>
+__device__ inline void list_walk(const TravNode* __restrict__ tn, int P, int end, int resume, double lx, double ly,
+                                 double lh, double lw, double fc, int item_nodes, LogWriter& log, int& cn, int& cf,
+                                 Item item) {
     // the position is uniform: records come through the scalar cache, all
     // 32 bytes in one load
     auto rec = [&](int p) {
@@ -1421,34 +1385,6 @@ __global__ __launch_bounds__(kBlock) void k_lists(NodeView nv, const TravNode* _
         __builtin_memcpy(reinterpret_cast<char*>(&r) + 16, &u1, 16);
         return r;
     };
-    const int P0 = __builtin_amdgcn_readfirstlane(E->node[q]);
-    const int dE = __builtin_amdgcn_readfirstlane(E->depth[q]);
-    const int lead = __builtin_amdgcn_readfirstlane(E->lead[q]);
-    // the entry's own record and its ancestors' are all loaded before any is
-    // used, so their latencies overlap
-    TravNode anc[kSplitDepth];
-#pragma unroll
-    for (int k = 0; k < kSplitDepth; k++)
-        if (k < dE) anc[k] = rec(__builtin_amdgcn_readfirstlane(E->anc[q][k]));
-    const int end = min(rec(P0).skip, nnodes);
-    // a lane takes part at positions >= resume
-    int resume = valid ? P0 : end;
-    // ancestors of the entry: the first far one (if any) cuts the whole entry
-#pragma unroll
-    for (int k = 0; k < kSplitDepth; k++) {
-        if (k >= dE || !valid || resume == end) continue;
-        const TravNode& a = anc[k];
-        const double dx = a.x - lx, dy = a.y - ly;
-        const double hp = a.hw + lh + lw;
-        if (dx * dx + dy * dy > fc * hp * hp) {
-            if ((lead >> k) & 1) {
-                if (far_list) far_list[pf++] = a.id;
-                cf++;
-            }
-            resume = end;
-        }
-    }
-    int P = __builtin_amdgcn_readfirstlane(__ballot(resume < end) != 0 ? P0 : end);
     while (P < end) {
         const TravNode r = rec(P);
         const int skip = __builtin_amdgcn_readfirstlane(r.skip);
@@ -1458,25 +1394,233 @@ __global__ __launch_bounds__(kBlock) void k_lists(NodeView nv, const TravNode* _
         const double dx = r.x - lx, dy = r.y - ly;
         const double hp = r.hw + lh + lw;
         const bool far = act && (dx * dx + dy * dy > fc * hp * hp);
+        const bool near = act && leaf && !far;
         if (far) {
-            if (far_list) far_list[pf++] = id;
             cf++;
             resume = skip;
-        } else if (act && leaf) {
-            if (near_list) near_list[pn++] = id;
-            cn++;
         }
-        const bool need = act && !far && !leaf;
-        P = __builtin_amdgcn_readfirstlane(__ballot(need) != 0 ? P + 1 : max(skip, P + 1));
+        if (near) cn++;
+        const uint64_t F = __ballot(far), N = __ballot(near);
+        const uint64_t need = leaf ? 0 : __ballot(act && !far);
+        if (F | N) log.push(id, F, N);
+        if (need == 0) {
+            P = max(skip, P + 1);
+        } else if (skip - P <= item_nodes) {
+            item(P, skip - P, need);
+            P = skip;
+        } else {
+            P = P + 1;
+        }
+        P = __builtin_amdgcn_readfirstlane(P);
     }
-    if (valid && near_cnt) near_cnt[slot] = cn;
-    if (valid && far_cnt) far_cnt[slot] = cf;
 }
 
-// Per-leaf CSR offsets from the per-(leaf, entry) offsets.
-__global__ void k_leaf_offsets(const int64_t* slot_off, int nleaf, int64_t* leaf_off) {
-    const int l = blockIdx.x * blockDim.x + threadIdx.x;
-    if (l <= nleaf) leaf_off[l] = slot_off[(size_t)l * kMaxEntries];
+__global__ __launch_bounds__(kBlock) void k_list_top(NodeView nv, const TravNode* __restrict__ tn,
+                                                     const int32_t* __restrict__ pre,
+                                                     const int32_t* __restrict__ groups, int ngroups,
+                                                     const int32_t* leaf_node, double fc, int item_nodes, ListLog G) {
+    const int grp = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave, lane = lane_id();
+    if (grp >= ngroups) return;
+    const int l = groups[3 * grp] + lane;
+    const bool valid = lane < groups[3 * grp + 1];
+    const int L = valid ? leaf_node[l] : 0;
+    const int P0 = __builtin_amdgcn_readfirstlane(pre[groups[3 * grp + 2]]);
+    const int end = __builtin_amdgcn_readfirstlane(tn[P0].skip);
+    const size_t o = (size_t)grp * G.R, io = (size_t)grp * G.S;
+    LogWriter log{G.tid + o, G.tfar + o, G.tnear + o, G.R, lane};
+    int cn = 0, cf = 0, ni = 0, nodes = 0;
+    list_walk(tn, P0, end, valid ? P0 : end, nv.x[L], nv.y[L], nv.h[L], nv.w[L], fc, item_nodes, log, cn, cf,
+              [&](int P, int size, uint64_t need) {
+                  if (lane == 0 && ni < G.S) {
+                      G.item[io + ni] = make_int2(P, nodes);
+                      G.item_mask[io + ni] = need;
+                  }
+                  log.push(-(ni + 1), 0, 0);
+                  ni++;
+                  nodes += size;
+              });
+    log.flush();
+    if (lane != 0) return;
+    G.head[grp] = make_int2((int)log.done, ni);
+    G.gnodes[grp] = nodes;
+    if (log.done > G.R) atomicMax(&G.most[0], (int)log.done);
+    if (ni > G.S) atomicMax(&G.most[1], ni);
+}
+
+__global__ __launch_bounds__(kBlock) void k_list_items(NodeView nv, const TravNode* __restrict__ tn,
+                                                       const int32_t* __restrict__ groups, int ngroups,
+                                                       const int32_t* leaf_node, double fc, ListLog G) {
+    const int lane = lane_id();
+    const int wave = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
+    // item k of all groups, then item k + 1: a group has about 20 of its S items,
+    // and with a group's items in neighbouring blocks these fell on the same few
+    // XCDs (S = 64: 1.6 against 0.53 ms at 1M)
+    const int grp = __builtin_amdgcn_readfirstlane(wave % ngroups), k = __builtin_amdgcn_readfirstlane(wave / ngroups);
+    if (k >= G.S || k >= G.head[grp].y) return;
+    const size_t it = (size_t)grp * G.S + k;
+    const int P0 = __builtin_amdgcn_readfirstlane(G.item[it].x);
+    const int end = __builtin_amdgcn_readfirstlane(tn[P0].skip);
+    const bool mine = (G.item_mask[it] >> lane) & 1;
+    const int l = groups[3 * grp] + lane;
+    const int L = mine ? leaf_node[l] : 0;
+    const int64_t o = G.gbase[grp] + G.item[it].y;
+    const int64_t room = min((int64_t)(end - P0), max((int64_t)0, G.cap - o));
+    LogWriter log{G.rid + o, G.rfar + o, G.rnear + o, room, lane};
+    int cn = 0, cf = 0;
+    list_walk(tn, P0 + 1, end, mine ? P0 : end, nv.x[L], nv.y[L], nv.h[L], nv.w[L], fc, 0, log, cn, cf,
+              [](int, int, uint64_t) {});
+    log.flush();
+    if (lane == 0) G.item_n[it] = (int)log.done;
+    G.lanes[it * kWave + lane] = make_int2(cn, cf);
+}
+
+// Reads 64 records of a log at once, one per lane, and hands them out in order.
+struct LogReader {
+    const int32_t* id;
+    const uint64_t *far, *near;
+    int32_t rid = 0;
+    uint64_t rf = 0, rn = 0;
+    __device__ inline void load(int64_t o, int left, int lane) {
+        if (lane < left) {
+            rid = id[o + lane];
+            rf = far[o + lane];
+            rn = near[o + lane];
+        }
+    }
+    __device__ static inline uint64_t pick(uint64_t v, int k) {
+        return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(v >> 32), k) << 32) |
+               (uint32_t)__builtin_amdgcn_readlane((int)v, k);
+    }
+};
+
+// One wave per group: what each lane lists before every item of the group's
+// log (left in lanes), and in all (the leaf's counts).
+__global__ __launch_bounds__(kBlock) void k_list_sums(const int32_t* __restrict__ groups, int ngroups, ListLog G,
+                                                      int32_t* near_cnt, int32_t* far_cnt) {
+    const int grp = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave, lane = lane_id();
+    if (grp >= ngroups) return;
+    const int nrec = min(G.head[grp].x, G.R);
+    const size_t io = (size_t)grp * G.S;
+    LogReader rd{G.tid + (size_t)grp * G.R, G.tfar + (size_t)grp * G.R, G.tnear + (size_t)grp * G.R};
+    int cn = 0, cf = 0;
+    const int ni = min(G.head[grp].y, G.S);
+    int2 ahead = ni > 0 ? G.lanes[io * kWave + lane] : make_int2(0, 0);   // the next item's counts
+    for (int r0 = 0; r0 < nrec; r0 += kWave) {
+        rd.load(r0, nrec - r0, lane);
+        const int m = min(kWave, nrec - r0);
+        for (int k = 0; k < m; k++) {
+            const int id = __builtin_amdgcn_readlane(rd.rid, k);
+            if (id >= 0) {
+                cf += __builtin_amdgcn_inverse_ballot_w64(LogReader::pick(rd.rf, k)) ? 1 : 0;
+                cn += __builtin_amdgcn_inverse_ballot_w64(LogReader::pick(rd.rn, k)) ? 1 : 0;
+            } else if (-id <= ni) {
+                int2* p = G.lanes + (io + (-id - 1)) * kWave + lane;
+                const int2 c = ahead;
+                if (-id < ni) ahead = p[kWave];
+                *p = make_int2(cn, cf);
+                cn += c.x;
+                cf += c.y;
+                G.after[(io + (-id - 1)) * kWave + lane] = make_int2(cn, cf);
+            }
+        }
+    }
+    if (lane < groups[3 * grp + 1]) {
+        const int l = groups[3 * grp] + lane;
+        near_cnt[l] = cn;
+        far_cnt[l] = cf;
+    }
+}
+
+// A lane's list, written four entries at a time: a store of single entries
+// touches a line per lane and record (57.7 M of them, 0.47 ms at 1M).
+typedef int32_t int4u __attribute__((ext_vector_type(4), aligned(4)));
+struct ListOut {
+    int32_t* p;
+    int32_t b0 = 0, b1 = 0, b2 = 0, b3 = 0;
+    int n = 0;
+    __device__ inline void push(int32_t id) {
+        b0 = b1;
+        b1 = b2;
+        b2 = b3;
+        b3 = id;
+        if (++n == 4) {
+            *reinterpret_cast<int4u*>(p) = int4u{b0, b1, b2, b3};
+            p += 4;
+            n = 0;
+        }
+    }
+    __device__ inline void flush() {   // the last n of b0..b3
+        if (n == 3) p[0] = b1;
+        if (n >= 2) p[n - 2] = b2;
+        if (n >= 1) p[n - 1] = b3;
+        p += n;
+        n = 0;
+    }
+};
+
+// The records to the lists: wave k of a group writes item k, one more wave the
+// group's own records.
+__global__ __launch_bounds__(kBlock) void k_list_replay(const int32_t* __restrict__ groups, int ngroups, ListLog G,
+                                                        const int64_t* near_off, const int64_t* far_off,
+                                                        int32_t* near_list, int32_t* far_list) {
+    const int lane = lane_id();
+    const int wave = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
+    const int grp = __builtin_amdgcn_readfirstlane(wave % ngroups), k = __builtin_amdgcn_readfirstlane(wave / ngroups);
+    if (k > G.S) return;
+    const int ni = G.head[grp].y;
+    if (k >= ni && k < G.S) return;
+    const int l = groups[3 * grp] + lane;
+    const bool valid = lane < groups[3 * grp + 1];
+    const size_t io = (size_t)grp * G.S;
+    ListOut near{near_list + (valid ? near_off[l] : 0)}, far{far_list + (valid ? far_off[l] : 0)};
+    auto emit = [&](const LogReader& rd, int q, int id) {
+        const uint64_t F = LogReader::pick(rd.rf, q), N = LogReader::pick(rd.rn, q);
+        if (__builtin_amdgcn_inverse_ballot_w64(F)) far.push(id);
+        if (N != 0 && __builtin_amdgcn_inverse_ballot_w64(N)) near.push(id);
+    };
+    if (k < G.S) {
+        const int2 c = G.lanes[(io + k) * kWave + lane];
+        near.p += c.x;
+        far.p += c.y;
+        const int64_t o = G.gbase[grp] + G.item[io + k].y;
+        const int n = G.item_n[io + k];
+        LogReader rd{G.rid, G.rfar, G.rnear}, next = rd;
+        next.load(o, n, lane);
+        for (int r0 = 0; r0 < n; r0 += kWave) {
+            rd = next;
+            if (r0 + kWave < n) next.load(o + r0 + kWave, n - r0 - kWave, lane);
+            const int m = min(kWave, n - r0);
+            for (int q = 0; q < m; q++) emit(rd, q, __builtin_amdgcn_readlane(rd.rid, q));
+        }
+        near.flush();
+        far.flush();
+        return;
+    }
+    // the group's own records: an item's entries are passed over, up to what
+    // the lane has listed before the next record
+    const int n = G.head[grp].x;
+    LogReader rd{G.tid + (size_t)grp * G.R, G.tfar + (size_t)grp * G.R, G.tnear + (size_t)grp * G.R};
+    int32_t *const bn = near.p, *const bf = far.p;   // the leaf's lists
+    for (int r0 = 0; r0 < n; r0 += kWave) {
+        rd.load(r0, n - r0, lane);
+        const int m = min(kWave, n - r0);
+        for (int q = 0; q < m; q++) {
+            const int id = __builtin_amdgcn_readlane(rd.rid, q);
+            if (id >= 0) {
+                emit(rd, q, id);
+                continue;
+            }
+            // after item i the lane stands where item i's entries end
+            const size_t it = io + (-id - 1);
+            const int2 c = G.after[it * kWave + lane];
+            near.flush();
+            far.flush();
+            near.p = bn + c.x;
+            far.p = bf + c.y;
+        }
+    }
+    near.flush();
+    far.flush();
 }
 
 // Segments: leaf of each segment, then stable order by (leaf, index).
@@ -1504,6 +1648,18 @@ __global__ void k_seg_off(const int32_t* seg_leaf, const int32_t* seg_list, int 
     seg_off[l] = lo;
 }
 
+// What the host needs of a walk, in one copy: the lists' lengths, the items'
+// nodes and the log's overflow marks, which are cleared for the next walk.
+__global__ void k_list_totals(const int64_t* near_end, const int64_t* far_end, const int64_t* nodes_end,
+                              int32_t* most, int64_t* out) {
+    const int k = threadIdx.x;
+    if (k < 3) out[k] = k == 0 ? *near_end : k == 1 ? *far_end : *nodes_end;
+    if (k == 3 || k == 4) {
+        out[k] = most[k - 3];
+        most[k - 3] = 0;
+    }
+}
+
 __global__ void k_iota(int32_t* a, int n) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k < n) a[k] = k;
@@ -1518,6 +1674,48 @@ template <typename T>
 void swap_buf(DBuf<T>& a, DBuf<T>& b) {
     std::swap(a.p, b.p);
     std::swap(a.cap, b.cap);
+}
+
+// Exclusive scans of int32 counts into int64 offsets (n + 1 outputs), one
+// block per array: for short arrays, where the library's two launches per scan
+// cost more than the scan.
+constexpr int kScanThreads = 1024, kScanPer = 8;
+__global__ __launch_bounds__(kScanThreads) void k_scan_block(const int32_t* in0, int64_t* out0, const int32_t* in1,
+                                                             int64_t* out1, int n) {
+    __shared__ int64_t s_w[kScanThreads / kWave];
+    const int32_t* in = blockIdx.x ? in1 : in0;
+    int64_t* out = blockIdx.x ? out1 : out0;
+    const int t = threadIdx.x, w = t / kWave, lane = lane_id();
+    int64_t carry = 0;
+    for (int b = 0; b <= n; b += kScanThreads * kScanPer) {
+        int v[kScanPer];
+        int64_t mine = 0;
+        for (int k = 0; k < kScanPer; k++) {
+            const int i = b + t * kScanPer + k;
+            v[k] = i < n ? in[i] : 0;
+            mine += v[k];
+        }
+        int64_t incl = mine;
+        for (int o = 1; o < kWave; o <<= 1) {
+            const int64_t u = __shfl_up(incl, o, kWave);
+            if (lane >= o) incl += u;
+        }
+        if (lane == kWave - 1) s_w[w] = incl;
+        __syncthreads();
+        int64_t before = carry, total = 0;
+        for (int q = 0; q < kScanThreads / kWave; q++) {
+            if (q < w) before += s_w[q];
+            total += s_w[q];
+        }
+        before += incl - mine;
+        for (int k = 0; k < kScanPer; k++) {
+            const int i = b + t * kScanPer + k;
+            if (i <= n) out[i] = before;
+            before += v[k];
+        }
+        carry += total;
+        __syncthreads();
+    }
 }
 
 // exclusive scan of int32 counts into int64 offsets (n+1 outputs)
@@ -1869,46 +2067,74 @@ void tree_lists(Ctx& c) {
     const int nl = t.nleaves_h;
     NodeView nv = view(t);
     hipStream_t s = c.stream;
-    const size_t nslot = (size_t)nl * kMaxEntries;
-    DBuf<int32_t>& cnt_n = t.cnt_near;
-    DBuf<int32_t>& cnt_f = t.cnt_far;
-    cnt_n.grow(nslot + 1);
-    cnt_f.grow(nslot + 1);
-    t.slot_near.grow(nslot + 1);
-    t.slot_far.grow(nslot + 1);
+    t.cnt_near.grow(nl + 1);
+    t.cnt_far.grow(nl + 1);
     t.near_off.grow(nl + 1);
     t.far_off.grow(nl + 1);
-    const int nroots = c.nsim;
     t.trav.grow((size_t)t.nnodes * sizeof(TravNode));
     TravNode* tn = reinterpret_cast<TravNode*>(t.trav.p);
+    t.log.most.grow(2);
+    t.log.totals.grow(5);
     hipLaunchKernelGGL(k_trav_nodes, dim3(nblocks(t.nnodes)), dim3(kBlock), 0, s, nv, t.nnodes, t.pre.p, t.nleaves.p,
-                       tn);
-    t.entries.grow(nroots * sizeof(ListEntries));
-    ListEntries* E = reinterpret_cast<ListEntries*>(t.entries.p);
-    hipLaunchKernelGGL(k_list_entries, dim3(nroots), dim3(kWave), 0, s, nv, t.pre.p, nroots, E);
-    VVHD_HIP(hipMemsetAsync(cnt_n.p, 0, (nslot + 1) * 4, s));
-    VVHD_HIP(hipMemsetAsync(cnt_f.p, 0, (nslot + 1) * 4, s));
+                       tn, t.log.most.p);
     const double fc = (double)t.far_criteria;
-    const int64_t waves = (int64_t)t.ngroups * kMaxEntries;
-    const int grid = (int)std::max<int64_t>(1, (waves + kBlock / kWave - 1) / (kBlock / kWave));
-    hipLaunchKernelGGL(k_lists, dim3(grid), dim3(kBlock), 0, s, nv, (const TravNode*)tn, (const ListEntries*)E,
-                       (const int32_t*)t.groups.p, t.ngroups, t.leaf_node.p, fc, t.nnodes, (const int64_t*)nullptr,
-                       (const int64_t*)nullptr, (int32_t*)nullptr, (int32_t*)nullptr, cnt_n.p, cnt_f.p);
-    scan_i32_to_i64(c, cnt_n.p, t.slot_near.p, (int)nslot);
-    scan_i32_to_i64(c, cnt_f.p, t.slot_far.p, (int)nslot);
-    hipLaunchKernelGGL(k_leaf_offsets, dim3(nblocks(nl + 1)), dim3(kBlock), 0, s, t.slot_near.p, nl, t.near_off.p);
-    hipLaunchKernelGGL(k_leaf_offsets, dim3(nblocks(nl + 1)), dim3(kBlock), 0, s, t.slot_far.p, nl, t.far_off.p);
-    int64_t tot[2];
-    VVHD_HIP(hipMemcpyAsync(&tot[0], t.slot_near.p + nslot, 8, hipMemcpyDeviceToHost, s));
-    VVHD_HIP(hipMemcpyAsync(&tot[1], t.slot_far.p + nslot, 8, hipMemcpyDeviceToHost, s));
-    VVHD_HIP(hipStreamSynchronize(s));
-    t.nnear = tot[0];
-    t.nfar = tot[1];
-    t.near_list.grow(t.nnear + 1);
-    t.far_list.grow(t.nfar + 1);
-    hipLaunchKernelGGL(k_lists, dim3(grid), dim3(kBlock), 0, s, nv, (const TravNode*)tn, (const ListEntries*)E,
-                       (const int32_t*)t.groups.p, t.ngroups, t.leaf_node.p, fc, t.nnodes, (const int64_t*)t.slot_near.p,
-                       (const int64_t*)t.slot_far.p, t.near_list.p, t.far_list.p, (int32_t*)nullptr, (int32_t*)nullptr);
+    // subtrees walked by waves of their own: a walk over the top of the tree
+    // has about 2 nnodes / item_nodes steps, one of an item at most item_nodes
+    const int item_nodes = std::min(512, std::max(32, (int)(1.4 * std::sqrt((double)t.nnodes))));
+    const int ng = t.ngroups;
+    auto wave_grid = [](int64_t waves) {
+        return dim3((unsigned)std::max<int64_t>(1, (waves + kBlock / kWave - 1) / (kBlock / kWave)));
+    };
+    ListLogBufs& b = t.log;
+    for (;;) {
+        // room for what the criteria in use need; a longer log is counted, its
+        // buffers grown and the walk repeated
+        b.grow(ng, (int64_t)ng * 6144);
+        ListLog G{b.R, b.S, (int64_t)b.rid.cap, b.tid.p, b.tfar.p, b.tnear.p, b.head.p, b.gnodes.p, b.gbase.p, b.item.p,
+                  b.item_mask.p, b.item_n.p, b.lanes.p, b.after.p, b.rid.p, b.rfar.p, b.rnear.p, b.most.p};
+        if (ng)
+            hipLaunchKernelGGL(k_list_top, wave_grid(ng), dim3(kBlock), 0, s, nv, (const TravNode*)tn,
+                               (const int32_t*)t.pre.p, (const int32_t*)t.groups.p, ng, t.leaf_node.p, fc, item_nodes,
+                               G);
+        // (one block scans 65536 counts in about 12 us)
+        if (ng <= 65536)
+            hipLaunchKernelGGL(k_scan_block, dim3(1), dim3(kScanThreads), 0, s, (const int32_t*)b.gnodes.p, b.gbase.p,
+                               (const int32_t*)nullptr, (int64_t*)nullptr, ng);
+        else
+            scan_i32_to_i64(c, b.gnodes.p, b.gbase.p, ng);
+        if (ng) {
+            hipLaunchKernelGGL(k_list_items, wave_grid((int64_t)ng * b.S), dim3(kBlock), 0, s, nv, (const TravNode*)tn,
+                               (const int32_t*)t.groups.p, ng, t.leaf_node.p, fc, G);
+            hipLaunchKernelGGL(k_list_sums, wave_grid(ng), dim3(kBlock), 0, s, (const int32_t*)t.groups.p, ng, G,
+                               t.cnt_near.p, t.cnt_far.p);
+        }
+        if (nl <= 65536) {
+            hipLaunchKernelGGL(k_scan_block, dim3(2), dim3(kScanThreads), 0, s, (const int32_t*)t.cnt_near.p,
+                               t.near_off.p, (const int32_t*)t.cnt_far.p, t.far_off.p, nl);
+        } else {
+            scan_i32_to_i64(c, t.cnt_near.p, t.near_off.p, nl);
+            scan_i32_to_i64(c, t.cnt_far.p, t.far_off.p, nl);
+        }
+        int64_t tot[5];   // near entries, far entries, items' nodes, most[0], most[1]
+        hipLaunchKernelGGL(k_list_totals, dim3(1), dim3(64), 0, s, (const int64_t*)t.near_off.p + nl,
+                           (const int64_t*)t.far_off.p + nl, (const int64_t*)b.gbase.p + ng, b.most.p, b.totals.p);
+        VVHD_HIP(hipMemcpyAsync(tot, b.totals.p, sizeof(tot), hipMemcpyDeviceToHost, s));
+        VVHD_HIP(hipStreamSynchronize(s));
+        if (tot[3] == 0 && tot[4] == 0 && tot[2] <= G.cap) {
+            t.nnear = tot[0];
+            t.nfar = tot[1];
+            t.near_list.grow(t.nnear + 1);
+            t.far_list.grow(t.nfar + 1);
+            if (ng)
+                hipLaunchKernelGGL(k_list_replay, wave_grid((int64_t)ng * (b.S + 1)), dim3(kBlock), 0, s,
+                                   (const int32_t*)t.groups.p, ng, G, (const int64_t*)t.near_off.p,
+                                   (const int64_t*)t.far_off.p, t.near_list.p, t.far_list.p);
+            return;
+        }
+        b.R = std::max(b.R, (int)tot[3]);
+        b.S = std::max(b.S, (int)tot[4]);
+        b.rid.grow(tot[2]);
+    }
 }
 
 }  // namespace vvhd
