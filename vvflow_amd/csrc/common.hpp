@@ -374,6 +374,8 @@ struct Ctx {
     // field evaluators: per-vortex weights, the grid map, running gsum
     DBuf<double> fld_a, fld_b, fld_gtmp;
     DBuf<float> fld_map;
+    DBuf<int32_t> vel_leaf;               // leaves of the points of a velocity call
+    DBuf<double4> vel_src;                // its packed sources
 
     // near-field work items and queue (persistent form), the autotuner's
     // choices per workload class, and the captured convective graphs

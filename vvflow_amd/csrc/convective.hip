@@ -452,70 +452,6 @@ __global__ void k_conv_finish_gs(const int32_t* vleaf, const double* nx, const d
     }
 }
 
-// MConvectiveFast::velocity for arbitrary points, FP64 (one wave per point).
-__global__ void k_velocity_points(TreeDev T, const double* x, const double* y, const double* g, const double* ie,
-                                  const double* pts, int64_t n, double inf_x, double inf_y, double* out) {
-    const int64_t p = (int64_t)blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
-    if (p >= n) return;
-    const double px = pts[2 * p], py = pts[2 * p + 1];
-    int node = 0;   // stree::findNode
-    while (T.ch1[node] >= 0) {
-        const int c = T.ch1[node];
-        if (T.nh[node] < T.nw[node])
-            node = (px < T.nx[node]) ? c : c + 1;
-        else
-            node = (py < T.ny[node]) ? c : c + 1;
-    }
-    const int l = T.leaf_rank[node];
-    double nx_ = 0, ny_ = 0, fx = 0, fy = 0;
-    for (int64_t e = T.near_off[l]; e < T.near_off[l + 1]; e++) {
-        const int M = T.near_list[e];
-        for (int j = T.v0[M] + lane_id(); j < T.v1[M]; j += kWave) {
-            const double gj = g[j];
-            if (!gj) continue;
-            const double dx = px - x[j], dy = py - y[j];
-            const double e1 = 1. / ie[j];
-            const double f = gj / (dx * dx + dy * dy + e1 * e1);
-            nx_ += -dy * f;
-            ny_ += dx * f;
-        }
-    }
-    for (int64_t e = T.far_off[l] + lane_id(); e < T.far_off[l + 1]; e += kWave) {
-        const int F = T.far_list[e];
-        {
-            const double dx = px - T.cmp_x[F], dy = py - T.cmp_y[F];
-            const double e1 = 1. / (double)T.cmp_ie[F];
-            const double f = T.cmp_g[F] / (dx * dx + dy * dy + e1 * e1);
-            fx += -dy * f;
-            fy += dx * f;
-        }
-        {
-            const double dx = px - T.cmm_x[F], dy = py - T.cmm_y[F];
-            const double e1 = 1. / (double)T.cmm_ie[F];
-            const double f = T.cmm_g[F] / (dx * dx + dy * dy + e1 * e1);
-            fx += -dy * f;
-            fy += dx * f;
-        }
-    }
-    nx_ = wave_sum(nx_);
-    ny_ = wave_sum(ny_);
-    fx = wave_sum(fx);
-    fy = wave_sum(fy);
-    if (lane_id() == 0) {
-        double rx = 0, ry = 0;
-        rx += nx_ * k1_2Pi;
-        ry += ny_ * k1_2Pi;
-        rx += fx * k1_2Pi;
-        ry += fy * k1_2Pi;
-        rx += 0.0;
-        ry += 0.0;
-        rx += inf_x;
-        ry += inf_y;
-        out[2 * p] = rx;
-        out[2 * p + 1] = ry;
-    }
-}
-
 // FP64 direct sum of the induced velocity, compensated; sources staged in
 // LDS, one thread per target.
 constexpr int kDsBlock = 256;
@@ -822,19 +758,6 @@ void convective_noalloc(Ctx& c, double inf_x, double inf_y, int kahan) {
     double4* taylor = (double4*)base;
     double2* near_out = (double2*)(base + align256((size_t)(c.t.nleaves_h + 1) * sizeof(double4)));
     convective_into(c, inf_x, inf_y, kahan, taylor, near_out, true);
-}
-
-void velocity_points(Ctx& c, const double* xy, int64_t n, double inf_x, double inf_y, double* v_out) {
-    if (n == 0) return;
-    const TreeDev T = tree_dev(c.t);
-    c.tmp.grow((size_t)n * 32);
-    double* dpts = (double*)c.tmp.p;
-    double* dout = dpts + 2 * n;
-    VVHD_HIP(hipMemcpyAsync(dpts, xy, (size_t)n * 16, hipMemcpyHostToDevice, c.stream));
-    hipLaunchKernelGGL(k_velocity_points, dim3((unsigned)((n + kWavesPerBlock - 1) / kWavesPerBlock)), dim3(kBlock), 0,
-                       c.stream, T, c.x.p, c.y.p, c.g.p, c.ie.p, dpts, n, inf_x, inf_y, dout);
-    VVHD_HIP(hipMemcpyAsync(v_out, dout, (size_t)n * 16, hipMemcpyDeviceToHost, c.stream));
-    VVHD_HIP(hipStreamSynchronize(c.stream));
 }
 
 void direct_sum(Ctx& c, const int64_t* targets, int64_t nt, double* v_out) {

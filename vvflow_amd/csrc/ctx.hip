@@ -257,6 +257,8 @@ void vvhd_destroy(vvhd_ctx* ctx) {
     for (auto* b : {&t.h0, &t.h1, &t.s0, &t.s1, &t.seg_keys, &t.seg_ids}) b->release();
     for (auto* b : {&c.fld_a, &c.fld_b, &c.fld_gtmp}) b->release();
     c.fld_map.release();
+    c.vel_leaf.release();
+    c.vel_src.release();
     if (c.lev_counters) (void)hipHostFree(c.lev_counters);
     if (c.fm_counts) (void)hipHostFree(c.fm_counts);
     (void)hipStreamDestroy(c.stream);

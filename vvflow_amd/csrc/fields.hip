@@ -13,6 +13,7 @@
 
 #include "api.hpp"
 #include "body_geom.hpp"
+#include "near_flat.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -72,16 +73,19 @@ __device__ inline double wave_min(double v) {
 // MEpsilonFast::eps2h(node, p): the second smallest non-zero squared distance
 // from p to the vortices of the near leaves of node (the smallest when there
 // is one, the lowest double when there is none), on the calling wave.
-__device__ double wave_eps2h(const TreeDev& T, const double* x, const double* y, int l, double px, double py) {
+__device__ double wave_eps2h(const TreeDev& T, const double* x, const double* y, int l, double px, double py,
+                             int* tab) {
     double r1 = INFINITY, r2 = INFINITY;
-    for (int64_t e = T.near_off[l]; e < T.near_off[l + 1]; e++) {
-        const int M = T.near_list[e];
-        for (int j = T.v0[M] + lane_id(); j < T.v1[M]; j += kWave) {
-            const double dx = px - x[j], dy = py - y[j];
-            const double d2 = dx * dx + dy * dy;
-            if (d2 != 0) top2_insert(d2, r1, r2);
-        }
-    }
+    wave_flat(T.near_list, T.near_off[l], T.near_off[l + 1], tab,
+              [&](int M, int& j0, int& cnt) {
+                  j0 = T.v0[M];
+                  cnt = T.v1[M] - j0;
+              },
+              [&](int j) {
+                  const double dx = px - x[j], dy = py - y[j];
+                  const double d2 = dx * dx + dy * dy;
+                  if (d2 != 0) top2_insert(d2, r1, r2);
+              });
     wave_top2(r1, r2);
     if (isfinite(r2)) return r2;
     if (isfinite(r1)) return r1;
@@ -112,39 +116,64 @@ __device__ inline bool in_any_body(const vvhd_body* bodies, int nbody, const vvh
     return false;
 }
 
-// MConvectiveFast::velocity(p) (MConvectiveFast.cpp:20-34, 139-151) on the
-// calling wave: near Lamb sum, far per-sign monopoles, U.
-__device__ void wave_velocity(const TreeDev& T, const double* x, const double* y, const double* g, const double* ie,
-                              double px, double py, double inf_x, double inf_y, double& ox, double& oy) {
-    const int l = T.leaf_rank[find_leaf_node(T, px, py)];
-    double nx_ = 0, ny_ = 0, fx = 0, fy = 0;
-    for (int64_t e = T.near_off[l]; e < T.near_off[l + 1]; e++) {
-        const int M = T.near_list[e];
-        for (int j = T.v0[M] + lane_id(); j < T.v1[M]; j += kWave) {
-            const double gj = g[j];
-            if (!gj) continue;
-            const double dx = px - x[j], dy = py - y[j];
-            const double e1 = 1. / ie[j];
-            const double f = gj / (dx * dx + dy * dy + e1 * e1);
-            nx_ += -dy * f;
-            ny_ += dx * f;
-        }
+// Sources of velocity sums as one 32-byte record each, {x, y, g, eps^2}: of
+// every vortex, and two (positive and negative) of every node.  Null where the
+// sums read the arrays themselves.
+struct VelSources {
+    const double4 *vort, *nodes;
+};
+
+__global__ void k_pack_sources(const double* x, const double* y, const double* g, const double* ie, int64_t n,
+                               TreeDev T, int nnodes, double4* vort, double4* nodes) {
+    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < n) {
+        const double e1 = 1. / ie[k];
+        vort[k] = make_double4(x[k], y[k], g[k], e1 * e1);
     }
+    if (k < nnodes) {
+        const double ep = 1. / (double)T.cmp_ie[k], em = 1. / (double)T.cmm_ie[k];
+        nodes[2 * k] = make_double4(T.cmp_x[k], T.cmp_y[k], T.cmp_g[k], ep * ep);
+        nodes[2 * k + 1] = make_double4(T.cmm_x[k], T.cmm_y[k], T.cmm_g[k], em * em);
+    }
+}
+
+// MConvectiveFast::velocity(p) (MConvectiveFast.cpp:20-34, 139-151) at p in
+// leaf l, on the calling wave: near Lamb sum, far per-sign monopoles, U.
+template <bool kPacked>
+__device__ void wave_velocity(const TreeDev& T, const double* x, const double* y, const double* g, const double* ie,
+                              const VelSources& S, int l, double px, double py, double inf_x, double inf_y, int* tab,
+                              double& ox, double& oy) {
+    double nx_ = 0, ny_ = 0, fx = 0, fy = 0;
+    auto add = [&](const double4 s, double& sx, double& sy) {
+        const double dx = px - s.x, dy = py - s.y;
+        const double f = s.z / (dx * dx + dy * dy + s.w);
+        sx += -dy * f;
+        sy += dx * f;
+    };
+    wave_flat(T.near_list, T.near_off[l], T.near_off[l + 1], tab,
+              [&](int M, int& j0, int& cnt) {
+                  j0 = T.v0[M];
+                  cnt = T.v1[M] - j0;
+              },
+              [&](int j) {
+                  double4 s;
+                  if (kPacked) {
+                      s = S.vort[j];
+                  } else {
+                      const double e1 = 1. / ie[j];
+                      s = make_double4(x[j], y[j], g[j], e1 * e1);
+                  }
+                  if (s.z) add(s, nx_, ny_);
+              });
     for (int64_t e = T.far_off[l] + lane_id(); e < T.far_off[l + 1]; e += kWave) {
         const int F = T.far_list[e];
-        {
-            const double dx = px - T.cmp_x[F], dy = py - T.cmp_y[F];
-            const double e1 = 1. / (double)T.cmp_ie[F];
-            const double f = T.cmp_g[F] / (dx * dx + dy * dy + e1 * e1);
-            fx += -dy * f;
-            fy += dx * f;
-        }
-        {
-            const double dx = px - T.cmm_x[F], dy = py - T.cmm_y[F];
-            const double e1 = 1. / (double)T.cmm_ie[F];
-            const double f = T.cmm_g[F] / (dx * dx + dy * dy + e1 * e1);
-            fx += -dy * f;
-            fy += dx * f;
+        if (kPacked) {
+            add(S.nodes[2 * (int64_t)F], fx, fy);
+            add(S.nodes[2 * (int64_t)F + 1], fx, fy);
+        } else {
+            const double ep = 1. / (double)T.cmp_ie[F], em = 1. / (double)T.cmm_ie[F];
+            add(make_double4(T.cmp_x[F], T.cmp_y[F], T.cmp_g[F], ep * ep), fx, fy);
+            add(make_double4(T.cmm_x[F], T.cmm_y[F], T.cmm_g[F], em * em), fx, fy);
         }
     }
     nx_ = wave_sum(nx_);
@@ -172,6 +201,7 @@ __global__ __launch_bounds__(kBlock) void k_eps2h_h2(TreeDev T, const double* x,
                                                      int64_t n, double* out) {
     const int64_t p = (int64_t)blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
     if (p >= n) return;
+    __shared__ int s_tab[kWavesPerBlock][kH2 ? 1 : kNearTab];
     double px, py;
     int l;
     if (pts) {
@@ -183,7 +213,7 @@ __global__ __launch_bounds__(kBlock) void k_eps2h_h2(TreeDev T, const double* x,
         py = y[p];
         l = T.vleaf[p];
     }
-    const double r = kH2 ? wave_h2(T, segs, l, px, py) : wave_eps2h(T, x, y, l, px, py);
+    const double r = kH2 ? wave_h2(T, segs, l, px, py) : wave_eps2h(T, x, y, l, px, py, s_tab[threadIdx.x / kWave]);
     if (lane_id() == 0) out[p] = r;
 }
 
@@ -197,7 +227,8 @@ __global__ __launch_bounds__(kBlock) void k_field_weights(TreeDev T, const doubl
                                                           double* b) {
     const int64_t i = (int64_t)blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
     if (i >= n) return;
-    const double e = wave_eps2h(T, x, y, T.vleaf[i], x[i], y[i]);
+    __shared__ int s_tab[kWavesPerBlock][kNearTab];
+    const double e = wave_eps2h(T, x, y, T.vleaf[i], x[i], y[i], s_tab[threadIdx.x / kWave]);
     if (lane_id() != 0) return;
     if (kStream) {
         a[i] = (m * m) * fmax(e * 0.25, (0.2 * dl) * (0.2 * dl));
@@ -353,7 +384,9 @@ __global__ __launch_bounds__(kBlock) void k_pressure_grid(TreeDev T, const doubl
     }
     cp = wave_sum(cp);
     double ux, uy;
-    wave_velocity(T, x, y, g, ie, px, py, inf_x, inf_y, ux, uy);
+    __shared__ int s_tab[kWavesPerBlock][kNearTab];
+    wave_velocity<false>(T, x, y, g, ie, VelSources{nullptr, nullptr}, T.leaf_rank[find_leaf_node(T, px, py)], px, py,
+                         inf_x, inf_y, s_tab[threadIdx.x / kWave], ux, uy);
     if (lane_id() == 0) {
         double c = k1_2Pi * cp + 0.5 * ((inf_x * inf_x + inf_y * inf_y) - (ux * ux + uy * uy));
         if (with_ref) c += 0.5 * ((ux - ref_x) * (ux - ref_x) + (uy - ref_y) * (uy - ref_y));
@@ -361,16 +394,47 @@ __global__ __launch_bounds__(kBlock) void k_pressure_grid(TreeDev T, const doubl
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_velocity_grid(TreeDev T, const double* x, const double* y,
-                                                          const double* g, const double* ie, Grid G, double inf_x,
-                                                          double inf_y, double ref_x, double ref_y, int comp,
-                                                          float* map) {
+// The leaf of every point (xy) or grid node (xy == nullptr), a thread each: in
+// the velocity kernel the descent would cost every wave its chain of loads.
+__global__ __launch_bounds__(kBlock) void k_point_leaves(TreeDev T, const double2* xy, Grid G, int64_t n,
+                                                         int32_t* leaf) {
+    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n) return;
+    double px, py;
+    if (xy) {
+        px = xy[k].x;
+        py = xy[k].y;
+    } else {
+        G.point(k, px, py);
+    }
+    leaf[k] = T.leaf_rank[find_leaf_node(T, px, py)];
+}
+
+// Velocities at points (out) or one component of the grid's (map), one wave
+// per point.  Bound by the FP64 operations of its terms, a division each.  A
+// leaf at a time, with the descent and two divisions a source, it took 680 us
+// for 20k grid nodes in 200k vortices; as one sequence of packed sources 136.
+template <bool kPacked>
+__global__ __launch_bounds__(kBlock) void k_velocity(TreeDev T, const double* x, const double* y, const double* g,
+                                                     const double* ie, VelSources S, const double2* xy, Grid G,
+                                                     const int32_t* leaf, int64_t n, double inf_x, double inf_y,
+                                                     double2* out, int comp, double ref, float* map) {
+    __shared__ int s_tab[kWavesPerBlock][kNearTab];
     const int64_t k = (int64_t)blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
-    if (k >= (int64_t)G.xres * G.yres) return;
+    if (k >= n) return;
     double px, py, ux, uy;
-    G.point(k, px, py);
-    wave_velocity(T, x, y, g, ie, px, py, inf_x, inf_y, ux, uy);
-    if (lane_id() == 0) map[k] = (float)(comp == 0 ? ux - ref_x : uy - ref_y);
+    if (xy) {
+        px = xy[k].x;
+        py = xy[k].y;
+    } else {
+        G.point(k, px, py);
+    }
+    wave_velocity<kPacked>(T, x, y, g, ie, S, leaf[k], px, py, inf_x, inf_y, s_tab[threadIdx.x / kWave], ux, uy);
+    if (lane_id() != 0) return;
+    if (out)
+        out[k] = make_double2(ux, uy);
+    else
+        map[k] = (float)((comp == 0 ? ux : uy) - ref);
 }
 
 // Running sum of gsum along each body's segments (XPressure.cpp:128-133).
@@ -385,6 +449,44 @@ __global__ void k_gsum_running(const vvhd_body* bodies, int nbody, const vvhd_se
 }
 
 }  // namespace
+
+// Velocities at xy, or on the grid where xy is null (all device pointers).
+static void velocities(Ctx& c, const TreeDev& T, const double2* xy, const Grid& G, int64_t n, double inf_x,
+                       double inf_y, double2* out, int comp, double ref, float* map) {
+    hipStream_t s = c.stream;
+    c.vel_leaf.grow((size_t)n);
+    hipLaunchKernelGGL(k_point_leaves, dim3(nblocks(n)), dim3(kBlock), 0, s, T, xy, G, n, c.vel_leaf.p);
+    // Packed records where the points read them often enough: in place against
+    // packed, 781 points in 200k vortices 360 and 284 us, 6060 points 406 and
+    // 338; 312 in 20k 147 and 138, 78 in 20k 139 and 144; 31 in 2k 38 and 42.
+    const int64_t m = std::max<int64_t>(c.n, c.t.nnodes);
+    if (n >= 256 && n * 256 >= m) {
+        c.vel_src.grow((size_t)(c.n + 2 * (int64_t)c.t.nnodes));
+        double4 *vort = c.vel_src.p, *nodes = vort + c.n;
+        hipLaunchKernelGGL(k_pack_sources, dim3(nblocks(m)), dim3(kBlock), 0, s, c.x.p, c.y.p, c.g.p, c.ie.p, c.n, T,
+                           c.t.nnodes, vort, nodes);
+        hipLaunchKernelGGL(k_velocity<true>, dim3(wave_blocks(n)), dim3(kBlock), 0, s, T, c.x.p, c.y.p, c.g.p,
+                           c.ie.p, VelSources{vort, nodes}, xy, G, (const int32_t*)c.vel_leaf.p, n, inf_x, inf_y, out,
+                           comp, ref, map);
+    } else {
+        hipLaunchKernelGGL(k_velocity<false>, dim3(wave_blocks(n)), dim3(kBlock), 0, s, T, c.x.p, c.y.p, c.g.p,
+                           c.ie.p, VelSources{nullptr, nullptr}, xy, G, (const int32_t*)c.vel_leaf.p, n, inf_x, inf_y,
+                           out, comp, ref, map);
+    }
+}
+
+void velocity_points(Ctx& c, const double* xy, int64_t n, double inf_x, double inf_y, double* v_out) {
+    if (n == 0) return;
+    const TreeDev T = tree_dev(c.t);
+    c.tmp.grow((size_t)n * 32);
+    double2* dpts = (double2*)c.tmp.p;
+    double2* dout = dpts + n;
+    VVHD_HIP(hipMemcpyAsync(dpts, xy, (size_t)n * 16, hipMemcpyHostToDevice, c.stream));
+    velocities(c, T, dpts, Grid{}, n, inf_x, inf_y, dout, 0, 0, nullptr);
+    VVHD_HIP(hipGetLastError());
+    VVHD_HIP(hipMemcpyAsync(v_out, dout, (size_t)n * 16, hipMemcpyDeviceToHost, c.stream));
+    VVHD_HIP(hipStreamSynchronize(c.stream));
+}
 
 void eps2h_h2(Ctx& c, bool h2, const double* xy, const int32_t* leaf, int64_t n, double* out) {
     const TreeDev T = tree_dev(c.t);
@@ -426,8 +528,8 @@ void grid_field(Ctx& c, int kind, const vvhd_grid& gr, double m, double dl, doub
     switch (kind) {
         case VVHD_FIELD_VX:
         case VVHD_FIELD_VY:
-            hipLaunchKernelGGL(k_velocity_grid, dim3(grid), dim3(kBlock), 0, s, T, c.x.p, c.y.p, c.g.p, c.ie.p, G,
-                               inf_x, inf_y, ref_x, ref_y, kind == VVHD_FIELD_VX ? 0 : 1, c.fld_map.p);
+            velocities(c, T, nullptr, G, npts, inf_x, inf_y, nullptr, kind == VVHD_FIELD_VX ? 0 : 1,
+                       kind == VVHD_FIELD_VX ? ref_x : ref_y, c.fld_map.p);
             break;
         case VVHD_FIELD_VORTICITY:
             if (c.n)
