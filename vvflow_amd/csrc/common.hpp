@@ -366,7 +366,8 @@ struct Ctx {
     bool mlp_loaded = false;
     DBuf<float> tr_x, tr_y, tr_w;            // training set on the device
     int64_t tr_n = 0;
-    DBuf<float> adam_m, adam_v, grad_part, grad_out;
+    DBuf<float> adam_m, adam_v, grad_part, grad_out, tr_loss;
+    DBuf<int32_t> frag_slots;                // per weight its elements of mlp_frags
     int64_t adam_t = 0;
     DBuf<int64_t> pair_off;
     DBuf<int32_t> pair_cnt, pair_t, pair_f;

@@ -397,65 +397,68 @@ __device__ inline bf16x8 input_frag(const float* f, bool ok, const float* P) {
     return x;
 }
 
+// The parameter behind fragment element t of the layouts above, -1 for padding.
+__device__ inline int frag_param(int t) {
+    const int base = t < fA2 ? fA1 : t < fA3 ? fA2 : t < fA3T ? fA3 : t < fA2T ? fA3T : t < fB1 ? fA2T
+                     : t < fB2 ? fB1 : t < fB3 ? fB2 : fB3;
+    const int set = (t - base) / kSet, rem = (t - base) % kSet;
+    const int lane = rem / 8, e = rem % 8, m = lane % 32, g = lane / 32;
+    const int m16 = lane % 16, g16 = lane / 16;   // 16x16x32 inference sets
+    switch (base) {
+        case fA1: {   // W1: A[m = unit][k = feature]
+            const int k = 8 * g + e;
+            return k < kFeat ? oW1 + (32 * set + m) * kFeat + k : -1;
+        }
+        case fA2:     // W2: block b = set / 4, K step st = set % 4
+            return oW2 + (32 * (set / 4) + m) * kHid + chain_unit(set % 4, g, e);
+        case fA3:     // W3 (rows 0, 1)
+            return m < kOut ? oW3 + m * kHid + chain_unit(set, g, e) : -1;
+        case fA3T: {  // W3^T: A[m = hidden unit][k = output]
+            const int k = 8 * g + e;
+            return k < kOut ? oW3 + k * kHid + 32 * set + m : -1;
+        }
+        case fA2T:    // W2^T: A[m = input unit][k = output unit in chained order]
+            return oW2 + chain_unit(set % 4, g, e) * kHid + 32 * (set / 4) + m;
+        case fB1: {   // W1' block set: rows 16 set + m16, K = feature 8 g16 + e
+            const int k = 8 * g16 + e;
+            return k < kFeat ? oW1 + (16 * set + m16) * kFeat + k : -1;
+        }
+        case fB2:     // W2: block b = set / 2, K step st = set % 2
+            return oW2 + (16 * (set / 2) + m16) * kHid + chain16(set % 2, g16, e);
+        default:      // W3' rows 0, 1, K step set
+            return m16 < kOut ? oW3 + m16 * kHid + chain16(set, g16, e) : -1;
+    }
+}
+
+// Element t's bits from the value w of its parameter p.  Layer 1 takes bf16
+// features; layers 2 and 3 of the inference sets take the fp16 hidden values.
+__device__ inline uint16_t frag_bits(int t, int p, float w, const float* P) {
+    float v = w;
+    if (t >= fB1 && t < fB2) v = (-kLog2e * w) * (1.f / P[oSd + (p - oW1) % kFeat]);
+    if (t >= fB3) v = w * -kLn2;
+    return t < fB2 ? bf16_bits(v) : __builtin_bit_cast(uint16_t, (_Float16)v);
+}
+
 // FP32 master parameters -> bf16 fragments in the layouts above.
 __global__ void k_pack_model(const float* P, uint16_t* frag) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= kFragElems) return;
-    int set, rem;
-    float v = 0.f;
-    auto decode = [&](int base) {
-        set = (t - base) / kSet;
-        rem = (t - base) % kSet;
-    };
-    if (t < fA2) {
-        decode(fA1);
-    } else if (t < fA3) {
-        decode(fA2);
-    } else if (t < fA3T) {
-        decode(fA3);
-    } else if (t < fA2T) {
-        decode(fA3T);
-    } else if (t < fB1) {
-        decode(fA2T);
-    } else if (t < fB2) {
-        decode(fB1);
-    } else if (t < fB3) {
-        decode(fB2);
-    } else {
-        decode(fB3);
-    }
-    const int lane = rem / 8, e = rem % 8, m = lane % 32, g = lane / 32;
-    if (t >= fB1) {   // 16x16x32 inference sets
-        const int m16 = lane % 16, g16 = lane / 16;
-        if (t < fB2) {   // W1' block set: rows 16 set + m16, K = feature 8 g16 + e
-            const int k = 8 * g16 + e;
-            if (k < kFeat) v = (-kLog2e * P[oW1 + (16 * set + m16) * kFeat + k]) * (1.f / P[oSd + k]);
-        } else if (t < fB3) {   // W2: block b = set / 2, K step st = set % 2
-            const int b = set / 2, st = set % 2;
-            v = P[oW2 + (16 * b + m16) * kHid + chain16(st, g16, e)];
-        } else {   // W3' rows 0, 1, K step set
-            if (m16 < kOut) v = P[oW3 + m16 * kHid + chain16(set, g16, e)] * -kLn2;
-        }
-        // layer 1 takes bf16 features; layers 2 and 3 take the fp16 hidden values
-        frag[t] = t < fB2 ? bf16_bits(v) : __builtin_bit_cast(uint16_t, (_Float16)v);
-        return;
-    }
-    if (t < fA2) {   // W1: A[m = unit][k = feature]
-        const int k = 8 * g + e;
-        if (k < kFeat) v = P[oW1 + (32 * set + m) * kFeat + k];
-    } else if (t < fA3) {   // W2: block b = set / 4, K step st = set % 4
-        const int b = set / 4, st = set % 4;
-        v = P[oW2 + (32 * b + m) * kHid + chain_unit(st, g, e)];
-    } else if (t < fA3T) {   // W3 (rows 0, 1)
-        if (m < kOut) v = P[oW3 + m * kHid + chain_unit(set, g, e)];
-    } else if (t < fA2T) {   // W3^T: A[m = hidden unit][k = output]
-        const int k = 8 * g + e;
-        if (k < kOut) v = P[oW3 + k * kHid + 32 * set + m];
-    } else {   // W2^T: A[m = input unit][k = output unit in chained order]
-        const int b = set / 4, st = set % 4;
-        v = P[oW2 + chain_unit(st, g, e) * kHid + 32 * b + m];
-    }
-    frag[t] = bf16_bits(v);
+    const int p = frag_param(t);
+    frag[t] = p < 0 ? (uint16_t)0 : frag_bits(t, p, P[p], P);
+}
+
+__global__ void k_fill_slots(int32_t* slots) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < 3 * kTrain) slots[k] = -1;
+}
+
+// The fragment elements of every weight (at most one in the forward, one in
+// the transposed and one in the inference sets), for the steps of training.
+__global__ void k_frag_slots(int32_t* slots) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= kFragElems) return;
+    const int p = frag_param(t);
+    if (p >= 0) slots[3 * p + (t >= fB1 ? 2 : t >= fA3T ? 1 : 0)] = t;
 }
 
 // -------------------------------------------------------------- inference
@@ -1003,16 +1006,25 @@ __device__ inline uint64_t mix64(uint64_t z) {
     return z ^ (z >> 31);
 }
 
-// Fused forward + backward of one tile of 32 samples per wave (block = one
-// wave).  Sample j of slot n: idx == nullptr -> j = tile*32 + n over the
-// data (full batch), else j = idx-hash of (seed, tile*32 + n) mod ndata.
-// Writes the tile's gradient and loss into part[tile].
-__global__ __launch_bounds__(64) void k_train_tile(const float* X, const float* Y, const float* Wt, int64_t ndata,
-                                                   int64_t nsamples, int hashed, uint64_t seed, float inv_b,
-                                                   const uint16_t* frag, const float* P, float* part) {
-    __shared__ uint16_t Tz2[kHid][32], Th1[kHid][32], Tz1[kHid][32], Th2[kHid][32], Tx[16][32], Tdy[2][32];
+// Fused forward + backward of one tile of 32 samples per block.  Sample j of
+// slot n: idx == nullptr -> j = tile*32 + n over the data (full batch), else
+// j = idx-hash of (seed, tile*32 + n) mod ndata.  Writes the tile's gradient
+// and loss into part[tile].
+// Bound by the latency of one wave's chain: a batch of 8192 is 256 tiles, a
+// wave each on a quarter of the chip's SIMDs, 19.8 us.  The four waves of a
+// block all run the forward pass; each then stages one operand in LDS (wave
+// 0 dZ2, 1 dZ1, 2 H1, 3 H2) and takes a quarter of the weight gradients.
+// LDS rows of 40 keep their 16-byte fragment reads off each other's banks.
+constexpr int kTrainRow = 40;
+__global__ __launch_bounds__(256) void k_train_tile(const float* X, const float* Y, const float* Wt, int64_t ndata,
+                                                    int64_t nsamples, int hashed, uint64_t seed, float inv_b,
+                                                    const uint16_t* __restrict__ frag, const float* __restrict__ P,
+                                                    float* __restrict__ part) {
+    __shared__ __align__(16) uint16_t Tz2[kHid][kTrainRow], Th1[kHid][kTrainRow], Tz1[kHid][kTrainRow],
+        Th2[kHid][kTrainRow], Tx[16][kTrainRow], Tdy[kOut][kTrainRow];
     const int64_t tile = blockIdx.x;
-    const int lane = threadIdx.x, g = lane >> 5, n = lane & 31;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int lane = lane_id(), g = lane >> 5, n = lane & 31;
     const int64_t slot = tile * 32 + n;
     int64_t j = -1;
     if (slot < nsamples) j = hashed ? (int64_t)(mix64(seed ^ (uint64_t)slot * 0xD1B54A32D192ED03ull) % (uint64_t)ndata)
@@ -1034,130 +1046,150 @@ __global__ __launch_bounds__(64) void k_train_tile(const float* X, const float* 
         dy0 = 2.f * wgt * r0 * inv_b;
         dy1 = 2.f * wgt * r1 * inv_b;
     }
-    bf16x8 dyf;
-    for (int e = 0; e < 8; e++) dyf[e] = to_bf16(g == 0 && e == 0 ? dy0 : (g == 0 && e == 1 ? dy1 : 0.f));
-    // dZ2 = (W3^T dY) * silu'(Z2)
-    f32x16 dz2[2];
-    for (int b = 0; b < 2; b++) {
-        f32x16 c = {};
-        c = mfma32(load_frag(frag, fA3T / kSet + b, lane), dyf, c);
-        for (int q = 0; q < 16; q++) dz2[b][q] = c[q] * dsilu_f(s.c2[b][q]);
-    }
-    bf16x8 z2b[4];
-    for (int st = 0; st < 4; st++)
-        for (int e = 0; e < 8; e++) z2b[st][e] = to_bf16(dz2[st >> 1][8 * (st & 1) + e]);
-    // dZ1 = (W2^T dZ2) * silu'(Z1)
-    f32x16 dz1[2];
-    for (int b = 0; b < 2; b++) {
-        f32x16 c = {};
-        for (int st = 0; st < 4; st++) c = mfma32(load_frag(frag, fA2T / kSet + 4 * b + st, lane), z2b[st], c);
-        for (int q = 0; q < 16; q++) dz1[b][q] = c[q] * dsilu_f(s.c1[b][q]);
-    }
-    // stage bf16 operands [unit][sample] for the weight gradients
-    for (int b = 0; b < 2; b++)
-        for (int j4 = 0; j4 < 4; j4++)
-            for (int i = 0; i < 4; i++) {
-                const int u = 32 * b + 8 * j4 + 4 * g + i, q = 4 * j4 + i;
-                Tz2[u][n] = bf16_bits(dz2[b][q]);
-                Tz1[u][n] = bf16_bits(dz1[b][q]);
-                Th1[u][n] = bf16_bits(silu_f(s.c1[b][q]));
-                Th2[u][n] = bf16_bits(silu_f(s.c2[b][q]));
-            }
-    for (int e = 0; e < 8; e++) {
+    float* out = part + tile * kPartStride;
+    // stages an operand's bf16 bits [unit][sample] for the weight gradients
+    auto stage = [&](uint16_t (*T)[kTrainRow], auto bits) {
+        for (int b = 0; b < 2; b++)
+            for (int q = 0; q < 16; q++) T[32 * b + 8 * (q >> 2) + 4 * g + (q & 3)][n] = bits(b, q);
+    };
+    auto raw = [](__bf16 v) {
         uint16_t b16;
-        const __bf16 v = xin[e];
         __builtin_memcpy(&b16, &v, 2);
-        Tx[8 * g + e][n] = b16;
-    }
-    if (g == 0) {
-        Tdy[0][n] = bf16_bits(dy0);
-        Tdy[1][n] = bf16_bits(dy1);
+        return b16;
+    };
+    // bias gradient: sums of the 32 units' deltas over the 32 samples.  At each
+    // step a lane keeps one half of its units and hands the other half on, so
+    // that 31 exchanges leave lane n the sum of unit n.
+    auto bias = [&](const f32x16* dz, float* o) {
+        float a[32];
+        for (int k = 0; k < 32; k++) a[k] = dz[k >> 4][k & 15];
+#pragma unroll
+        for (int h = 16; h > 0; h >>= 1) {
+            const bool hi = (n & h) != 0;
+#pragma unroll
+            for (int k = 0; k < h; k++) {
+                const float keep = hi ? a[k + h] : a[k], give = hi ? a[k] : a[k + h];
+                a[k] = keep + __shfl_xor(give, h, kWave);
+            }
+        }
+        const int q = n & 15;
+        o[32 * (n >> 4) + 8 * (q >> 2) + 4 * g + (q & 3)] = a[0];
+    };
+    if (w < 2) {
+        bf16x8 dyf;
+        for (int e = 0; e < 8; e++) dyf[e] = to_bf16(g == 0 && e == 0 ? dy0 : (g == 0 && e == 1 ? dy1 : 0.f));
+        // dZ2 = (W3^T dY) * silu'(Z2)
+        f32x16 dz2[2];
+        for (int b = 0; b < 2; b++) {
+            f32x16 c = {};
+            c = mfma32(load_frag(frag, fA3T / kSet + b, lane), dyf, c);
+            for (int q = 0; q < 16; q++) dz2[b][q] = c[q] * dsilu_f(s.c2[b][q]);
+        }
+        if (w == 0) {
+            stage(Tz2, [&](int b, int q) { return bf16_bits(dz2[b][q]); });
+            bias(dz2, out + oB2);
+        } else {
+            bf16x8 z2b[4];
+            for (int st = 0; st < 4; st++)
+                for (int e = 0; e < 8; e++) z2b[st][e] = to_bf16(dz2[st >> 1][8 * (st & 1) + e]);
+            // dZ1 = (W2^T dZ2) * silu'(Z1)
+            f32x16 dz1[2];
+            for (int b = 0; b < 2; b++) {
+                f32x16 c = {};
+                for (int st = 0; st < 4; st++)
+                    c = mfma32(load_frag(frag, fA2T / kSet + 4 * b + st, lane), z2b[st], c);
+                for (int q = 0; q < 16; q++) dz1[b][q] = c[q] * dsilu_f(s.c1[b][q]);
+            }
+            stage(Tz1, [&](int b, int q) { return bf16_bits(dz1[b][q]); });
+            bias(dz1, out + oB1);
+        }
+    } else if (w == 2) {
+        stage(Th1, [&](int b, int q) { return raw(s.h1[2 * b + (q >> 3)][q & 7]); });
+        for (int e = 0; e < 8; e++) Tx[8 * g + e][n] = raw(xin[e]);
+    } else {
+        stage(Th2, [&](int b, int q) { return raw(s.h2[2 * b + (q >> 3)][q & 7]); });
+        if (g == 0) {
+            Tdy[0][n] = bf16_bits(dy0);
+            Tdy[1][n] = bf16_bits(dy1);
+        }
+        float b0 = dy0, b1 = dy1, ls = loss;
+        for (int o = 1; o < 64; o <<= 1) {
+            b0 += __shfl_xor(b0, o, kWave);
+            b1 += __shfl_xor(b1, o, kWave);
+            ls += __shfl_xor(ls, o, kWave);
+        }
+        if (lane == 0) {
+            out[oB3] = b0;
+            out[oB3 + 1] = b1;
+            out[kTrain] = ls;
+        }
     }
     __syncthreads();
-    float* out = part + tile * kPartStride;
-    auto frag_lds = [&](const uint16_t* row0, int stride, int nrows, int row, int t) {
-        // A or B fragment: 8 samples 16t + 8g .. +8 of one row (zero past nrows)
-        bf16x8 r;
-        for (int e = 0; e < 8; e++) {
-            const uint16_t b16 = row < nrows ? row0[row * stride + 16 * t + 8 * g + e] : (uint16_t)0;
-            __bf16 v;
-            __builtin_memcpy(&v, &b16, 2);
-            r[e] = v;
-        }
+    // A or B fragment: 8 samples 16t + 8g .. +8 of one row (zero past nrows)
+    auto frag_lds = [&](const uint16_t (*T)[kTrainRow], int nrows, int row, int t) {
+        bf16x8 r = {};
+        if (row < nrows) r = *reinterpret_cast<const bf16x8*>(&T[row][16 * t + 8 * g]);
         return r;
     };
-    // dW2[out][in]
-    for (int bo = 0; bo < 2; bo++)
-        for (int bi = 0; bi < 2; bi++) {
-            f32x16 c = {};
-            for (int t = 0; t < 2; t++)
-                c = mfma32(frag_lds(&Tz2[0][0], 32, kHid, 32 * bo + n, t), frag_lds(&Th1[0][0], 32, kHid, 32 * bi + n, t),
-                           c);
-            for (int j4 = 0; j4 < 4; j4++)
-                for (int i = 0; i < 4; i++) {
-                    const int o = 32 * bo + 8 * j4 + 4 * g + i, in = 32 * bi + n;
-                    out[oW2 + o * kHid + in] = c[4 * j4 + i];
-                }
-        }
-    // dW1[out][feature]
-    for (int bo = 0; bo < 2; bo++) {
+    // dW2[out][in], a block of 32 x 32 each wave
+    {
+        const int bo = w >> 1, bi = w & 1;
         f32x16 c = {};
-        for (int t = 0; t < 2; t++)
-            c = mfma32(frag_lds(&Tz1[0][0], 32, kHid, 32 * bo + n, t), frag_lds(&Tx[0][0], 32, kFeat, n, t), c);
-        if (n < kFeat)
-            for (int j4 = 0; j4 < 4; j4++)
-                for (int i = 0; i < 4; i++) out[oW1 + (32 * bo + 8 * j4 + 4 * g + i) * kFeat + n] = c[4 * j4 + i];
+        for (int t = 0; t < 2; t++) c = mfma32(frag_lds(Tz2, kHid, 32 * bo + n, t), frag_lds(Th1, kHid, 32 * bi + n, t), c);
+        for (int q = 0; q < 16; q++) out[oW2 + (32 * bo + 8 * (q >> 2) + 4 * g + (q & 3)) * kHid + 32 * bi + n] = c[q];
     }
-    // dW3[k][in]
-    for (int bi = 0; bi < 2; bi++) {
+    if (w < 2) {   // dW1[out][feature]
         f32x16 c = {};
-        for (int t = 0; t < 2; t++)
-            c = mfma32(frag_lds(&Tdy[0][0], 32, kOut, n, t), frag_lds(&Th2[0][0], 32, kHid, 32 * bi + n, t), c);
+        for (int t = 0; t < 2; t++) c = mfma32(frag_lds(Tz1, kHid, 32 * w + n, t), frag_lds(Tx, kFeat, n, t), c);
+        if (n < kFeat)
+            for (int q = 0; q < 16; q++) out[oW1 + (32 * w + 8 * (q >> 2) + 4 * g + (q & 3)) * kFeat + n] = c[q];
+    } else {       // dW3[k][in]
+        const int bi = w - 2;
+        f32x16 c = {};
+        for (int t = 0; t < 2; t++) c = mfma32(frag_lds(Tdy, kOut, n, t), frag_lds(Th2, kHid, 32 * bi + n, t), c);
         if (g == 0)
             for (int i = 0; i < kOut; i++) out[oW3 + i * kHid + 32 * bi + n] = c[i];
     }
-    // bias gradients: sums over the 32 samples (lanes of one group)
-    for (int b = 0; b < 2; b++)
-        for (int q = 0; q < 16; q++) {
-            float a1 = dz1[b][q], a2 = dz2[b][q];
-            for (int o = 1; o < 32; o <<= 1) {
-                a1 += __shfl_xor(a1, o, kWave);
-                a2 += __shfl_xor(a2, o, kWave);
-            }
-            if (n == 0) {
-                const int u = 32 * b + 8 * (q >> 2) + 4 * g + (q & 3);
-                out[oB1 + u] = a1;
-                out[oB2 + u] = a2;
-            }
-        }
-    float b0 = dy0, b1 = dy1, ls = loss;
-    for (int o = 1; o < 64; o <<= 1) {
-        b0 += __shfl_xor(b0, o, kWave);
-        b1 += __shfl_xor(b1, o, kWave);
-        ls += __shfl_xor(ls, o, kWave);
-    }
-    if (lane == 0) {
-        out[oB3] = b0;
-        out[oB3 + 1] = b1;
-        out[kTrain] = ls;
-    }
 }
 
-// Sum of the tile partials in tile order (deterministic); optional Adam step.
-__global__ void k_reduce_adam(const float* part, int ntiles, float* grad, float* P, float* m, float* v, int update,
-                              float lr, float bc1, float bc2) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p > kTrain) return;
+// Sum of the tile partials (deterministic: each wave adds a run of tiles in
+// order, then the runs in order); optional Adam step, which writes the updated
+// weight's fragment elements too.  A block takes 64 parameters.  Bound by the
+// latency of the loads: one thread a parameter and tile after tile took 60 us
+// for 256 tiles, and packing the fragments another launch of 6.
+constexpr int kReduceWaves = 16;
+__global__ __launch_bounds__(kReduceWaves* kWave) void k_reduce_adam(const float* part, int ntiles, float* grad,
+                                                                    float* P, float* m, float* v, int update, float lr,
+                                                                    float bc1, float bc2, const int32_t* slots,
+                                                                    uint16_t* frag, float* loss) {
+    __shared__ float s_sum[kReduceWaves][kWave];
+    const int w = threadIdx.x / kWave, lane = lane_id();
+    const int p = blockIdx.x * kWave + lane;
+    const int per = (ntiles + kReduceWaves - 1) / kReduceWaves;
+    const int t1 = min(ntiles, (w + 1) * per);
     float s = 0.f;
-    for (int t = 0; t < ntiles; t++) s += part[(size_t)t * kPartStride + p];
+    if (p <= kTrain) {
+#pragma unroll 8
+        for (int t = w * per; t < t1; t++) s += part[(size_t)t * kPartStride + p];
+    }
+    s_sum[w][lane] = s;
+    __syncthreads();
+    if (w != 0 || p > kTrain) return;
+    for (int q = 1; q < kReduceWaves; q++) s += s_sum[q][lane];
     grad[p] = s;
+    if (p == kTrain && loss) *loss = s;
     if (!update || p == kTrain) return;
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
     const float mm = b1 * m[p] + (1.f - b1) * s;
     const float vv = b2 * v[p] + (1.f - b2) * s * s;
     m[p] = mm;
     v[p] = vv;
-    P[p] -= lr * (mm / bc1) / (sqrtf(vv / bc2) + eps);
+    const float np = P[p] - lr * (mm / bc1) / (sqrtf(vv / bc2) + eps);
+    P[p] = np;
+    for (int k = 0; k < 3; k++) {
+        const int t = slots[3 * p + k];
+        if (t >= 0) frag[t] = frag_bits(t, p, np, P);
+    }
 }
 
 // ----------------------------------------------------------- training data
@@ -1270,13 +1302,19 @@ void pack_model(Ctx& c) {
 }
 
 // Runs the tile kernel over nsamples and reduces (optionally with an Adam step).
-float train_pass(Ctx& c, const float* X, const float* Y, const float* Wt, int64_t ndata, int64_t nsamples, int hashed,
-                 uint64_t seed, float inv_b, int update, float lr) {
+// loss: device address for the batch's loss, or null.
+void train_pass(Ctx& c, const float* X, const float* Y, const float* Wt, int64_t ndata, int64_t nsamples, int hashed,
+                uint64_t seed, float inv_b, int update, float lr, float* loss) {
     const int64_t ntiles = (nsamples + 31) / 32;
     VVHD_CHECK(ntiles <= (1 << 20), VVHD_EINVAL, "learned far field: batch too large");
     c.grad_part.grow((size_t)ntiles * kPartStride);
     c.grad_out.grow(kPartStride);
-    hipLaunchKernelGGL(k_train_tile, dim3((unsigned)ntiles), dim3(64), 0, c.stream, X, Y, Wt, ndata, nsamples, hashed,
+    if (update && !c.frag_slots.p) {
+        c.frag_slots.grow(3 * kTrain);
+        hipLaunchKernelGGL(k_fill_slots, dim3(nblocks(3 * kTrain)), dim3(kBlock), 0, c.stream, c.frag_slots.p);
+        hipLaunchKernelGGL(k_frag_slots, dim3(nblocks(kFragElems)), dim3(kBlock), 0, c.stream, c.frag_slots.p);
+    }
+    hipLaunchKernelGGL(k_train_tile, dim3((unsigned)ntiles), dim3(256), 0, c.stream, X, Y, Wt, ndata, nsamples, hashed,
                        seed, inv_b, c.mlp_frags.p, c.mlp_params.p, c.grad_part.p);
     float bc1 = 1.f, bc2 = 1.f;
     if (update) {
@@ -1284,10 +1322,9 @@ float train_pass(Ctx& c, const float* X, const float* Y, const float* Wt, int64_
         bc1 = 1.f - std::pow(0.9f, (float)c.adam_t);
         bc2 = 1.f - std::pow(0.999f, (float)c.adam_t);
     }
-    hipLaunchKernelGGL(k_reduce_adam, dim3(nblocks(kTrain + 1)), dim3(kBlock), 0, c.stream, c.grad_part.p, (int)ntiles,
-                       c.grad_out.p, c.mlp_params.p, c.adam_m.p, c.adam_v.p, update, lr, bc1, bc2);
-    if (update) pack_model(c);
-    return 0.f;
+    hipLaunchKernelGGL(k_reduce_adam, dim3(nblocks(kTrain + 1, kWave)), dim3(kReduceWaves * kWave), 0, c.stream,
+                       (const float*)c.grad_part.p, (int)ntiles, c.grad_out.p, c.mlp_params.p, c.adam_m.p, c.adam_v.p,
+                       update, lr, bc1, bc2, (const int32_t*)c.frag_slots.p, c.mlp_frags.p, loss);
 }
 
 }  // namespace
@@ -1301,7 +1338,8 @@ void farfield_release(Ctx& c) {
     c.mlp_params.release();
     c.mlp_frags.release();
     c.mlp_loaded = false;
-    for (auto* b : {&c.tr_x, &c.tr_y, &c.tr_w, &c.adam_m, &c.adam_v, &c.grad_part, &c.grad_out}) b->release();
+    for (auto* b : {&c.tr_x, &c.tr_y, &c.tr_w, &c.adam_m, &c.adam_v, &c.grad_part, &c.grad_out, &c.tr_loss}) b->release();
+    c.frag_slots.release();
     c.pair_off.release();
     for (auto* b : {&c.pair_cnt, &c.pair_t, &c.pair_f}) b->release();
 }
@@ -1455,7 +1493,7 @@ int vvhd_far_gradients(vvhd_ctx* ctx, const float* X, const float* Y, const floa
     VVHD_HIP(hipMemcpyAsync(dX.p, X, (size_t)n * kFeat * 4, hipMemcpyHostToDevice, c.stream));
     VVHD_HIP(hipMemcpyAsync(dY.p, Y, (size_t)n * 2 * 4, hipMemcpyHostToDevice, c.stream));
     VVHD_HIP(hipMemcpyAsync(dW.p, W, (size_t)n * 4, hipMemcpyHostToDevice, c.stream));
-    train_pass(c, dX.p, dY.p, dW.p, n, n, 0, 0, 1.f / (float)n, 0, 0.f);
+    train_pass(c, dX.p, dY.p, dW.p, n, n, 0, 0, 1.f / (float)n, 0, 0.f, nullptr);
     std::vector<float> h(kTrain + 1);
     VVHD_HIP(hipMemcpyAsync(h.data(), c.grad_out.p, (kTrain + 1) * 4, hipMemcpyDeviceToHost, c.stream));
     VVHD_HIP(hipStreamSynchronize(c.stream));
@@ -1493,14 +1531,13 @@ int vvhd_far_train(vvhd_ctx* ctx, int32_t steps, int32_t batch, const float* lr,
     VVHD_CHECK(c.tr_n > 0, VVHD_ESTATE, "far_train: no training data");
     require_model(c);
     VVHD_HIP(hipSetDevice(c.device));
-    std::vector<float> lsum(steps, 0.f);
-    for (int s = 0; s < steps; s++) {
+    if (loss) c.tr_loss.grow(std::max(steps, 1));
+    for (int s = 0; s < steps; s++)
         train_pass(c, c.tr_x.p, c.tr_y.p, c.tr_w.p, c.tr_n, batch, 1, seed + (uint64_t)s * 0x9E3779B97F4A7C15ull,
-                   1.f / (float)batch, 1, lr[s]);
-        if (loss) VVHD_HIP(hipMemcpyAsync(&lsum[s], c.grad_out.p + kTrain, 4, hipMemcpyDeviceToHost, c.stream));
-    }
+                   1.f / (float)batch, 1, lr[s], loss ? c.tr_loss.p + s : nullptr);
+    if (loss && steps)
+        VVHD_HIP(hipMemcpyAsync(loss, c.tr_loss.p, (size_t)steps * 4, hipMemcpyDeviceToHost, c.stream));
     VVHD_HIP(hipStreamSynchronize(c.stream));
-    if (loss) std::memcpy(loss, lsum.data(), (size_t)steps * 4);
     API_END(ctx)
 }
 
