@@ -61,7 +61,8 @@ __device__ inline double slot_sum(double v, int t, int ntc, int nslot) {
     return s;
 }
 
-constexpr int kStage = 512;   // staged sources per wave
+constexpr int kStage = 256;   // staged sources of a wave
+constexpr int kFold = 8;      // terms between two folds of the partial sums
 
 // One wave per leaf and chunk of up to 16 targets.  The sources of the near
 // leaves within the cutoff are staged in LDS (FP32, relative to the leaf
@@ -74,27 +75,23 @@ constexpr int kStage = 512;   // staged sources per wave
 // dvx/dvy non-null (no segments only): the increment is stored there for
 // k_add_diffusive instead of being added to vx/vy.
 template <bool kSeg>
-__global__ __launch_bounds__(kBlock) void k_diffusive(TreeDev T, const double* __restrict__ x,
+__global__ __launch_bounds__(kWave) void k_diffusive(TreeDev T, const double* __restrict__ x,
                                                       const double* __restrict__ y, const double* __restrict__ g,
                                                       const double* __restrict__ ie, const vvhd_seg* segs, int nseg,
                                                       double* vx, double* vy, double re_one, const double* sim_re,
                                                       const int32_t* leaf_sim, double* dvx, double* dvy) {
-    __shared__ float s_x[kWavesPerBlock][kStage], s_y[kWavesPerBlock][kStage], s_g[kWavesPerBlock][kStage];
-    __shared__ int s_idx[kWavesPerBlock][kStage];   // vortex index of each slot of the chunk being staged
-    const int w = threadIdx.x / kWave;
-    const int l = xcd_block(blockIdx.x, gridDim.x) * kWavesPerBlock + w;
+    __shared__ __align__(16) float4 src[kStage];   // {x, y, circulation}
+    __shared__ int sidx[kStage];                   // vortex index of each slot of the chunk being staged
+    const int l = xcd_block(blockIdx.x, gridDim.x);
     if (l >= T.nleaf) return;
     const int lane = lane_id();
     const int L = T.leaf_node[l];
     const int v0 = T.v0[L], v1 = T.v1[L];
     if (v0 == v1) return;
     const double cx = T.nx[L], cy = T.ny[L];
+    const double4 box = T.pbox[L];
     const int64_t e0 = T.near_off[l], e1 = T.near_off[l + 1];
     const double re = sim_re ? sim_re[leaf_sim[l]] : re_one;   // Reynolds number of the leaf's simulation
-    float* sx = s_x[w];
-    float* sy = s_y[w];
-    float* sg = s_g[w];
-    int* sidx = s_idx[w];
 
     for (int base = v0; base < v1; base += 16) {
         const int ntc = min(16, v1 - base);
@@ -122,29 +119,37 @@ __global__ __launch_bounds__(kBlock) void k_diffusive(TreeDev T, const double* _
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
             if (active) {
-                const int k0 = pos ? 0 : kStage - nneg, k1 = pos ? npos : kStage;
-                int nk = 0;
-                for (int k = k0 + slot; k < k1; k += nslot) {
-                    // the partial sums fold every eight sources of this lane
-                    if ((++nk & 7) == 0) {
-                        s2x.fold();
-                        s2y.fold();
-                        s1.fold();
-                    }
-                    const float gj = sg[k];
-                    const float dx = tx - sx[k];
-                    const float dy = ty - sy[k];
-                    if (fabsf(dx) + fabsf(dy) < 1e-10f) continue;
+                const int n = pos ? npos : nneg;
+                const int step = pos ? nslot : -nslot;
+                int k = pos ? slot : kStage - 1 - slot;
+                auto term = [&](const float4 v) {
+                    const float dx = tx - v.x;
+                    const float dy = ty - v.y;
                     const float d2 = __builtin_fmaf(dx, dx, dy * dy);
                     const float rinv = __builtin_amdgcn_rsqf(d2);
                     const float exparg = -(d2 * rinv) * ief;
-                    if (exparg < (float)kExpArgLimit) continue;
-                    const float i1 = gj * __expf(exparg);
-                    const float f = i1 * rinv;
+                    const bool on = !(fabsf(dx) + fabsf(dy) < 1e-10f) & !(exparg < (float)kExpArgLimit);
+                    const float i1 = on ? v.z * __expf(exparg) : 0.f;
+                    const float f = i1 * (on ? rinv : 0.f);
                     s2x.q = __builtin_fmaf(dx, f, s2x.q);
                     s2y.q = __builtin_fmaf(dy, f, s2y.q);
                     s1.q += i1;
+                };
+                int q = slot;
+                for (; q + (kFold - 1) * nslot < n; q += kFold * nslot) {
+                    float4 v[kFold];
+#pragma unroll
+                    for (int u = 0; u < kFold; u++, k += step) v[u] = src[k];
+#pragma unroll
+                    for (int u = 0; u < kFold; u++) term(v[u]);
+                    s2x.fold();
+                    s2y.fold();
+                    s1.fold();
                 }
+                for (; q < n; q += nslot, k += step) term(src[k]);
+                s2x.fold();
+                s2y.fold();
+                s1.fold();
             }
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
@@ -177,20 +182,20 @@ __global__ __launch_bounds__(kBlock) void k_diffusive(TreeDev T, const double* _
                     float gv = 0.f, xv = 0.f, yv = 0.f;
                     if (q < take) {
                         const int j = sidx[q];
-                        gv = (float)g[j];
-                        xv = (float)(x[j] - cx);
-                        yv = (float)(y[j] - cy);
+                        const double xj = x[j], yj = y[j];
+                        xv = (float)(xj - cx);
+                        yv = (float)(yj - cy);
+                        // beyond the cutoff of every target: not staged
+                        const double bx = fmax(0.0, fmax(box.x - xj, xj - box.z));
+                        const double by = fmax(0.0, fmax(box.y - yj, yj - box.w));
+                        if (!(bx * bx + by * by > R2 * (1.0 + 1e-5))) gv = (float)g[j];
                     }
                     const uint64_t pm = __ballot(gv > 0.f), nm = __ballot(gv < 0.f);
                     const uint64_t below = (1ull << lane) - 1;
                     int k = -1;
                     if (gv > 0.f) k = npos + __popcll(pm & below);
                     if (gv < 0.f) k = kStage - 1 - (nneg + __popcll(nm & below));
-                    if (k >= 0) {
-                        sx[k] = xv;
-                        sy[k] = yv;
-                        sg[k] = gv;
-                    }
+                    if (k >= 0) src[k] = make_float4(xv, yv, gv, 0.f);
                     npos += __popcll(pm);
                     nneg += __popcll(nm);
                 }
@@ -363,7 +368,7 @@ void diffusive(Ctx& c, bool overlap) {
     if (overlap && nseg == 0) {
         c.dvx.grow(c.n + 1);
         c.dvy.grow(c.n + 1);
-        hipLaunchKernelGGL(k_diffusive<false>, dim3(grid), dim3(kBlock), 0, c.stream2, T, c.x.p, c.y.p, c.g.p, c.ie.p,
+        hipLaunchKernelGGL(k_diffusive<false>, dim3(nl), dim3(kWave), 0, c.stream2, T, c.x.p, c.y.p, c.g.p, c.ie.p,
                            c.segs.p, nseg, c.vx.p, c.vy.p, c.re, sim_re, (const int32_t*)c.t.leaf_sim.p, c.dvx.p,
                            c.dvy.p);
         VVHD_HIP(hipEventRecord(c.ev[7], c.stream2));
@@ -374,11 +379,11 @@ void diffusive(Ctx& c, bool overlap) {
         return;
     }
     if (nseg)
-        hipLaunchKernelGGL(k_diffusive<true>, dim3(grid), dim3(kBlock), 0, c.stream, T, c.x.p, c.y.p, c.g.p, c.ie.p,
+        hipLaunchKernelGGL(k_diffusive<true>, dim3(nl), dim3(kWave), 0, c.stream, T, c.x.p, c.y.p, c.g.p, c.ie.p,
                            c.segs.p, nseg, c.vx.p, c.vy.p, c.re, sim_re, (const int32_t*)c.t.leaf_sim.p,
                            (double*)nullptr, (double*)nullptr);
     else
-        hipLaunchKernelGGL(k_diffusive<false>, dim3(grid), dim3(kBlock), 0, c.stream, T, c.x.p, c.y.p, c.g.p, c.ie.p,
+        hipLaunchKernelGGL(k_diffusive<false>, dim3(nl), dim3(kWave), 0, c.stream, T, c.x.p, c.y.p, c.g.p, c.ie.p,
                            c.segs.p, nseg, c.vx.p, c.vy.p, c.re, sim_re, (const int32_t*)c.t.leaf_sim.p,
                            (double*)nullptr, (double*)nullptr);
     if (nseg) {
