@@ -181,7 +181,7 @@ __global__ __launch_bounds__(kBlock) void k_leaf_criteria(TreeDev T, const vvhd_
     restr_out[l] = restr;
 }
 
-constexpr int kStageE = 384;   // staged sources per wave (pass 1)
+constexpr int kStageE = 256;   // staged sources of a wave (pass 1)
 
 // Pass 1: top-2 of every target on the unmodified state, one wave per leaf
 // and chunk of up to 16 targets.  The sources (g != 0) of the selected near
@@ -189,27 +189,25 @@ constexpr int kStageE = 384;   // staged sources per wave (pass 1)
 // s = l / ntc) runs over every nslot-th of them; the slots' top-2s combine
 // afterwards (the top-2 under (d^2, index) does not depend on the order).
 // First the leaves touching the target leaf, then those whose box lies
-// within the largest second-neighbour distance found.
-__global__ __launch_bounds__(kBlock) void k_eps_top2(TreeDev T, const double* x, const double* y, const double* g,
+// within the largest second-neighbour distance found, without the sources
+// that are farther than it from the target leaf's box.
+// Bound by the latency of the staging loads.  A leaf per block: four leaves of
+// unequal work in one held 32 KB of LDS until the last had finished, and each
+// staged source was found by a search over the entries' offsets.
+__global__ __launch_bounds__(kWave) void k_eps_top2(TreeDev T, const double* x, const double* y, const double* g,
                                                      int merge, const double* leaf_crit, int32_t* nn1, int32_t* nn2,
                                                      double* d1o, double* d2o, uint8_t* eflag, int32_t* ecount,
                                                      int32_t* flag_list) {
-    __shared__ double s_x[kWavesPerBlock][kStageE], s_y[kWavesPerBlock][kStageE];
-    __shared__ int s_j[kWavesPerBlock][kStageE];
-    __shared__ int s_off[kWavesPerBlock][kWave], s_j0[kWavesPerBlock][kWave];
-    const int w = threadIdx.x / kWave;
-    const int l = xcd_block(blockIdx.x, gridDim.x) * kWavesPerBlock + w;
+    __shared__ double sx[kStageE], sy[kStageE];
+    __shared__ int sj[kStageE], sidx[kStageE];   // sidx: the vortices being staged
+    const int l = xcd_block(blockIdx.x, gridDim.x);
     if (l >= T.nleaf) return;
     const int lane = lane_id();
     const int L = T.leaf_node[l];
     const int v0 = T.v0[L], v1 = T.v1[L];
     const double crit = leaf_crit[l];
+    const double4 box = T.pbox[L];
     const int64_t e0 = T.near_off[l], e1 = T.near_off[l + 1];
-    double* sx = s_x[w];
-    double* sy = s_y[w];
-    int* sj = s_j[w];
-    int* soff = s_off[w];
-    int* sj0 = s_j0[w];
     auto wave_sync = [] {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -225,11 +223,25 @@ __global__ __launch_bounds__(kBlock) void k_eps_top2(TreeDev T, const double* x,
         Top2 st = top2_empty();
         auto compute = [&](int nsrc) {
             wave_sync();
-            if (active)
-                for (int k = slot; k < nsrc; k += nslot) {
-                    const int j = sj[k];
-                    if (j >= 0 && j != i) top2_insert(st, dist2(tx, ty, sx[k], sy[k]), j);
+            if (active) {
+                auto one = [&](int j, double px, double py) {
+                    if (j != i) top2_insert(st, dist2(tx, ty, px, py), j);
+                };
+                int k = slot;
+                for (; k + 3 * nslot < nsrc; k += 4 * nslot) {
+                    int j[4];
+                    double px[4], py[4];
+#pragma unroll
+                    for (int u = 0; u < 4; u++) {
+                        j[u] = sj[k + u * nslot];
+                        px[u] = sx[k + u * nslot];
+                        py[u] = sy[k + u * nslot];
+                    }
+#pragma unroll
+                    for (int u = 0; u < 4; u++) one(j[u], px[u], py[u]);
                 }
+                for (; k < nsrc; k += nslot) one(sj[k], sx[k], sy[k]);
+            }
             wave_sync();
         };
         // sources of the near leaves with lo < box distance <= hi
@@ -247,36 +259,43 @@ __global__ __launch_bounds__(kBlock) void k_eps_top2(TreeDev T, const double* x,
                     }
                 }
                 const int incl = wave_incl_scan(cnt);
+                const int off = incl - cnt;
                 const int tot = __shfl(incl, kWave - 1, kWave);
                 if (tot == 0) continue;
-                soff[lane] = incl - cnt;
-                sj0[lane] = j0;
-                wave_sync();
                 for (int done = 0; done < tot;) {
                     const int take = min(tot - done, kStageE - fill);
-                    for (int q = lane; q < take; q += kWave) {
-                        const int gidx = done + q;
-                        int a = 0, b = kWave - 1;   // last lane whose offset <= gidx
-                        while (a < b) {
-                            const int mid = (a + b + 1) >> 1;
-                            if (soff[mid] <= gidx)
-                                a = mid;
-                            else
-                                b = mid - 1;
+                    // each lane lists the vortices of its leaf that fall in this chunk
+                    for (int k = max(off, done); k < min(off + cnt, done + take); k++) sidx[k - done] = j0 + (k - off);
+                    wave_sync();
+                    for (int q0 = 0; q0 < take; q0 += kWave) {
+                        const int q = q0 + lane;
+                        int j = 0;
+                        double px = 0, py = 0;
+                        bool on = false;
+                        if (q < take) {
+                            j = sidx[q];
+                            px = x[j];
+                            py = y[j];
+                            const double bx = fmax(0.0, fmax(box.x - px, px - box.z));
+                            const double by = fmax(0.0, fmax(box.y - py, py - box.w));
+                            on = g[j] != 0 && (hi <= 0.0 || !(bx * bx + by * by > hi));
                         }
-                        const int j = sj0[a] + (gidx - soff[a]);
-                        sx[fill + q] = x[j];
-                        sy[fill + q] = y[j];
-                        sj[fill + q] = g[j] != 0 ? j : -1;
+                        const uint64_t m = __ballot(on);
+                        if (on) {
+                            const int k = fill + __popcll(m & ((1ull << lane) - 1));
+                            sx[k] = px;
+                            sy[k] = py;
+                            sj[k] = j;
+                        }
+                        fill += __popcll(m);
                     }
-                    fill += take;
                     done += take;
                     if (fill == kStageE) {
                         compute(fill);
                         fill = 0;
                     }
+                    wave_sync();   // the next chunk rewrites the index list
                 }
-                wave_sync();
             }
             if (fill) compute(fill);
         };
@@ -852,7 +871,7 @@ void epsilon(Ctx& c, int merge, int32_t* nn1_out, int32_t* nn2_out, int32_t* mer
                        (const int32_t*)c.sim_body.p, (const int32_t*)c.t.leaf_sim.p,
                        merge, c.leaf_crit.p, c.leaf_restr.p);
     if (nl > 0)
-        hipLaunchKernelGGL(k_eps_top2, dim3((nl + kWavesPerBlock - 1) / kWavesPerBlock), dim3(kBlock), 0, s, T, c.x.p,
+        hipLaunchKernelGGL(k_eps_top2, dim3(nl), dim3(kWave), 0, s, T, c.x.p,
                            c.y.p, c.g.p, merge, c.leaf_crit.p, c.nn1.p, c.nn2.p, c.d1.p, c.d2.p, c.eflag.p,
                            c.ecount.p, c.flag_list.p);
     int32_t flags = 0, merged = 0;
