@@ -116,9 +116,7 @@ __global__ __launch_bounds__(kWave) void k_diffusive(TreeDev T, const double* __
         // own sign's part only
         int npos = 0, nneg = 0;
         auto compute = [&]() {
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            wave_sync();
             if (active) {
                 const int n = pos ? npos : nneg;
                 const int step = pos ? nslot : -nslot;
@@ -152,9 +150,7 @@ __global__ __launch_bounds__(kWave) void k_diffusive(TreeDev T, const double* __
                 s2y.fold();
                 s1.fold();
             }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            wave_sync();
         };
         int fill = 0;
         for (int64_t eb = e0; eb < e1; eb += kWave) {
@@ -175,9 +171,7 @@ __global__ __launch_bounds__(kWave) void k_diffusive(TreeDev T, const double* __
                 const int take = min(tot - done, kStage - fill);
                 // each lane lists the vortices of its leaf that fall in this chunk
                 for (int k = max(off, done); k < min(off + cnt, done + take); k++) sidx[k - done] = j0 + (k - off);
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                wave_sync();
                 for (int q0 = 0; q0 < take; q0 += kWave) {
                     const int q = q0 + lane;
                     float gv = 0.f, xv = 0.f, yv = 0.f;
@@ -207,33 +201,36 @@ __global__ __launch_bounds__(kWave) void k_diffusive(TreeDev T, const double* __
                     npos = nneg = fill = 0;
                 }
                 // the next chunk rewrites the index list
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                wave_sync();
             }
         }
         if (fill) compute();
         // body segments of the near leaves within the cutoff (FP64)
         double s3x = 0, s3y = 0, s0 = 0;
         if (kSeg && nseg) {
+            // the segments of 64 entries at a time, all slots on them
             for (int64_t eb = e0; eb < e1; eb += kWave) {
                 const int64_t e = eb + lane;
-                int M = -1;
-                bool q = false;
+                int j0 = 0, cnt = 0;
                 if (e < e1) {
-                    M = T.near_list[e];
+                    const int M = T.near_list[e];
                     const int m = T.leaf_rank[M];
-                    q = T.seg_off[m + 1] > T.seg_off[m] && box_dist2p(T, L, M) <= R2;
+                    const int64_t q0 = T.seg_off[m], q1 = T.seg_off[m + 1];
+                    if (q1 > q0 && box_dist2p(T, L, M) <= R2) {
+                        j0 = (int)q0;
+                        cnt = (int)(q1 - q0);
+                    }
                 }
-                uint64_t mask = __ballot(q);
-                while (mask) {
-                    const int b = (int)__builtin_ctzll(mask);
-                    mask &= mask - 1;
-                    const int m = T.leaf_rank[__shfl(M, b, kWave)];
-                    for (int64_t qq = T.seg_off[m] + slot; qq < T.seg_off[m + 1]; qq += nslot) {
-                        if (!active) continue;
-                        const int sid = T.seg_list[qq];
-                        const vvhd_seg sgm = segs[sid];
+                const int incl = wave_incl_scan(cnt);
+                const int off = incl - cnt;
+                const int tot = __shfl(incl, kWave - 1, kWave);
+                for (int done = 0; done < tot; done += kStage) {
+                    const int take = min(tot - done, kStage);
+                    for (int k = max(off, done); k < min(off + cnt, done + take); k++)
+                        sidx[k - done] = T.seg_list[j0 + (k - off)];
+                    wave_sync();
+                    for (int k = slot; active && k < take; k += nslot) {
+                        const vvhd_seg& sgm = segs[sidx[k]];
                         const double drx = xi - sgm.x, dry = yi - sgm.y;
                         const double drabs2 = drx * drx + dry * dry;
                         const double drabs = sqrt(drabs2);
@@ -245,6 +242,7 @@ __global__ __launch_bounds__(kWave) void k_diffusive(TreeDev T, const double* __
                         s3y += dSy * expres;
                         s0 += (drabs * iei + 1) / drabs2 * (drx * dSx + dry * dSy) * expres;
                     }
+                    wave_sync();   // the next chunk rewrites the index list
                 }
             }
         }

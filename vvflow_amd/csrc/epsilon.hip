@@ -26,6 +26,7 @@
 // the same monotone rounded operations, so pruning never drops a candidate.
 
 #include "common.hpp"
+#include "near_flat.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -208,11 +209,6 @@ __global__ __launch_bounds__(kWave) void k_eps_top2(TreeDev T, const double* x, 
     const double crit = leaf_crit[l];
     const double4 box = T.pbox[L];
     const int64_t e0 = T.near_off[l], e1 = T.near_off[l + 1];
-    auto wave_sync = [] {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    };
     for (int base = v0; base < v1; base += 16) {
         const int ntc = min(16, v1 - base);
         const int nslot = kWave / ntc;
@@ -360,17 +356,20 @@ __device__ inline uint64_t d2_key(double d2) { return ord_from_double(isnan(d2) 
 
 // Upper bound of the second-neighbour distance over the searched targets of
 // every leaf (-1 for a leaf without one): a merge farther from the leaf's box
-// than this changes none of its targets.
-__global__ void k_leaf_maxd2(TreeDev T, const int32_t* r0, const int32_t* r1, int base, const double* d2a,
+// than this changes none of its targets.  16 lanes a leaf: a lane alone spent
+// 20 us on the leaves of 3k vortices, one load after another.
+constexpr int kMaxLanes = 16;
+__global__ __launch_bounds__(kBlock) void k_leaf_maxd2(TreeDev T, const int32_t* r0, const int32_t* r1, int base, const double* d2a,
                              const uint8_t* eflag, uint64_t* maxd2) {
-    const int l = blockIdx.x * blockDim.x + threadIdx.x;
+    const int l = blockIdx.x * (kBlock / kMaxLanes) + threadIdx.x / kMaxLanes, sub = threadIdx.x % kMaxLanes;
     if (l >= T.nleaf) return;
     const int L = T.leaf_node[l];
     uint64_t m = ord_from_double(-1.0);
     if (d2a)
-        for (int i = r0[L] - base; i < r1[L] - base; i++)
+        for (int i = r0[L] - base + sub; i < r1[L] - base; i += kMaxLanes)
             if (eflag[i] & 1) m = max(m, d2_key(d2a[i]));
-    maxd2[l] = m;
+    for (int o = kMaxLanes / 2; o > 0; o >>= 1) m = max(m, (uint64_t)__shfl_xor((unsigned long long)m, o, kMaxLanes));
+    if (sub == 0) maxd2[l] = m;
 }
 
 // The list being merged (the vortices, or the heat particles) and the state
@@ -432,11 +431,6 @@ __device__ Top2 seen_top2(const MergeArgs& A, int l, int L, int i, int excl, dou
     const int lane = lane_id();
     const int64_t e0 = T.near_off[l], e1 = T.near_off[l + 1];
     constexpr int kPer = 4;
-    auto wave_sync = [] {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    };
     auto scan = [&](bool touching, double bound) {
         Top2 st = top2_empty();
         const int w = G == 1 ? 0 : threadIdx.x / kWave;
@@ -673,6 +667,7 @@ __global__ __launch_bounds__(kMergeThreads) void k_merge_apply(MergeArgs A, int 
 // and new partner, which it kills or revives.  Work items are (change, 256
 // leaves): leaves before the element's hold no later target.
 __global__ __launch_bounds__(kBlock) void k_merge_mark(MergeArgs A, int parity, int chunks, int tag) {
+    __shared__ int s_tab[kWavesPerBlock][kNearTab];
     const TreeDev& T = A.T;
     const int nc = A.ctr[2 + parity];
     int32_t* list = parity ? A.list0 : A.list1;
@@ -689,31 +684,38 @@ __global__ __launch_bounds__(kBlock) void k_merge_mark(MergeArgs A, int parity, 
             if (p0 > q) push(p0);
             if (p1 > q) push(p1);
         }
+        // the leaves it may reach, then their targets, a lane each
         const int l = lq + ch * kBlock + threadIdx.x;
-        if (l >= lend) continue;
         const double4 b = A.cbox[e];
-        const int L = T.leaf_node[l];
-        const double m = double_from_ord(A.maxd2[l]);
-        {
+        int j0 = 0, cnt = 0;
+        if (l < lend) {
+            const int L = T.leaf_node[l];
+            const double m = double_from_ord(A.maxd2[l]);
             const double dx = fmax(0.0, fmax(b.x - double_from_ord(T.trx[L]), double_from_ord(T.blx[L]) - b.z));
             const double dy = fmax(0.0, fmax(b.y - double_from_ord(T.try_[L]), double_from_ord(T.bly[L]) - b.w));
-            if (dx * dx + dy * dy > m) continue;
+            if (!(dx * dx + dy * dy > m)) {
+                j0 = max(A.r0[L] - A.base, q + 1);
+                cnt = max(0, A.r1[L] - A.base - j0);
+            }
         }
         auto reach = [&](double px, double py, double d2) {
             const double dx = fmax(0.0, fmax(b.x - px, px - b.z)), dy = fmax(0.0, fmax(b.y - py, py - b.w));
             return !(dx * dx + dy * dy > d2);
         };
-        for (int i = A.r0[L] - A.base; i < A.r1[L] - A.base; i++) {
-            if (i <= q || !(A.eflag[i] & 1)) continue;
-            bool hit;
-            if (A.info[i].x >= 0) {
-                const double4 r = A.rec[i];
-                hit = reach(A.x[i], A.y[i], A.fd2[i]) || reach(r.x, r.y, A.d2[i]);
-            } else {
-                hit = reach(A.x[i], A.y[i], A.d2[i]);
+        wave_lay_out(j0, cnt, s_tab[threadIdx.x / kWave], [&](int m) {
+            for (int k = lane_id(); k < m; k += kWave) {
+                const int i = s_tab[threadIdx.x / kWave][k];
+                if (!(A.eflag[i] & 1)) continue;
+                bool hit;
+                if (A.info[i].x >= 0) {
+                    const double4 r = A.rec[i];
+                    hit = reach(A.x[i], A.y[i], A.fd2[i]) || reach(r.x, r.y, A.d2[i]);
+                } else {
+                    hit = reach(A.x[i], A.y[i], A.d2[i]);
+                }
+                if (hit) push(i);
             }
-            if (hit) push(i);
-        }
+        });
     }
 }
 
@@ -881,7 +883,7 @@ void epsilon(Ctx& c, int merge, int32_t* nn1_out, int32_t* nn2_out, int32_t* mer
         const MergeArgs A = merge_args(c, c.x.p, c.y.p, c.g.p, T.v0, T.v1, 0, n, 0, c.nn1.p, c.nn2.p, c.d1.p, c.d2.p,
                                        c.eflag.p, c.flag_list.p);
         hipLaunchKernelGGL(k_merge_init, dim3(nblocks(n)), dim3(kBlock), 0, s, A);
-        hipLaunchKernelGGL(k_leaf_maxd2, dim3(nblocks(nl)), dim3(kBlock), 0, s, T, A.r0, A.r1, 0,
+        hipLaunchKernelGGL(k_leaf_maxd2, dim3(nblocks(nl, kBlock / kMaxLanes)), dim3(kBlock), 0, s, T, A.r0, A.r1, 0,
                            (const double*)c.d2.p, (const uint8_t*)c.eflag.p, A.maxd2);
         merge_rounds(c, A, c.x.p, c.y.p, c.g.p, c.ecount.p + 5);
     }
@@ -925,7 +927,7 @@ int heat_epsilon(Ctx& c, int merge) {
     const int32_t start[8] = {(int32_t)nh, 0, 0, 0, 0, 0, 0, 0};
     VVHD_HIP(hipMemcpyAsync(c.ecount.p, start, sizeof(start), hipMemcpyHostToDevice, s));
     hipLaunchKernelGGL(k_merge_init, dim3(nblocks(nh)), dim3(kBlock), 0, s, A);
-    hipLaunchKernelGGL(k_leaf_maxd2, dim3(nblocks(T.nleaf)), dim3(kBlock), 0, s, T, A.r0, A.r1, A.base,
+    hipLaunchKernelGGL(k_leaf_maxd2, dim3(nblocks(T.nleaf, kBlock / kMaxLanes)), dim3(kBlock), 0, s, T, A.r0, A.r1, A.base,
                        (const double*)nullptr, (const uint8_t*)nullptr, A.maxd2);
     merge_rounds(c, A, c.heat.x.p, c.heat.y.p, c.heat.g.p, c.ecount.p + 5);
     hipLaunchKernelGGL(k_heat_eps_apply, dim3(nblocks(nh)), dim3(kBlock), 0, s, T.vleaf + T.hbase,

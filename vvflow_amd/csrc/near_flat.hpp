@@ -14,11 +14,25 @@ __device__ inline void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// The elements j of the ranges that range(list[e], j0, count) gives for e in
-// [e0, e1), in order: some of them at a time in tab[0..m), then chunk(m).  A
-// leaf has about 12 elements: taken leaf by leaf, four of five lanes idle, and
-// every leaf waits for its own chain of loads (list, range, element).  Here 64
-// entries are looked up at once, a lane each, and their elements laid out in
+// The elements [j0, j0 + cnt) of every lane's range, in lane order: some of
+// them at a time in tab[0..m), then chunk(m).
+template <typename Chunk>
+__device__ inline void wave_lay_out(int j0, int cnt, int* tab, Chunk chunk) {
+    const int incl = wave_incl_scan(cnt);
+    const int total = __builtin_amdgcn_readlane(incl, kWave - 1);
+    for (int done = 0; done < total; done += kNearTab) {
+        const int o = incl - cnt - done;
+        for (int t = max(0, -o); t < cnt && o + t < kNearTab; t++) tab[o + t] = j0 + t;
+        wave_sync();
+        chunk(min(kNearTab, total - done));
+        wave_sync();
+    }
+}
+
+// The same for the ranges that range(list[e], j0, cnt) gives for e in [e0, e1).
+// A leaf has about 12 elements: taken leaf by leaf, four of five lanes idle,
+// and every leaf waits for its own chain of loads (list, range, element).  Here
+// 64 entries are looked up at once, a lane each, and their elements laid out in
 // LDS.
 template <typename Range, typename Chunk>
 __device__ inline void wave_lay_out(const int32_t* list, int64_t e0, int64_t e1, int* tab, Range range, Chunk chunk) {
@@ -26,15 +40,7 @@ __device__ inline void wave_lay_out(const int32_t* list, int64_t e0, int64_t e1,
     for (int64_t eb = e0; eb < e1; eb += kWave) {
         int j0 = 0, cnt = 0;
         if (eb + lane < e1) range(list[eb + lane], j0, cnt);
-        const int incl = wave_incl_scan(cnt);
-        const int total = __builtin_amdgcn_readlane(incl, kWave - 1);
-        for (int done = 0; done < total; done += kNearTab) {
-            const int o = incl - cnt - done;
-            for (int t = max(0, -o); t < cnt && o + t < kNearTab; t++) tab[o + t] = j0 + t;
-            wave_sync();
-            chunk(min(kNearTab, total - done));
-            wave_sync();
-        }
+        wave_lay_out(j0, cnt, tab, chunk);
     }
 }
 
