@@ -448,6 +448,12 @@ __device__ inline double box_dist2(const TreeDev& T, int a, int b) {
     return dx * dx + dy * dy;
 }
 
+// Blocks that share a leaf's chunks of 16 targets in the kernels with a wave
+// per leaf.  A leaf that the least node size keeps whole has ten chunks and
+// more, one wave's work a whole launch waited for where the leaves are few;
+// where they are many, blocks without a chunk cost more than it gives.
+inline unsigned leaf_parts(int nleaf) { return (unsigned)std::clamp(16384 / std::max(nleaf, 1), 1, 8); }
+
 // host helpers implemented in ctx.hip
 void ensure_vortex_capacity(Ctx& c, int64_t n);
 // Refreshes the device copies of the simulation table (one simulation over

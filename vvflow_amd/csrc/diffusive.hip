@@ -88,13 +88,13 @@ __global__ __launch_bounds__(kWave) void k_diffusive(TreeDev T, const double* __
     const int lane = lane_id();
     const int L = T.leaf_node[l];
     const int v0 = T.v0[L], v1 = T.v1[L];
-    if (v0 == v1) return;
+    if (v0 + 16 * (int)blockIdx.y >= v1) return;
     const double cx = T.nx[L], cy = T.ny[L];
     const double4 box = T.pbox[L];
     const int64_t e0 = T.near_off[l], e1 = T.near_off[l + 1];
     const double re = sim_re ? sim_re[leaf_sim[l]] : re_one;   // Reynolds number of the leaf's simulation
 
-    for (int base = v0; base < v1; base += 16) {
+    for (int base = v0 + 16 * (int)blockIdx.y; base < v1; base += 16 * (int)gridDim.y) {
         const int ntc = min(16, v1 - base);
         const int nslot = kWave / ntc;
         const int t = lane % ntc, slot = lane / ntc;
@@ -367,7 +367,7 @@ void diffusive(Ctx& c, bool overlap) {
     if (overlap && nseg == 0) {
         c.dvx.grow(c.n + 1);
         c.dvy.grow(c.n + 1);
-        hipLaunchKernelGGL(k_diffusive<false>, dim3(nl), dim3(kWave), 0, c.stream2, T, c.x.p, c.y.p, c.g.p, c.ie.p,
+        hipLaunchKernelGGL(k_diffusive<false>, dim3(nl, leaf_parts(nl)), dim3(kWave), 0, c.stream2, T, c.x.p, c.y.p, c.g.p, c.ie.p,
                            c.segs.p, nseg, c.vx.p, c.vy.p, c.re, sim_re, (const int32_t*)c.t.leaf_sim.p, c.dvx.p,
                            c.dvy.p);
         VVHD_HIP(hipEventRecord(c.ev[7], c.stream2));
@@ -378,11 +378,11 @@ void diffusive(Ctx& c, bool overlap) {
         return;
     }
     if (nseg)
-        hipLaunchKernelGGL(k_diffusive<true>, dim3(nl), dim3(kWave), 0, c.stream, T, c.x.p, c.y.p, c.g.p, c.ie.p,
+        hipLaunchKernelGGL(k_diffusive<true>, dim3(nl, leaf_parts(nl)), dim3(kWave), 0, c.stream, T, c.x.p, c.y.p, c.g.p, c.ie.p,
                            c.segs.p, nseg, c.vx.p, c.vy.p, c.re, sim_re, (const int32_t*)c.t.leaf_sim.p,
                            (double*)nullptr, (double*)nullptr);
     else
-        hipLaunchKernelGGL(k_diffusive<false>, dim3(nl), dim3(kWave), 0, c.stream, T, c.x.p, c.y.p, c.g.p, c.ie.p,
+        hipLaunchKernelGGL(k_diffusive<false>, dim3(nl, leaf_parts(nl)), dim3(kWave), 0, c.stream, T, c.x.p, c.y.p, c.g.p, c.ie.p,
                            c.segs.p, nseg, c.vx.p, c.vy.p, c.re, sim_re, (const int32_t*)c.t.leaf_sim.p,
                            (double*)nullptr, (double*)nullptr);
     if (nseg) {

@@ -209,7 +209,7 @@ __global__ __launch_bounds__(kWave) void k_eps_top2(TreeDev T, const double* x, 
     const double crit = leaf_crit[l];
     const double4 box = T.pbox[L];
     const int64_t e0 = T.near_off[l], e1 = T.near_off[l + 1];
-    for (int base = v0; base < v1; base += 16) {
+    for (int base = v0 + 16 * (int)blockIdx.y; base < v1; base += 16 * (int)gridDim.y) {
         const int ntc = min(16, v1 - base);
         const int nslot = kWave / ntc;
         const int t = lane % ntc, slot = lane / ntc;
@@ -873,7 +873,7 @@ void epsilon(Ctx& c, int merge, int32_t* nn1_out, int32_t* nn2_out, int32_t* mer
                        (const int32_t*)c.sim_body.p, (const int32_t*)c.t.leaf_sim.p,
                        merge, c.leaf_crit.p, c.leaf_restr.p);
     if (nl > 0)
-        hipLaunchKernelGGL(k_eps_top2, dim3(nl), dim3(kWave), 0, s, T, c.x.p,
+        hipLaunchKernelGGL(k_eps_top2, dim3(nl, leaf_parts(nl)), dim3(kWave), 0, s, T, c.x.p,
                            c.y.p, c.g.p, merge, c.leaf_crit.p, c.nn1.p, c.nn2.p, c.d1.p, c.d2.p, c.eflag.p,
                            c.ecount.p, c.flag_list.p);
     int32_t flags = 0, merged = 0;
