@@ -734,6 +734,21 @@ __global__ void k_slip_cells(SlaeMap M, const vvhd_seg* segs, int nseg, double* 
     A[(size_t)sys * M.n * M.n + (size_t)col * M.n + row] = xi_g(sm.cx, sm.cy, segs[i], rd) * k1_2Pi;
 }
 
+// First row of every body in its system, its system, and each system's bodies.
+__global__ void k_slae_layout(const vvhd_body* bodies, const int32_t* sim_body, int nsys, int32_t* base,
+                              int32_t* body_sys, int32_t* sys_body) {
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= nsys) return;
+    int row = 0;
+    for (int b = sim_body[q]; b < sim_body[q + 1]; b++) {
+        base[b] = row;
+        body_sys[b] = q;
+        row += bodies[b].nseg + 9;
+    }
+    sys_body[q] = sim_body[q];
+    if (q == nsys - 1) sys_body[nsys] = sim_body[nsys];
+}
+
 // Right-hand side of the slip rows, one wave (= one block) per segment:
 // rotl(U) . dl minus NodeInfluence (:398-418) of the leaf holding the
 // segment centre (stree::findNode, TSortedTree.cpp:284-303).  The terms of 64
@@ -1113,7 +1128,10 @@ __global__ __launch_bounds__(kBodyBlock) void k_writeback(CoreMap C, vvhd_body* 
 
 }  // namespace
 
-void sync_bodies_to_host(Ctx& c) {
+// Steps change the bodies on the device only; a copy of them to the host after
+// each of five calls a step waited for the stream every time.
+void fetch_bodies(Ctx& c) {
+    if (!c.bodies_stale) return;
     const int ns = (int)c.segs_h.size(), nb = (int)c.bodies_h.size();
     if (ns)
         VVHD_HIP(hipMemcpyAsync(c.segs_h.data(), c.segs.p, (size_t)ns * sizeof(vvhd_seg), hipMemcpyDeviceToHost,
@@ -1122,6 +1140,7 @@ void sync_bodies_to_host(Ctx& c) {
         VVHD_HIP(hipMemcpyAsync(c.bodies_h.data(), c.bodies_d.p, (size_t)nb * sizeof(vvhd_body),
                                 hipMemcpyDeviceToHost, c.stream));
     VVHD_HIP(hipStreamSynchronize(c.stream));
+    c.bodies_stale = false;
 }
 
 static void exclusive_scan_i32(Ctx& c, const int32_t* in, int32_t* out, size_t n) {
@@ -1142,7 +1161,7 @@ void bodies_prepare(Ctx& c) {
                             c.stream));
     hipLaunchKernelGGL(k_body_properties, dim3(nb), dim3(kBodyBlock), 0, c.stream, c.bodies_d.p, c.segs.p,
                        c.body_geo.p);
-    sync_bodies_to_host(c);
+    c.bodies_stale = true;
 }
 
 void bodies_release(Ctx& c) {
@@ -1238,7 +1257,7 @@ void move_and_clean(Ctx& c, int remove, int64_t* cleaned) {
         c.sim_off_h[c.nsim] = c.n;
     }
     if (c.heat.n || c.streak.n) passive_move_and_clean(c);
-    if (nb) sync_bodies_to_host(c);
+    if (nb) c.bodies_stale = true;
 }
 
 void vortex_shed(Ctx& c) {
@@ -1280,7 +1299,7 @@ void vortex_shed(Ctx& c) {
         for (int q = 1; q <= ns; q++) c.sim_off_h[q] += pos[seg0[q]];
         c.n += pos[nseg];
         c.t.built = false;
-        sync_bodies_to_host(c);
+        c.bodies_stale = true;
         return;
     }
     hipLaunchKernelGGL(k_shed_write, dim3(nblocks(nseg)), dim3(kBlock), 0, c.stream, c.segs.p, nseg, c.iscratch0.p,
@@ -1290,7 +1309,7 @@ void vortex_shed(Ctx& c) {
     VVHD_HIP(hipStreamSynchronize(c.stream));
     c.n += added;
     c.t.built = false;
-    sync_bodies_to_host(c);
+    c.bodies_stale = true;
 }
 
 void calc_forces(Ctx& c) {
@@ -1310,7 +1329,7 @@ void calc_forces(Ctx& c) {
     hipLaunchKernelGGL(k_calc_forces, dim3(nb), dim3(kBodyBlock), 0, c.stream, c.bodies_d.p, c.segs.p, c.fric.p,
                        c.re, c.dt, c.pr, batch ? (const double*)c.sim_re.p : (const double*)nullptr,
                        (const int32_t*)body_sim);
-    sync_bodies_to_host(c);
+    c.bodies_stale = true;
 }
 
 void zero_forces(Ctx& c) {
@@ -1318,7 +1337,7 @@ void zero_forces(Ctx& c) {
     if (!nb) return;
     hipLaunchKernelGGL(k_zero_forces, dim3(nb), dim3(kBodyBlock), 0, c.stream, c.bodies_d.p, c.segs.p, c.fric.p);
     heat_layer_reset(c);
-    sync_bodies_to_host(c);
+    c.bodies_stale = true;
 }
 
 void calc_circulation(Ctx& c, double infx, double infy) {
@@ -1329,15 +1348,12 @@ void calc_circulation(Ctx& c, double infx, double infy) {
     // one system per simulation, all of the same order
     sim_sync(c);
     const int nsys = c.nsim;
-    std::vector<int32_t> base(nb), body_sys(nb);
     int n = -1, max_segs = 0;
     for (int q = 0; q < nsys; q++) {
         const int b0 = c.sim_body_h[q], b1 = c.sim_body_h[q + 1];
         VVHD_CHECK(b1 > b0, VVHD_EUNSUPPORTED, "calc_circulation: a simulation without bodies in the batch");
         int acc = 0, segs_q = 0;
         for (int b = b0; b < b1; b++) {
-            base[b] = acc;
-            body_sys[b] = q;
             acc += c.bodies_h[b].nseg + 9;
             segs_q += c.bodies_h[b].nseg;
         }
@@ -1350,9 +1366,8 @@ void calc_circulation(Ctx& c, double infx, double infy) {
     int32_t* d_base = c.slae_base.p;
     int32_t* d_body_sys = c.slae_base.p + nb;
     int32_t* d_sys_body = c.slae_base.p + 2 * nb;
-    VVHD_HIP(hipMemcpyAsync(d_base, base.data(), (size_t)nb * 4, hipMemcpyHostToDevice, s));
-    VVHD_HIP(hipMemcpyAsync(d_body_sys, body_sys.data(), (size_t)nb * 4, hipMemcpyHostToDevice, s));
-    VVHD_HIP(hipMemcpyAsync(d_sys_body, c.sim_body_h.data(), (size_t)(nsys + 1) * 4, hipMemcpyHostToDevice, s));
+    hipLaunchKernelGGL(k_slae_layout, dim3(nblocks(nsys)), dim3(kBlock), 0, s, c.bodies_d.p, (const int32_t*)c.sim_body.p,
+                       nsys, d_base, d_body_sys, d_sys_body);
     const size_t nn = (size_t)n * n, nall = nn * nsys;
     c.slae_A.grow(nall);
     c.slae_b.grow((size_t)n * nsys + 1);
@@ -1427,7 +1442,7 @@ void calc_circulation(Ctx& c, double infx, double infy) {
     hipLaunchKernelGGL(k_core_mv<kMvCorrect>, rows, dim3(kBlock), 0, s, C);
     hipLaunchKernelGGL(k_writeback, dim3(nb), dim3(kBodyBlock), 0, s, C, c.bodies_d.p, c.segs.p,
                        (const double*)c.slae_A.p, (const double*)c.slae_b.p, (const int32_t*)d_body_sys);
-    sync_bodies_to_host(c);
+    c.bodies_stale = true;
 }
 
 }  // namespace vvhd
@@ -1515,7 +1530,7 @@ int vvhd_zero_profiles(vvhd_ctx* ctx) {
     const int nseg = (int)c.segs_h.size();
     if (nseg) {
         hipLaunchKernelGGL(k_zero_profiles, dim3(nblocks(nseg)), dim3(kBlock), 0, c.stream, c.segs.p, nseg);
-        sync_bodies_to_host(c);
+        c.bodies_stale = true;
     }
     API_END(ctx)
 }

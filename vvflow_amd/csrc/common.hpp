@@ -153,6 +153,8 @@ struct ListLogBufs {
     }
 };
 
+constexpr int kMaxLevels = 126;   // deepest tree accepted
+constexpr int kLevCounters = 16 + 2 * (kMaxLevels + 2);   // ints of Ctx::lev_counters
 constexpr int kSubLevels = 128;   // levels of a subtree in TreeArrays::sub_lev
 
 struct TreeArrays {
@@ -323,6 +325,7 @@ struct Ctx {
     // segments and bodies (host copy is authoritative between calls)
     std::vector<vvhd_seg> segs_h;
     std::vector<vvhd_body> bodies_h;
+    bool bodies_stale = false;            // the device has changed them since (ranges and counts hold always)
     DBuf<vvhd_seg> segs;
     DBuf<double> fric;                       // per segment friction accumulator
     DBuf<int32_t> body_range;                // per body: first segment, count
@@ -394,7 +397,7 @@ struct Ctx {
 
     // timing
     hipEvent_t ev[16] = {};
-    int32_t* lev_counters = nullptr;      // pinned: the tree build's counters
+    int32_t* lev_counters = nullptr;      // pinned: the tree build's counters, then its levels' ranges
     int32_t* fm_counts = nullptr;         // pinned: flow-move survivors, removals in bodies, scan error
     bool phase_recorded[8] = {false, false, false, false, false, false, false, false};
 
@@ -501,7 +504,7 @@ void heat_layer_reset(Ctx& c);
 void list_append(Ctx& c, PList& L, const double* o6, int64_t m);
 void list_download(Ctx& c, PList& L, double* o6);
 void far_taylor(Ctx& c, double4* taylor);
-void sync_bodies_to_host(Ctx& c);
+void fetch_bodies(Ctx& c);   // segs_h and bodies_h from the device, where it has changed them
 __global__ void k_leaf_lists(TreeDev T, int32_t* out);
 void eps2h_h2(Ctx& c, bool h2, const double* xy, const int32_t* leaf, int64_t n, double* out);
 void grid_field(Ctx& c, int kind, const vvhd_grid& gr, double m, double dl, double inf_x, double inf_y, int with_ref,

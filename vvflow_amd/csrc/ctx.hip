@@ -85,17 +85,35 @@ __global__ void k_integrals_final(const double* part, int nb, double* out) {
 
 void reserve_vortices(Ctx& c, int64_t n, bool preserve);
 
+// The ranges of one simulation, written on the device.
+static __global__ void k_sim_one(int64_t* sim_off, int64_t n, int32_t* sim_body, int nb, double* sim_re, double re,
+                                 int32_t* seg_root, int nseg) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < nseg) seg_root[i] = 0;
+    if (i != 0) return;
+    sim_off[0] = 0;
+    sim_off[1] = n;
+    sim_body[0] = 0;
+    sim_body[1] = nb;
+    sim_re[0] = re;
+}
+
 void sim_sync(Ctx& c) {
-    if (c.nsim == 1) {
+    const int ns = c.nsim, nseg = (int)c.segs_h.size();
+    if (ns == 1) {
         c.sim_off_h = {0, c.n};
         c.sim_body_h = {0, (int32_t)c.bodies_h.size()};
         c.sim_re_h = {c.re};
     }
-    const int ns = c.nsim, nseg = (int)c.segs_h.size();
     c.sim_off.grow(ns + 1);
     c.sim_body.grow(ns + 1);
     c.sim_re.grow(ns);
     c.seg_root.grow(std::max(nseg, 1));
+    if (ns == 1) {   // four copies and a wait cost 60 us and more a tree
+        hipLaunchKernelGGL(k_sim_one, dim3(nblocks(nseg)), dim3(kBlock), 0, c.stream, c.sim_off.p, c.n, c.sim_body.p,
+                           c.sim_body_h[1], c.sim_re.p, c.re, c.seg_root.p, nseg);
+        return;
+    }
     std::vector<int32_t> root(nseg, 0);
     for (int s = 0; s < ns; s++)
         for (int b = c.sim_body_h[s]; b < c.sim_body_h[s + 1]; b++)
@@ -174,7 +192,7 @@ int vvhd_create(int device, vvhd_ctx** out) {
         delete ctx;
         return VVHD_EHIP;
     }
-    if (hipHostMalloc((void**)&ctx->c.lev_counters, 16 * sizeof(int32_t), hipHostMallocDefault) !=
+    if (hipHostMalloc((void**)&ctx->c.lev_counters, kLevCounters * sizeof(int32_t), hipHostMallocDefault) !=
             hipSuccess ||
         hipHostMalloc((void**)&ctx->c.fm_counts, 4 * sizeof(int32_t), hipHostMallocDefault) != hipSuccess) {
         delete ctx;
@@ -367,6 +385,7 @@ int vvhd_upload_bodies(vvhd_ctx* ctx, const vvhd_seg* segs, int32_t nseg, const 
     VVHD_CHECK(expect == nseg, VVHD_EINVAL, "upload_bodies: segment count mismatch");
     c.segs_h.assign(segs, segs + nseg);
     c.bodies_h.assign(bodies, bodies + nbody);
+    c.bodies_stale = false;
     c.nsim = 1;
     c.body_range.grow(2 * std::max(nbody, 1));
     if (nbody) {
@@ -474,6 +493,7 @@ int vvhd_download_bodies(vvhd_ctx* ctx, vvhd_seg* segs, int32_t nseg, vvhd_body*
     Ctx& c = ctx->c;
     VVHD_CHECK(nseg == (int32_t)c.segs_h.size() && nbody == (int32_t)c.bodies_h.size(), VVHD_EINVAL,
                "download_bodies: counts do not match");
+    fetch_bodies(c);
     if (nseg) {
         std::vector<double> fr(nseg);
         VVHD_HIP(hipMemcpyAsync(fr.data(), c.fric.p, (size_t)nseg * 8, hipMemcpyDeviceToHost, c.stream));

@@ -701,7 +701,7 @@ int vvhd_heat_shed(vvhd_ctx* ctx) {
     API_BEGIN
     REQUIRE_ONE_SIM(ctx->c, "heat_shed");
     vvhd::heat_shed(ctx->c);
-    vvhd::sync_bodies_to_host(ctx->c);
+    ctx->c.bodies_stale = true;
     API_END(ctx)
 }
 

@@ -46,7 +46,6 @@ namespace vvhd {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kMaxLevels = 126;   // deepest tree accepted
 
 inline int nblocks(int64_t n, int b = kBlock) { return (int)std::max<int64_t>(1, (n + b - 1) / b); }
 
@@ -1665,9 +1664,16 @@ __global__ void k_iota(int32_t* a, int n) {
     if (k < n) a[k] = k;
 }
 
-__global__ void k_fill_i32(int32_t* a, int n, int32_t v) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < n) a[k] = v;
+// Leaves and leaf groups of a single simulation.
+__global__ void k_one_root_leaves(int nl, int32_t* leaf_sim, int32_t* groups) {
+    const int l = blockIdx.x * blockDim.x + threadIdx.x;
+    if (l >= nl) return;
+    leaf_sim[l] = 0;
+    if (l % kWave) return;
+    int32_t* g = groups + 3 * (l / kWave);
+    g[0] = l;
+    g[1] = min(kWave, nl - l);
+    g[2] = 0;
 }
 
 template <typename T>
@@ -1944,6 +1950,7 @@ void tree_build(Ctx& c, int far_criteria, double min_node, double max_node, int3
                            enode.p, c.x.p, c.y.p, c.id.p, (const vvhd_seg*)c.segs.p, nseg, seg_node.p, t.sub_lev.p,
                            t.sub_nlev.p, sub_cap);
         VVHD_HIP(hipMemcpyAsync(hc, t.counters.p, 10 * sizeof(int32_t), hipMemcpyDeviceToHost, s));
+        VVHD_HIP(hipMemcpyAsync(hc + 16, t.lev_d.p, (depth + 1) * sizeof(int2), hipMemcpyDeviceToHost, s));
         VVHD_HIP(hipStreamSynchronize(s));
         VVHD_CHECK(hc[4] != 1, VVHD_ENOMEM, "tree_build: node capacity exceeded");
         VVHD_CHECK(hc[4] == 0 && depth < kMaxLevels - 1, VVHD_EUNSUPPORTED, "tree_build: tree deeper than supported");
@@ -1956,13 +1963,9 @@ void tree_build(Ctx& c, int far_criteria, double min_node, double max_node, int3
     t.max_depth = hc[5];
     t.nsub = std::min(hc[7], sub_cap);
     // node ranges of the levels over the whole list
-    const int nlev = depth + 1;
-    std::vector<int2> lv(nlev);
-    VVHD_HIP(hipMemcpyAsync(lv.data(), t.lev_d.p, nlev * sizeof(int2), hipMemcpyDeviceToHost, s));
-    VVHD_HIP(hipStreamSynchronize(s));
     std::vector<std::pair<int, int>>& levels = t.levels;
     levels.clear();
-    for (const int2& q : lv) levels.push_back({q.x, q.y});
+    for (int d = 0; d <= depth; d++) levels.push_back({hc[16 + 2 * d], hc[17 + 2 * d]});
     const int nl = t.nleaves_h;
 
     // tree order of the remaining fields
@@ -2006,12 +2009,13 @@ void tree_build(Ctx& c, int far_criteria, double min_node, double max_node, int3
                            t.pre.p);
     // leaf -> simulation and the list builder's leaf groups (64 leaves of one root)
     t.leaf_sim.grow(nl + 1);
-    std::vector<int32_t> grp;
     if (nroots == 1) {
-        if (nl) hipLaunchKernelGGL(k_fill_i32, dim3(nblocks(nl)), dim3(kBlock), 0, s, t.leaf_sim.p, nl, 0);
-        for (int f = 0; f < nl; f += kWave) grp.insert(grp.end(), {f, std::min(kWave, nl - f), 0});
+        t.ngroups = (nl + kWave - 1) / kWave;
+        t.groups.grow(3 * (size_t)t.ngroups + 3);
+        if (nl)
+            hipLaunchKernelGGL(k_one_root_leaves, dim3(nblocks(nl)), dim3(kBlock), 0, s, nl, t.leaf_sim.p, t.groups.p);
     } else {
-        std::vector<int32_t> rf(nroots + 1);
+        std::vector<int32_t> rf(nroots + 1), grp;
         VVHD_HIP(hipMemcpyAsync(rf.data(), t.root_first.p, (nroots + 1) * 4, hipMemcpyDeviceToHost, s));
         VVHD_HIP(hipStreamSynchronize(s));
         if (nl)
@@ -2019,11 +2023,11 @@ void tree_build(Ctx& c, int far_criteria, double min_node, double max_node, int3
                                nroots, nl, t.leaf_sim.p);
         for (int r = 0; r < nroots; r++)
             for (int f = rf[r]; f < rf[r + 1]; f += kWave) grp.insert(grp.end(), {f, std::min(kWave, rf[r + 1] - f), r});
+        t.ngroups = (int)grp.size() / 3;
+        t.groups.grow(grp.size() + 3);
+        if (!grp.empty())
+            VVHD_HIP(hipMemcpyAsync(t.groups.p, grp.data(), grp.size() * 4, hipMemcpyHostToDevice, s));
     }
-    t.ngroups = (int)grp.size() / 3;
-    t.groups.grow(grp.size() + 3);
-    if (!grp.empty())
-        VVHD_HIP(hipMemcpyAsync(t.groups.p, grp.data(), grp.size() * 4, hipMemcpyHostToDevice, s));
     // segments per leaf
     t.seg_off.grow(nl + 1);
     t.seg_leaf.grow(nseg + 1);
