@@ -585,80 +585,99 @@ __global__ __launch_bounds__(kEvalThreads) void k_merge_eval(MergeArgs A, int pa
         merge_eval<1>(A, parity, nd, s_tab, s_parts);
 }
 
-// Second part, one workgroup: the changed records take effect, the deaths
-// follow from all records, and every change gets the box of the positions it
-// involves (the element's own before and after, and its old and new
-// partner's).  Node boxes grow by the new positions, so that box distances
-// stay lower bounds.
+// Second part: the changed records take effect, the deaths follow from all
+// records, and every change gets the box of the positions it involves (the
+// element's own before and after, and its old and new partner's).  Node boxes
+// grow by the new positions, so that box distances stay lower bounds.  Three
+// phases, each over all changes before the next; thread tid of stride.
+__device__ inline void grow_box(double4& b, double px, double py) {
+    b.x = fmin(b.x, px);
+    b.y = fmin(b.y, py);
+    b.z = fmax(b.z, px);
+    b.w = fmax(b.w, py);
+}
+
+template <int kPhase>
+__device__ void merge_apply(const MergeArgs& A, int parity, int tid, int stride) {
+    const int nc = A.ctr[2 + parity];
+    if (kPhase == 0) {
+        for (int e = tid; e < nc; e += stride) {
+            const int q = A.chg[e], p = A.info[q].x;
+            double4 b = make_double4(A.x[q], A.y[q], A.x[q], A.y[q]);
+            A.chg_p[e] = p;
+            if (p >= 0) {
+                const double4 r = A.rec[q];
+                grow_box(b, r.x, r.y);
+                grow_box(b, A.x[p], A.y[p]);
+                A.info[p].y = INT32_MAX;
+            }
+            A.cbox[e] = b;
+        }
+    } else if (kPhase == 1) {
+        for (int e = tid; e < nc; e += stride) {
+            const int q = A.chg[e];
+            const double4 r = A.cand[q];
+            const int p = (int)r.w;
+            if (A.info[q].x == -1) A.ever[atomicAdd(&A.ctr[4], 1)] = q;
+            A.info[q].x = p >= 0 ? p : -2;
+            A.rec[q] = r;
+            if (p >= 0) {
+                double4 b = A.cbox[e];
+                grow_box(b, r.x, r.y);
+                grow_box(b, A.x[p], A.y[p]);
+                A.cbox[e] = b;
+                const int Lq = A.T.leaf_node[A.T.vleaf[A.base + q]];
+                if (!isnan(r.x)) {
+                    atomicMin((unsigned long long*)&A.blx[Lq], (unsigned long long)ord_from_double(r.x));
+                    atomicMax((unsigned long long*)&A.trx[Lq], (unsigned long long)ord_from_double(r.x));
+                }
+                if (!isnan(r.y)) {
+                    atomicMin((unsigned long long*)&A.bly[Lq], (unsigned long long)ord_from_double(r.y));
+                    atomicMax((unsigned long long*)&A.try_[Lq], (unsigned long long)ord_from_double(r.y));
+                }
+            }
+        }
+    } else {
+        const int ne = A.ctr[4];
+        for (int k = tid; k < ne; k += stride) {
+            const int q = A.ever[k], p = A.info[q].x;
+            if (p >= 0) atomicMin(&A.info[p].y, q);
+        }
+        // a partner that has merged itself is seen at its merged position too
+        for (int e = tid; e < nc; e += stride) {
+            const int q = A.chg[e];
+            double4 b = A.cbox[e];
+            for (int which = 0; which < 2; which++) {
+                const int p = which ? A.chg_p[e] : A.info[q].x;
+                if (p < 0 || A.info[p].x < 0) continue;
+                const double4 r = A.rec[p];
+                grow_box(b, r.x, r.y);
+            }
+            A.cbox[e] = b;
+        }
+        if (tid == 0) {
+            A.ctr[parity] = 0;
+            A.ctr[2 + (parity ^ 1)] = 0;
+        }
+    }
+}
+
+// All phases in one workgroup: 12 us for up to a few hundred changes.
 constexpr int kMergeThreads = 1024;
 __global__ __launch_bounds__(kMergeThreads) void k_merge_apply(MergeArgs A, int parity) {
-    const int nc = A.ctr[2 + parity], tid = threadIdx.x;
-    auto grow = [](double4& b, double px, double py) {
-        b.x = fmin(b.x, px);
-        b.y = fmin(b.y, py);
-        b.z = fmax(b.z, px);
-        b.w = fmax(b.w, py);
-    };
-    for (int e = tid; e < nc; e += kMergeThreads) {
-        const int q = A.chg[e], p = A.info[q].x;
-        double4 b = make_double4(A.x[q], A.y[q], A.x[q], A.y[q]);
-        A.chg_p[e] = p;
-        if (p >= 0) {
-            const double4 r = A.rec[q];
-            grow(b, r.x, r.y);
-            grow(b, A.x[p], A.y[p]);
-            A.info[p].y = INT32_MAX;
-        }
-        A.cbox[e] = b;
-    }
+    merge_apply<0>(A, parity, threadIdx.x, kMergeThreads);
     __threadfence();
     __syncthreads();
-    for (int e = tid; e < nc; e += kMergeThreads) {
-        const int q = A.chg[e];
-        const double4 r = A.cand[q];
-        const int p = (int)r.w;
-        if (A.info[q].x == -1) A.ever[atomicAdd(&A.ctr[4], 1)] = q;
-        A.info[q].x = p >= 0 ? p : -2;
-        A.rec[q] = r;
-        if (p >= 0) {
-            double4 b = A.cbox[e];
-            grow(b, r.x, r.y);
-            grow(b, A.x[p], A.y[p]);
-            A.cbox[e] = b;
-            const int Lq = A.T.leaf_node[A.T.vleaf[A.base + q]];
-            if (!isnan(r.x)) {
-                atomicMin((unsigned long long*)&A.blx[Lq], (unsigned long long)ord_from_double(r.x));
-                atomicMax((unsigned long long*)&A.trx[Lq], (unsigned long long)ord_from_double(r.x));
-            }
-            if (!isnan(r.y)) {
-                atomicMin((unsigned long long*)&A.bly[Lq], (unsigned long long)ord_from_double(r.y));
-                atomicMax((unsigned long long*)&A.try_[Lq], (unsigned long long)ord_from_double(r.y));
-            }
-        }
-    }
+    merge_apply<1>(A, parity, threadIdx.x, kMergeThreads);
     __threadfence();
     __syncthreads();
-    const int ne = A.ctr[4];
-    for (int k = tid; k < ne; k += kMergeThreads) {
-        const int q = A.ever[k], p = A.info[q].x;
-        if (p >= 0) atomicMin(&A.info[p].y, q);
-    }
-    // a partner that has merged itself is seen at its merged position too
-    for (int e = tid; e < nc; e += kMergeThreads) {
-        const int q = A.chg[e];
-        double4 b = A.cbox[e];
-        for (int which = 0; which < 2; which++) {
-            const int p = which ? A.chg_p[e] : A.info[q].x;
-            if (p < 0 || A.info[p].x < 0) continue;
-            const double4 r = A.rec[p];
-            grow(b, r.x, r.y);
-        }
-        A.cbox[e] = b;
-    }
-    if (tid == 0) {
-        A.ctr[parity] = 0;
-        A.ctr[2 + (parity ^ 1)] = 0;
-    }
+    merge_apply<2>(A, parity, threadIdx.x, kMergeThreads);
+}
+
+// A phase a launch, over the chip.
+template <int kPhase>
+__global__ __launch_bounds__(kBlock) void k_merge_apply_part(MergeArgs A, int parity) {
+    merge_apply<kPhase>(A, parity, blockIdx.x * kBlock + threadIdx.x, gridDim.x * kBlock);
 }
 
 // Third part: the targets after a changed element whose second-neighbour
@@ -805,7 +824,9 @@ namespace {
 // (three to about ten).  One workgroup committing merge after merge took
 // about 45 us each (5.8 ms a step for a cylinder wake of 3k vortices); a
 // round of all of them takes about 25 us.
-void merge_rounds(Ctx& c, MergeArgs A, double* x, double* y, double* g, int32_t* merged) {
+// left: the targets listed for the first round.
+constexpr int kApplyOne = 2048;
+void merge_rounds(Ctx& c, MergeArgs A, int32_t left, double* x, double* y, double* g, int32_t* merged) {
     hipStream_t s = c.stream;
     int most = 1;   // most leaves of one simulation
     if (c.nsim == 1) {
@@ -817,14 +838,19 @@ void merge_rounds(Ctx& c, MergeArgs A, double* x, double* y, double* g, int32_t*
         for (int q = 0; q < c.nsim; q++) most = std::max(most, rf[q + 1] - rf[q]);
     }
     const int chunks = (most + kBlock - 1) / kBlock;
-    int32_t left = 1;
     for (int64_t round = 0; left > 0; ) {
         VVHD_CHECK(round <= (int64_t)A.n + 8, VVHD_EHIP, "epsilon: the merges do not settle");
         for (int k = 0; k < 4; k++, round++) {
             const int par = (int)(round & 1);
             hipLaunchKernelGGL(k_merge_eval, dim3(kEvalBlocks), dim3(kEvalThreads), 0, s, A, par);
-            hipLaunchKernelGGL(k_merge_apply, dim3(1), dim3(kMergeThreads), 0, s, A, par);
-            hipLaunchKernelGGL(k_merge_mark, dim3(1024), dim3(kBlock), 0, s, A, par, chunks, (int)round + 1);
+            if (left <= kApplyOne) {
+                hipLaunchKernelGGL(k_merge_apply, dim3(1), dim3(kMergeThreads), 0, s, A, par);
+            } else {
+                hipLaunchKernelGGL(k_merge_apply_part<0>, dim3(256), dim3(kBlock), 0, s, A, par);
+                hipLaunchKernelGGL(k_merge_apply_part<1>, dim3(256), dim3(kBlock), 0, s, A, par);
+                hipLaunchKernelGGL(k_merge_apply_part<2>, dim3(256), dim3(kBlock), 0, s, A, par);
+            }
+            hipLaunchKernelGGL(k_merge_mark, dim3(2048), dim3(kBlock), 0, s, A, par, chunks, (int)round + 1);
         }
         VVHD_HIP(hipMemcpyAsync(&left, A.ctr + (round & 1), 4, hipMemcpyDeviceToHost, s));
         VVHD_HIP(hipStreamSynchronize(s));
@@ -885,7 +911,7 @@ void epsilon(Ctx& c, int merge, int32_t* nn1_out, int32_t* nn2_out, int32_t* mer
         hipLaunchKernelGGL(k_merge_init, dim3(nblocks(n)), dim3(kBlock), 0, s, A);
         hipLaunchKernelGGL(k_leaf_maxd2, dim3(nblocks(nl, kBlock / kMaxLanes)), dim3(kBlock), 0, s, T, A.r0, A.r1, 0,
                            (const double*)c.d2.p, (const uint8_t*)c.eflag.p, A.maxd2);
-        merge_rounds(c, A, c.x.p, c.y.p, c.g.p, c.ecount.p + 5);
+        merge_rounds(c, A, flags, c.x.p, c.y.p, c.g.p, c.ecount.p + 5);
     }
     hipLaunchKernelGGL(k_eps_apply, dim3(nblocks(n)), dim3(kBlock), 0, s, T, c.g.p, c.ie.p, n, c.nn1.p, c.nn2.p,
                        c.d1.p, c.d2.p, c.eflag.p, c.leaf_restr.p, c.src_ge.p);
@@ -929,7 +955,7 @@ int heat_epsilon(Ctx& c, int merge) {
     hipLaunchKernelGGL(k_merge_init, dim3(nblocks(nh)), dim3(kBlock), 0, s, A);
     hipLaunchKernelGGL(k_leaf_maxd2, dim3(nblocks(T.nleaf, kBlock / kMaxLanes)), dim3(kBlock), 0, s, T, A.r0, A.r1, A.base,
                        (const double*)nullptr, (const uint8_t*)nullptr, A.maxd2);
-    merge_rounds(c, A, c.heat.x.p, c.heat.y.p, c.heat.g.p, c.ecount.p + 5);
+    merge_rounds(c, A, (int32_t)nh, c.heat.x.p, c.heat.y.p, c.heat.g.p, c.ecount.p + 5);
     hipLaunchKernelGGL(k_heat_eps_apply, dim3(nblocks(nh)), dim3(kBlock), 0, s, T.vleaf + T.hbase,
                        (const int32_t*)b.hn1.p, (const int32_t*)b.hn2.p, (const double*)b.hd1.p,
                        (const double*)b.hd2.p, (const uint8_t*)b.hflag.p, (const double*)c.leaf_restr.p, c.heat.ie.p,

@@ -345,21 +345,87 @@ __global__ void k_fill_i32v(int32_t* a, int64_t n, int32_t v) {
 
 // MFlowmove::heat_shed (MFlowmove.cpp:237-273), bodies and segments in
 // order, appending at nh (capacity checked by the host); the new count goes
-// to out_n.
-__global__ void k_heat_shed(const vvhd_body* bodies, int nbody, vvhd_seg* segs, const int32_t* cond,
-                            const float* heat_const, const int64_t* layer, double* hx, double* hy, double* hg,
-                            double* hvx, double* hvy, double* hie, int64_t nh, int64_t* out_n, int32_t* err) {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    int64_t n = nh;
-    auto push = [&](double px, double py, double g) {
-        hx[n] = px;
-        hy[n] = py;
-        hg[n] = g;
-        hvx[n] = 0;
-        hvy[n] = 0;
-        hie[n] = 0;
-        n++;
+// to out_n.  used: zeros, one per particle.  Bound by latency: one thread for
+// all segments took 265 us for 350 of them.  A block's threads take a segment
+// each; where segments depend on each other through a layer particle, one
+// thread goes through them in order.
+constexpr int kShedThreads = 1024;
+__global__ __launch_bounds__(kShedThreads) void k_heat_shed(const vvhd_body* bodies, int nbody, vvhd_seg* segs,
+                                                            const int32_t* cond, const float* heat_const,
+                                                            const int64_t* layer, double* hx, double* hy, double* hg,
+                                                            double* hvx, double* hvy, double* hie, int64_t nh,
+                                                            int32_t* used, int64_t* out_n, int32_t* err) {
+    __shared__ int s_serial, s_cnt[kShedThreads / kWave];
+    const int t = threadIdx.x;
+    auto put = [&](int64_t at, double px, double py, double g) {
+        hx[at] = px;
+        hy[at] = py;
+        hg[at] = g;
+        hvx[at] = 0;
+        hvy[at] = 0;
+        hie[at] = 0;
     };
+    // a layer particle of two segments, or one shed in this call or missing:
+    // what a segment finds there depends on those before it
+    if (t == 0) s_serial = 0;
+    __syncthreads();
+    for (int b = 0; b < nbody; b++) {
+        if (cond[b] != 2) continue;
+        for (int k = t; k < bodies[b].nseg; k += kShedThreads) {
+            const int64_t no = layer[bodies[b].first_seg + k];
+            if (no >= nh || (no >= 0 && atomicExch(&used[no], 1) != 0)) s_serial = 1;
+        }
+    }
+    __syncthreads();
+    int64_t n = nh;
+    if (!s_serial) {
+        for (int b = 0; b < nbody; b++) {
+            const int c = cond[b], first = bodies[b].first_seg, ns = bodies[b].nseg;
+            if (c < 1 || c > 3) continue;
+            for (int k0 = 0; k0 < ns; k0 += kShedThreads) {
+                const int i = first + k0 + t;
+                bool shed = false;
+                double px = 0, py = 0, g = 0;
+                if (k0 + t < ns) {
+                    vvhd_seg& s = segs[i];
+                    px = s.x + (-s.dly) * 0.5;
+                    py = s.y + s.dlx * 0.5;
+                    if (c == 1) {
+                        shed = s.hsum != 0;
+                        if (shed) {
+                            g = -s.hsum;
+                            s.hsum = 0;
+                        }
+                    } else {
+                        g = (s.dlx * s.dlx + s.dly * s.dly) * (double)heat_const[i];
+                        const int64_t no = c == 2 ? layer[i] : -1;
+                        if (no >= 0) {
+                            s.hsum += g - hg[no];
+                            hg[no] = g;
+                        } else {
+                            s.hsum += g;
+                            shed = true;
+                        }
+                    }
+                }
+                const uint64_t m = __ballot(shed);
+                if (lane_id() == 0) s_cnt[t / kWave] = __popcll(m);
+                __syncthreads();
+                int before = 0, total = 0;
+                for (int w = 0; w < kShedThreads / kWave; w++) {
+                    if (w < t / kWave) before += s_cnt[w];
+                    total += s_cnt[w];
+                }
+                if (shed) put(n + before + __popcll(m & ((1ull << lane_id()) - 1)), px, py, g);
+                n += total;
+                __syncthreads();
+            }
+        }
+        if (t == 0) *out_n = n;
+        return;
+    }
+    if (t != 0) return;
+    auto push = [&](double px, double py, double g) { put(n++, px, py, g); };
     for (int b = 0; b < nbody; b++) {
         const int c = cond[b];
         for (int k = 0; k < bodies[b].nseg; k++) {
@@ -500,11 +566,11 @@ void heat_shed(Ctx& c) {
     hipStream_t s = c.stream;
     c.heat.reserve(c.heat.n + nseg + 1, true, s);
     c.lscratch0.grow(2);
-    c.iscratch4.grow(2);
-    hipLaunchKernelGGL(k_fill_i32v, dim3(1), dim3(64), 0, s, c.iscratch4.p, (int64_t)2, 0);
-    hipLaunchKernelGGL(k_heat_shed, dim3(1), dim3(1), 0, s, c.bodies_d.p, nb, c.segs.p, (const int32_t*)c.heat_cond.p,
+    c.iscratch4.grow(c.heat.n + 2);   // error, then the particles seen as a layer's
+    hipLaunchKernelGGL(k_fill_i32v, dim3(nblocks(c.heat.n + 2)), dim3(kBlock), 0, s, c.iscratch4.p, c.heat.n + 2, 0);
+    hipLaunchKernelGGL(k_heat_shed, dim3(1), dim3(kShedThreads), 0, s, c.bodies_d.p, nb, c.segs.p, (const int32_t*)c.heat_cond.p,
                        (const float*)c.heat_const.p, (const int64_t*)c.heat_layer.p, c.heat.x.p, c.heat.y.p,
-                       c.heat.g.p, c.heat.vx.p, c.heat.vy.p, c.heat.ie.p, c.heat.n, c.lscratch0.p, c.iscratch4.p);
+                       c.heat.g.p, c.heat.vx.p, c.heat.vy.p, c.heat.ie.p, c.heat.n, c.iscratch4.p + 2, c.lscratch0.p, c.iscratch4.p);
     int64_t n = 0;
     int32_t err = 0;
     VVHD_HIP(hipMemcpyAsync(&n, c.lscratch0.p, 8, hipMemcpyDeviceToHost, s));
