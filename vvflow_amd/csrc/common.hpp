@@ -256,7 +256,7 @@ struct MergeBufs {
     DBuf<double4> rec, cand, cbox;                // records, next records, boxes of the changes
     DBuf<double> fd2;                             // second-neighbour distance before a merge
     DBuf<int32_t> stamp, list, chg, chg_p, ever;
-    DBuf<uint64_t> maxd2;                         // per leaf: bound of the second-neighbour distance
+    DBuf<uint64_t> maxd2, lbox, cbound;           // per leaf: bound of the second-neighbour distance, box; of chunks
     DBuf<int32_t> hn1, hn2, hlist;                // heat list: search results
     DBuf<double> hd1, hd2;
     DBuf<uint8_t> hflag;
@@ -266,6 +266,8 @@ struct MergeBufs {
         for (auto* b : {&fd2, &hd1, &hd2}) b->release();
         for (auto* b : {&stamp, &list, &chg, &chg_p, &ever, &hn1, &hn2, &hlist}) b->release();
         maxd2.release();
+        lbox.release();
+        cbound.release();
         hflag.release();
     }
 };

@@ -356,11 +356,12 @@ __device__ inline uint64_t d2_key(double d2) { return ord_from_double(isnan(d2) 
 
 // Upper bound of the second-neighbour distance over the searched targets of
 // every leaf (-1 for a leaf without one): a merge farther from the leaf's box
-// than this changes none of its targets.  16 lanes a leaf: a lane alone spent
+// than this changes none of its targets.  And the leaves' boxes in their order
+// (lbox: four arrays), which the rounds read and grow.  16 lanes a leaf: a lane alone spent
 // 20 us on the leaves of 3k vortices, one load after another.
 constexpr int kMaxLanes = 16;
 __global__ __launch_bounds__(kBlock) void k_leaf_maxd2(TreeDev T, const int32_t* r0, const int32_t* r1, int base, const double* d2a,
-                             const uint8_t* eflag, uint64_t* maxd2) {
+                             const uint8_t* eflag, uint64_t* maxd2, uint64_t* lbox) {
     const int l = blockIdx.x * (kBlock / kMaxLanes) + threadIdx.x / kMaxLanes, sub = threadIdx.x % kMaxLanes;
     if (l >= T.nleaf) return;
     const int L = T.leaf_node[l];
@@ -370,6 +371,31 @@ __global__ __launch_bounds__(kBlock) void k_leaf_maxd2(TreeDev T, const int32_t*
             if (eflag[i] & 1) m = max(m, d2_key(d2a[i]));
     for (int o = kMaxLanes / 2; o > 0; o >>= 1) m = max(m, (uint64_t)__shfl_xor((unsigned long long)m, o, kMaxLanes));
     if (sub == 0) maxd2[l] = m;
+    if (sub < 4) lbox[(size_t)sub * T.nleaf + l] = sub == 0 ? T.blx[L] : sub == 1 ? T.bly[L] : sub == 2 ? T.trx[L] : T.try_[L];
+}
+
+// The same bound and box over every kChunk leaves (cbound: least x, least y,
+// most x, most y, bound; five arrays).
+constexpr int kChunk = kBlock;
+__global__ __launch_bounds__(kBlock) void k_chunk_bounds(int nleaf, const uint64_t* maxd2, const uint64_t* lbox,
+                                                         uint64_t* cbound) {
+    __shared__ uint64_t s_part[kWavesPerBlock][5];
+    const int l = min(blockIdx.x * kChunk + (int)threadIdx.x, nleaf - 1), w = threadIdx.x / kWave;
+    uint64_t v[5];
+    for (int k = 0; k < 5; k++) v[k] = k < 4 ? lbox[(size_t)k * nleaf + l] : maxd2[l];
+    for (int o = kWave / 2; o > 0; o >>= 1)
+        for (int k = 0; k < 5; k++) {
+            const uint64_t u = __shfl_xor((unsigned long long)v[k], o, kWave);
+            v[k] = k < 2 ? min(v[k], u) : max(v[k], u);
+        }
+    if (lane_id() == 0)
+        for (int k = 0; k < 5; k++) s_part[w][k] = v[k];
+    __syncthreads();
+    const int k = threadIdx.x;
+    if (k >= 5) return;
+    uint64_t r = s_part[0][k];
+    for (int q = 1; q < kWavesPerBlock; q++) r = k < 2 ? min(r, s_part[q][k]) : max(r, s_part[q][k]);
+    cbound[(size_t)k * gridDim.x + blockIdx.x] = r;
 }
 
 // The list being merged (the vortices, or the heat particles) and the state
@@ -392,7 +418,8 @@ struct MergeArgs {
     int32_t *nn1, *nn2;
     double *d1, *d2;
     uint8_t* eflag;
-    uint64_t* maxd2;
+    uint64_t *maxd2, *lbox, *cbound;
+    int nchunk;
     int2* info;
     double4 *rec, *cand;
     double* fd2;
@@ -499,6 +526,34 @@ __global__ void k_merge_init(MergeArgs A) {
     }
 }
 
+// Entries that a block collects for a list in global memory: one claim of the
+// list's counter a block (12 ns each, 8000 and more of them a round where every
+// wave claimed its own).  Entries past the room go to the list at once.
+struct BlockList {
+    static constexpr int kRoom = 512;
+    int n, base;
+    int32_t at[kRoom];
+    __device__ void begin() {   // all threads
+        if (threadIdx.x == 0) n = 0;
+        __syncthreads();
+    }
+    __device__ void push(int32_t v, int32_t* list, int32_t* count) {
+        const int k = atomicAdd(&n, 1);
+        if (k < kRoom)
+            at[k] = v;
+        else
+            list[atomicAdd(count, 1)] = v;
+    }
+    __device__ void end(int32_t* list, int32_t* count) {   // all threads
+        __syncthreads();
+        const int m = min(n, kRoom);
+        if (m == 0) return;
+        if (threadIdx.x == 0) base = atomicAdd(count, m);
+        __syncthreads();
+        for (int k = threadIdx.x; k < m; k += blockDim.x) list[base + k] = at[k];
+    }
+};
+
 // One round, first part: every listed target is visited as the reference does
 // when the merges of the targets before it are those of the last round.  Its
 // search results are written in place (only the marking pass reads them), its
@@ -508,7 +563,8 @@ __global__ void k_merge_init(MergeArgs A) {
 // round with a wave each, 64 with a block).
 constexpr int kEvalThreads = 512, kEvalWaves = kEvalThreads / kWave, kEvalBlocks = 512;
 template <int G>
-__device__ void merge_eval(const MergeArgs& A, int parity, int nd, int (*s_tab)[kMergeTab], Top2* parts) {
+__device__ void merge_eval(const MergeArgs& A, int parity, int nd, int (*s_tab)[kMergeTab], Top2* parts,
+                           BlockList& changes) {
     const TreeDev& T = A.T;
     const int w = threadIdx.x / kWave, lane = lane_id();
     const int32_t* list = parity ? A.list1 : A.list0;
@@ -559,6 +615,7 @@ __device__ void merge_eval(const MergeArgs& A, int parity, int nd, int (*s_tab)[
         if (alive) {
             const uint64_t key = max(d2_key(st.d2), d2_key(first_d2));
             atomicMax((unsigned long long*)&A.maxd2[l], (unsigned long long)key);
+            atomicMax((unsigned long long*)&A.cbound[4 * (size_t)A.nchunk + l / kChunk], (unsigned long long)key);
         }
         bool changed = partner != max(own.x, -1);
         if (!changed && partner >= 0) {
@@ -570,7 +627,7 @@ __device__ void merge_eval(const MergeArgs& A, int parity, int nd, int (*s_tab)[
         if (changed) {
             rec.w = (double)partner;
             A.cand[i] = rec;
-            A.chg[atomicAdd(&A.ctr[2 + parity], 1)] = i;
+            changes.push(i, A.chg, &A.ctr[2 + parity]);
         }
     }
 }
@@ -578,11 +635,14 @@ __device__ void merge_eval(const MergeArgs& A, int parity, int nd, int (*s_tab)[
 __global__ __launch_bounds__(kEvalThreads) void k_merge_eval(MergeArgs A, int parity) {
     __shared__ int s_tab[kEvalWaves][kMergeTab];
     __shared__ Top2 s_parts[kEvalWaves];
+    __shared__ BlockList s_changes;
     const int nd = A.ctr[parity];
+    s_changes.begin();
     if (nd <= (int)gridDim.x)
-        merge_eval<kEvalWaves>(A, parity, nd, s_tab, s_parts);
+        merge_eval<kEvalWaves>(A, parity, nd, s_tab, s_parts, s_changes);
     else
-        merge_eval<1>(A, parity, nd, s_tab, s_parts);
+        merge_eval<1>(A, parity, nd, s_tab, s_parts, s_changes);
+    s_changes.end(A.chg, &A.ctr[2 + parity]);
 }
 
 // Second part: the changed records take effect, the deaths follow from all
@@ -626,14 +686,31 @@ __device__ void merge_apply(const MergeArgs& A, int parity, int tid, int stride)
                 grow_box(b, r.x, r.y);
                 grow_box(b, A.x[p], A.y[p]);
                 A.cbox[e] = b;
-                const int Lq = A.T.leaf_node[A.T.vleaf[A.base + q]];
-                if (!isnan(r.x)) {
-                    atomicMin((unsigned long long*)&A.blx[Lq], (unsigned long long)ord_from_double(r.x));
-                    atomicMax((unsigned long long*)&A.trx[Lq], (unsigned long long)ord_from_double(r.x));
-                }
-                if (!isnan(r.y)) {
-                    atomicMin((unsigned long long*)&A.bly[Lq], (unsigned long long)ord_from_double(r.y));
-                    atomicMax((unsigned long long*)&A.try_[Lq], (unsigned long long)ord_from_double(r.y));
+                const int lq = A.T.vleaf[A.base + q], Lq = A.T.leaf_node[lq], nl = A.T.nleaf;
+                const size_t ck = lq / kChunk, nk = A.nchunk;
+                // mostly inside already: the leaf's copy tells for the node, too
+                auto least = [](uint64_t* a, uint64_t key) {
+                    if (key >= *a) return false;
+                    atomicMin((unsigned long long*)a, (unsigned long long)key);
+                    return true;
+                };
+                auto most = [](uint64_t* a, uint64_t key) {
+                    if (key <= *a) return false;
+                    atomicMax((unsigned long long*)a, (unsigned long long)key);
+                    return true;
+                };
+                for (int k = 0; k < 2; k++) {
+                    const double v = k == 0 ? r.x : r.y;
+                    if (isnan(v)) continue;
+                    const uint64_t key = ord_from_double(v);
+                    if (least(&A.lbox[k * (size_t)nl + lq], key)) {
+                        least(k == 0 ? &A.blx[Lq] : &A.bly[Lq], key);
+                        least(&A.cbound[k * nk + ck], key);
+                    }
+                    if (most(&A.lbox[(2 + k) * (size_t)nl + lq], key)) {
+                        most(k == 0 ? &A.trx[Lq] : &A.try_[Lq], key);
+                        most(&A.cbound[(2 + k) * nk + ck], key);
+                    }
                 }
             }
         }
@@ -683,59 +760,82 @@ __global__ __launch_bounds__(kBlock) void k_merge_apply_part(MergeArgs A, int pa
 // Third part: the targets after a changed element whose second-neighbour
 // distance reaches its box are visited again in the next round (those it
 // does not reach cannot take or lose a neighbour by it), and so are its old
-// and new partner, which it kills or revives.  Work items are (change, 256
-// leaves): leaves before the element's hold no later target.
-__global__ __launch_bounds__(kBlock) void k_merge_mark(MergeArgs A, int parity, int chunks, int tag) {
+// and new partner, which it kills or revives.
+// A block per change: each wave tests the chunks of leaves from the element's
+// on (leaves before it hold no later target), a lane each; the block's threads
+// the leaves of a chunk that may be reached; and their targets a lane each.
+// Testing every leaf for every change took 120 us a round in the batch of 16
+// cylinders, 14 us behind one in 100k vortices; now 18 and 8.5.
+__global__ __launch_bounds__(kBlock) void k_merge_mark(MergeArgs A, int parity, int tag) {
     __shared__ int s_tab[kWavesPerBlock][kNearTab];
+    __shared__ BlockList s_next;
     const TreeDev& T = A.T;
-    const int nc = A.ctr[2 + parity];
+    const int nc = A.ctr[2 + parity], lane = lane_id();
     int32_t* list = parity ? A.list0 : A.list1;
     auto push = [&](int i) {
-        if (atomicExch(&A.stamp[i], tag) != tag) list[atomicAdd(&A.ctr[parity ^ 1], 1)] = i;
+        if (atomicExch(&A.stamp[i], tag) != tag) s_next.push(i, list, &A.ctr[parity ^ 1]);
     };
-    for (int64_t it = blockIdx.x; it < (int64_t)nc * chunks; it += gridDim.x) {
-        const int e = (int)(it / chunks), ch = (int)(it % chunks);
+    auto far = [](const double4& b, uint64_t blx, uint64_t bly, uint64_t trx, uint64_t try_, double m) {
+        const double dx = fmax(0.0, fmax(b.x - double_from_ord(trx), double_from_ord(blx) - b.z));
+        const double dy = fmax(0.0, fmax(b.y - double_from_ord(try_), double_from_ord(bly) - b.w));
+        return dx * dx + dy * dy > m;
+    };
+    s_next.begin();
+    for (int e = blockIdx.x; e < nc; e += gridDim.x) {
         const int q = A.chg[e];
+        const double4 b = A.cbox[e];
         const int lq = T.vleaf[A.base + q];
         const int lend = A.root_first[A.leaf_sim[lq] + 1];
-        if (ch == 0 && threadIdx.x == 0) {
+        if (threadIdx.x == 0) {
             const int p0 = A.chg_p[e], p1 = A.info[q].x;
             if (p0 > q) push(p0);
             if (p1 > q) push(p1);
-        }
-        // the leaves it may reach, then their targets, a lane each
-        const int l = lq + ch * kBlock + threadIdx.x;
-        const double4 b = A.cbox[e];
-        int j0 = 0, cnt = 0;
-        if (l < lend) {
-            const int L = T.leaf_node[l];
-            const double m = double_from_ord(A.maxd2[l]);
-            const double dx = fmax(0.0, fmax(b.x - double_from_ord(T.trx[L]), double_from_ord(T.blx[L]) - b.z));
-            const double dy = fmax(0.0, fmax(b.y - double_from_ord(T.try_[L]), double_from_ord(T.bly[L]) - b.w));
-            if (!(dx * dx + dy * dy > m)) {
-                j0 = max(A.r0[L] - A.base, q + 1);
-                cnt = max(0, A.r1[L] - A.base - j0);
-            }
         }
         auto reach = [&](double px, double py, double d2) {
             const double dx = fmax(0.0, fmax(b.x - px, px - b.z)), dy = fmax(0.0, fmax(b.y - py, py - b.w));
             return !(dx * dx + dy * dy > d2);
         };
-        wave_lay_out(j0, cnt, s_tab[threadIdx.x / kWave], [&](int m) {
-            for (int k = lane_id(); k < m; k += kWave) {
-                const int i = s_tab[threadIdx.x / kWave][k];
-                if (!(A.eflag[i] & 1)) continue;
-                bool hit;
-                if (A.info[i].x >= 0) {
-                    const double4 r = A.rec[i];
-                    hit = reach(A.x[i], A.y[i], A.fd2[i]) || reach(r.x, r.y, A.d2[i]);
-                } else {
-                    hit = reach(A.x[i], A.y[i], A.d2[i]);
+        auto leaves = [&](int l) {
+            const double m = l >= lq && l < lend ? double_from_ord(A.maxd2[l]) : -1.0;
+            int j0 = 0, cnt = 0;
+            if (!(m < 0)) {
+                const uint64_t* lb = A.lbox + l;
+                const size_t nl = T.nleaf;
+                if (!far(b, lb[0], lb[nl], lb[2 * nl], lb[3 * nl], m)) {
+                    const int L = T.leaf_node[l];
+                    j0 = max(A.r0[L] - A.base, q + 1);
+                    cnt = max(0, A.r1[L] - A.base - j0);
                 }
-                if (hit) push(i);
             }
-        });
+            wave_lay_out(j0, cnt, s_tab[threadIdx.x / kWave], [&](int n) {
+                for (int k = lane; k < n; k += kWave) {
+                    const int i = s_tab[threadIdx.x / kWave][k];
+                    if (!(A.eflag[i] & 1)) continue;
+                    bool hit;
+                    if (A.info[i].x >= 0) {
+                        const double4 r = A.rec[i];
+                        hit = reach(A.x[i], A.y[i], A.fd2[i]) || reach(r.x, r.y, A.d2[i]);
+                    } else {
+                        hit = reach(A.x[i], A.y[i], A.d2[i]);
+                    }
+                    if (hit) push(i);
+                }
+            });
+        };
+        const int ck1 = (lend - 1) / kChunk;
+        for (int c0 = lq / kChunk; c0 <= ck1; c0 += kWave) {
+            bool may = false;
+            if (c0 + lane <= ck1) {
+                const uint64_t* cb = A.cbound + c0 + lane;
+                const size_t nk = A.nchunk;
+                const double m = double_from_ord(cb[4 * nk]);
+                may = !(m < 0) && !far(b, cb[0], cb[nk], cb[2 * nk], cb[3 * nk], m);
+            }
+            for (uint64_t mask = __ballot(may); mask; mask &= mask - 1)
+                leaves((c0 + (int)__builtin_ctzll(mask)) * kChunk + threadIdx.x);
+        }
     }
+    s_next.end(list, &A.ctr[parity ^ 1]);
 }
 
 // The converged merges written to the list, one workgroup: every merging
@@ -828,16 +928,8 @@ namespace {
 constexpr int kApplyOne = 2048;
 void merge_rounds(Ctx& c, MergeArgs A, int32_t left, double* x, double* y, double* g, int32_t* merged) {
     hipStream_t s = c.stream;
-    int most = 1;   // most leaves of one simulation
-    if (c.nsim == 1) {
-        most = A.T.nleaf;
-    } else {
-        std::vector<int32_t> rf(c.nsim + 1);
-        VVHD_HIP(hipMemcpyAsync(rf.data(), c.t.root_first.p, rf.size() * 4, hipMemcpyDeviceToHost, s));
-        VVHD_HIP(hipStreamSynchronize(s));
-        for (int q = 0; q < c.nsim; q++) most = std::max(most, rf[q + 1] - rf[q]);
-    }
-    const int chunks = (most + kBlock - 1) / kBlock;
+    hipLaunchKernelGGL(k_chunk_bounds, dim3(A.nchunk), dim3(kBlock), 0, s, A.T.nleaf, (const uint64_t*)A.maxd2,
+                       (const uint64_t*)A.lbox, A.cbound);
     for (int64_t round = 0; left > 0; ) {
         VVHD_CHECK(round <= (int64_t)A.n + 8, VVHD_EHIP, "epsilon: the merges do not settle");
         for (int k = 0; k < 4; k++, round++) {
@@ -850,7 +942,7 @@ void merge_rounds(Ctx& c, MergeArgs A, int32_t left, double* x, double* y, doubl
                 hipLaunchKernelGGL(k_merge_apply_part<1>, dim3(256), dim3(kBlock), 0, s, A, par);
                 hipLaunchKernelGGL(k_merge_apply_part<2>, dim3(256), dim3(kBlock), 0, s, A, par);
             }
-            hipLaunchKernelGGL(k_merge_mark, dim3(2048), dim3(kBlock), 0, s, A, par, chunks, (int)round + 1);
+            hipLaunchKernelGGL(k_merge_mark, dim3(1024), dim3(kBlock), 0, s, A, par, (int)round + 1);
         }
         VVHD_HIP(hipMemcpyAsync(&left, A.ctr + (round & 1), 4, hipMemcpyDeviceToHost, s));
         VVHD_HIP(hipStreamSynchronize(s));
@@ -870,9 +962,12 @@ MergeArgs merge_args(Ctx& c, const double* x, const double* y, const double* g, 
     b.fd2.grow(n);
     for (auto* p : {&b.stamp, &b.list, &b.chg, &b.chg_p, &b.ever}) p->grow(n);
     b.maxd2.grow(c.t.nleaves_h + 1);
+    b.lbox.grow(4 * (size_t)c.t.nleaves_h + 1);
+    const int nchunk = nblocks(c.t.nleaves_h, kChunk);
+    b.cbound.grow(5 * (size_t)nchunk);
     TreeArrays& t = c.t;
     return MergeArgs{tree_dev(t), x, y, g, r0, r1, base, (int)n, heat, c.leaf_crit.p, nn1, nn2, d1, d2, eflag,
-                     b.maxd2.p, b.info.p, b.rec.p, b.cand.p, b.fd2.p, b.stamp.p, list0, b.list.p, b.chg.p, b.chg_p.p,
+                     b.maxd2.p, b.lbox.p, b.cbound.p, nchunk, b.info.p, b.rec.p, b.cand.p, b.fd2.p, b.stamp.p, list0, b.list.p, b.chg.p, b.chg_p.p,
                      b.ever.p, b.cbox.p, c.ecount.p, t.blx.p, t.bly.p, t.trx.p, t.try_.p, t.leaf_sim.p,
                      t.root_first.p};
 }
@@ -910,7 +1005,7 @@ void epsilon(Ctx& c, int merge, int32_t* nn1_out, int32_t* nn2_out, int32_t* mer
                                        c.eflag.p, c.flag_list.p);
         hipLaunchKernelGGL(k_merge_init, dim3(nblocks(n)), dim3(kBlock), 0, s, A);
         hipLaunchKernelGGL(k_leaf_maxd2, dim3(nblocks(nl, kBlock / kMaxLanes)), dim3(kBlock), 0, s, T, A.r0, A.r1, 0,
-                           (const double*)c.d2.p, (const uint8_t*)c.eflag.p, A.maxd2);
+                           (const double*)c.d2.p, (const uint8_t*)c.eflag.p, A.maxd2, A.lbox);
         merge_rounds(c, A, flags, c.x.p, c.y.p, c.g.p, c.ecount.p + 5);
     }
     hipLaunchKernelGGL(k_eps_apply, dim3(nblocks(n)), dim3(kBlock), 0, s, T, c.g.p, c.ie.p, n, c.nn1.p, c.nn2.p,
@@ -954,7 +1049,7 @@ int heat_epsilon(Ctx& c, int merge) {
     VVHD_HIP(hipMemcpyAsync(c.ecount.p, start, sizeof(start), hipMemcpyHostToDevice, s));
     hipLaunchKernelGGL(k_merge_init, dim3(nblocks(nh)), dim3(kBlock), 0, s, A);
     hipLaunchKernelGGL(k_leaf_maxd2, dim3(nblocks(T.nleaf, kBlock / kMaxLanes)), dim3(kBlock), 0, s, T, A.r0, A.r1, A.base,
-                       (const double*)nullptr, (const uint8_t*)nullptr, A.maxd2);
+                       (const double*)nullptr, (const uint8_t*)nullptr, A.maxd2, A.lbox);
     merge_rounds(c, A, (int32_t)nh, c.heat.x.p, c.heat.y.p, c.heat.g.p, c.ecount.p + 5);
     hipLaunchKernelGGL(k_heat_eps_apply, dim3(nblocks(nh)), dim3(kBlock), 0, s, T.vleaf + T.hbase,
                        (const int32_t*)b.hn1.p, (const int32_t*)b.hn2.p, (const double*)b.hd1.p,
