@@ -151,12 +151,24 @@ __global__ void k_fill_roots(int32_t* enode, int n, const int64_t* sim_off, int 
     enode[k] = lo;
 }
 
+// Adds 1 to count[node] for every active lane, a claim for all lanes of a node:
+// a counter takes one every 12 ns or so, and neighbouring segments share theirs.
+// Called by all lanes of the wave.
+__device__ inline void count_wave(int32_t* count, int node, bool active) {
+    for (uint64_t left = __ballot(active); left;) {
+        const int lead = __builtin_amdgcn_readlane(node, (int)__builtin_ctzll(left));
+        const uint64_t same = __ballot(active && node == lead);
+        if (lane_id() == (int)__builtin_ctzll(left)) atomicAdd(&count[lead], (int)__popcll(same));
+        left &= ~same;
+    }
+}
+
 // Segments start at the root of their body's simulation.
 __global__ void k_seg_roots(NodeView nv, const int32_t* seg_root, int nseg, int32_t* seg_node) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nseg) return;
-    seg_node[i] = seg_root[i];
-    atomicAdd(&nv.nseg[seg_root[i]], 1);
+    const int r = i < nseg ? seg_root[i] : 0;
+    if (i < nseg) seg_node[i] = r;
+    count_wave(nv.nseg, r, i < nseg);
 }
 
 // Adds a point to a node's bounding box; NaN coordinates are ignored, as by
@@ -336,10 +348,20 @@ __global__ void k_child_boxes(NodeView nv, const int32_t* counters, const double
     }
 }
 
+// Adds the lanes' segments to their nodes: counts and boxes.  Most nodes' boxes
+// hold them already, with their vortices': those need no claim.
+__device__ inline void add_segs_wave(NodeView nv, int node, double px, double py, bool active) {
+    count_wave(nv.nseg, node, active);
+    const bool in = active && ord_from_double(px) >= nv.blx[node] && ord_from_double(px) <= nv.trx[node] &&
+                    ord_from_double(py) >= nv.bly[node] && ord_from_double(py) <= nv.try_[node];
+    bbox_add_wave(nv, node, px, py, active && !in);
+}
+
 // Segments of the root bounding boxes.
 __global__ void k_root_segs(NodeView nv, const vvhd_seg* segs, const int32_t* seg_root, int nseg) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < nseg) bbox_add(nv, seg_root[i], segs[i].x, segs[i].y);
+    const bool on = i < nseg;
+    bbox_add_wave(nv, on ? seg_root[i] : 0, on ? segs[i].x : 0, on ? segs[i].y : 0, on);
 }
 
 // Root bounding boxes when there are more roots than k_bbox_top handles.
@@ -565,15 +587,18 @@ __global__ void k_swap(NodeView nv, int32_t* enode, const int32_t* flag, const i
 // Segments descend one level (stable partition == per-segment descent).
 __global__ void k_seg_step(NodeView nv, const vvhd_seg* segs, int nseg, int32_t* seg_node) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nseg) return;
-    const int node = seg_node[s];
-    if (nv.split[node] != 2) return;
-    const int c = nv.ch1[node] + (goes_left(nv, node, segs[s].x, segs[s].y) ? 0 : 1);
-    seg_node[s] = c;
-    atomicAdd(&nv.nseg[c], 1);
-    bbox_add(nv, c, segs[s].x, segs[s].y);
+    const int node = s < nseg ? seg_node[s] : 0;
+    const bool active = s < nseg && nv.split[node] == 2;
+    int c = 0;
+    double px = 0, py = 0;
+    if (active) {
+        px = segs[s].x;
+        py = segs[s].y;
+        c = nv.ch1[node] + (goes_left(nv, node, px, py) ? 0 : 1);
+        seg_node[s] = c;
+    }
+    add_segs_wave(nv, c, px, py, active);
 }
-
 
 // The ids that k_subtree took lie before the children of the level's other
 // nodes.
