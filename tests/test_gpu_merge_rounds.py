@@ -47,16 +47,26 @@ def cloud(n, seed):
     return o
 
 
+def wide(n, seed):
+    """Such layers strung out downstream: leaves by the ten thousand."""
+    o = cloud(n, seed)
+    o[:, 0] += np.floor(np.random.default_rng(seed + 1).uniform(0, 800, n)) * 1.3
+    return o
+
+
+KINDS = {"ring": None, "cloud": cloud, "wide": wide}
 CASES = [("ring", 1, 0.1, "same"), ("ring", 2, 0.1, "same"), ("ring", 3, 0.1, "alternating"),
          ("ring", 17, 0.05, "same"), ("ring", 65, 0.2, "equal and opposite"), ("ring", 300, 0.02, "same"),
-         ("ring", 700, 0.3, "alternating"), ("cloud", 500, 5, ""), ("cloud", 3000, 6, "")]
+         ("ring", 700, 0.3, "alternating"), ("cloud", 500, 5, ""), ("cloud", 3000, 6, ""),
+         # more targets than one workgroup applies, and more chunks of 256 leaves than a wave tests at once
+         ("cloud", 30000, 7, ""), ("wide", 250000, 8, "")]
 
 
 @pytest.mark.parametrize("kind,n,a,signs", CASES)
 def test_merge_rounds_vs_oracle(ctx, kind, n, a, signs):
     print(f"case merge rounds {kind} n={n} {a} {signs}", flush=True)
-    v = ring(n, a, signs, n) if kind == "ring" else cloud(n, a)
-    h = ring(n, a, "same", n + 1) if kind == "ring" else cloud(n, a + 100)
+    v = ring(n, a, signs, n) if kind == "ring" else KINDS[kind](n, a)
+    h = ring(n, a, "same", n + 1) if kind == "ring" else KINDS[kind](n, a + 100)
     h[:, 2] = np.abs(h[:, 2])
     corners = cylinder_corners(200)
     dl = 200 * np.sin(np.pi / 200) / 199
