@@ -189,6 +189,7 @@ struct TreeArrays {
     ListLogBufs log;                                    // records of the list builder's walks
     DBuf<uint8_t> trav;                                 // packed node records of the list builder
     DBuf<double4> pbox;                                 // packed node boxes (pack_boxes)
+    DBuf<double2> cmk;                                  // packed monopoles of the nodes, 64 bytes each
     DBuf<int32_t> groups;                               // list builder leaf groups: {first leaf, count, root}
     int ngroups = 0;
     DBuf<int32_t> leaf_sim;                             // per leaf: its simulation (root)
@@ -420,6 +421,7 @@ struct TreeDev {
     const double4* pbox;   // per node {blx, bly, trx, try} as doubles (pack_boxes)
     const int32_t *h0, *h1, *s0, *s1;   // heat / streak ranges (element numbering)
     int hbase, sbase;                   // first heat and first streak element
+    const double2* cmk;                 // per node {cmp_x, cmp_y}, {cmp_g, cmm_g}, {cmm_x, cmm_y}, unused (k_trav_nodes)
 };
 
 inline TreeDev tree_dev(const TreeArrays& t) {
@@ -428,7 +430,7 @@ inline TreeDev tree_dev(const TreeArrays& t) {
                    t.far_off.p, t.seg_off.p, t.near_list.p, t.far_list.p, t.seg_list.p, t.vleaf.p,  t.cmp_x.p,
                    t.cmp_y.p,   t.cmp_g.p,  t.cmm_x.p,   t.cmm_y.p,   t.cmm_g.p,   t.cmp_ie.p,  t.cmm_ie.p,
                    t.nleaves_h, t.pbox.p, t.h0.p,   t.h1.p,      t.s0.p,      t.s1.p,      t.hbase,
-                   t.sbase};
+                   t.sbase,     t.cmk.p};
 }
 
 // box_dist2 from the packed copy of the boxes: one 32-byte load per node.

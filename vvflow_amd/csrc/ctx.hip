@@ -244,6 +244,7 @@ void vvhd_destroy(vvhd_ctx* ctx) {
     for (auto* b : {&t.near_off, &t.far_off, &t.seg_off}) b->release();
     for (auto* b : {&t.groups, &t.leaf_sim, &t.root_first, &t.pre}) b->release();
     t.log.release();
+    t.cmk.release();
     t.lev_d.release();
     t.sub_lev.release();
     t.trav.release();

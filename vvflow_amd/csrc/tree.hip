@@ -1009,6 +1009,10 @@ struct CMView {
     float *pie, *mie;
 };
 
+CMView cm_view(const TreeArrays& t) {
+    return CMView{t.cmp_x.p, t.cmp_y.p, t.cmp_g.p, t.cmm_x.p, t.cmm_y.p, t.cmm_g.p, t.cmp_ie.p, t.cmm_ie.p};
+}
+
 // Per-sign monopoles of a node (CMp, CMm); ie is _1_eps, infinite or 0.
 struct Monopoles {
     double px, py, pg, mx, my, mg;
@@ -1311,10 +1315,13 @@ struct TravNode {
 static_assert(sizeof(TravNode) == 32, "TravNode layout");
 
 __global__ void k_trav_nodes(NodeView nv, int nnodes, const int32_t* pre, const int32_t* nleaves, TravNode* out,
-                             int32_t* most) {
+                             int32_t* most, CMView cm, double2* cmk) {
     const int id = blockIdx.x * blockDim.x + threadIdx.x;
     if (id < 2) most[id] = 0;
     if (id >= nnodes) return;
+    cmk[4 * (size_t)id] = make_double2(cm.px[id], cm.py[id]);
+    cmk[4 * (size_t)id + 1] = make_double2(cm.pg[id], cm.mg[id]);
+    cmk[4 * (size_t)id + 2] = make_double2(cm.mx[id], cm.my[id]);
     TravNode r;
     r.x = nv.x[id];
     r.y = nv.y[id];
@@ -2013,7 +2020,7 @@ void tree_build(Ctx& c, int far_criteria, double min_node, double max_node, int3
     }
 
     // leaf counts and monopoles bottom-up, DFS ranks top-down
-    CMView cm{t.cmp_x.p, t.cmp_y.p, t.cmp_g.p, t.cmm_x.p, t.cmm_y.p, t.cmm_g.p, t.cmp_ie.p, t.cmm_ie.p};
+    const CMView cm = cm_view(t);
     if (t.nsub)
         hipLaunchKernelGGL(k_up_subs, dim3(t.nsub), dim3(kBlock), 0, s, nv, cm, (const int2*)t.sub_lev.p,
                            (const int32_t*)t.sub_nlev.p, c.x.p, c.y.p, c.g.p, t.nleaves.p);
@@ -2104,8 +2111,9 @@ void tree_lists(Ctx& c) {
     TravNode* tn = reinterpret_cast<TravNode*>(t.trav.p);
     t.log.most.grow(2);
     t.log.totals.grow(5);
+    t.cmk.grow(4 * (size_t)t.nnodes + 1);
     hipLaunchKernelGGL(k_trav_nodes, dim3(nblocks(t.nnodes)), dim3(kBlock), 0, s, nv, t.nnodes, t.pre.p, t.nleaves.p,
-                       tn, t.log.most.p);
+                       tn, t.log.most.p, cm_view(t), t.cmk.p);
     const double fc = (double)t.far_criteria;
     // subtrees walked by waves of their own: a walk over the top of the tree
     // has about 2 nnodes / item_nodes steps, one of an item at most item_nodes
