@@ -1,6 +1,6 @@
 // convective.hip -- MConvectiveFast::process_all_lists (MConvectiveFast.cpp:
-// 36-114), MConvectiveFast::velocity (:20-34) and the FP64 direct sum used as
-// the accuracy yardstick.
+// 36-114) and the FP64 direct sum used as the accuracy yardstick
+// (MConvectiveFast::velocity is in fields.hip).
 //
 // process_all_lists runs as three kernels:
 //  1. k_far_taylor, one wave per leaf: the reference's first-order Taylor
@@ -67,8 +67,8 @@ __device__ inline float readlane_f(float v, int k) {
 
 // Far-field Taylor coefficients of every leaf (MConvectiveFast.cpp:48-69).
 // Bound by the gathers of the far nodes: with six words from six arrays the
-// batch of 16 cylinders took 350 us, with three loads from one 64-byte record
-// 190 (4M vortices, beside the near field: 29.3 and 28.5 ms a pass).
+// batch of 16 cylinders took 350 us and 4M vortices 2.6 ms, with three loads
+// from one 64-byte record 190 us and 1.5 ms.
 __global__ __launch_bounds__(kBlock) void k_far_taylor(TreeDev T, double4* taylor) {
     const int w = threadIdx.x / kWave;
     const int l = blockIdx.x * kWavesPerBlock + w;

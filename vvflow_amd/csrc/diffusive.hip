@@ -73,10 +73,15 @@ constexpr int kFold = 8;      // terms between two folds of the partial sums
 // |dr| / eps_i <= 8; |dr| and 1/|dr| from one reciprocal square root.
 // kSeg: the FP64 segment terms are compiled in (their library exp and sqrt
 // take registers that would cost the vortex-only launches occupancy).
+// Bound by VALU issue, with a reciprocal root and an exp a pair at a quarter of
+// the rate.  Four leaves to a block kept 32 KB of LDS until the longest had
+// finished, 1.7 waves a SIMD: 7.2 ms alone at 4M vortices, 4.7 with a leaf
+// (5 KB) a block, 16-byte records and selections in place of branches, 4.5
+// with registers for a fifth wave (87 in place of 100).
 // dvx/dvy non-null (no segments only): the increment is stored there for
 // k_add_diffusive instead of being added to vx/vy.
 template <bool kSeg>
-__global__ __launch_bounds__(kWave) void k_diffusive(TreeDev T, const double* __restrict__ x,
+__global__ __launch_bounds__(kWave, kSeg ? 4 : 5) void k_diffusive(TreeDev T, const double* __restrict__ x,
                                                       const double* __restrict__ y, const double* __restrict__ g,
                                                       const double* __restrict__ ie, const vvhd_seg* segs, int nseg,
                                                       double* vx, double* vy, double re_one, const double* sim_re,
