@@ -137,7 +137,7 @@ int vvhd_download_bodies(vvhd_ctx* ctx, vvhd_seg* segs, int32_t nseg,
  * simulation in the same launches; no list, merge or sum crosses
  * simulations, and the direct sum of a target runs over its own simulation.
  * calc_circulation solves one boundary system per simulation (all of one
- * order: strided-batched LU), vortex_shed appends each simulation's new
+ * order), vortex_shed appends each simulation's new
  * vortices after its own, move_and_clean removes each vortex only against
  * its own simulation's bodies, and calc_forces uses each simulation's
  * Reynolds number; the ranges then move (vvhd_batch_offsets).  Holds until
@@ -282,7 +282,8 @@ int vvhd_vortex_shed(vvhd_ctx* ctx);
 
 /* ---- boundary-condition SLAE: MConvectiveFast::calc_circulation -------
  * (:235-273, fill :882-1017) with Matrix::solveUsingInverseMatrix
- * (TMatrix.cpp:166-259): FP64 fill and LU solve on the device; writes the
+ * (TMatrix.cpp:166-259): FP64 fill and solve on the device, with the kept
+ * inverse of the segment rows and a step of residual correction; writes the
  * bound circulations, speed_slae, force_hydro and force_holder. */
 int vvhd_calc_circulation(vvhd_ctx* ctx, double inf_x, double inf_y);
 /* The system filled by the last vvhd_calc_circulation: order into *n; when
