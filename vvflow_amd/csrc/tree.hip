@@ -1935,10 +1935,10 @@ void tree_build(Ctx& c, int far_criteria, double min_node, double max_node, int3
                            (const int32_t*)c.seg_root.p, nseg);
 
     // One level per iteration over the whole list, its kernels taking their node
-    // range from the device counters.  No node can fit a workgroup before the
-    // largest root has been halved down to kSubElems elements, so the levels up
-    // to there are queued without asking; from there on k_subtree takes what
-    // fits, and the host reads after it whether anything is left.
+    // range from the device counters.  Few nodes fit a workgroup before a root
+    // has been halved down to kSubElems elements, so the levels up to there are
+    // queued without asking; from there on k_subtree takes what fits, and the
+    // host reads after it whether anything is left.
     auto launch_level = [&](int d) {
         const int node_blocks = 1024;
         hipLaunchKernelGGL(k_decide, dim3(node_blocks), dim3(kBlock), 0, s, nv, t.counters.p, cap, min_node, max_node);
@@ -1968,13 +1968,16 @@ void tree_build(Ctx& c, int far_criteria, double min_node, double max_node, int3
         if (nseg)
             hipLaunchKernelGGL(k_seg_step, dim3(nblocks(nseg)), dim3(kBlock), 0, s, nv, c.segs.p, nseg, seg_node.p);
     };
-    int64_t largest = n;   // elements of the largest root
-    if (nroots > 1) {
-        largest = 0;
-        for (int q = 0; q < nroots; q++) largest = std::max(largest, c.sim_off_h[q + 1] - c.sim_off_h[q]);
+    // Elements of the root whose nodes fit first.  Roots of a batch differ: 64 of
+    // 14k to 400k elements, taken when the largest one's nodes fitted, gave 25k
+    // subtrees of a few elements each (a tree 23 ms, now 13).
+    int64_t start = n;
+    for (int q = 0; nroots > 1 && q < nroots; q++) {
+        const int64_t m = c.sim_off_h[q + 1] - c.sim_off_h[q];
+        if (m > 0) start = std::min(start, m);
     }
     int depth = 0;
-    for (; (largest >> depth) > kSubElems; depth++) launch_level(depth);
+    for (; (start >> depth) > kSubElems; depth++) launch_level(depth);
     int32_t* hc = c.lev_counters;   // pinned
     for (;; depth++) {
         const int grid = (int)std::min<int64_t>(2 * c.n_cu, (int64_t)nroots << std::min(depth, 20));
