@@ -755,8 +755,9 @@ __global__ void k_slae_layout(const vvhd_body* bodies, const int32_t* sim_body, 
 // sources at a time are evaluated together and added in the reference's order
 // (near nodes and their vortices in list order, then each far node's
 // positive and negative monopole).  Bound by latency: a near leaf at a time,
-// its terms added by one lane, 186 us for a cylinder in 100k vortices; now 72.  Also the speed cells (_2PI_A123, :375-396)
-// of a rigid body with no prescribed rotation.
+// its terms added by one lane, 186 us for a cylinder in 100k vortices; now 72.
+// Also the speed cells (_2PI_A123, :375-396) of a rigid body with no prescribed
+// rotation.
 __global__ __launch_bounds__(64) void k_slip_rhs(SlaeMap M, TreeDev T, const vvhd_seg* segs, int nseg,
                                                  const double* x, const double* y, const double* g, const double* ie,
                                                  double infx, double infy, double* A, double* rhs) {
