@@ -124,32 +124,32 @@ __device__ inline int xcd_block(int b, int nblocks) {
 
 // ------------------------------------------------------------------ context --
 
-// Log of the list builder (tree.hip: ListLog): R records and S items a group.
+// Log of the list builder (tree.hip: ListLog) for `groups` groups, with room for
+// `top` records and `items` items of theirs and `records` records of the items.
 struct ListLogBufs {
-    int R = 512, S = 64;
-    DBuf<int32_t> tid, gnodes, item_n, rid, most;
+    DBuf<int32_t> tid, nrec, nitem, gnodes, item_n, item_grp, rid, most;
     DBuf<uint64_t> tfar, tnear, item_mask, rfar, rnear;
-    DBuf<int64_t> gbase, totals;
-    DBuf<int2> head, item, lanes, after;
-    void grow(int64_t groups, int64_t records) {
-        for (auto* b : {&tfar, &tnear}) b->grow(groups * R + 1);
-        tid.grow(groups * R + 1);
-        gnodes.grow(groups + 1);
-        gbase.grow(groups + 1);
-        head.grow(groups + 1);
-        item.grow(groups * S + 1);
-        item_mask.grow(groups * S + 1);
-        item_n.grow(groups * S + 1);
-        for (auto* b : {&lanes, &after}) b->grow((groups * S + 1) * 64);
+    DBuf<int64_t> gbase, tbase, ibase, totals;
+    DBuf<int2> item, lanes, after;
+    // of the last walk: most records and items of a group, and of all groups
+    int64_t last_recs = 0, last_items = 0, last_all_recs = 0, last_all_items = 0;
+    void grow(int64_t groups, int64_t top, int64_t items, int64_t records) {
+        for (auto* b : {&tfar, &tnear}) b->grow(top + 1);
+        tid.grow(top + 1);
+        for (auto* b : {&nrec, &nitem, &gnodes}) b->grow(groups + 1);
+        for (auto* b : {&gbase, &tbase, &ibase}) b->grow(groups + 1);
+        item.grow(items + 1);
+        item_mask.grow(items + 1);
+        for (auto* b : {&item_n, &item_grp}) b->grow(items + 1);
+        for (auto* b : {&lanes, &after}) b->grow((items + 1) * 64);
         rid.grow(records + 1);
         for (auto* b : {&rfar, &rnear}) b->grow(rid.cap);
     }
     void release() {
-        for (auto* b : {&tid, &gnodes, &item_n, &rid, &most}) b->release();
+        for (auto* b : {&tid, &nrec, &nitem, &gnodes, &item_n, &item_grp, &rid, &most}) b->release();
         for (auto* b : {&tfar, &tnear, &item_mask, &rfar, &rnear}) b->release();
-        gbase.release();
-        totals.release();
-        for (auto* b : {&head, &item, &lanes, &after}) b->release();
+        for (auto* b : {&gbase, &tbase, &ibase, &totals}) b->release();
+        for (auto* b : {&item, &lanes, &after}) b->release();
     }
 };
 

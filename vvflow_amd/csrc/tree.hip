@@ -1352,20 +1352,37 @@ __global__ void k_trav_nodes(NodeView nv, int nnodes, const int32_t* pre, const 
 // steps were walked twice, to count and to write.  No counter is shared
 // between waves (50k claims of one address cost 0.7 ms).
 struct ListLog {
-    int R, S;                    // records and items a group has room for
+    int R, S;                    // records and items every group has room for,
+    const int64_t *tbase, *ibase;   // or (not null) where each group's begin: room for as many as it has
+    int slots;                   // items there is room for in all groups
     int64_t cap;                 // records of all items
-    int32_t* tid;                // groups x R: node, or -(item of the group + 1)
+    int32_t* tid;                // a group's records: node, or -(item of the group + 1)
     uint64_t *tfar, *tnear;
-    int2* head;                  // per group: records, items
+    int32_t *nrec, *nitem;       // per group: records, items
     int32_t* gnodes;             // per group: nodes of its items (their records at most)
     const int64_t* gbase;        // their exclusive sums
-    int2* item;                  // groups x S: position, first record within the group's
+    int2* item;                  // a group's items: position, first record within the group's
     uint64_t* item_mask;         // lanes that need it
     int32_t* item_n;             // its records
-    int2 *lanes, *after;         // groups x S x 64: near and far nodes a lane lists in the item, then before it; and after it
+    int32_t* item_grp;           // its group (written where ibase is given)
+    int2 *lanes, *after;         // items x 64: near and far nodes a lane lists in the item, then before it; and after it
     int32_t* rid;
     uint64_t *rfar, *rnear;
-    int32_t* most;               // [0] records, [1] items of a group beyond its room
+    int32_t* most;               // not 0 where a group's records [0] or items [1] ran out of room
+    __device__ int64_t rec0(int g) const { return tbase ? tbase[g] : (int64_t)g * R; }
+    __device__ int64_t item0(int g) const { return ibase ? ibase[g] : (int64_t)g * S; }
+    __device__ int recs(int g) const { return tbase ? (int)(tbase[g + 1] - tbase[g]) : R; }
+    __device__ int items(int g) const { return ibase ? (int)(ibase[g + 1] - ibase[g]) : S; }
+    // Item of slot w, its group in grp; -1 where the slot holds none.
+    __device__ int64_t slot(int w, int ngroups, int& grp) const {
+        if (ibase) {
+            grp = __builtin_amdgcn_readfirstlane(item_grp[w]);
+            return w;
+        }
+        grp = __builtin_amdgcn_readfirstlane(w % ngroups);
+        const int k = __builtin_amdgcn_readfirstlane(w / ngroups);
+        return k < nitem[grp] ? (int64_t)grp * S + k : -1;
+    }
 };
 
 // The records of one walk at [o, o + limit): record k of every 64 is collected
@@ -1457,14 +1474,16 @@ __global__ __launch_bounds__(kBlock) void k_list_top(NodeView nv, const TravNode
     const int L = valid ? leaf_node[l] : 0;
     const int P0 = __builtin_amdgcn_readfirstlane(pre[groups[3 * grp + 2]]);
     const int end = __builtin_amdgcn_readfirstlane(tn[P0].skip);
-    const size_t o = (size_t)grp * G.R, io = (size_t)grp * G.S;
-    LogWriter log{G.tid + o, G.tfar + o, G.tnear + o, G.R, lane};
+    const int64_t o = G.rec0(grp), io = G.item0(grp);
+    const int R = G.recs(grp), S = G.items(grp);
+    LogWriter log{G.tid + o, G.tfar + o, G.tnear + o, R, lane};
     int cn = 0, cf = 0, ni = 0, nodes = 0;
     list_walk(tn, P0, end, valid ? P0 : end, nv.x[L], nv.y[L], nv.h[L], nv.w[L], fc, item_nodes, log, cn, cf,
               [&](int P, int size, uint64_t need) {
-                  if (lane == 0 && ni < G.S) {
+                  if (lane == 0 && ni < S) {
                       G.item[io + ni] = make_int2(P, nodes);
                       G.item_mask[io + ni] = need;
+                      if (G.ibase) G.item_grp[io + ni] = grp;
                   }
                   log.push(-(ni + 1), 0, 0);
                   ni++;
@@ -1472,37 +1491,41 @@ __global__ __launch_bounds__(kBlock) void k_list_top(NodeView nv, const TravNode
               });
     log.flush();
     if (lane != 0) return;
-    G.head[grp] = make_int2((int)log.done, ni);
+    G.nrec[grp] = (int)log.done;
+    G.nitem[grp] = ni;
     G.gnodes[grp] = nodes;
-    if (log.done > G.R) atomicMax(&G.most[0], (int)log.done);
-    if (ni > G.S) atomicMax(&G.most[1], ni);
+    if (log.done > R) G.most[0] = 1;
+    if (ni > S) G.most[1] = 1;
 }
 
 __global__ __launch_bounds__(kBlock) void k_list_items(NodeView nv, const TravNode* __restrict__ tn,
                                                        const int32_t* __restrict__ groups, int ngroups,
                                                        const int32_t* leaf_node, double fc, ListLog G) {
     const int lane = lane_id();
-    const int wave = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
+    if (G.most[0] | G.most[1]) return;   // the walk is repeated
     // item k of all groups, then item k + 1: a group has about 20 of its S items,
     // and with a group's items in neighbouring blocks these fell on the same few
     // XCDs (S = 64: 1.6 against 0.53 ms at 1M)
-    const int grp = __builtin_amdgcn_readfirstlane(wave % ngroups), k = __builtin_amdgcn_readfirstlane(wave / ngroups);
-    if (k >= G.S || k >= G.head[grp].y) return;
-    const size_t it = (size_t)grp * G.S + k;
-    const int P0 = __builtin_amdgcn_readfirstlane(G.item[it].x);
-    const int end = __builtin_amdgcn_readfirstlane(tn[P0].skip);
-    const bool mine = (G.item_mask[it] >> lane) & 1;
-    const int l = groups[3 * grp] + lane;
-    const int L = mine ? leaf_node[l] : 0;
-    const int64_t o = G.gbase[grp] + G.item[it].y;
-    const int64_t room = min((int64_t)(end - P0), max((int64_t)0, G.cap - o));
-    LogWriter log{G.rid + o, G.rfar + o, G.rnear + o, room, lane};
-    int cn = 0, cf = 0;
-    list_walk(tn, P0 + 1, end, mine ? P0 : end, nv.x[L], nv.y[L], nv.h[L], nv.w[L], fc, 0, log, cn, cf,
-              [](int, int, uint64_t) {});
-    log.flush();
-    if (lane == 0) G.item_n[it] = (int)log.done;
-    G.lanes[it * kWave + lane] = make_int2(cn, cf);
+    const int step = gridDim.x * (kBlock / kWave);
+    for (int w = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave; w < G.slots; w += step) {
+        int grp;
+        const int64_t it = G.slot(w, ngroups, grp);
+        if (it < 0) continue;
+        const int P0 = __builtin_amdgcn_readfirstlane(G.item[it].x);
+        const int end = __builtin_amdgcn_readfirstlane(tn[P0].skip);
+        const bool mine = (G.item_mask[it] >> lane) & 1;
+        const int l = groups[3 * grp] + lane;
+        const int L = mine ? leaf_node[l] : 0;
+        const int64_t o = G.gbase[grp] + G.item[it].y;
+        const int64_t room = min((int64_t)(end - P0), max((int64_t)0, G.cap - o));
+        LogWriter log{G.rid + o, G.rfar + o, G.rnear + o, room, lane};
+        int cn = 0, cf = 0;
+        list_walk(tn, P0 + 1, end, mine ? P0 : end, nv.x[L], nv.y[L], nv.h[L], nv.w[L], fc, 0, log, cn, cf,
+                  [](int, int, uint64_t) {});
+        log.flush();
+        if (lane == 0) G.item_n[it] = (int)log.done;
+        G.lanes[it * kWave + lane] = make_int2(cn, cf);
+    }
 }
 
 // Reads 64 records of a log at once, one per lane, and hands them out in order.
@@ -1530,11 +1553,11 @@ __global__ __launch_bounds__(kBlock) void k_list_sums(const int32_t* __restrict_
                                                       int32_t* near_cnt, int32_t* far_cnt) {
     const int grp = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave, lane = lane_id();
     if (grp >= ngroups) return;
-    const int nrec = min(G.head[grp].x, G.R);
-    const size_t io = (size_t)grp * G.S;
-    LogReader rd{G.tid + (size_t)grp * G.R, G.tfar + (size_t)grp * G.R, G.tnear + (size_t)grp * G.R};
+    const bool whole = (G.most[0] | G.most[1]) == 0;   // otherwise the walk is repeated
+    const int nrec = whole ? G.nrec[grp] : 0, ni = whole ? G.nitem[grp] : 0;
+    const int64_t io = G.item0(grp), to = G.rec0(grp);
+    LogReader rd{G.tid + to, G.tfar + to, G.tnear + to};
     int cn = 0, cf = 0;
-    const int ni = min(G.head[grp].y, G.S);
     int2 ahead = ni > 0 ? G.lanes[io * kWave + lane] : make_int2(0, 0);   // the next item's counts
     for (int r0 = 0; r0 < nrec; r0 += kWave) {
         rd.load(r0, nrec - r0, lane);
@@ -1589,69 +1612,70 @@ struct ListOut {
     }
 };
 
-// The records to the lists: wave k of a group writes item k, one more wave the
+// The records to the lists: a wave an item, then a wave a group for the
 // group's own records.
 __global__ __launch_bounds__(kBlock) void k_list_replay(const int32_t* __restrict__ groups, int ngroups, ListLog G,
                                                         const int64_t* near_off, const int64_t* far_off,
                                                         int32_t* near_list, int32_t* far_list) {
     const int lane = lane_id();
-    const int wave = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
-    const int grp = __builtin_amdgcn_readfirstlane(wave % ngroups), k = __builtin_amdgcn_readfirstlane(wave / ngroups);
-    if (k > G.S) return;
-    const int ni = G.head[grp].y;
-    if (k >= ni && k < G.S) return;
-    const int l = groups[3 * grp] + lane;
-    const bool valid = lane < groups[3 * grp + 1];
-    const size_t io = (size_t)grp * G.S;
-    ListOut near{near_list + (valid ? near_off[l] : 0)}, far{far_list + (valid ? far_off[l] : 0)};
-    auto emit = [&](const LogReader& rd, int q, int id) {
+    auto emit = [&](const LogReader& rd, ListOut& near, ListOut& far, int q, int id) {
         const uint64_t F = LogReader::pick(rd.rf, q), N = LogReader::pick(rd.rn, q);
         if (__builtin_amdgcn_inverse_ballot_w64(F)) far.push(id);
         if (N != 0 && __builtin_amdgcn_inverse_ballot_w64(N)) near.push(id);
     };
-    if (k < G.S) {
-        const int2 c = G.lanes[(io + k) * kWave + lane];
-        near.p += c.x;
-        far.p += c.y;
-        const int64_t o = G.gbase[grp] + G.item[io + k].y;
-        const int n = G.item_n[io + k];
-        LogReader rd{G.rid, G.rfar, G.rnear}, next = rd;
-        next.load(o, n, lane);
+    const int step = gridDim.x * (kBlock / kWave);
+    for (int w = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave; w < G.slots + ngroups; w += step) {
+        const bool own = w >= G.slots;
+        int grp = __builtin_amdgcn_readfirstlane(w - G.slots);
+        const int64_t it = own ? 0 : G.slot(w, ngroups, grp);
+        if (it < 0) continue;
+        const int l = groups[3 * grp] + lane;
+        const bool valid = lane < groups[3 * grp + 1];
+        ListOut near{near_list + (valid ? near_off[l] : 0)}, far{far_list + (valid ? far_off[l] : 0)};
+        if (!own) {
+            const int2 c = G.lanes[it * kWave + lane];
+            near.p += c.x;
+            far.p += c.y;
+            const int64_t o = G.gbase[grp] + G.item[it].y;
+            const int n = G.item_n[it];
+            LogReader rd{G.rid, G.rfar, G.rnear}, next = rd;
+            next.load(o, n, lane);
+            for (int r0 = 0; r0 < n; r0 += kWave) {
+                rd = next;
+                if (r0 + kWave < n) next.load(o + r0 + kWave, n - r0 - kWave, lane);
+                const int m = min(kWave, n - r0);
+                for (int q = 0; q < m; q++) emit(rd, near, far, q, __builtin_amdgcn_readlane(rd.rid, q));
+            }
+            near.flush();
+            far.flush();
+            continue;
+        }
+        // the group's own records: an item's entries are passed over, up to what
+        // the lane has listed before the next record
+        const int n = G.nrec[grp];
+        const int64_t io = G.item0(grp), to = G.rec0(grp);
+        LogReader rd{G.tid + to, G.tfar + to, G.tnear + to};
+        int32_t *const bn = near.p, *const bf = far.p;   // the leaf's lists
         for (int r0 = 0; r0 < n; r0 += kWave) {
-            rd = next;
-            if (r0 + kWave < n) next.load(o + r0 + kWave, n - r0 - kWave, lane);
+            rd.load(r0, n - r0, lane);
             const int m = min(kWave, n - r0);
-            for (int q = 0; q < m; q++) emit(rd, q, __builtin_amdgcn_readlane(rd.rid, q));
+            for (int q = 0; q < m; q++) {
+                const int id = __builtin_amdgcn_readlane(rd.rid, q);
+                if (id >= 0) {
+                    emit(rd, near, far, q, id);
+                    continue;
+                }
+                // after item i the lane stands where item i's entries end
+                const int2 c = G.after[(io + (-id - 1)) * kWave + lane];
+                near.flush();
+                far.flush();
+                near.p = bn + c.x;
+                far.p = bf + c.y;
+            }
         }
         near.flush();
         far.flush();
-        return;
     }
-    // the group's own records: an item's entries are passed over, up to what
-    // the lane has listed before the next record
-    const int n = G.head[grp].x;
-    LogReader rd{G.tid + (size_t)grp * G.R, G.tfar + (size_t)grp * G.R, G.tnear + (size_t)grp * G.R};
-    int32_t *const bn = near.p, *const bf = far.p;   // the leaf's lists
-    for (int r0 = 0; r0 < n; r0 += kWave) {
-        rd.load(r0, n - r0, lane);
-        const int m = min(kWave, n - r0);
-        for (int q = 0; q < m; q++) {
-            const int id = __builtin_amdgcn_readlane(rd.rid, q);
-            if (id >= 0) {
-                emit(rd, q, id);
-                continue;
-            }
-            // after item i the lane stands where item i's entries end
-            const size_t it = io + (-id - 1);
-            const int2 c = G.after[it * kWave + lane];
-            near.flush();
-            far.flush();
-            near.p = bn + c.x;
-            far.p = bf + c.y;
-        }
-    }
-    near.flush();
-    far.flush();
 }
 
 // Segments: leaf of each segment, then stable order by (leaf, index).
@@ -1680,15 +1704,41 @@ __global__ void k_seg_off(const int32_t* seg_leaf, const int32_t* seg_list, int 
 }
 
 // What the host needs of a walk, in one copy: the lists' lengths, the items'
-// nodes and the log's overflow marks, which are cleared for the next walk.
-__global__ void k_list_totals(const int64_t* near_end, const int64_t* far_end, const int64_t* nodes_end,
-                              int32_t* most, int64_t* out) {
+// nodes, whether a group ran out of room (the marks are cleared for the next
+// walk), and the most of a group and the sum of the groups' records and items.
+constexpr int kTotals = 8, kTotalsThreads = 1024;
+__global__ __launch_bounds__(kTotalsThreads) void k_list_totals(const int64_t* near_end, const int64_t* far_end,
+                                                                const int64_t* nodes_end, ListLog G, int ngroups,
+                                                                int64_t* out) {
+    __shared__ int64_t s_part[kTotalsThreads / kWave][4];
     const int k = threadIdx.x;
-    if (k < 3) out[k] = k == 0 ? *near_end : k == 1 ? *far_end : *nodes_end;
-    if (k == 3 || k == 4) {
-        out[k] = most[k - 3];
-        most[k - 3] = 0;
+    int64_t v[4] = {0, 0, 0, 0};   // most records, most items, all records, all items
+    for (int g = k; g < ngroups; g += kTotalsThreads) {
+        const int64_t r = G.nrec[g], i = G.nitem[g];
+        v[0] = max(v[0], r);
+        v[1] = max(v[1], i);
+        v[2] += r;
+        v[3] += i;
     }
+    auto join = [](int64_t* a, const int64_t* b) {
+        for (int q = 0; q < 4; q++) a[q] = q < 2 ? max(a[q], b[q]) : a[q] + b[q];
+    };
+    for (int o = kWave / 2; o > 0; o >>= 1) {
+        int64_t u[4];
+        for (int q = 0; q < 4; q++) u[q] = __shfl_xor((long long)v[q], o, kWave);
+        join(v, u);
+    }
+    if (lane_id() == 0)
+        for (int q = 0; q < 4; q++) s_part[k / kWave][q] = v[q];
+    __syncthreads();
+    if (k != 0) return;
+    for (int w = 1; w < kTotalsThreads / kWave; w++) join(v, s_part[w]);
+    out[0] = *near_end;
+    out[1] = *far_end;
+    out[2] = *nodes_end;
+    out[3] = G.most[0] | G.most[1];
+    for (int q = 0; q < 4; q++) out[4 + q] = v[q];
+    G.most[0] = G.most[1] = 0;
 }
 
 __global__ void k_iota(int32_t* a, int n) {
@@ -2113,7 +2163,7 @@ void tree_lists(Ctx& c) {
     t.trav.grow((size_t)t.nnodes * sizeof(TravNode));
     TravNode* tn = reinterpret_cast<TravNode*>(t.trav.p);
     t.log.most.grow(2);
-    t.log.totals.grow(5);
+    t.log.totals.grow(kTotals);
     t.cmk.grow(4 * (size_t)t.nnodes + 1);
     hipLaunchKernelGGL(k_trav_nodes, dim3(nblocks(t.nnodes)), dim3(kBlock), 0, s, nv, t.nnodes, t.pre.p, t.nleaves.p,
                        tn, t.log.most.p, cm_view(t), t.cmk.p);
@@ -2122,16 +2172,35 @@ void tree_lists(Ctx& c) {
     // has about 2 nnodes / item_nodes steps, one of an item at most item_nodes
     const int item_nodes = std::min(512, std::max(32, (int)(1.4 * std::sqrt((double)t.nnodes))));
     const int ng = t.ngroups;
+    // a wave each, or what a launch may hold of them (its threads are a 32-bit
+    // number): the kernels over items go round the rest
     auto wave_grid = [](int64_t waves) {
-        return dim3((unsigned)std::max<int64_t>(1, (waves + kBlock / kWave - 1) / (kBlock / kWave)));
+        return dim3((unsigned)std::clamp<int64_t>((waves + kBlock / kWave - 1) / (kBlock / kWave), 1, 1 << 22));
     };
     ListLogBufs& b = t.log;
+    // The same room for every group, as the last walk needed it, unless one
+    // group among many needed far more than the others (a leaf spread wide
+    // around the rest is near to all of them) and it comes to more than 128
+    // MiB: the floors then, which most groups stay under.  Where they do not
+    // do, the counts of the first walk over the groups give every group the
+    // room that it needs in a second (55 us at 1M, against 400 us for the
+    // items' walk).  With the widest group's room for all, ten strays round 4M
+    // vortices took 24 GiB, and round 8M the build failed.
+    auto room = [&](int64_t most, int64_t all, int64_t floor, int64_t small) {
+        const int64_t r = std::max(floor, most + most / 8);
+        return r * ng <= std::max(small, 4 * all + floor * ng) ? r : floor;
+    };
+    int64_t R = room(b.last_recs, b.last_all_recs, 512, 1 << 22), S = room(b.last_items, b.last_all_items, 64, 1 << 17);
+    int64_t recs = R * ng, items = S * ng;   // room in all
+    bool exact = false;
+    // the items' records: what the criteria in use need, or what was counted
+    int64_t nodes = (int64_t)ng * 6144;
     for (;;) {
-        // room for what the criteria in use need; a longer log is counted, its
-        // buffers grown and the walk repeated
-        b.grow(ng, (int64_t)ng * 6144);
-        ListLog G{b.R, b.S, (int64_t)b.rid.cap, b.tid.p, b.tfar.p, b.tnear.p, b.head.p, b.gnodes.p, b.gbase.p, b.item.p,
-                  b.item_mask.p, b.item_n.p, b.lanes.p, b.after.p, b.rid.p, b.rfar.p, b.rnear.p, b.most.p};
+        VVHD_CHECK(items < (1 << 30), VVHD_ENOMEM, "tree_build: too many parts of the list walk");
+        b.grow(ng, recs, items, nodes);
+        ListLog G{(int)R, (int)S, exact ? b.tbase.p : nullptr, exact ? b.ibase.p : nullptr, (int)items, (int64_t)b.rid.cap,
+                  b.tid.p, b.tfar.p, b.tnear.p, b.nrec.p, b.nitem.p, b.gnodes.p, b.gbase.p, b.item.p, b.item_mask.p,
+                  b.item_n.p, b.item_grp.p, b.lanes.p, b.after.p, b.rid.p, b.rfar.p, b.rnear.p, b.most.p};
         if (ng)
             hipLaunchKernelGGL(k_list_top, wave_grid(ng), dim3(kBlock), 0, s, nv, (const TravNode*)tn,
                                (const int32_t*)t.pre.p, (const int32_t*)t.groups.p, ng, t.leaf_node.p, fc, item_nodes,
@@ -2143,7 +2212,7 @@ void tree_lists(Ctx& c) {
         else
             scan_i32_to_i64(c, b.gnodes.p, b.gbase.p, ng);
         if (ng) {
-            hipLaunchKernelGGL(k_list_items, wave_grid((int64_t)ng * b.S), dim3(kBlock), 0, s, nv, (const TravNode*)tn,
+            hipLaunchKernelGGL(k_list_items, wave_grid(items), dim3(kBlock), 0, s, nv, (const TravNode*)tn,
                                (const int32_t*)t.groups.p, ng, t.leaf_node.p, fc, G);
             hipLaunchKernelGGL(k_list_sums, wave_grid(ng), dim3(kBlock), 0, s, (const int32_t*)t.groups.p, ng, G,
                                t.cnt_near.p, t.cnt_far.p);
@@ -2155,25 +2224,37 @@ void tree_lists(Ctx& c) {
             scan_i32_to_i64(c, t.cnt_near.p, t.near_off.p, nl);
             scan_i32_to_i64(c, t.cnt_far.p, t.far_off.p, nl);
         }
-        int64_t tot[5];   // near entries, far entries, items' nodes, most[0], most[1]
-        hipLaunchKernelGGL(k_list_totals, dim3(1), dim3(64), 0, s, (const int64_t*)t.near_off.p + nl,
-                           (const int64_t*)t.far_off.p + nl, (const int64_t*)b.gbase.p + ng, b.most.p, b.totals.p);
+        // lengths of the near and the far lists, the items' nodes, out of room, then
+        // most and all of the records and of the items
+        int64_t tot[kTotals];
+        hipLaunchKernelGGL(k_list_totals, dim3(1), dim3(kTotalsThreads), 0, s, (const int64_t*)t.near_off.p + nl,
+                           (const int64_t*)t.far_off.p + nl, (const int64_t*)b.gbase.p + ng, G, ng, b.totals.p);
+        VVHD_HIP(hipGetLastError());   // no lengths from a launch that was refused
         VVHD_HIP(hipMemcpyAsync(tot, b.totals.p, sizeof(tot), hipMemcpyDeviceToHost, s));
         VVHD_HIP(hipStreamSynchronize(s));
-        if (tot[3] == 0 && tot[4] == 0 && tot[2] <= G.cap) {
-            t.nnear = tot[0];
-            t.nfar = tot[1];
-            t.near_list.grow(t.nnear + 1);
-            t.far_list.grow(t.nfar + 1);
-            if (ng)
-                hipLaunchKernelGGL(k_list_replay, wave_grid((int64_t)ng * (b.S + 1)), dim3(kBlock), 0, s,
-                                   (const int32_t*)t.groups.p, ng, G, (const int64_t*)t.near_off.p,
-                                   (const int64_t*)t.far_off.p, t.near_list.p, t.far_list.p);
-            return;
+        b.last_recs = tot[4];
+        b.last_items = tot[5];
+        b.last_all_recs = tot[6];
+        b.last_all_items = tot[7];
+        nodes = std::max(nodes, tot[2]);
+        if (tot[3]) {
+            scan_i32_to_i64(c, b.nrec.p, b.tbase.p, ng);
+            scan_i32_to_i64(c, b.nitem.p, b.ibase.p, ng);
+            exact = true;
+            recs = tot[6];
+            items = tot[7];
+            continue;
         }
-        b.R = std::max(b.R, (int)tot[3]);
-        b.S = std::max(b.S, (int)tot[4]);
-        b.rid.grow(tot[2]);
+        if (tot[2] > G.cap) continue;
+        t.nnear = tot[0];
+        t.nfar = tot[1];
+        t.near_list.grow(t.nnear + 1);
+        t.far_list.grow(t.nfar + 1);
+        if (ng)
+            hipLaunchKernelGGL(k_list_replay, wave_grid(items + ng), dim3(kBlock), 0, s, (const int32_t*)t.groups.p,
+                               ng, G, (const int64_t*)t.near_off.p, (const int64_t*)t.far_off.p, t.near_list.p,
+                               t.far_list.p);
+        return;
     }
 }
 
