@@ -1389,6 +1389,10 @@ void calc_circulation(Ctx& c, double infx, double infy) {
     // the core of each system, and whether its inverse is kept
     const int nc = max_segs;
     const size_t cc = (size_t)nc * nc, call = cc * nsys;
+    // from here the core may be another than the inverted one: an error before
+    // its own inverse is there leaves none behind
+    bool refactor = !(c.time > 0) || c.slae_n != nc || c.slae_nsys_factored != nsys;
+    c.slae_n = -1;
     c.slae_core.grow(call);
     c.slae_inv.grow(call);
     c.slae_v.grow(3 * (size_t)nc * nsys);
@@ -1400,7 +1404,6 @@ void calc_circulation(Ctx& c, double infx, double infy) {
     const int tiles = (nc + 31) / 32;
     hipLaunchKernelGGL(k_core_gather, dim3(tiles, tiles, nsys), dim3(kBlock), 0, s, C, (const double*)c.slae_A.p,
                        d_differ);
-    bool refactor = !(c.time > 0) || c.slae_n != nc || c.slae_nsys_factored != nsys;
     if (!refactor) {
         int32_t differ = 0;
         VVHD_HIP(hipMemcpyAsync(&differ, d_differ, 4, hipMemcpyDeviceToHost, s));
@@ -1415,7 +1418,6 @@ void calc_circulation(Ctx& c, double infx, double infy) {
         }
         rocblas_handle h = (rocblas_handle)c.rocblas;
         VVHD_CHECK(rocblas_set_stream(h, s) == rocblas_status_success, VVHD_EHIP, "rocblas_set_stream failed");
-        c.slae_n = -1;
         c.slae_ipiv.grow((size_t)nc * nsys + 1);
         VVHD_HIP(hipMemcpyAsync(c.slae_inv.p, c.slae_core.p, call * 8, hipMemcpyDeviceToDevice, s));
         // a row-major core is the transpose to the library, whose inverse is the row-major inverse
@@ -1432,9 +1434,9 @@ void calc_circulation(Ctx& c, double infx, double infy) {
         VVHD_CHECK(rocsolver_dgetri_strided_batched(h, nc, c.slae_inv.p, nc, (rocblas_stride)cc, c.slae_ipiv.p,
                                                     (rocblas_stride)nc, c.slae_info.p, nsys) == rocblas_status_success,
                    VVHD_EHIP, "rocsolver_dgetri_strided_batched failed");
-        c.slae_n = nc;
-        c.slae_nsys_factored = nsys;
     }
+    c.slae_n = nc;
+    c.slae_nsys_factored = nsys;
     hipLaunchKernelGGL(k_core_rhs, dim3(nblocks(nc), nsys), dim3(kBlock), 0, s, C, (const double*)c.slae_A.p,
                        (const double*)c.slae_b.p);
     const dim3 rows((nc + kBlock / kWave - 1) / (kBlock / kWave), nsys);
