@@ -282,9 +282,9 @@ int vvhd_vortex_shed(vvhd_ctx* ctx);
 
 /* ---- boundary-condition SLAE: MConvectiveFast::calc_circulation -------
  * (:235-273, fill :882-1017) with Matrix::solveUsingInverseMatrix
- * (TMatrix.cpp:166-259): FP64 fill and solve on the device, with the kept
- * inverse of the segment rows and a step of residual correction; writes the
- * bound circulations, speed_slae, force_hydro and force_holder. */
+ * (TMatrix.cpp:166-259): FP64 fill and solve on the device, with the factors
+ * of the segment rows or, where they are the last call's, their kept inverse
+ * and a step of residual correction; writes the bound circulations, speed_slae, force_hydro and force_holder. */
 int vvhd_calc_circulation(vvhd_ctx* ctx, double inf_x, double inf_y);
 /* The system filled by the last vvhd_calc_circulation: order into *n; when
  * non-NULL, the matrix row-major into A (n*n) and the right-hand side into

@@ -21,9 +21,9 @@
 //    per system).  The solve uses that the system of rigid bodies is block
 //    triangular: the speeds are given, the segments' circulations follow from
 //    the segment rows alone (the core), the forces from the circulations.  The
-//    core's inverse is kept while the core is bit-identical to the inverted
-//    one, the condition under which the reference reuses its inverse
-//    (TMatrix.cpp:225-259).
+//    core's factors, and from its second use on its inverse, are kept while the
+//    core is bit-identical to the factored one, the condition under which the
+//    reference reuses its inverse (TMatrix.cpp:225-259).
 
 #include "api.hpp"
 #include "body_geom.hpp"
@@ -1389,8 +1389,8 @@ void calc_circulation(Ctx& c, double infx, double infy) {
     // the core of each system, and whether its inverse is kept
     const int nc = max_segs;
     const size_t cc = (size_t)nc * nc, call = cc * nsys;
-    // from here the core may be another than the inverted one: an error before
-    // its own inverse is there leaves none behind
+    // from here the core may be another than the factored one: an error before
+    // its own factors are there leaves none behind
     bool refactor = !(c.time > 0) || c.slae_n != nc || c.slae_nsys_factored != nsys;
     c.slae_n = -1;
     c.slae_core.grow(call);
@@ -1410,7 +1410,7 @@ void calc_circulation(Ctx& c, double infx, double infy) {
         VVHD_HIP(hipStreamSynchronize(s));
         refactor = differ != 0;
     }
-    if (refactor) {
+    auto handle = [&]() {
         if (!c.rocblas) {
             rocblas_handle h = nullptr;
             VVHD_CHECK(rocblas_create_handle(&h) == rocblas_status_success, VVHD_EHIP, "rocblas_create_handle failed");
@@ -1418,6 +1418,15 @@ void calc_circulation(Ctx& c, double infx, double infy) {
         }
         rocblas_handle h = (rocblas_handle)c.rocblas;
         VVHD_CHECK(rocblas_set_stream(h, s) == rocblas_status_success, VVHD_EHIP, "rocblas_set_stream failed");
+        return h;
+    };
+    // A core seen for the first time is solved with its factors, the inverse
+    // made from them when it is seen again: bodies that change every call pay
+    // for no inverse (500 segments: factors and solve 2.9 ms, inverse 2.0 ms
+    // more; a solve with the inverse 0.1, with the factors 0.4).
+    if (refactor) {
+        rocblas_handle h = handle();
+        c.slae_inverted = false;
         c.slae_ipiv.grow((size_t)nc * nsys + 1);
         VVHD_HIP(hipMemcpyAsync(c.slae_inv.p, c.slae_core.p, call * 8, hipMemcpyDeviceToDevice, s));
         // a row-major core is the transpose to the library, whose inverse is the row-major inverse
@@ -1431,18 +1440,28 @@ void calc_circulation(Ctx& c, double infx, double infy) {
             if (info[q] != 0)
                 throw Error(VVHD_ESINGULAR, "calc_circulation: singular matrix of simulation " + std::to_string(q) +
                                                 ", column " + std::to_string(info[q]));
-        VVHD_CHECK(rocsolver_dgetri_strided_batched(h, nc, c.slae_inv.p, nc, (rocblas_stride)cc, c.slae_ipiv.p,
+    } else if (!c.slae_inverted) {
+        VVHD_CHECK(rocsolver_dgetri_strided_batched(handle(), nc, c.slae_inv.p, nc, (rocblas_stride)cc, c.slae_ipiv.p,
                                                     (rocblas_stride)nc, c.slae_info.p, nsys) == rocblas_status_success,
                    VVHD_EHIP, "rocsolver_dgetri_strided_batched failed");
+        c.slae_inverted = true;
+    }
+    hipLaunchKernelGGL(k_core_rhs, dim3(nblocks(nc), nsys), dim3(kBlock), 0, s, C, (const double*)c.slae_A.p,
+                       (const double*)c.slae_b.p);
+    if (c.slae_inverted) {
+        const dim3 rows((nc + kBlock / kWave - 1) / (kBlock / kWave), nsys);
+        hipLaunchKernelGGL(k_core_mv<kMvFirst>, rows, dim3(kBlock), 0, s, C);
+        hipLaunchKernelGGL(k_core_mv<kMvResidual>, rows, dim3(kBlock), 0, s, C);
+        hipLaunchKernelGGL(k_core_mv<kMvCorrect>, rows, dim3(kBlock), 0, s, C);
+    } else {
+        VVHD_HIP(hipMemcpyAsync(C.x, C.b, (size_t)nc * nsys * 8, hipMemcpyDeviceToDevice, s));
+        VVHD_CHECK(rocsolver_dgetrs_strided_batched(handle(), rocblas_operation_transpose, nc, 1, c.slae_inv.p, nc,
+                                                    (rocblas_stride)cc, c.slae_ipiv.p, (rocblas_stride)nc, C.x, nc,
+                                                    (rocblas_stride)nc, nsys) == rocblas_status_success,
+                   VVHD_EHIP, "rocsolver_dgetrs_strided_batched failed");
     }
     c.slae_n = nc;
     c.slae_nsys_factored = nsys;
-    hipLaunchKernelGGL(k_core_rhs, dim3(nblocks(nc), nsys), dim3(kBlock), 0, s, C, (const double*)c.slae_A.p,
-                       (const double*)c.slae_b.p);
-    const dim3 rows((nc + kBlock / kWave - 1) / (kBlock / kWave), nsys);
-    hipLaunchKernelGGL(k_core_mv<kMvFirst>, rows, dim3(kBlock), 0, s, C);
-    hipLaunchKernelGGL(k_core_mv<kMvResidual>, rows, dim3(kBlock), 0, s, C);
-    hipLaunchKernelGGL(k_core_mv<kMvCorrect>, rows, dim3(kBlock), 0, s, C);
     hipLaunchKernelGGL(k_writeback, dim3(nb), dim3(kBodyBlock), 0, s, C, c.bodies_d.p, c.segs.p,
                        (const double*)c.slae_A.p, (const double*)c.slae_b.p, (const int32_t*)d_body_sys);
     c.bodies_stale = true;

@@ -338,10 +338,11 @@ struct Ctx {
 
     // boundary-condition system (column-major, LAPACK convention)
     DBuf<double> slae_A, slae_b, slae_x;
-    DBuf<double> slae_core, slae_inv, slae_v;   // segment rows and columns, their inverse, vectors of the solve
+    DBuf<double> slae_core, slae_inv, slae_v;   // segment rows and columns, their factors or inverse, vectors of the solve
     DBuf<int32_t> slae_base, slae_ipiv, slae_info;
-    int slae_n = -1;                         // order of the kept inverse
-    int slae_nsys = 1, slae_nsys_factored = 0;   // systems filled / inverted (one per simulation)
+    int slae_n = -1;                         // order of the kept factors or inverse (slae_inv)
+    bool slae_inverted = false;              // slae_inv: the inverse, otherwise the factors
+    int slae_nsys = 1, slae_nsys_factored = 0;   // systems filled / factored (one per simulation)
     int slae_filled = 0;                     // order of the last filled system
     void* rocblas = nullptr;                 // rocblas_handle
 
