@@ -459,8 +459,10 @@ static void velocities(Ctx& c, const TreeDev& T, const double2* xy, const Grid& 
     // Packed records where the points read them often enough: in place against
     // packed, 781 points in 200k vortices 360 and 284 us, 6060 points 406 and
     // 338; 312 in 20k 147 and 138, 78 in 20k 139 and 144; 31 in 2k 38 and 42.
+    // Leaves of hundreds of elements are read along the arrays as they are (909
+    // on average, 2000 points: 203 us packed, 187 in place).
     const int64_t m = std::max<int64_t>(c.n, c.t.nnodes);
-    if (n >= 256 && n * 256 >= m) {
+    if (n >= 256 && n * 256 >= m && c.n <= 128 * (int64_t)c.t.nleaves_h) {
         c.vel_src.grow((size_t)(c.n + 2 * (int64_t)c.t.nnodes));
         double4 *vort = c.vel_src.p, *nodes = vort + c.n;
         hipLaunchKernelGGL(k_pack_sources, dim3(nblocks(m)), dim3(kBlock), 0, s, c.x.p, c.y.p, c.g.p, c.ie.p, c.n, T,
