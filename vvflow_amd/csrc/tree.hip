@@ -1374,8 +1374,9 @@ struct ListLog {
     __device__ int recs(int g) const { return tbase ? (int)(tbase[g + 1] - tbase[g]) : R; }
     __device__ int items(int g) const { return ibase ? (int)(ibase[g + 1] - ibase[g]) : S; }
     // Item of slot w, its group in grp; -1 where the slot holds none.
+    template <bool kExact>
     __device__ int64_t slot(int w, int ngroups, int& grp) const {
-        if (ibase) {
+        if (kExact) {
             grp = __builtin_amdgcn_readfirstlane(item_grp[w]);
             return w;
         }
@@ -1498,6 +1499,8 @@ __global__ __launch_bounds__(kBlock) void k_list_top(NodeView nv, const TravNode
     if (ni > S) G.most[1] = 1;
 }
 
+// kExact: room as counted (ibase); a wave may then take several items.
+template <bool kExact>
 __global__ __launch_bounds__(kBlock) void k_list_items(NodeView nv, const TravNode* __restrict__ tn,
                                                        const int32_t* __restrict__ groups, int ngroups,
                                                        const int32_t* leaf_node, double fc, ListLog G) {
@@ -1509,8 +1512,8 @@ __global__ __launch_bounds__(kBlock) void k_list_items(NodeView nv, const TravNo
     const int step = gridDim.x * (kBlock / kWave);
     for (int w = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave; w < G.slots; w += step) {
         int grp;
-        const int64_t it = G.slot(w, ngroups, grp);
-        if (it < 0) continue;
+        const int64_t it = G.slot<kExact>(w, ngroups, grp);
+        if (it < 0) return;
         const int P0 = __builtin_amdgcn_readfirstlane(G.item[it].x);
         const int end = __builtin_amdgcn_readfirstlane(tn[P0].skip);
         const bool mine = (G.item_mask[it] >> lane) & 1;
@@ -1525,6 +1528,7 @@ __global__ __launch_bounds__(kBlock) void k_list_items(NodeView nv, const TravNo
         log.flush();
         if (lane == 0) G.item_n[it] = (int)log.done;
         G.lanes[it * kWave + lane] = make_int2(cn, cf);
+        if (!kExact) return;
     }
 }
 
@@ -1614,6 +1618,7 @@ struct ListOut {
 
 // The records to the lists: a wave an item, then a wave a group for the
 // group's own records.
+template <bool kExact>
 __global__ __launch_bounds__(kBlock) void k_list_replay(const int32_t* __restrict__ groups, int ngroups, ListLog G,
                                                         const int64_t* near_off, const int64_t* far_off,
                                                         int32_t* near_list, int32_t* far_list) {
@@ -1627,8 +1632,8 @@ __global__ __launch_bounds__(kBlock) void k_list_replay(const int32_t* __restric
     for (int w = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave; w < G.slots + ngroups; w += step) {
         const bool own = w >= G.slots;
         int grp = __builtin_amdgcn_readfirstlane(w - G.slots);
-        const int64_t it = own ? 0 : G.slot(w, ngroups, grp);
-        if (it < 0) continue;
+        const int64_t it = own ? 0 : G.slot<kExact>(w, ngroups, grp);
+        if (it < 0) return;
         const int l = groups[3 * grp] + lane;
         const bool valid = lane < groups[3 * grp + 1];
         ListOut near{near_list + (valid ? near_off[l] : 0)}, far{far_list + (valid ? far_off[l] : 0)};
@@ -1648,6 +1653,7 @@ __global__ __launch_bounds__(kBlock) void k_list_replay(const int32_t* __restric
             }
             near.flush();
             far.flush();
+            if (!kExact) return;
             continue;
         }
         // the group's own records: an item's entries are passed over, up to what
@@ -1675,6 +1681,7 @@ __global__ __launch_bounds__(kBlock) void k_list_replay(const int32_t* __restric
         }
         near.flush();
         far.flush();
+        if (!kExact) return;
     }
 }
 
@@ -2173,9 +2180,9 @@ void tree_lists(Ctx& c) {
     const int item_nodes = std::min(512, std::max(32, (int)(1.4 * std::sqrt((double)t.nnodes))));
     const int ng = t.ngroups;
     // a wave each, or what a launch may hold of them (its threads are a 32-bit
-    // number): the kernels over items go round the rest
+    // number): with room as counted the kernels over items go round the rest
     auto wave_grid = [](int64_t waves) {
-        return dim3((unsigned)std::clamp<int64_t>((waves + kBlock / kWave - 1) / (kBlock / kWave), 1, 1 << 22));
+        return dim3((unsigned)std::clamp<int64_t>((waves + kBlock / kWave - 1) / (kBlock / kWave), 1, (1 << 24) - 1));
     };
     ListLogBufs& b = t.log;
     // The same room for every group, as the last walk needed it, unless one
@@ -2186,11 +2193,17 @@ void tree_lists(Ctx& c) {
     // room that it needs in a second (55 us at 1M, against 400 us for the
     // items' walk).  With the widest group's room for all, ten strays round 4M
     // vortices took 24 GiB, and round 8M the build failed.
+    // (Room of no use costs, too: 150 us at 4M for nine idle items a group.)
     auto room = [&](int64_t most, int64_t all, int64_t floor, int64_t small) {
-        const int64_t r = std::max(floor, most + most / 8);
+        const int64_t r = std::max(floor, most);
         return r * ng <= std::max(small, 4 * all + floor * ng) ? r : floor;
     };
+    // what successive walks need stays where it does not fall by a fifth
+    auto follow = [](int64_t& most, int64_t now) {
+        if (now > most || 5 * now < 4 * most) most = now;
+    };
     int64_t R = room(b.last_recs, b.last_all_recs, 512, 1 << 22), S = room(b.last_items, b.last_all_items, 64, 1 << 17);
+    S = std::min<int64_t>(S, (1 << 25) / std::max(ng, 1));   // a wave each in one launch
     int64_t recs = R * ng, items = S * ng;   // room in all
     bool exact = false;
     // the items' records: what the criteria in use need, or what was counted
@@ -2212,7 +2225,7 @@ void tree_lists(Ctx& c) {
         else
             scan_i32_to_i64(c, b.gnodes.p, b.gbase.p, ng);
         if (ng) {
-            hipLaunchKernelGGL(k_list_items, wave_grid(items), dim3(kBlock), 0, s, nv, (const TravNode*)tn,
+            hipLaunchKernelGGL(exact ? k_list_items<true> : k_list_items<false>, wave_grid(items), dim3(kBlock), 0, s, nv, (const TravNode*)tn,
                                (const int32_t*)t.groups.p, ng, t.leaf_node.p, fc, G);
             hipLaunchKernelGGL(k_list_sums, wave_grid(ng), dim3(kBlock), 0, s, (const int32_t*)t.groups.p, ng, G,
                                t.cnt_near.p, t.cnt_far.p);
@@ -2232,8 +2245,8 @@ void tree_lists(Ctx& c) {
         VVHD_HIP(hipGetLastError());   // no lengths from a launch that was refused
         VVHD_HIP(hipMemcpyAsync(tot, b.totals.p, sizeof(tot), hipMemcpyDeviceToHost, s));
         VVHD_HIP(hipStreamSynchronize(s));
-        b.last_recs = tot[4];
-        b.last_items = tot[5];
+        follow(b.last_recs, tot[4]);
+        follow(b.last_items, tot[5]);
         b.last_all_recs = tot[6];
         b.last_all_items = tot[7];
         nodes = std::max(nodes, tot[2]);
@@ -2251,7 +2264,7 @@ void tree_lists(Ctx& c) {
         t.near_list.grow(t.nnear + 1);
         t.far_list.grow(t.nfar + 1);
         if (ng)
-            hipLaunchKernelGGL(k_list_replay, wave_grid(items + ng), dim3(kBlock), 0, s, (const int32_t*)t.groups.p,
+            hipLaunchKernelGGL(exact ? k_list_replay<true> : k_list_replay<false>, wave_grid(items + ng), dim3(kBlock), 0, s, (const int32_t*)t.groups.p,
                                ng, G, (const int64_t*)t.near_off.p, (const int64_t*)t.far_off.p, t.near_list.p,
                                t.far_list.p);
         return;
