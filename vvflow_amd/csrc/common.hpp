@@ -257,6 +257,7 @@ struct MergeBufs {
     DBuf<double4> rec, cand, cbox;                // records, next records, boxes of the changes
     DBuf<double> fd2;                             // second-neighbour distance before a merge
     DBuf<int32_t> stamp, list, chg, chg_p, ever;
+    DBuf<int32_t> next;                           // per simulation: the order's next element; simulations left
     DBuf<uint64_t> maxd2, lbox, cbound;           // per leaf: bound of the second-neighbour distance, box; of chunks
     DBuf<int32_t> hn1, hn2, hlist;                // heat list: search results
     DBuf<double> hd1, hd2;
@@ -265,7 +266,7 @@ struct MergeBufs {
         info.release();
         for (auto* b : {&rec, &cand, &cbox}) b->release();
         for (auto* b : {&fd2, &hd1, &hd2}) b->release();
-        for (auto* b : {&stamp, &list, &chg, &chg_p, &ever, &hn1, &hn2, &hlist}) b->release();
+        for (auto* b : {&stamp, &list, &chg, &chg_p, &ever, &next, &hn1, &hn2, &hlist}) b->release();
         maxd2.release();
         lbox.release();
         cbound.release();

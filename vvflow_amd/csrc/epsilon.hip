@@ -18,7 +18,8 @@
 // changed against the merges assumed so far, seen as of i, until no merge
 // changes.  After k rounds every target whose chain of dependencies is
 // shorter than k holds its sequential result, and a state that a round leaves
-// unchanged is the sequential one.
+// unchanged is the sequential one.  Where chains are long, the targets left
+// are visited one by one in order (k_merge_in_order).
 //
 // Pass 1 prunes near leaves by box distance: leaves touching the target leaf
 // are scanned first, then only leaves whose box distance does not exceed the
@@ -461,7 +462,11 @@ __device__ Top2 seen_top2(const MergeArgs& A, int l, int L, int i, int excl, dou
     auto scan = [&](bool touching, double bound) {
         Top2 st = top2_empty();
         const int w = G == 1 ? 0 : threadIdx.x / kWave;
-        for (int64_t eb = e0 + (int64_t)w * kPer * kWave; eb < e1; eb += (int64_t)G * kPer * kWave) {
+        // waves take places of the list in turn, or share the candidates of the
+        // only ones (a wide leaf's neighbours may be few and wide)
+        const bool share = G > 1 && e1 - e0 <= kPer * kWave;
+        const int q0 = share ? w * kWave : 0, qstep = share ? G * kWave : kWave;
+        for (int64_t eb = share ? e0 : e0 + (int64_t)w * kPer * kWave; eb < e1; eb += (int64_t)G * kPer * kWave) {
             int M[kPer], j0[kPer], cnt[kPer], mine = 0;
 #pragma unroll
             for (int k = 0; k < kPer; k++) {
@@ -483,12 +488,15 @@ __device__ Top2 seen_top2(const MergeArgs& A, int l, int L, int i, int excl, dou
                 int o = incl - mine - done;
 #pragma unroll
                 for (int k = 0; k < kPer; k++) {
-                    for (int t = max(0, -o); t < cnt[k] && o + t < kMergeTab; t++) tab[o + t] = j0[k] + t;
+                    if (cnt[k] <= kWide)
+                        for (int t = max(0, -o); t < cnt[k] && o + t < kMergeTab; t++) tab[o + t] = j0[k] + t;
+                    for (uint64_t wide = __ballot(cnt[k] > kWide); wide; wide &= wide - 1)
+                        wave_write_range(j0[k], cnt[k], o, (int)__builtin_ctzll(wide), tab, kMergeTab);
                     o += cnt[k];
                 }
                 wave_sync();
                 const int m = min(kMergeTab, total - done);
-                for (int q = lane; q < m; q += kWave) {
+                for (int q = q0 + lane; q < m; q += qstep) {
                     const int j = tab[q];
                     if (j == i || j == excl) continue;
                     const int2 f = A.info[j];
@@ -520,6 +528,7 @@ __global__ void k_merge_init(MergeArgs A) {
     if (i >= A.n) return;
     A.info[i] = make_int2(-1, INT32_MAX);
     A.stamp[i] = 0;
+    A.ever[i] = -1;
     if (A.heat) {   // no parallel pass before the rounds: every particle is a target of the first
         A.list0[i] = i;
         A.d2[i] = -1.;
@@ -554,58 +563,66 @@ struct BlockList {
     }
 };
 
-// One round, first part: every listed target is visited as the reference does
-// when the merges of the targets before it are those of the last round.  Its
-// search results are written in place (only the marking pass reads them), its
-// merge goes to cand and the list of changes.  A wave takes a target, or while
-// there are no more targets than blocks a whole block: the near list of a wide
-// leaf at a cluster's rim runs to thousands of leaves (4M vortices: 310 us a
-// round with a wave each, 64 with a block).
-constexpr int kEvalThreads = 512, kEvalWaves = kEvalThreads / kWave, kEvalBlocks = 512;
-template <int G>
-__device__ void merge_eval(const MergeArgs& A, int parity, int nd, int (*s_tab)[kMergeTab], Top2* parts,
-                           BlockList& changes) {
+// Raises *a to key: by an atomic, or where the block's one writer is the only
+// one that touches it by a store, which the block's later loads see.
+template <bool kAlone>
+__device__ inline void raise_key(uint64_t* a, uint64_t key) {
+    if (kAlone) {
+        if (key > *a) *a = key;
+    } else {
+        atomicMax((unsigned long long*)a, (unsigned long long)key);
+    }
+}
+
+// Target i is visited as the reference does when the merges of the targets
+// before it are those assumed now.  Its search results are written in place
+// (only the marking pass reads them), its merge to cand; true where that is
+// not the assumed one (the same on all lanes).  G waves share the search.
+template <int G, bool kAlone>
+__device__ bool merge_visit(const MergeArgs& A, int i, int* tab, Top2* parts) {
     const TreeDev& T = A.T;
-    const int w = threadIdx.x / kWave, lane = lane_id();
-    const int32_t* list = parity ? A.list1 : A.list0;
-    const int k0 = G == 1 ? blockIdx.x * kEvalWaves + w : blockIdx.x;
-    for (int k = k0; k < nd; k += G == 1 ? gridDim.x * kEvalWaves : gridDim.x) {
-        const int i = list[k];
-        const double gi = A.g[i];
-        const int2 own = A.info[i];
-        const int l = T.vleaf[A.base + i], L = T.leaf_node[l];
-        Top2 st = top2_empty();
-        int partner = -1;
-        double4 rec = make_double4(0, 0, 0, 0);
-        const bool alive = gi != 0 && own.y >= i;
-        double first_d2 = -1.;
-        if (alive) {
-            double px = A.x[i], py = A.y[i];
-            st = seen_top2<G>(A, l, L, i, -1, px, py, s_tab[w], parts);
-            first_d2 = st.d2;
-            const double crit = A.crit[l];
-            if (st.i1 >= 0 && st.i2 >= 0 && !isnan(crit)) {
-                const Seen a = seen_of(A, st.i1, i, A.info[st.i1]), b = seen_of(A, st.i2, i, A.info[st.i2]);
-                const double s1 = sgn(a.g), s2 = sgn(b.g), si = sgn(gi);
-                if ((st.d1 < crit) || (!A.heat && (s1 == s2) && (s1 != si))) {
-                    // MergeVortexes (:111-126), then the search without merging
-                    partner = st.i1;
-                    if (si == s1) {
-                        const double inv = 1. / (gi + a.g);
-                        const double nx = (px * gi + a.x * a.g) * inv;
-                        const double ny = (py * gi + a.y * a.g) * inv;
-                        px = nx;
-                        py = ny;
-                    } else if (fabs(gi) < fabs(a.g)) {
-                        px = a.x;
-                        py = a.y;
-                    }
-                    rec = make_double4(px, py, gi + a.g, 0);
-                    st = seen_top2<G>(A, l, L, i, partner, px, py, s_tab[w], parts);
+    const double gi = A.g[i];
+    const int2 own = A.info[i];
+    const int l = T.vleaf[A.base + i], L = T.leaf_node[l];
+    Top2 st = top2_empty();
+    int partner = -1;
+    double4 rec = make_double4(0, 0, 0, 0);
+    const bool alive = gi != 0 && own.y >= i;
+    double first_d2 = -1.;
+    if (alive) {
+        double px = A.x[i], py = A.y[i];
+        st = seen_top2<G>(A, l, L, i, -1, px, py, tab, parts);
+        first_d2 = st.d2;
+        const double crit = A.crit[l];
+        if (st.i1 >= 0 && st.i2 >= 0 && !isnan(crit)) {
+            const Seen a = seen_of(A, st.i1, i, A.info[st.i1]), b = seen_of(A, st.i2, i, A.info[st.i2]);
+            const double s1 = sgn(a.g), s2 = sgn(b.g), si = sgn(gi);
+            if ((st.d1 < crit) || (!A.heat && (s1 == s2) && (s1 != si))) {
+                // MergeVortexes (:111-126), then the search without merging
+                partner = st.i1;
+                if (si == s1) {
+                    const double inv = 1. / (gi + a.g);
+                    const double nx = (px * gi + a.x * a.g) * inv;
+                    const double ny = (py * gi + a.y * a.g) * inv;
+                    px = nx;
+                    py = ny;
+                } else if (fabs(gi) < fabs(a.g)) {
+                    px = a.x;
+                    py = a.y;
                 }
+                rec = make_double4(px, py, gi + a.g, 0);
+                st = seen_top2<G>(A, l, L, i, partner, px, py, tab, parts);
             }
         }
-        if (lane != 0 || (G > 1 && w != 0)) continue;
+    }
+    bool changed = partner != max(own.x, -1);
+    if (!changed && partner >= 0) {
+        const double4 o = A.rec[i];
+        changed = __double_as_longlong(o.x) != __double_as_longlong(rec.x) ||
+                  __double_as_longlong(o.y) != __double_as_longlong(rec.y) ||
+                  __double_as_longlong(o.z) != __double_as_longlong(rec.z);
+    }
+    if (lane_id() == 0 && (G == 1 || threadIdx.x / kWave == 0)) {
         A.nn1[i] = st.i1;
         A.nn2[i] = st.i2;
         A.d1[i] = st.d1;
@@ -614,21 +631,34 @@ __device__ void merge_eval(const MergeArgs& A, int parity, int nd, int (*s_tab)[
         A.eflag[i] = alive ? 1 : 0;
         if (alive) {
             const uint64_t key = max(d2_key(st.d2), d2_key(first_d2));
-            atomicMax((unsigned long long*)&A.maxd2[l], (unsigned long long)key);
-            atomicMax((unsigned long long*)&A.cbound[4 * (size_t)A.nchunk + l / kChunk], (unsigned long long)key);
-        }
-        bool changed = partner != max(own.x, -1);
-        if (!changed && partner >= 0) {
-            const double4 o = A.rec[i];
-            changed = __double_as_longlong(o.x) != __double_as_longlong(rec.x) ||
-                      __double_as_longlong(o.y) != __double_as_longlong(rec.y) ||
-                      __double_as_longlong(o.z) != __double_as_longlong(rec.z);
+            raise_key<kAlone>(&A.maxd2[l], key);
+            // (leaves of several simulations share a chunk)
+            raise_key<false>(&A.cbound[4 * (size_t)A.nchunk + l / kChunk], key);
         }
         if (changed) {
             rec.w = (double)partner;
             A.cand[i] = rec;
-            changes.push(i, A.chg, &A.ctr[2 + parity]);
         }
+    }
+    return changed;
+}
+
+// One round, first part: every listed target is visited, those whose merge
+// differs go to the list of changes.  A wave takes a target, or while
+// there are no more targets than blocks a whole block: the near list of a wide
+// leaf at a cluster's rim runs to thousands of leaves (4M vortices: 310 us a
+// round with a wave each, 64 with a block).
+constexpr int kEvalThreads = 512, kEvalWaves = kEvalThreads / kWave, kEvalBlocks = 512;
+template <int G>
+__device__ void merge_eval(const MergeArgs& A, int parity, int nd, int (*s_tab)[kMergeTab], Top2* parts,
+                           BlockList& changes) {
+    const int w = threadIdx.x / kWave;
+    const int32_t* list = parity ? A.list1 : A.list0;
+    const int k0 = G == 1 ? blockIdx.x * kEvalWaves + w : blockIdx.x;
+    for (int k = k0; k < nd; k += G == 1 ? gridDim.x * kEvalWaves : gridDim.x) {
+        const int i = list[k];
+        if (merge_visit<G, false>(A, i, s_tab[w], parts) && lane_id() == 0 && (G == 1 || w == 0))
+            changes.push(i, A.chg, &A.ctr[2 + parity]);
     }
 }
 
@@ -655,6 +685,43 @@ __device__ inline void grow_box(double4& b, double px, double py) {
     b.y = fmin(b.y, py);
     b.z = fmax(b.z, px);
     b.w = fmax(b.w, py);
+}
+
+// The leaf of element q holds (px, py) too: its boxes grow (mostly inside
+// already: the leaf's copy tells for the node, too).
+template <bool kAlone>
+__device__ inline void grow_leaf(const MergeArgs& A, int q, double px, double py) {
+    const int lq = A.T.vleaf[A.base + q], Lq = A.T.leaf_node[lq], nl = A.T.nleaf;
+    const size_t ck = lq / kChunk, nk = A.nchunk;
+    auto least = [](uint64_t* a, uint64_t key, bool alone) {
+        if (key >= *a) return false;
+        if (alone)
+            *a = key;
+        else
+            atomicMin((unsigned long long*)a, (unsigned long long)key);
+        return true;
+    };
+    auto most = [](uint64_t* a, uint64_t key, bool alone) {
+        if (key <= *a) return false;
+        if (alone)
+            *a = key;
+        else
+            atomicMax((unsigned long long*)a, (unsigned long long)key);
+        return true;
+    };
+    for (int k = 0; k < 2; k++) {
+        const double v = k == 0 ? px : py;
+        if (isnan(v)) continue;
+        const uint64_t key = ord_from_double(v);
+        if (least(&A.lbox[k * (size_t)nl + lq], key, kAlone)) {
+            least(k == 0 ? &A.blx[Lq] : &A.bly[Lq], key, kAlone);
+            atomicMin((unsigned long long*)&A.cbound[k * nk + ck], (unsigned long long)key);
+        }
+        if (most(&A.lbox[(2 + k) * (size_t)nl + lq], key, kAlone)) {
+            most(k == 0 ? &A.trx[Lq] : &A.try_[Lq], key, kAlone);
+            atomicMax((unsigned long long*)&A.cbound[(2 + k) * nk + ck], (unsigned long long)key);
+        }
+    }
 }
 
 template <int kPhase>
@@ -686,32 +753,7 @@ __device__ void merge_apply(const MergeArgs& A, int parity, int tid, int stride)
                 grow_box(b, r.x, r.y);
                 grow_box(b, A.x[p], A.y[p]);
                 A.cbox[e] = b;
-                const int lq = A.T.vleaf[A.base + q], Lq = A.T.leaf_node[lq], nl = A.T.nleaf;
-                const size_t ck = lq / kChunk, nk = A.nchunk;
-                // mostly inside already: the leaf's copy tells for the node, too
-                auto least = [](uint64_t* a, uint64_t key) {
-                    if (key >= *a) return false;
-                    atomicMin((unsigned long long*)a, (unsigned long long)key);
-                    return true;
-                };
-                auto most = [](uint64_t* a, uint64_t key) {
-                    if (key <= *a) return false;
-                    atomicMax((unsigned long long*)a, (unsigned long long)key);
-                    return true;
-                };
-                for (int k = 0; k < 2; k++) {
-                    const double v = k == 0 ? r.x : r.y;
-                    if (isnan(v)) continue;
-                    const uint64_t key = ord_from_double(v);
-                    if (least(&A.lbox[k * (size_t)nl + lq], key)) {
-                        least(k == 0 ? &A.blx[Lq] : &A.bly[Lq], key);
-                        least(&A.cbound[k * nk + ck], key);
-                    }
-                    if (most(&A.lbox[(2 + k) * (size_t)nl + lq], key)) {
-                        most(k == 0 ? &A.trx[Lq] : &A.try_[Lq], key);
-                        most(&A.cbound[(2 + k) * nk + ck], key);
-                    }
-                }
+                grow_leaf<false>(A, q, r.x, r.y);
             }
         }
     } else {
@@ -757,85 +799,208 @@ __global__ __launch_bounds__(kBlock) void k_merge_apply_part(MergeArgs A, int pa
     merge_apply<kPhase>(A, parity, blockIdx.x * kBlock + threadIdx.x, gridDim.x * kBlock);
 }
 
-// Third part: the targets after a changed element whose second-neighbour
-// distance reaches its box are visited again in the next round (those it
-// does not reach cannot take or lose a neighbour by it), and so are its old
-// and new partner, which it kills or revives.
+// Does a change in the box b reach target i: before its own merge or after?
+__device__ inline bool change_reaches(const MergeArgs& A, const double4& b, int i) {
+    auto reach = [&](double px, double py, double d2) {
+        const double dx = fmax(0.0, fmax(b.x - px, px - b.z)), dy = fmax(0.0, fmax(b.y - py, py - b.w));
+        return !(dx * dx + dy * dy > d2);
+    };
+    if (!(A.eflag[i] & 1)) return false;
+    if (A.info[i].x < 0) return reach(A.x[i], A.y[i], A.d2[i]);
+    const double4 r = A.rec[i];
+    return reach(A.x[i], A.y[i], A.fd2[i]) || reach(r.x, r.y, A.d2[i]);
+}
+
+// The targets after a changed element q whose second-neighbour distance
+// reaches the change's box b have to be visited again (those it does not reach
+// cannot take or lose a neighbour by it), and so have its old and new partner
+// p0 and p1, which it kills or revives: push(target) for each, by any thread.
 // A block per change: each wave tests the chunks of leaves from the element's
-// on (leaves before it hold no later target), a lane each; the block's threads
-// the leaves of a chunk that may be reached; and their targets a lane each.
+// on (leaves before it hold no later target), a lane each; the block's first
+// threads the leaves of a chunk that may be reached; and their targets a lane
+// each.  tab: the wave's.
 // Testing every leaf for every change took 120 us a round in the batch of 16
 // cylinders, 14 us behind one in 100k vortices; now 18 and 8.5.
-__global__ __launch_bounds__(kBlock) void k_merge_mark(MergeArgs A, int parity, int tag) {
-    __shared__ int s_tab[kWavesPerBlock][kNearTab];
-    __shared__ BlockList s_next;
+// kRaised: other blocks raise the chunks' bounds meanwhile, by atomics.  Ranges
+// of more than kWide targets go to wide(j0, cnt), which says whether it takes them.
+template <bool kRaised, typename Push, typename Wide>
+__device__ inline void mark_change(const MergeArgs& A, int q, const double4& b, int p0, int p1, int* tab, Push push,
+                                   Wide wide) {
     const TreeDev& T = A.T;
-    const int nc = A.ctr[2 + parity], lane = lane_id();
-    int32_t* list = parity ? A.list0 : A.list1;
-    auto push = [&](int i) {
-        if (atomicExch(&A.stamp[i], tag) != tag) s_next.push(i, list, &A.ctr[parity ^ 1]);
-    };
-    auto far = [](const double4& b, uint64_t blx, uint64_t bly, uint64_t trx, uint64_t try_, double m) {
+    const int lane = lane_id();
+    auto far = [&](uint64_t blx, uint64_t bly, uint64_t trx, uint64_t try_, double m) {
         const double dx = fmax(0.0, fmax(b.x - double_from_ord(trx), double_from_ord(blx) - b.z));
         const double dy = fmax(0.0, fmax(b.y - double_from_ord(try_), double_from_ord(bly) - b.w));
         return dx * dx + dy * dy > m;
     };
+    const int lq = T.vleaf[A.base + q];
+    const int lend = A.root_first[A.leaf_sim[lq] + 1];
+    if (threadIdx.x == 0) {
+        if (p0 > q) push(p0);
+        if (p1 > q) push(p1);
+    }
+    auto leaves = [&](int l) {
+        const double m = l >= lq && l < lend ? double_from_ord(A.maxd2[l]) : -1.0;
+        int j0 = 0, cnt = 0;
+        if (!(m < 0)) {
+            const uint64_t* lb = A.lbox + l;
+            const size_t nl = T.nleaf;
+            if (!far(lb[0], lb[nl], lb[2 * nl], lb[3 * nl], m)) {
+                const int L = T.leaf_node[l];
+                j0 = max(A.r0[L] - A.base, q + 1);
+                cnt = max(0, A.r1[L] - A.base - j0);
+                if (cnt > kWide && wide(j0, cnt)) cnt = 0;
+            }
+        }
+        wave_lay_out(j0, cnt, tab, [&](int n) {
+            for (int k = lane; k < n; k += kWave)
+                if (change_reaches(A, b, tab[k])) push(tab[k]);
+        });
+    };
+    const int ck1 = (lend - 1) / kChunk;
+    for (int c0 = lq / kChunk; c0 <= ck1; c0 += kWave) {
+        bool may = false;
+        if (c0 + lane <= ck1) {
+            uint64_t cb[5];
+            for (int k = 0; k < 5; k++) {
+                const uint64_t* p = A.cbound + k * (size_t)A.nchunk + c0 + lane;
+                cb[k] = kRaised ? __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *p;
+            }
+            const double m = double_from_ord(cb[4]);
+            may = !(m < 0) && !far(cb[0], cb[1], cb[2], cb[3], m);
+        }
+        for (uint64_t mask = __ballot(may); mask; mask &= mask - 1)
+            if (threadIdx.x < kChunk) leaves((c0 + (int)__builtin_ctzll(mask)) * kChunk + threadIdx.x);
+    }
+}
+
+// Third part of a round: what the changes reach is listed for the next one.
+__global__ __launch_bounds__(kBlock) void k_merge_mark(MergeArgs A, int parity, int tag) {
+    __shared__ int s_tab[kWavesPerBlock][kNearTab];
+    __shared__ BlockList s_next;
+    const int nc = A.ctr[2 + parity];
+    int32_t* list = parity ? A.list0 : A.list1;
     s_next.begin();
     for (int e = blockIdx.x; e < nc; e += gridDim.x) {
         const int q = A.chg[e];
-        const double4 b = A.cbox[e];
-        const int lq = T.vleaf[A.base + q];
-        const int lend = A.root_first[A.leaf_sim[lq] + 1];
-        if (threadIdx.x == 0) {
-            const int p0 = A.chg_p[e], p1 = A.info[q].x;
-            if (p0 > q) push(p0);
-            if (p1 > q) push(p1);
-        }
-        auto reach = [&](double px, double py, double d2) {
-            const double dx = fmax(0.0, fmax(b.x - px, px - b.z)), dy = fmax(0.0, fmax(b.y - py, py - b.w));
-            return !(dx * dx + dy * dy > d2);
-        };
-        auto leaves = [&](int l) {
-            const double m = l >= lq && l < lend ? double_from_ord(A.maxd2[l]) : -1.0;
-            int j0 = 0, cnt = 0;
-            if (!(m < 0)) {
-                const uint64_t* lb = A.lbox + l;
-                const size_t nl = T.nleaf;
-                if (!far(b, lb[0], lb[nl], lb[2 * nl], lb[3 * nl], m)) {
-                    const int L = T.leaf_node[l];
-                    j0 = max(A.r0[L] - A.base, q + 1);
-                    cnt = max(0, A.r1[L] - A.base - j0);
-                }
-            }
-            wave_lay_out(j0, cnt, s_tab[threadIdx.x / kWave], [&](int n) {
-                for (int k = lane; k < n; k += kWave) {
-                    const int i = s_tab[threadIdx.x / kWave][k];
-                    if (!(A.eflag[i] & 1)) continue;
-                    bool hit;
-                    if (A.info[i].x >= 0) {
-                        const double4 r = A.rec[i];
-                        hit = reach(A.x[i], A.y[i], A.fd2[i]) || reach(r.x, r.y, A.d2[i]);
-                    } else {
-                        hit = reach(A.x[i], A.y[i], A.d2[i]);
-                    }
-                    if (hit) push(i);
-                }
-            });
-        };
-        const int ck1 = (lend - 1) / kChunk;
-        for (int c0 = lq / kChunk; c0 <= ck1; c0 += kWave) {
-            bool may = false;
-            if (c0 + lane <= ck1) {
-                const uint64_t* cb = A.cbound + c0 + lane;
-                const size_t nk = A.nchunk;
-                const double m = double_from_ord(cb[4 * nk]);
-                may = !(m < 0) && !far(b, cb[0], cb[nk], cb[2 * nk], cb[3 * nk], m);
-            }
-            for (uint64_t mask = __ballot(may); mask; mask &= mask - 1)
-                leaves((c0 + (int)__builtin_ctzll(mask)) * kChunk + threadIdx.x);
-        }
+        mark_change<false>(A, q, A.cbox[e], A.chg_p[e], A.info[q].x, s_tab[threadIdx.x / kWave], [&](int i) {
+            if (atomicExch(&A.stamp[i], tag) != tag) s_next.push(i, list, &A.ctr[parity ^ 1]);
+        }, [](int, int) { return false; });
     }
     s_next.end(list, &A.ctr[parity ^ 1]);
+}
+
+// The targets still to be visited (stamp == tag) one after another in their
+// order, a block per simulation: every target is visited once, when all before
+// it are settled.  For chains of merges that wait for each other one by one,
+// where each round settles a single one and visits all behind it in vain.
+// next: the block's first element to look at; a launch visits kInOrder targets
+// of a simulation at most, *left then counts the simulations that have more.
+// What is written here is read by the same block only (stores, and barriers
+// that wait for them), but for the chunk bounds and the list of elements that
+// have a record, of which an entry of another simulation does nothing.
+constexpr int kInOrder = 2048;
+__global__ __launch_bounds__(kEvalThreads) void k_merge_in_order(MergeArgs A, int tag, int32_t* next, int32_t* left) {
+    __shared__ int s_tab[kEvalWaves][kNearTab];
+    __shared__ Top2 s_parts[kEvalWaves];
+    __shared__ int s_first[kEvalWaves], s_death[2], s_nwide;
+    __shared__ int2 s_wide[kChunk];   // ranges of targets that all threads share
+    __shared__ double4 s_box;
+    static_assert(kNearTab >= kMergeTab && kEvalThreads >= kChunk, "tables of the searches and leaves of a chunk");
+    const int sim = blockIdx.x, t = threadIdx.x, w = t / kWave, lane = lane_id();
+    const int end = A.r1[sim] - A.base;
+    auto sync = [] {
+        __threadfence_block();
+        __syncthreads();
+    };
+    int cur = next[sim];
+    for (int visits = 0; cur < end && visits < kInOrder;) {
+        // the first one listed from cur on
+        constexpr int kPer = 4;
+        int first = INT32_MAX;
+        for (int k = kPer - 1; k >= 0; k--) {
+            const int i = cur + k * kEvalThreads + t;
+            const uint64_t m = __ballot(i < end && A.stamp[i] == tag);
+            if (m) first = i - lane + (int)__builtin_ctzll(m);
+        }
+        if (lane == 0) s_first[w] = first;
+        __syncthreads();
+        for (int q = 0; q < kEvalWaves; q++) first = min(first, s_first[q]);
+        if (first == INT32_MAX) {
+            cur += kPer * kEvalThreads;
+            __syncthreads();
+            continue;
+        }
+        const int i = first;
+        visits++;
+        cur = i + 1;
+        const int p0 = A.info[i].x;
+        const bool changed = merge_visit<kEvalWaves, true>(A, i, s_tab[w], s_parts);
+        sync();
+        if (!changed) continue;
+        // the record takes effect (see merge_apply)
+        const double4 r = A.cand[i];
+        const int p1 = (int)r.w;
+        if (t == 0) {
+            double4 b = make_double4(A.x[i], A.y[i], A.x[i], A.y[i]);
+            if (p0 >= 0) {
+                const double4 o = A.rec[i];
+                grow_box(b, o.x, o.y);
+                grow_box(b, A.x[p0], A.y[p0]);
+            }
+            if (p0 == -1) A.ever[atomicAdd(&A.ctr[4], 1)] = i;
+            A.info[i].x = p1 >= 0 ? p1 : -2;
+            A.rec[i] = r;
+            if (p1 >= 0) {
+                grow_box(b, r.x, r.y);
+                grow_box(b, A.x[p1], A.y[p1]);
+                grow_leaf<true>(A, i, r.x, r.y);
+            }
+            for (int p : {p0, p1})
+                if (p >= 0 && A.info[p].x >= 0) {
+                    const double4 o = A.rec[p];
+                    grow_box(b, o.x, o.y);
+                }
+            s_box = b;
+            s_death[0] = s_death[1] = INT32_MAX;
+            s_nwide = 0;
+        }
+        sync();
+        // deaths of the old and the new partner
+        const int ne = __hip_atomic_load(&A.ctr[4], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int k = t; k < ne; k += kEvalThreads) {
+            const int q = A.ever[k], p = q >= 0 ? A.info[q].x : -1;
+            if (p < 0) continue;
+            if (p == p0) atomicMin(&s_death[0], q);
+            if (p == p1) atomicMin(&s_death[1], q);
+        }
+        __syncthreads();
+        if (t == 0) {
+            if (p0 >= 0) A.info[p0].y = s_death[0];
+            if (p1 >= 0) A.info[p1].y = s_death[1];
+        }
+        auto push = [&](int k) { A.stamp[k] = tag; };
+        mark_change<true>(A, i, s_box, p0, p1, s_tab[w], push, [&](int j0, int cnt) {
+            const int k = atomicAdd(&s_nwide, 1);
+            if (k < kChunk) s_wide[k] = make_int2(j0, cnt);
+            return k < kChunk;
+        });
+        __syncthreads();
+        for (int r = 0; r < min(s_nwide, kChunk); r++)
+            for (int k = t; k < s_wide[r].y; k += kEvalThreads)
+                if (change_reaches(A, s_box, s_wide[r].x + k)) push(s_wide[r].x + k);
+        sync();
+    }
+    if (t == 0) {
+        next[sim] = cur;
+        if (cur < end) atomicAdd(left, 1);
+    }
+}
+
+// The first element of every simulation.
+__global__ void k_merge_first(MergeArgs A, int nsim, int32_t* next) {
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s < nsim) next[s] = A.r0[s] - A.base;
 }
 
 // The converged merges written to the list, one workgroup: every merging
@@ -926,10 +1091,17 @@ namespace {
 // round of all of them takes about 25 us.
 // left: the targets listed for the first round.
 constexpr int kApplyOne = 2048;
+// A round takes about 25 us and 1/16 us a target, a visit in order 10 to 18.
+// Rounds are given up for the order when they have taken about a third of what
+// the targets left would take in it; most lists have settled long before.  A
+// line of 2000 merges: 350 ms in rounds alone, 38 so (121 where one workgroup
+// committed merge after merge); 300 round a body 14.2, 3.5 (6.1).
+constexpr int64_t kInOrderShare = 3, kInOrderAfter = 16;
 void merge_rounds(Ctx& c, MergeArgs A, int32_t left, double* x, double* y, double* g, int32_t* merged) {
     hipStream_t s = c.stream;
     hipLaunchKernelGGL(k_chunk_bounds, dim3(A.nchunk), dim3(kBlock), 0, s, A.T.nleaf, (const uint64_t*)A.maxd2,
                        (const uint64_t*)A.lbox, A.cbound);
+    int64_t spent = 0;
     for (int64_t round = 0; left > 0; ) {
         VVHD_CHECK(round <= (int64_t)A.n + 8, VVHD_EHIP, "epsilon: the merges do not settle");
         for (int k = 0; k < 4; k++, round++) {
@@ -946,6 +1118,19 @@ void merge_rounds(Ctx& c, MergeArgs A, int32_t left, double* x, double* y, doubl
         }
         VVHD_HIP(hipMemcpyAsync(&left, A.ctr + (round & 1), 4, hipMemcpyDeviceToHost, s));
         VVHD_HIP(hipStreamSynchronize(s));
+        spent += 4 * (25 + (int64_t)left / 16);
+        if (round < kInOrderAfter || spent < kInOrderShare * (int64_t)left) continue;
+        // the rounds do not pay: the rest in order
+        c.mg.next.grow(c.nsim + 1);
+        int32_t* more = c.mg.next.p + c.nsim;
+        hipLaunchKernelGGL(k_merge_first, dim3(nblocks(c.nsim)), dim3(kBlock), 0, s, A, c.nsim, c.mg.next.p);
+        while (left > 0) {
+            VVHD_HIP(hipMemsetAsync(more, 0, 4, s));
+            hipLaunchKernelGGL(k_merge_in_order, dim3(c.nsim), dim3(kEvalThreads), 0, s, A, (int)round, c.mg.next.p,
+                               more);
+            VVHD_HIP(hipMemcpyAsync(&left, more, 4, hipMemcpyDeviceToHost, s));
+            VVHD_HIP(hipStreamSynchronize(s));
+        }
     }
     hipLaunchKernelGGL(k_merge_finish, dim3(1), dim3(kMergeThreads), 0, s, A, x, y, g, merged);
 }

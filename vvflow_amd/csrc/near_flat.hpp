@@ -19,6 +19,15 @@ __device__ inline void wave_sync() {
 // of more than kWide elements is written by all lanes, range after range (a
 // leaf that the least node size keeps whole may hold thousands).
 constexpr int kWide = 32;
+
+// The part of lane b's range [j0, j0 + cnt) that falls in tab[0..room), its
+// first element at tab[o] (before the table where o < 0).
+__device__ inline void wave_write_range(int j0, int cnt, int o, int b, int* tab, int room) {
+    const int ob = __builtin_amdgcn_readlane(o, b), j = __builtin_amdgcn_readlane(j0, b) - ob;
+    const int end = min(ob + __builtin_amdgcn_readlane(cnt, b), room);
+    for (int t = max(0, ob) + lane_id(); t < end; t += kWave) tab[t] = j + t;
+}
+
 template <typename Chunk>
 __device__ inline void wave_lay_out(int j0, int cnt, int* tab, Chunk chunk) {
     const int incl = wave_incl_scan(cnt);
@@ -28,12 +37,8 @@ __device__ inline void wave_lay_out(int j0, int cnt, int* tab, Chunk chunk) {
         const int o = incl - cnt - done;
         if (cnt <= kWide)
             for (int t = max(0, -o); t < cnt && o + t < kNearTab; t++) tab[o + t] = j0 + t;
-        for (uint64_t w = wide; w; w &= w - 1) {
-            const int b = (int)__builtin_ctzll(w);
-            const int ob = __builtin_amdgcn_readlane(o, b), j = __builtin_amdgcn_readlane(j0, b) - ob;
-            const int end = min(ob + __builtin_amdgcn_readlane(cnt, b), kNearTab);
-            for (int t = max(0, ob) + lane_id(); t < end; t += kWave) tab[t] = j + t;
-        }
+        for (uint64_t w = wide; w; w &= w - 1)
+            wave_write_range(j0, cnt, o, (int)__builtin_ctzll(w), tab, kNearTab);
         wave_sync();
         chunk(min(kNearTab, total - done));
         wave_sync();
