@@ -477,8 +477,10 @@ void sync(Ctx& c);
 void tree_build(Ctx& c, int far_criteria, double min_node, double max_node, int32_t* perm_out);
 void tree_lists(Ctx& c);
 // Calls run(first level, end level, blocks) for the levels over the whole list,
-// deepest first when up: consecutive small levels together for one block.
-void for_level_runs(const TreeArrays& t, bool up, const std::function<void(int, int, int)>& run);
+// deepest first when up: consecutive levels of at most `small` nodes together for
+// one block, larger ones each on blocks of `threads`.
+void for_level_runs(const TreeArrays& t, bool up, const std::function<void(int, int, int)>& run, int small,
+                    int threads);
 void epsilon(Ctx& c, int merge, int32_t* nn1, int32_t* nn2, int32_t* merged);
 void convective(Ctx& c, double inf_x, double inf_y, int kahan);
 // beside: the near field runs beside the far-field kernels (tuned among the

@@ -261,8 +261,12 @@ __device__ inline void node_moments(const int32_t* ch1, const double* nx, const 
 
 // Bottom-up over the levels [l0, l1) of the whole list (one block for several,
 // or one level spread over the grid), and over each subtree's levels (one
-// block per subtree).
-constexpr int kMomThreads = 1024;
+// wave per subtree).  They run beside the near field, whose waves fill the
+// chip: a block waits for as many free slots on one CU as it has waves.  At 1M
+// one block of 1024 threads for the levels took 413 us and 256 threads a
+// subtree 480; 256 for levels of up to as many nodes and a wave a subtree
+// take 52 and 38 (a launch for each of all the tree's levels 280).
+constexpr int kMomThreads = 256;
 __global__ __launch_bounds__(kMomThreads) void k_moments_levels(const int32_t* ch1, const int32_t* split,
                                                                 const double* nx, const double* ny, MomView M,
                                                                 const int2* lev, int l0, int l1) {
@@ -274,12 +278,12 @@ __global__ __launch_bounds__(kMomThreads) void k_moments_levels(const int32_t* c
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_moments_subs(const int32_t* ch1, const int32_t* split, const double* nx,
-                                                         const double* ny, MomView M, const int2* sub_lev,
-                                                         const int32_t* sub_nlev) {
+__global__ __launch_bounds__(kWave) void k_moments_subs(const int32_t* ch1, const int32_t* split, const double* nx,
+                                                        const double* ny, MomView M, const int2* sub_lev,
+                                                        const int32_t* sub_nlev) {
     const int2* lev = sub_lev + (size_t)blockIdx.x * kSubLevels;
     for (int d = sub_nlev[blockIdx.x] - 2; d >= 0; d--) {   // the last level holds leaves only
-        for (int i = threadIdx.x; i < lev[d].y; i += kBlock)
+        for (int i = threadIdx.x; i < lev[d].y; i += kWave)
             if (split[lev[d].x + i] == 2) node_moments(ch1, nx, ny, M, lev[d].x + i);
         __threadfence_block();
         __syncthreads();
@@ -1284,12 +1288,12 @@ MomView moments(Ctx& c) {
                            t.nleaves_h, t.v0.p, t.v1.p, t.x.p, t.y.p, c.x.p, c.y.p, c.g.p, c.ie.p, M);
     // internal nodes: the subtrees, then the levels above them
     if (t.nsub)
-        hipLaunchKernelGGL(k_moments_subs, dim3(t.nsub), dim3(kBlock), 0, c.stream, t.ch1.p, t.split.p, t.x.p, t.y.p, M,
+        hipLaunchKernelGGL(k_moments_subs, dim3(t.nsub), dim3(kWave), 0, c.stream, t.ch1.p, t.split.p, t.x.p, t.y.p, M,
                            (const int2*)t.sub_lev.p, (const int32_t*)t.sub_nlev.p);
     for_level_runs(t, true, [&](int l0, int l1, int grid) {
         hipLaunchKernelGGL(k_moments_levels, dim3(grid), dim3(kMomThreads), 0, c.stream, t.ch1.p, t.split.p, t.x.p,
                            t.y.p, M, (const int2*)t.lev_d.p, l0, l1);
-    });
+    }, kMomThreads, kMomThreads);
     return M;
 }
 

@@ -1890,15 +1890,16 @@ void scan_flags(Ctx& c, const GoesLeftFlag& f, int32_t* flag, int32_t* P, int32_
 
 }  // namespace
 
-void for_level_runs(const TreeArrays& t, bool up, const std::function<void(int, int, int)>& run) {
+void for_level_runs(const TreeArrays& t, bool up, const std::function<void(int, int, int)>& run, int small,
+                    int threads) {
     const int n = (int)t.levels.size();
     auto size = [&](int d) { return t.levels[d].second - t.levels[d].first; };
     std::vector<std::array<int, 3>> runs;
     for (int d = 0; d < n;) {
         int e = d + 1;
-        if (size(d) <= kPassNodes)
-            while (e < n && size(e) <= kPassNodes) e++;
-        runs.push_back({d, e, size(d) <= kPassNodes ? 1 : nblocks(size(d), kPassThreads)});
+        if (size(d) <= small)
+            while (e < n && size(e) <= small) e++;
+        runs.push_back({d, e, size(d) <= small ? 1 : nblocks(size(d), threads)});
         d = e;
     }
     if (up) std::reverse(runs.begin(), runs.end());
@@ -2087,14 +2088,14 @@ void tree_build(Ctx& c, int far_criteria, double min_node, double max_node, int3
     for_level_runs(t, true, [&](int l0, int l1, int grid) {
         hipLaunchKernelGGL(k_up_levels, dim3(grid), dim3(kPassThreads), 0, s, nv, cm, (const int2*)t.lev_d.p, l0, l1,
                            c.x.p, c.y.p, c.g.p, t.nleaves.p);
-    });
+    }, kPassNodes, kPassThreads);
     int32_t* first = t.arrive.p;
     t.root_first.grow(nroots + 1);
     hipLaunchKernelGGL(k_root_first, dim3(1), dim3(1), 0, s, t.nleaves.p, nroots, first, t.root_first.p, t.pre.p);
     for_level_runs(t, false, [&](int l0, int l1, int grid) {
         hipLaunchKernelGGL(k_down_levels, dim3(grid), dim3(kPassThreads), 0, s, nv, (const int2*)t.lev_d.p, l0, l1,
                            t.nleaves.p, first, t.leaf_rank.p, t.leaf_node.p, t.vleaf.p, t.pre.p);
-    });
+    }, kPassNodes, kPassThreads);
     if (t.nsub)
         hipLaunchKernelGGL(k_down_subs, dim3(t.nsub), dim3(kBlock), 0, s, nv, (const int2*)t.sub_lev.p,
                            (const int32_t*)t.sub_nlev.p, t.nleaves.p, first, t.leaf_rank.p, t.leaf_node.p, t.vleaf.p,
