@@ -48,7 +48,7 @@ def test_sums_over_unequal_leaves(ctx, sizes):
     o.epsilon(False)
     ctx.epsilon(False)
     r = np.random.default_rng(5)
-    for npts in (7, 300):   # in place and packed
+    for npts in (7, 300):   # sources in place and, where leaves average up to 128, packed
         pts = r.uniform(-1, 1, (npts, 2))
         pts[::3] = objs[r.integers(0, n, len(pts[::3])), :2]
         ref, got = o.velocity(pts), ctx.velocity(pts, inf=(1.0, 0.0))

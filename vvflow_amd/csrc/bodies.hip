@@ -57,7 +57,9 @@ __device__ inline double dot2(double ax, double ay, double bx, double by) { retu
 // chunk of segments are computed by all threads and staged in LDS, then one
 // lane per sum adds them in segment order, so every FP64 quantity rounds as
 // in the reference.  One thread per body waited for each segment's loads in
-// turn (290-410 us for 350-500 segments; 5-12 us so).
+// turn: 290-410 us for 350-500 segments.  Now k_calc_forces takes 9-11 us,
+// k_dead 25-43, k_body_move and k_body_properties 31-34 (their sums, one after
+// another, are what is left).
 constexpr int kBodyBlock = 256;
 constexpr int kBodyChunk = 512;
 
@@ -201,12 +203,6 @@ __global__ __launch_bounds__(kBodyBlock) void k_body_move(vvhd_body* bodies, vvh
             B.speed_slae_prev[i] = B.speed_slae[i];
         }
     body_properties(B, segs, geo + 5 * b, sh, acc);
-}
-
-__device__ inline int body_of_seg(const vvhd_body* bodies, int nbody, int s) {
-    int b = 0;
-    while (b + 1 < nbody && bodies[b + 1].first_seg <= s) b++;
-    return b;
 }
 
 // ---------------------------------------------------------------- flow-move

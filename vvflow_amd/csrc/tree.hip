@@ -531,11 +531,11 @@ __global__ void k_ranks(NodeView nv, const int32_t* enode, const int32_t* P, int
     }
 }
 
-// Hoare swaps, child bounding boxes and element -> child node.
-// With bbox false the child boxes are left to k_bbox_top.
+// Hoare swaps and element -> child node (the children's boxes follow from the
+// elements in their places: k_bbox_top, k_child_boxes).
 __global__ void k_swap(NodeView nv, int32_t* enode, const int32_t* flag, const int32_t* P, int n, int hbase,
                        int sbase, int cap, const int32_t* node_L, const int32_t* node_m, const int32_t* left_pos,
-                       const int32_t* right_pos, double* x, double* y, int32_t* id, bool bbox) {
+                       const int32_t* right_pos, double* x, double* y, int32_t* id) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     bool active = false;
     int node = 0, Labs = 0, v0 = 0, f = 0, c = 0, slot = 0;
@@ -553,27 +553,12 @@ __global__ void k_swap(NodeView nv, int32_t* enode, const int32_t* flag, const i
         c = nv.ch1[node];
     }
     const bool left_mis = active && k < Labs && !f;
-    const bool right_mis = active && k >= Labs && f;
-    // Bounding boxes by element identity: each element's own flag decides its
-    // child.  A misplaced pair is accounted by its left thread (the right
-    // thread's coordinates may already be swapped and are not used).
-    const double px = active ? x[k] : 0, py = active ? y[k] : 0;
-    double qx = 0, qy = 0;
-    int partner = -1;
+    if (active) enode[k] = (k < Labs) ? c : c + 1;
+    // Only the left thread of a misplaced pair reads and writes either position.
     if (left_mis) {
         const int r = (k - v0) - (P[k] - P[v0]);
-        partner = right_pos[v0 + node_m[slot] - 1 - r];
-        qx = x[partner];
-        qy = y[partner];
-    }
-    if (bbox) {
-        const bool own = active && !right_mis;
-        bbox_add_wave(nv, c + (f ? 0 : 1), px, py, own);
-        bbox_add_wave(nv, c, qx, qy, left_mis);
-    }
-    if (active) enode[k] = (k < Labs) ? c : c + 1;
-    // Only the left thread of a misplaced pair writes either position.
-    if (left_mis) {
+        const int partner = right_pos[v0 + node_m[slot] - 1 - r];
+        const double px = x[k], py = y[k], qx = x[partner], qy = y[partner];
         const int32_t ik = id[k], ip = id[partner];
         x[k] = qx;
         y[k] = qy;
@@ -2006,7 +1991,7 @@ void tree_build(Ctx& c, int far_criteria, double min_node, double max_node, int3
         // the children of level d number at most nroots 2^(d+1)
         const bool top = ((int64_t)nroots << std::min<int>(d + 1, 30)) <= kTopNodes;
         hipLaunchKernelGGL(k_swap, dim3(nblocks(n)), dim3(kBlock), 0, s, nv, enode.p, flag, P, n, t.hbase, t.sbase,
-                           cap, node_L.p, node_m.p, left_pos, right_pos, c.x.p, c.y.p, c.id.p, false);
+                           cap, node_L.p, node_m.p, left_pos, right_pos, c.x.p, c.y.p, c.id.p);
         if (top && n)
             hipLaunchKernelGGL(k_bbox_top, dim3(nblocks(n, kTopChunk)), dim3(kBlock), 0, s, nv,
                                (const int32_t*)(t.counters.p + 2), (const int32_t*)enode.p, c.x.p, c.y.p, n);
@@ -2193,7 +2178,8 @@ void tree_lists(Ctx& c) {
     // do, the counts of the first walk over the groups give every group the
     // room that it needs in a second (55 us at 1M, against 400 us for the
     // items' walk).  With the widest group's room for all, ten strays round 4M
-    // vortices took 24 GiB, and round 8M the build failed.
+    // vortices took 24 GiB, and round 8M the launches of 12020 x 6211 waves
+    // were larger than a grid may be.
     // (Room of no use costs, too: 150 us at 4M for nine idle items a group.)
     auto room = [&](int64_t most, int64_t all, int64_t floor, int64_t small) {
         const int64_t r = std::max(floor, most);
