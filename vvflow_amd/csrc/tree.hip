@@ -2189,9 +2189,15 @@ void tree_lists(Ctx& c) {
     auto follow = [](int64_t& most, int64_t now) {
         if (now > most || 5 * now < 4 * most) most = now;
     };
-    int64_t R = room(b.last_recs, b.last_all_recs, 512, 1 << 22), S = room(b.last_items, b.last_all_items, 64, 1 << 17);
-    S = std::min<int64_t>(S, (1 << 25) / std::max(ng, 1));   // a wave each in one launch
-    int64_t recs = R * ng, items = S * ng;   // room in all
+    int64_t R, S, recs, items;   // room of a group, and in all
+    auto same_room = [&]() {
+        R = room(b.last_recs, b.last_all_recs, 512, 1 << 22);
+        S = room(b.last_items, b.last_all_items, 64, 1 << 17);
+        S = std::min<int64_t>(S, (1 << 25) / std::max(ng, 1));   // a wave each in one launch
+        recs = R * ng;
+        items = S * ng;
+    };
+    same_room();
     bool exact = false;
     // the items' records: what the criteria in use need, or what was counted
     int64_t nodes = (int64_t)ng * 6144;
@@ -2238,11 +2244,14 @@ void tree_lists(Ctx& c) {
         b.last_all_items = tot[7];
         nodes = std::max(nodes, tot[2]);
         if (tot[3]) {
-            scan_i32_to_i64(c, b.nrec.p, b.tbase.p, ng);
-            scan_i32_to_i64(c, b.nitem.p, b.ibase.p, ng);
-            exact = true;
-            recs = tot[6];
-            items = tot[7];
+            same_room();
+            exact = R < tot[4] || S < tot[5];
+            if (exact) {
+                scan_i32_to_i64(c, b.nrec.p, b.tbase.p, ng);
+                scan_i32_to_i64(c, b.nitem.p, b.ibase.p, ng);
+                recs = tot[6];
+                items = tot[7];
+            }
             continue;
         }
         if (tot[2] > G.cap) continue;
