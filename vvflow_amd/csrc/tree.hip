@@ -1705,7 +1705,7 @@ __global__ __launch_bounds__(kTotalsThreads) void k_list_totals(const int64_t* n
     __shared__ int64_t s_part[kTotalsThreads / kWave][4];
     const int k = threadIdx.x;
     int64_t v[4] = {0, 0, 0, 0};   // most records, most items, all records, all items
-    for (int g = k; g < ngroups; g += kTotalsThreads) {
+    for (int g = k; g < ngroups; g += blockDim.x) {
         const int64_t r = G.nrec[g], i = G.nitem[g];
         v[0] = max(v[0], r);
         v[1] = max(v[1], i);
@@ -1724,7 +1724,7 @@ __global__ __launch_bounds__(kTotalsThreads) void k_list_totals(const int64_t* n
         for (int q = 0; q < 4; q++) s_part[k / kWave][q] = v[q];
     __syncthreads();
     if (k != 0) return;
-    for (int w = 1; w < kTotalsThreads / kWave; w++) join(v, s_part[w]);
+    for (int w = 1; w < (int)blockDim.x / kWave; w++) join(v, s_part[w]);
     out[0] = *near_end;
     out[1] = *far_end;
     out[2] = *nodes_end;
@@ -2233,7 +2233,7 @@ void tree_lists(Ctx& c) {
         // lengths of the near and the far lists, the items' nodes, out of room, then
         // most and all of the records and of the items
         int64_t tot[kTotals];
-        hipLaunchKernelGGL(k_list_totals, dim3(1), dim3(kTotalsThreads), 0, s, (const int64_t*)t.near_off.p + nl,
+        hipLaunchKernelGGL(k_list_totals, dim3(1), dim3(std::clamp((ng + 255) / 256 * kWave, kWave, kTotalsThreads)), 0, s, (const int64_t*)t.near_off.p + nl,
                            (const int64_t*)t.far_off.p + nl, (const int64_t*)b.gbase.p + ng, G, ng, b.totals.p);
         VVHD_HIP(hipGetLastError());   // no lengths from a launch that was refused
         VVHD_HIP(hipMemcpyAsync(tot, b.totals.p, sizeof(tot), hipMemcpyDeviceToHost, s));
