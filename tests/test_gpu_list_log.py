@@ -73,3 +73,40 @@ def test_memory_of_strays():
             ctx.close()
     print(f"  {used[0]:.0f} and {used[1]:.0f} MiB", flush=True)
     assert used[1] < 1.25 * used[0]
+
+
+def test_little_memory_left():
+    """A tree of 2.2M vortices with 2.9 GiB of device memory left: its lists are
+    walked in parts, and are those that a walk of all has."""
+    n = 2200000
+    objs = V.gen_wake(n)
+    out = []
+    for left in (None, 2.9):
+        print(f"case list log n={n}, GiB left: {left}", flush=True)
+        ctx = V.Context(0)
+        hog = None
+        try:
+            ctx.upload(objs)
+            ctx.snapshot()
+            torch.cuda.synchronize()
+            if left:
+                torch.cuda.empty_cache()
+                hog = torch.empty(torch.cuda.mem_get_info()[0] - int(left * 2**30), dtype=torch.uint8, device="cuda")
+            for _ in range(2):   # without and with the buffers of the build before
+                ctx.restore()
+                ctx.tree_build(8)
+            hog = None
+            torch.cuda.empty_cache()
+            near = ctx.tree_lists()
+            ctx.epsilon(False)
+            ctx.convective((1.0, 0.0))
+            out.append((near["off"], near["path"], near["depth"], ctx.download()))
+            ctx.restore()
+            ctx.tree_build(8)   # memory again
+            ctx.epsilon(False)
+            ctx.convective((1.0, 0.0))
+            assert np.array_equal(ctx.download(), out[0][3])
+        finally:
+            ctx.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)

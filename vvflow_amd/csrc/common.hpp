@@ -52,6 +52,7 @@ struct DBuf {
         cap = 0;
         if (hipMalloc(&p, nc * sizeof(T)) != hipSuccess) {
             p = nullptr;
+            (void)hipGetLastError();   // reported here, not by the next call
             throw Error(VVHD_ENOMEM, "hipMalloc of " + std::to_string(nc * sizeof(T)) + " bytes failed");
         }
         cap = nc;
@@ -131,8 +132,11 @@ struct ListLogBufs {
     DBuf<uint64_t> tfar, tnear, item_mask, rfar, rnear;
     DBuf<int64_t> gbase, tbase, ibase, totals;
     DBuf<int2> item, lanes, after;
-    // of the last walk: most records and items of a group, and of all groups
-    int64_t last_recs = 0, last_items = 0, last_all_recs = 0, last_all_items = 0;
+    // of the last walk: most records and items of a group, and of all groups;
+    // nodes of a group's items on average
+    int64_t last_recs = 0, last_items = 0, last_all_recs = 0, last_all_items = 0, last_nodes = 0;
+    // bytes of the records and items
+    int64_t bytes() const { return (int64_t)(20 * tid.cap + 20 * rid.cap + 24 * item.cap + 16 * lanes.cap); }
     void grow(int64_t groups, int64_t top, int64_t items, int64_t records) {
         for (auto* b : {&tfar, &tnear}) b->grow(top + 1);
         tid.grow(top + 1);
@@ -145,11 +149,15 @@ struct ListLogBufs {
         rid.grow(records + 1);
         for (auto* b : {&rfar, &rnear}) b->grow(rid.cap);
     }
-    void release() {
-        for (auto* b : {&tid, &nrec, &nitem, &gnodes, &item_n, &item_grp, &rid, &most}) b->release();
+    void release_walk() {
+        for (auto* b : {&tid, &item_n, &item_grp, &rid}) b->release();
         for (auto* b : {&tfar, &tnear, &item_mask, &rfar, &rnear}) b->release();
-        for (auto* b : {&gbase, &tbase, &ibase, &totals}) b->release();
         for (auto* b : {&item, &lanes, &after}) b->release();
+    }
+    void release() {
+        release_walk();
+        for (auto* b : {&nrec, &nitem, &gnodes, &most}) b->release();
+        for (auto* b : {&gbase, &tbase, &ibase, &totals}) b->release();
     }
 };
 

@@ -2181,7 +2181,8 @@ void tree_lists(Ctx& c) {
     // vortices took 24 GiB, and round 8M the launches of 12020 x 6211 waves
     // were larger than a grid may be.
     // (Room of no use costs, too: 150 us at 4M for nine idle items a group.)
-    auto room = [&](int64_t most, int64_t all, int64_t floor, int64_t small) {
+    constexpr int64_t kRecFloor = 512, kItemFloor = 64, kNodeFloor = 6144;   // of a group
+    auto room = [](int ng, int64_t most, int64_t all, int64_t floor, int64_t small) {
         const int64_t r = std::max(floor, most);
         return r * ng <= std::max(small, 4 * all + floor * ng) ? r : floor;
     };
@@ -2189,40 +2190,37 @@ void tree_lists(Ctx& c) {
     auto follow = [](int64_t& most, int64_t now) {
         if (now > most || 5 * now < 4 * most) most = now;
     };
-    int64_t R, S, recs, items;   // room of a group, and in all
-    auto same_room = [&]() {
-        R = room(b.last_recs, b.last_all_recs, 512, 1 << 22);
-        S = room(b.last_items, b.last_all_items, 64, 1 << 17);
-        S = std::min<int64_t>(S, (1 << 25) / std::max(ng, 1));   // a wave each in one launch
-        recs = R * ng;
-        items = S * ng;
+    // The log takes 0.5 to 0.7 KB a vortex.  Where that is more than an eighth of
+    // the memory free (some 50M vortices, or little memory left), the groups are
+    // walked in parts, once for the counts and once more for the lists.  In one
+    // part the tree of 96M vortices took 264 GiB, so 156; 150M did not fit.
+    auto need = [&]() {
+        return ng * (20 * room(ng, b.last_recs, b.last_all_recs, kRecFloor, 1 << 22) +
+                     1048 * room(ng, b.last_items, b.last_all_items, kItemFloor, 1 << 17) +
+                     20 * std::max(kNodeFloor, b.last_nodes));
     };
-    same_room();
-    bool exact = false;
-    // the items' records: what the criteria in use need, or what was counted
-    int64_t nodes = (int64_t)ng * 6144;
-    for (;;) {
-        VVHD_CHECK(items < (1 << 30), VVHD_ENOMEM, "tree_build: too many parts of the list walk");
-        b.grow(ng, recs, items, nodes);
-        ListLog G{(int)R, (int)S, exact ? b.tbase.p : nullptr, exact ? b.ibase.p : nullptr, (int)items, (int64_t)b.rid.cap,
-                  b.tid.p, b.tfar.p, b.tnear.p, b.nrec.p, b.nitem.p, b.gnodes.p, b.gbase.p, b.item.p, b.item_mask.p,
-                  b.item_n.p, b.item_grp.p, b.lanes.p, b.after.p, b.rid.p, b.rfar.p, b.rnear.p, b.most.p};
-        if (ng)
-            hipLaunchKernelGGL(k_list_top, wave_grid(ng), dim3(kBlock), 0, s, nv, (const TravNode*)tn,
-                               (const int32_t*)t.pre.p, (const int32_t*)t.groups.p, ng, t.leaf_node.p, fc, item_nodes,
-                               G);
-        // (one block scans 65536 counts in about 12 us)
-        if (ng <= 65536)
-            hipLaunchKernelGGL(k_scan_block, dim3(1), dim3(kScanThreads), 0, s, (const int32_t*)b.gnodes.p, b.gbase.p,
-                               (const int32_t*)nullptr, (int64_t*)nullptr, ng);
-        else
-            scan_i32_to_i64(c, b.gnodes.p, b.gbase.p, ng);
-        if (ng) {
-            hipLaunchKernelGGL(exact ? k_list_items<true> : k_list_items<false>, wave_grid(items), dim3(kBlock), 0, s, nv, (const TravNode*)tn,
-                               (const int32_t*)t.groups.p, ng, t.leaf_node.p, fc, G);
-            hipLaunchKernelGGL(k_list_sums, wave_grid(ng), dim3(kBlock), 0, s, (const int32_t*)t.groups.p, ng, G,
-                               t.cnt_near.p, t.cnt_far.p);
-        }
+    auto parts_of = [&]() {
+        const int64_t want = need(), have = b.bytes();
+        if (want <= (1 << 30) || want <= have) return 1;
+        size_t free_b = 0, all_b = 0;
+        VVHD_HIP(hipMemGetInfo(&free_b, &all_b));
+        const int64_t may = std::max<int64_t>(1 << 29, ((int64_t)free_b + have) / 8);
+        return (int)std::min<int64_t>((want + may - 1) / may, ng);
+    };
+    int parts = parts_of();
+    auto first_of = [&](int k) { return (int)((int64_t)t.ngroups * k / parts); };
+    // The walk of the groups of part k: their logs, which a replay reads, and
+    // their leaves' counts; where it is the only part also the lists' offsets and
+    // lengths.  plan: where the counts ask for more parts, only their number.
+    struct Walk {
+        ListLog G;
+        const int32_t* groups;
+        int ng;
+        bool exact;
+        int64_t nnear, nfar;
+        int parts;
+    };
+    auto scan_counts = [&]() {
         if (nl <= 65536) {
             hipLaunchKernelGGL(k_scan_block, dim3(2), dim3(kScanThreads), 0, s, (const int32_t*)t.cnt_near.p,
                                t.near_off.p, (const int32_t*)t.cnt_far.p, t.far_off.p, nl);
@@ -2230,41 +2228,122 @@ void tree_lists(Ctx& c) {
             scan_i32_to_i64(c, t.cnt_near.p, t.near_off.p, nl);
             scan_i32_to_i64(c, t.cnt_far.p, t.far_off.p, nl);
         }
-        // lengths of the near and the far lists, the items' nodes, out of room, then
-        // most and all of the records and of the items
-        int64_t tot[kTotals];
-        hipLaunchKernelGGL(k_list_totals, dim3(1), dim3(std::clamp((ng + 255) / 256 * kWave, kWave, kTotalsThreads)), 0, s, (const int64_t*)t.near_off.p + nl,
-                           (const int64_t*)t.far_off.p + nl, (const int64_t*)b.gbase.p + ng, G, ng, b.totals.p);
-        VVHD_HIP(hipGetLastError());   // no lengths from a launch that was refused
-        VVHD_HIP(hipMemcpyAsync(tot, b.totals.p, sizeof(tot), hipMemcpyDeviceToHost, s));
-        VVHD_HIP(hipStreamSynchronize(s));
-        follow(b.last_recs, tot[4]);
-        follow(b.last_items, tot[5]);
-        b.last_all_recs = tot[6];
-        b.last_all_items = tot[7];
-        nodes = std::max(nodes, tot[2]);
-        if (tot[3]) {
-            same_room();
-            exact = R < tot[4] || S < tot[5];
-            if (exact) {
-                scan_i32_to_i64(c, b.nrec.p, b.tbase.p, ng);
-                scan_i32_to_i64(c, b.nitem.p, b.ibase.p, ng);
-                recs = tot[6];
-                items = tot[7];
+    };
+    auto walk = [&](int k, bool plan) {
+        const int g0 = first_of(k), ng = first_of(k + 1) - g0;
+        const bool all = parts == 1;
+        Walk W{};
+        W.parts = parts;
+        W.groups = (const int32_t*)t.groups.p + 3 * (size_t)g0;
+        W.ng = ng;
+        int64_t R, S, recs, items;   // room of a group, and in all
+        auto same_room = [&]() {
+            R = room(ng, b.last_recs, b.last_all_recs, kRecFloor, 1 << 22);
+            S = room(ng, b.last_items, b.last_all_items, kItemFloor, 1 << 17);
+            S = std::min<int64_t>(S, (1 << 25) / std::max(ng, 1));   // a wave each in one launch
+            recs = R * ng;
+            items = S * ng;
+        };
+        same_room();
+        // the items' records: what the criteria in use need, or what was counted
+        int64_t nodes = ng * kNodeFloor;
+        for (;;) {
+            VVHD_CHECK(items < (1 << 30), VVHD_ENOMEM, "tree_build: too many parts of the list walk");
+            b.grow(ng, recs, items, nodes);
+            W.G = ListLog{(int)R, (int)S, W.exact ? b.tbase.p : nullptr, W.exact ? b.ibase.p : nullptr, (int)items,
+                          (int64_t)b.rid.cap, b.tid.p, b.tfar.p, b.tnear.p, b.nrec.p, b.nitem.p, b.gnodes.p, b.gbase.p,
+                          b.item.p, b.item_mask.p, b.item_n.p, b.item_grp.p, b.lanes.p, b.after.p, b.rid.p, b.rfar.p,
+                          b.rnear.p, b.most.p};
+            if (ng)
+                hipLaunchKernelGGL(k_list_top, wave_grid(ng), dim3(kBlock), 0, s, nv, (const TravNode*)tn,
+                                   (const int32_t*)t.pre.p, W.groups, ng, t.leaf_node.p, fc, item_nodes, W.G);
+            // (one block scans 65536 counts in about 12 us)
+            if (ng <= 65536)
+                hipLaunchKernelGGL(k_scan_block, dim3(1), dim3(kScanThreads), 0, s, (const int32_t*)b.gnodes.p,
+                                   b.gbase.p, (const int32_t*)nullptr, (int64_t*)nullptr, ng);
+            else
+                scan_i32_to_i64(c, b.gnodes.p, b.gbase.p, ng);
+            if (ng) {
+                hipLaunchKernelGGL(W.exact ? k_list_items<true> : k_list_items<false>, wave_grid(items), dim3(kBlock), 0,
+                                   s, nv, (const TravNode*)tn, W.groups, ng, t.leaf_node.p, fc, W.G);
+                hipLaunchKernelGGL(k_list_sums, wave_grid(ng), dim3(kBlock), 0, s, W.groups, ng, W.G, t.cnt_near.p,
+                                   t.cnt_far.p);
             }
-            continue;
+            if (all) scan_counts();
+            // lengths of the near and the far lists (of all groups), the items'
+            // nodes, out of room, then most and all of the records and the items
+            int64_t tot[kTotals];
+            hipLaunchKernelGGL(k_list_totals, dim3(1),
+                               dim3(std::clamp((ng + 255) / 256 * kWave, kWave, kTotalsThreads)), 0, s,
+                               (const int64_t*)t.near_off.p + nl, (const int64_t*)t.far_off.p + nl,
+                               (const int64_t*)b.gbase.p + ng, W.G, ng, b.totals.p);
+            VVHD_HIP(hipGetLastError());   // no lengths from a launch that was refused
+            VVHD_HIP(hipMemcpyAsync(tot, b.totals.p, sizeof(tot), hipMemcpyDeviceToHost, s));
+            VVHD_HIP(hipStreamSynchronize(s));
+            follow(b.last_recs, tot[4]);
+            follow(b.last_items, tot[5]);
+            b.last_all_recs = tot[6];
+            b.last_all_items = tot[7];
+            b.last_nodes = tot[2] / std::max(ng, 1);
+            nodes = std::max(nodes, tot[2]);
+            if (plan && (tot[3] || tot[2] > W.G.cap)) {
+                W.parts = std::max(parts, parts_of());
+                if (W.parts > parts) return W;
+            }
+            if (tot[3]) {
+                same_room();
+                W.exact = R < tot[4] || S < tot[5];
+                if (W.exact) {
+                    scan_i32_to_i64(c, b.nrec.p, b.tbase.p, ng);
+                    scan_i32_to_i64(c, b.nitem.p, b.ibase.p, ng);
+                    recs = tot[6];
+                    items = tot[7];
+                }
+                continue;
+            }
+            if (tot[2] > W.G.cap) continue;
+            W.nnear = tot[0];
+            W.nfar = tot[1];
+            return W;
         }
-        if (tot[2] > G.cap) continue;
-        t.nnear = tot[0];
-        t.nfar = tot[1];
-        t.near_list.grow(t.nnear + 1);
-        t.far_list.grow(t.nfar + 1);
-        if (ng)
-            hipLaunchKernelGGL(exact ? k_list_replay<true> : k_list_replay<false>, wave_grid(items + ng), dim3(kBlock), 0, s, (const int32_t*)t.groups.p,
-                               ng, G, (const int64_t*)t.near_off.p, (const int64_t*)t.far_off.p, t.near_list.p,
-                               t.far_list.p);
-        return;
+    };
+    auto replay = [&](const Walk& W) {
+        if (W.ng)
+            hipLaunchKernelGGL(W.exact ? k_list_replay<true> : k_list_replay<false>, wave_grid((int64_t)W.G.slots + W.ng),
+                               dim3(kBlock), 0, s, W.groups, W.ng, W.G, (const int64_t*)t.near_off.p,
+                               (const int64_t*)t.far_off.p, t.near_list.p, t.far_list.p);
+    };
+    Walk last{};
+    for (int k = 0; k < parts; k++) {
+        last = walk(k, true);
+        if (last.parts == parts) continue;
+        parts = last.parts;   // from the first one, with smaller ones
+        if (b.bytes() / 5 > need() / (4 * parts)) b.release_walk();
+        k = -1;
     }
+    bool again = false;   // the last part, too, in smaller ones
+    if (parts > 1) {
+        scan_counts();
+        int64_t ends[2];
+        VVHD_HIP(hipMemcpyAsync(&ends[0], t.near_off.p + nl, 8, hipMemcpyDeviceToHost, s));
+        VVHD_HIP(hipMemcpyAsync(&ends[1], t.far_off.p + nl, 8, hipMemcpyDeviceToHost, s));
+        VVHD_HIP(hipStreamSynchronize(s));
+        last.nnear = ends[0];
+        last.nfar = ends[1];
+        size_t free_b = 0, all_b = 0;
+        VVHD_HIP(hipMemGetInfo(&free_b, &all_b));
+        again = 4 * (ends[0] + ends[1]) + (1 << 30) > (int64_t)free_b && t.far_list.cap <= (size_t)ends[1];
+        if (again) b.release_walk();   // the lists first
+    }
+    t.nnear = last.nnear;
+    t.nfar = last.nfar;
+    t.near_list.grow(t.nnear + 1);
+    t.far_list.grow(t.nfar + 1);
+    if (again)
+        parts = std::max(parts, parts_of());
+    else
+        replay(last);
+    for (int k = 0; k < parts - !again; k++) replay(walk(k, false));
 }
 
 }  // namespace vvhd
