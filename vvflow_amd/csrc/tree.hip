@@ -1893,6 +1893,7 @@ void for_level_runs(const TreeArrays& t, bool up, const std::function<void(int, 
 
 void tree_build(Ctx& c, int far_criteria, double min_node, double max_node, int32_t* perm_out) {
     TreeArrays& t = c.t;
+    t.built = false;   // until all of it is there: an error on the way leaves no tree
     const int nvort = (int)c.n;
     const int nh = (int)c.heat.n, nst = (int)c.streak.n;
     const int nseg = (int)c.segs_h.size();
@@ -2131,9 +2132,9 @@ void tree_build(Ctx& c, int far_criteria, double min_node, double max_node, int3
     } else {
         VVHD_HIP(hipMemsetAsync(t.seg_off.p, 0, (size_t)(nl + 1) * 8, s));
     }
-    t.built = true;
     tree_lists(c);
     pack_boxes(c);
+    t.built = true;
 }
 
 void pack_boxes(Ctx& c) {
