@@ -1,4 +1,5 @@
-"""Tree builds that end in an error: no call takes what is there for a tree."""
+"""Tree builds that end in an error: the list keeps its records, and no call
+takes what is there for a tree."""
 import numpy as np
 import pytest
 import torch
@@ -40,6 +41,9 @@ def test_a_tree_without_an_end(n, built):
         with pytest.raises(V.VVHDError, match="tree_build"):
             ctx.tree_build(8, -1.0, 0.0)
         refused(ctx)
+        assert np.array_equal(rows(ctx.download()), rows(v))
+        assert np.array_equal(rows(ctx.download_list(HEAT)), rows(h))
+        assert np.array_equal(rows(ctx.download_list(STREAK)), rows(h[:7]))
         ctx.tree_build(8)
         ctx.epsilon(False)
     finally:

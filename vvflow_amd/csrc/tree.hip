@@ -2031,12 +2031,21 @@ void tree_build(Ctx& c, int far_criteria, double min_node, double max_node, int3
         VVHD_HIP(hipMemcpyAsync(hc, t.counters.p, 10 * sizeof(int32_t), hipMemcpyDeviceToHost, s));
         VVHD_HIP(hipMemcpyAsync(hc + 16, t.lev_d.p, (depth + 1) * sizeof(int2), hipMemcpyDeviceToHost, s));
         VVHD_HIP(hipStreamSynchronize(s));
-        VVHD_CHECK(hc[4] != 1, VVHD_ENOMEM, "tree_build: node capacity exceeded");
-        VVHD_CHECK(hc[4] == 0 && depth < kMaxLevels - 1, VVHD_EUNSUPPORTED, "tree_build: tree deeper than supported");
-        if (hc[6] == 0) break;   // the level's nodes are all decided
+        if (hc[4] != 0 || depth >= kMaxLevels - 1) break;   // refused below
+        if (hc[6] == 0) break;                              // the level's nodes are all decided
         hipLaunchKernelGGL(k_level_begin, dim3(1), dim3(64), 0, s, t.counters.p);
         launch_level(depth);
     }
+    // tree order of the remaining fields (also where the build is refused: the
+    // positions have been moved)
+    hipLaunchKernelGGL(k_gather, dim3(nblocks(nvort)), dim3(kBlock), 0, s, c.id.p, nvort, c.g.p, c.vx.p, c.vy.p,
+                       c.ie.p, c.g2.p, c.vx2.p, c.vy2.p, c.ie2.p);
+    swap_buf(c.g, c.g2);
+    swap_buf(c.vx, c.vx2);
+    swap_buf(c.vy, c.vy2);
+    swap_buf(c.ie, c.ie2);
+    VVHD_CHECK(hc[4] != 1, VVHD_ENOMEM, "tree_build: node capacity exceeded");
+    VVHD_CHECK(hc[4] == 0 && depth < kMaxLevels - 1, VVHD_EUNSUPPORTED, "tree_build: tree deeper than supported");
     t.nnodes = hc[0];
     t.nleaves_h = hc[1];
     t.max_depth = hc[5];
@@ -2047,13 +2056,6 @@ void tree_build(Ctx& c, int far_criteria, double min_node, double max_node, int3
     for (int d = 0; d <= depth; d++) levels.push_back({hc[16 + 2 * d], hc[17 + 2 * d]});
     const int nl = t.nleaves_h;
 
-    // tree order of the remaining fields
-    hipLaunchKernelGGL(k_gather, dim3(nblocks(nvort)), dim3(kBlock), 0, s, c.id.p, nvort, c.g.p, c.vx.p, c.vy.p,
-                       c.ie.p, c.g2.p, c.vx2.p, c.vy2.p, c.ie2.p);
-    swap_buf(c.g, c.g2);
-    swap_buf(c.vx, c.vx2);
-    swap_buf(c.vy, c.vy2);
-    swap_buf(c.ie, c.ie2);
     if (perm_out && nvort) VVHD_HIP(hipMemcpyAsync(perm_out, c.id.p, (size_t)nvort * 4, hipMemcpyDeviceToHost, s));
     // the heat and streak lists in their new order
     for (int q = 0; q < 2; q++) {
