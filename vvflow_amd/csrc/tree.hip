@@ -2180,8 +2180,8 @@ void tree_lists(Ctx& c) {
     // MiB: the floors then, which most groups stay under.  Where they do not
     // do, the counts of the first walk over the groups give every group the
     // room that it needs in a second (55 us at 1M, against 400 us for the
-    // items' walk).  With the widest group's room for all, ten strays round 4M
-    // vortices took 24 GiB, and round 8M the launches of 12020 x 6211 waves
+    // items' walk).  With the widest group's room for all, ten strays around 4M
+    // vortices took 24 GiB, and around 8M the launches of 12020 x 6211 waves
     // were larger than a grid may be.
     // (Room of no use costs, too: 150 us at 4M for nine idle items a group.)
     constexpr int64_t kRecFloor = 512, kItemFloor = 64, kNodeFloor = 6144;   // of a group
